@@ -22,7 +22,7 @@ __global__ void k_nodal(DevGrid g, const NodalCell *cells, int ncells,
                         const float *values, int nsrc, int n, const int *dn,
                         int serial) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (dn) n = *dn;  // graph replay: step index lives on the device
+  if (dn) n += *dn;  // graph replay: the step index lives on the device
   const int lo = serial ? 0 : t, hi = serial ? (t == 0 ? ncells : 0) : min(t + 1, ncells);
   for (int c = lo; c < hi; ++c) {
     const NodalCell cell = cells[c];
@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) k_tfsf_list(const PwRun *runs, const long
   cc[f.axis] = f.fixed;
   cc[ua] = f.lo[ua] + (int)(c % r.nu);
   cc[va] = f.lo[va] + (int)(c / r.nu);
-  const int step = r.dn ? *r.dn : n;
+  const int step = r.dn ? *r.dn + n : n;
   const float tm = r.half ? (float)(r.tiempo[step] + (double)0.5f * r.dt) : (float)r.tiempo[step];
   const float ehi = pw_incid(f, r.wave, r.phys, r.pstride, tm, cc);
   const long long p = (long long)(cc[2] + 1) * r.pxy + (long long)(cc[1] + 1) * r.px + r.xoff + cc[0];
@@ -368,15 +368,38 @@ int launch_tick_many(int *const *counters, int n, void *stream) {
   return (int)hipGetLastError();
 }
 
-// Frequency-domain sums of one box at step n (or *dn), observation.F90:
-// 3553-3600: one thread per (point, frequency); the three components of the
-// point are read once per thread and multiplied by the complex(8) phase
-// factor of the step (each part scaled by the real sample).
-__global__ void __launch_bounds__(256) k_dft(DevGrid g, DftDev d, int n, const int *dn) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long npt = (long long)d.cnt[0] * d.cnt[1] * d.cnt[2];
-  if (t >= npt * d.nfreq) return;
-  if (dn) n = *dn;
+// UpdateObservation (observation.F90:2620-2672 point probes, :3553-3600
+// frequency-domain sums) of one grid after a step.  Block 0 samples the
+// probes: one row per call, *count advancing on the device so that a recorded
+// step can be replayed.  The other blocks take one (point, frequency) pair of
+// a frequency-domain box per thread: the three components of the point are
+// read once and multiplied by the complex(8) phase factor of the step (each
+// part scaled by the real sample).  Both only read the fields, and no block
+// reads what another writes.  One launch, not one each: a launch of a few
+// hundred threads costs 4.4 us here whatever it does, half the time of a pass
+// over a 64^3 grid.
+__device__ __forceinline__ void observe_block(const DevGrid &g, const Observe &o, int n, int blk,
+                                              bool probes, bool dft) {
+  if (blk == 0) {
+    if (!probes || o.np <= 0) return;
+    __shared__ int row;
+    if (threadIdx.x == 0) row = *o.count;
+    __syncthreads();
+    if (row < o.cap) {
+      for (int t = threadIdx.x; t < o.np; t += blockDim.x)
+        o.buf[(long long)row * o.np + t] = field_ld(g, o.pr[t].comp, o.pr[t].p);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && row < o.cap) *o.count = row + 1;
+    return;
+  }
+  const long long w = (long long)(blk - 1) * blockDim.x + threadIdx.x;
+  if (!dft || w >= o.total) return;
+  if (o.dn) n += *o.dn;
+  int q = 0;
+  while (q + 1 < o.ndft && o.dft[q + 1].start <= w) ++q;
+  const DftDev &d = o.dft[q];
+  const long long t = w - d.start;
   const long long pt = t / d.nfreq;
   const int f = (int)(t - pt * d.nfreq);
   const int it = (int)(pt % d.cnt[0]);
@@ -388,62 +411,41 @@ __global__ void __launch_bounds__(256) k_dft(DevGrid g, DftDev d, int n, const i
   for (int c = 0; c < 3; ++c) {
     const double v = (double)field_ld(g, 3 * d.kind + c, p);
     double2 *acc = d.acc + (pt * 3 + c) * d.nfreq + f;
-    const double2 o = *acc;
-    *acc = make_double2(o.x + a.x * v, o.y + a.y * v);
+    const double2 o2 = *acc;
+    *acc = make_double2(o2.x + a.x * v, o2.y + a.y * v);
   }
 }
 
-int launch_dft(const DevGrid &g, const DftDev &d, int n, const int *dn, void *stream) {
-  const long long work = (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
-  if (work <= 0) return 0;
-  const unsigned blocks = (unsigned)((work + 255) / 256);
-  hipLaunchKernelGGL(k_dft, dim3(blocks), dim3(256), 0, (hipStream_t)stream, g, d, n, dn);
+__global__ void __launch_bounds__(256) k_observe(DevGrid g, Observe o, int n, int probes, int dft) {
+  observe_block(g, o, n, blockIdx.x, probes != 0, dft != 0);
+}
+
+__global__ void __launch_bounds__(256) k_observe_many(const DevGrid *grids, const ObserveGrid *obs,
+                                                      const int *start, int nobs) {
+  int lo = 0, hi = nobs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (start[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+  }
+  const ObserveGrid &s = obs[lo];
+  observe_block(grids[s.grid], s.o, 0, (int)blockIdx.x - start[lo], true, true);
+}
+
+int observe_blocks(const Observe &o) { return 1 + (int)((o.total + 255) / 256); }
+
+int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, void *stream) {
+  const bool p = probes && o.np > 0, d = dft && o.total > 0;
+  if (!p && !d) return 0;
+  hipLaunchKernelGGL(k_observe, dim3(d ? (unsigned)observe_blocks(o) : 1u), dim3(256), 0,
+                     (hipStream_t)stream, g, o, n, p ? 1 : 0, d ? 1 : 0);
   return (int)hipGetLastError();
 }
 
-// UpdateObservation point probes (observation.F90:2620-2672): one row of
-// samples per call; *count advances on the device so captured graphs can
-// replay it.
-__global__ void k_probes(DevGrid g, const ProbeDev *pr, int np, float *buf,
-                         int *count, int cap) {
-  __shared__ int row;
-  if (threadIdx.x == 0) row = *count;
-  __syncthreads();
-  if (row < cap) {
-    for (int t = threadIdx.x; t < np; t += blockDim.x)
-      buf[(long long)row * np + t] = field_ld(g, pr[t].comp, pr[t].p);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && row < cap) *count = row + 1;
-}
-
-// one block per probe set, as k_probes
-__global__ void k_probes_many(const DevGrid *grids, const ProbeSet *sets) {
-  const ProbeSet &ps = sets[blockIdx.x];
-  const DevGrid &g = grids[ps.grid];
-  __shared__ int row;
-  if (threadIdx.x == 0) row = *ps.count;
-  __syncthreads();
-  if (row < ps.cap) {
-    for (int t = threadIdx.x; t < ps.np; t += blockDim.x)
-      ps.buf[(long long)row * ps.np + t] = field_ld(g, ps.pr[t].comp, ps.pr[t].p);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && row < ps.cap) *ps.count = row + 1;
-}
-
-int launch_probes_many(const DevGrid *grids, const ProbeSet *sets, int nsets, void *stream) {
-  if (nsets <= 0) return 0;
-  hipLaunchKernelGGL(k_probes_many, dim3(nsets), dim3(256), 0, (hipStream_t)stream, grids,
-                     sets);
-  return (int)hipGetLastError();
-}
-
-int launch_probes(const DevGrid &g, const ProbeDev *pr, int np, float *buf,
-                  int *count, int cap, void *stream) {
-  if (np <= 0) return 0;
-  hipLaunchKernelGGL(k_probes, dim3(1), dim3(256), 0, (hipStream_t)stream, g, pr, np,
-                     buf, count, cap);
+int launch_observe_many(const DevGrid *grids, const ObserveGrid *obs, const int *start, int nobs,
+                        int blocks, void *stream) {
+  if (nobs <= 0 || blocks <= 0) return 0;
+  hipLaunchKernelGGL(k_observe_many, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
+                     grids, obs, start, nobs);
   return (int)hipGetLastError();
 }
 
@@ -552,13 +554,18 @@ int launch_mur(const DevGrid &g, const MurRun *runs, int nrun, long long total, 
   return (int)hipGetLastError();
 }
 
-__global__ void k_tick(int *dn) { *dn = *dn + 1; }
+__global__ void k_tick(int *dn, int by) { *dn = *dn + by; }
+__global__ void k_set_step(int *dn, int n) { *dn = n; }
 
-int launch_tick(int *dn, void *stream) {
-  hipLaunchKernelGGL(k_tick, dim3(1), dim3(1), 0, (hipStream_t)stream, dn);
+int launch_tick(int *dn, int by, void *stream) {
+  hipLaunchKernelGGL(k_tick, dim3(1), dim3(1), 0, (hipStream_t)stream, dn, by);
   return (int)hipGetLastError();
 }
 
+int launch_set_step(int *dn, int n, void *stream) {
+  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, (hipStream_t)stream, dn, n);
+  return (int)hipGetLastError();
+}
 
 __global__ void k_fill_i16(int16_t *a, long long n, int16_t v) {
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;

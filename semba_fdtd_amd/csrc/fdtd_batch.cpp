@@ -9,8 +9,7 @@
 //   nodal E                           one launch per grid with E sources
 //   H face pass of all grids          one persistent launch
 //   plane-wave H faces, nodal H       as above
-//   probes                            one launch for all grids
-//   frequency-domain sums             per grid
+//   probes, frequency-domain sums     one launch for all grids
 //   step counters                     one launch for all grids
 // captured once per membership in a HIP graph and replayed.  Each grid keeps
 // its own step counter (its dstep), so grids admitted at different times
@@ -24,8 +23,8 @@
 //                                      shape and media width) over the tiles
 //                                      of every grid's own tile plan
 //   Mur faces                          per grid with Mur faces
-//   probes, step counters              one launch each for all grids
-//   frequency-domain sums              per grid
+//   probes and frequency-domain sums,
+//   step counters                      one launch each for all grids
 // An odd last step runs the two-pass step above.
 #include <hip/hip_runtime.h>
 
@@ -79,8 +78,9 @@ struct fdtd_batch {
   size_t ade_lds[2] = {0, 0};
   int ade_tbl[2] = {1, 1};
   long long ade_nmax[2] = {0, 0};
-  ProbeSet *dprobes = nullptr;
-  int nprobesets = 0;
+  ObserveGrid *dobs = nullptr;
+  int *dobstart = nullptr;
+  int nobs = 0, obs_blocks = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   // one launch per step: rows per block (0: two passes) and planes per chunk
@@ -240,7 +240,8 @@ int build_descriptors(fdtd_batch *b) {
   // pole stage and probes: one launch each for the whole batch
   {
     const bool exact = b->mode == FDTD_MODE_EXACT;
-    std::vector<ProbeSet> sets;
+    std::vector<ObserveGrid> sets;
+    std::vector<int> obstart(1, 0);
     std::vector<int> al[2];
     for (int side = 0; side < 2; ++side) {
       b->ade_lds[side] = 0;
@@ -263,15 +264,12 @@ int build_descriptors(fdtd_batch *b) {
         b->ade_lds[side] = std::max(b->ade_lds[side], la);
         if (h->g.nmedia + 1 > 4096) b->ade_tbl[side] = 0;
       }
-      if (h->nprobe) {
-        ProbeSet ps{};
-        ps.pr = h->dprobes;
-        ps.buf = h->dpbuf;
-        ps.count = h->dpcount;
-        ps.np = h->nprobe;
-        ps.cap = h->pcap;
-        ps.grid = gi;
-        sets.push_back(ps);
+      if (h->nprobe || !h->dfts.empty()) {
+        ObserveGrid og{};
+        og.o = observe_desc(h, h->dstep);
+        og.grid = gi;
+        sets.push_back(og);
+        obstart.push_back(obstart.back() + observe_blocks(og.o));
       }
       ++gi;
     }
@@ -282,9 +280,13 @@ int build_descriptors(fdtd_batch *b) {
       if (!al[side].empty() && (rc = bupload(b, &b->dade[side], al[side].data(), al[side].size())))
         return rc;
     }
-    b->nprobesets = (int)sets.size();
-    b->dprobes = nullptr;
-    if (!sets.empty() && (rc = bupload(b, &b->dprobes, sets.data(), sets.size()))) return rc;
+    b->nobs = (int)sets.size();
+    b->obs_blocks = obstart.back();
+    b->dobs = nullptr;
+    b->dobstart = nullptr;
+    if (!sets.empty() && ((rc = bupload(b, &b->dobs, sets.data(), sets.size())) ||
+                          (rc = bupload(b, &b->dobstart, obstart.data(), obstart.size()))))
+      return rc;
   }
   // plane-wave groups across the batch, in each grid's face order: per half,
   // per wave index, per face axis (the runs read each grid's own counter)
@@ -419,7 +421,7 @@ int build_step_descriptors(fdtd_batch *b) {
 // one step of a pair for every grid, direction d (0: A -> B, 1: B -> A)
 int launch_step_dir(fdtd_batch *b, int d, bool exact_prev) {
   const bool exact = b->mode == FDTD_MODE_EXACT;
-  int e, rc;
+  int e;
   if (b->njobs &&
       launch_pw_incident_many(b->djobs, b->njobs, b->maxnf, b->maxcells, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch incident-field launch failed");
@@ -436,15 +438,8 @@ int launch_step_dir(fdtd_batch *b, int d, bool exact_prev) {
     if (launch_mur(h->sd[d].go, h->dmur, (int)h->mur_runs.size(), h->mur_total, exact, b->stream))
       return bfail(b, FDTD_ERR_HIP, "batch Mur launch failed");
   }
-  if (launch_probes_many(b->dgo[d], b->dprobes, b->nprobesets, b->stream))
-    return bfail(b, FDTD_ERR_HIP, "batch probe launch failed");
-  for (fdtd_handle *h : b->slots) {
-    if (!h) continue;
-    for (const DftDev &df : h->dfts)
-      if (launch_dft(h->sd[d].go, df, 0, h->dstep, b->stream))
-        return bfail(b, FDTD_ERR_HIP, "batch DFT launch failed");
-  }
-  (void)rc;
+  if (launch_observe_many(b->dgo[d], b->dobs, b->dobstart, b->nobs, b->obs_blocks, b->stream))
+    return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
   if (launch_tick_many(b->dcounters, b->ncounters, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
   return FDTD_OK;
@@ -484,10 +479,8 @@ int launch_step(fdtd_batch *b) {
   }
   for (fdtd_handle *h : b->slots)
     if (h && (rc = run_mur(h))) return bfail(b, rc, "grid: %s", h->err.c_str());
-  if (launch_probes_many(b->bd.grids, b->dprobes, b->nprobesets, b->stream))
-    return bfail(b, FDTD_ERR_HIP, "batch probe launch failed");
-  for (fdtd_handle *h : b->slots)
-    if (h && (rc = run_dft(h, 0, h->dstep))) return bfail(b, rc, "grid: %s", h->err.c_str());
+  if (launch_observe_many(b->bd.grids, b->dobs, b->dobstart, b->nobs, b->obs_blocks, b->stream))
+    return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
   if (launch_tick_many(b->dcounters, b->ncounters, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
   return FDTD_OK;

@@ -118,6 +118,7 @@ struct fdtd_handle {
   // frequency-domain observation
   std::vector<sfd_host::DftIn> dftin;
   std::vector<sfd::DftDev> dfts;
+  sfd::DftDev *ddfts = nullptr;       // device copy of dfts
   bool dft_ready = false;
   std::vector<void *> dft_allocs;     // phase tables (rebuilt with the time vector)
   std::vector<void *> dft_sums;       // running sums (kept across rebuilds)
@@ -208,7 +209,11 @@ int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);
 int run_nodal(fdtd_handle *h, int half, int n, const int *dn);
-int run_dft(fdtd_handle *h, int n, const int *dn);
+// UpdateObservation of grid g (h->g or the written copy of a one-launch step)
+// at step n (or *dn + n): point probes and frequency-domain sums
+sfd::Observe observe_desc(const fdtd_handle *h, const int *dn);
+int run_observe(fdtd_handle *h, const sfd::DevGrid &g, int n, const int *dn, bool probes,
+                bool dft);
 int run_mur(fdtd_handle *h);
 int run_ade(fdtd_handle *h, int side);
 void invalidate_graph(fdtd_handle *h);

@@ -823,13 +823,8 @@ static int run_step(fdtd_handle *h, int dir, bool exact_prev = false) {
       launch_mur(sd.go, h->dmur, (int)h->mur_runs.size(), h->mur_total,
                  h->mode == FDTD_MODE_EXACT, h->stream))
     return fail(h, FDTD_ERR_HIP, "Mur launch failed");
-  if (h->nprobe &&
-      launch_probes(sd.go, h->dprobes, h->nprobe, h->dpbuf, h->dpcount, h->pcap, h->stream))
-    return fail(h, FDTD_ERR_HIP, "probe launch failed");
-  for (const DftDev &d : h->dfts)
-    if (launch_dft(sd.go, d, 0, h->dstep, h->stream))
-      return fail(h, FDTD_ERR_HIP, "DFT launch failed");
-  if (launch_tick(h->dstep, h->stream)) return fail(h, FDTD_ERR_HIP, "tick failed");
+  if ((e = run_observe(h, sd.go, 0, h->dstep, true, true))) return e;
+  if (launch_tick(h->dstep, 1, h->stream)) return fail(h, FDTD_ERR_HIP, "tick failed");
   return FDTD_OK;
 }
 
@@ -1143,6 +1138,13 @@ int build_dfts(fdtd_handle *h) {
     if ((rc = upload(h, &da, aux.data(), aux.size(), &h->dft_allocs))) return rc;
     h->dfts[q].aux = da;
   }
+  long long start = 0;
+  for (DftDev &d : h->dfts) {
+    d.start = start;
+    start += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+  }
+  h->ddfts = nullptr;
+  if ((rc = upload(h, &h->ddfts, h->dfts.data(), h->dfts.size(), &h->dft_allocs))) return rc;
   h->dft_ready = true;
   return FDTD_OK;
 }
@@ -1186,16 +1188,23 @@ int run_h(fdtd_handle *h, int yee, int cpml, int ade) {
 
 int run_ade(fdtd_handle *h, int side) { return side ? run_h(h, 0, 0, 1) : run_e(h, 0, 0, 1); }
 
-// UpdateObservation's frequency-domain sums at step n (or *dn)
-int run_dft(fdtd_handle *h, int n, const int *dn) {
-  if (h->dfts.empty()) return FDTD_OK;
-  if (!dn && (n < 0 || n >= (int)h->tiempo.size()))
-    return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
-                (int)h->tiempo.size() - 1);
-  for (const DftDev &d : h->dfts) {
-    int e = launch_dft(h->g, d, n, dn, h->stream);
-    if (e) return fail(h, FDTD_ERR_HIP, "DFT launch failed: %s", hipGetErrorString((hipError_t)e));
-  }
+Observe observe_desc(const fdtd_handle *h, const int *dn) {
+  Observe o{};
+  o.pr = h->dprobes;
+  o.buf = h->dpbuf;
+  o.count = h->dpcount;
+  o.np = h->nprobe;
+  o.cap = h->pcap;
+  o.dft = h->ddfts;
+  o.ndft = (int)h->dfts.size();
+  for (const DftDev &d : h->dfts) o.total += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+  o.dn = dn;
+  return o;
+}
+
+int run_observe(fdtd_handle *h, const DevGrid &g, int n, const int *dn, bool probes, bool dft) {
+  const int e = launch_observe(g, observe_desc(h, dn), n, probes, dft, h->stream);
+  if (e) return fail(h, FDTD_ERR_HIP, "observation launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
 
@@ -1690,11 +1699,14 @@ int fdtd_update_observation(fdtd_handle *h, int32_t n) {
   int rc = prepare(h);
   if (rc) return rc;
   if ((rc = probe_room(h, 1))) return rc;
-  if (h->nprobe && launch_probes(h->g, h->dprobes, h->nprobe, h->dpbuf, h->dpcount, h->pcap,
-                                 h->stream))
-    return fail(h, FDTD_ERR_HIP, "probe launch failed");
+  // a step outside the time vector still samples the probes
+  const bool in = n >= 0 && n < (int)h->tiempo.size();
+  if ((rc = run_observe(h, h->g, n, nullptr, true, in))) return rc;
   h->pbuffered += h->nprobe ? 1 : 0;
-  return run_dft(h, n, nullptr);
+  if (!in && !h->dfts.empty())
+    return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
+                (int)h->tiempo.size() - 1);
+  return FDTD_OK;
 }
 
 int fdtd_set_lines(fdtd_handle *h, const float *line_x, const float *line_y,
@@ -1800,7 +1812,7 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
     return fail(h, FDTD_ERR_ARG, "steps %d..%d beyond the time vector", n0, n0 + nsteps - 1);
   // the step counter lives on the device so one captured step replays for
   // every n
-  HIPCHK(h, hipMemcpyAsync(h->dstep, &n0, 4, hipMemcpyHostToDevice, h->stream));
+  if (launch_set_step(h->dstep, n0, h->stream)) return fail(h, FDTD_ERR_HIP, "step launch failed");
   // one-launch steps go in pairs (A -> B -> A); an odd last step, and every
   // step when they are off, replays the two-pass step
   const bool paired = h->step_rows > 0 && nsteps >= 2;
@@ -1835,25 +1847,22 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
   }
   if (singles == 0) return FDTD_OK;
   if ((rc = build_tile_media(h))) return rc;
-  // one two-pass step, reading the step number from the device counter and
-  // advancing it, recorded nrep times into one graph
+  // nrep two-pass steps in one graph: step r of it reads the step number
+  // *dstep + r, and the counter advances once, at the end
   auto capture = [h](int nrep, hipGraph_t *gout, hipGraphExec_t *xout) -> int {
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int r2 = 0;
     for (int r = 0; r < nrep && !r2; ++r) {
       r2 = run_e(h, 1, 1, 1);
-      if (!r2) r2 = run_pw(h, 0, 0, h->dstep);
-      if (!r2) r2 = run_nodal(h, 0, 0, h->dstep);
+      if (!r2) r2 = run_pw(h, 0, r, h->dstep);
+      if (!r2) r2 = run_nodal(h, 0, r, h->dstep);
       if (!r2) r2 = run_h(h, 1, 1, 1);
-      if (!r2) r2 = run_pw(h, 1, 0, h->dstep);
-      if (!r2) r2 = run_nodal(h, 1, 0, h->dstep);
+      if (!r2) r2 = run_pw(h, 1, r, h->dstep);
+      if (!r2) r2 = run_nodal(h, 1, r, h->dstep);
       if (!r2) r2 = run_mur(h);
-      if (!r2 && h->nprobe)
-        r2 = launch_probes(h->g, h->dprobes, h->nprobe, h->dpbuf, h->dpcount, h->pcap, h->stream)
-                 ? fail(h, FDTD_ERR_HIP, "probe launch failed") : 0;
-      if (!r2) r2 = run_dft(h, 0, h->dstep);
-      if (!r2) r2 = launch_tick(h->dstep, h->stream) ? fail(h, FDTD_ERR_HIP, "tick failed") : 0;
+      if (!r2) r2 = run_observe(h, h->g, r, h->dstep, true, true);
     }
+    if (!r2) r2 = launch_tick(h->dstep, nrep, h->stream) ? fail(h, FDTD_ERR_HIP, "tick failed") : 0;
     hipGraph_t graph = nullptr;
     hipError_t ec = hipStreamEndCapture(h->stream, &graph);
     if (r2) { if (graph) hipGraphDestroy(graph); return r2; }
@@ -2070,8 +2079,7 @@ int fdtd_sample_probes(fdtd_handle *h) {
   if (int rc = refuse_batched(h)) return rc;
   if (int rc = probe_room(h, 1)) return rc;
   hipSetDevice(h->device);
-  if (launch_probes(h->g, h->dprobes, h->nprobe, h->dpbuf, h->dpcount, h->pcap, h->stream))
-    return fail(h, FDTD_ERR_HIP, "probe launch failed");
+  if (int rc = run_observe(h, h->g, 0, nullptr, true, false)) return rc;
   h->pbuffered += 1;
   return FDTD_OK;
 }

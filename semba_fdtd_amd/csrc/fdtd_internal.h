@@ -172,6 +172,8 @@ struct DftDev {
   int kind;                   // 0: Ex,Ey,Ez  1: Hx,Hy,Hz
   int first[3], stride[3], cnt[3];
   int nfreq;
+  long long start;            // first (point, frequency) pair of the box in the
+                              // observation launch of its grid
   const double2 *aux;         // [step][freq]
   double2 *acc;               // [pt][3][freq], pt = (kt*cnt1 + jt)*cnt0 + it
 };
@@ -179,6 +181,19 @@ struct DftDev {
 struct ProbeDev {
   long long p;
   int comp;
+};
+
+// The observation of one grid after a step: its point probes and the
+// frequency-domain boxes, one launch (launch_observe)
+struct Observe {
+  const ProbeDev *pr;         // point probes, their buffer and sample count
+  float *buf;
+  int *count;
+  int np, cap;
+  const DftDev *dft;          // frequency-domain boxes (device), in the order
+  int ndft;                   // of their start
+  long long total;            // (point, frequency) pairs of all boxes
+  const int *dn;              // device step counter (null: the launch's n)
 };
 
 // TF/SF faces per half that a one-launch step handles (one bit each in the
@@ -393,8 +408,24 @@ SFD_DECLARE_LAUNCHERS(exact)
 int launch_nodal(const DevGrid &g, const NodalCell *cells, int ncells,
                  const float *values, int nsrc, int n, const int *dn, int serial,
                  void *stream);
-int launch_tick(int *dn, void *stream);
-int launch_dft(const DevGrid &g, const DftDev &d, int n, const int *dn, void *stream);
+// A step number is *dn + n where a device step counter dn is given (n: the
+// step's place in the recorded sequence, the counter moving once at its end),
+// else n.
+// *dn += by / *dn = n
+int launch_tick(int *dn, int by, void *stream);
+int launch_set_step(int *dn, int n, void *stream);
+// the observation of a grid at step n: probes sampled (when probes), then
+// frequency-domain sums advanced (when dft)
+int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, void *stream);
+// the same for many grids: blocks start[s] .. start[s+1]-1 of the launch
+// serve obs[s] on grids[grid[s]]
+struct ObserveGrid {
+  Observe o;
+  int grid;
+};
+int launch_observe_many(const DevGrid *grids, const ObserveGrid *obs, const int *start, int nobs,
+                        int blocks, void *stream);
+int observe_blocks(const Observe &o);
 // a group of TF/SF faces at step n (or each run's *dn): F += sign * G *
 // Incid(t) * id, t the real(4) time stamp of the half step (E: tiempo(n), H:
 // tiempo(n) + dt/2); runs[r] covers cells start[r] .. start[r+1]-1 of total
@@ -433,16 +464,6 @@ int launch_pw_incident_many(const PwIncJob *jobs, int njobs, int maxnf, long lon
                             void *stream);
 // increments every counter of the list (per-grid step counters of a batch)
 int launch_tick_many(int *const *counters, int n, void *stream);
-int launch_probes(const DevGrid &g, const ProbeDev *pr, int np, float *buf,
-                  int *count, int cap, void *stream);
-// the probes of several grids of a batch in one launch
-struct ProbeSet {
-  const ProbeDev *pr;
-  float *buf;
-  int *count;
-  int np, cap, grid;          // grid: index into the batch's descriptors
-};
-int launch_probes_many(const DevGrid *grids, const ProbeSet *sets, int nsets, void *stream);
 // bounding box {xmin,ymin,zmin,xmax,ymax,zmax} of the dispersive edges of
 // component comp; out must hold {INT_MAX x3, INT_MIN x3} on entry
 int launch_disp_bbox(const DevGrid &g, int side, int c, int32_t *out, void *stream);
