@@ -368,18 +368,80 @@ int launch_tick_many(int *const *counters, int n, void *stream) {
   return (int)hipGetLastError();
 }
 
+// The TF/SF term +-G * Incid * id (AdvancePlaneWaveE/H, planewaves.F90:878-1475)
+// of cell w of the faces' cells at step n: what pw_apply adds to the field,
+// with the same roundings.
+__device__ __forceinline__ void pw_term_cell(const PwTerms &t, long long w, int n) {
+#pragma clang fp contract(off)
+  int lo = 0, hi = t.nf - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (t.start[mid] <= w) lo = mid; else hi = mid - 1;
+  }
+  const PwFace &f = t.faces[lo];
+  const int half = lo >= t.nf0 ? 1 : 0;
+  const int ua = f.axis == 0 ? 1 : 0, va = f.axis == 2 ? 1 : 2;
+  const int c = (int)(w - t.start[lo]), nu = f.hi[ua] - f.lo[ua] + 1;
+  int cc[3];
+  cc[f.axis] = f.fixed;
+  cc[ua] = f.lo[ua] + c % nu;
+  cc[va] = f.lo[va] + c / nu;
+  const float tm = half ? (float)(t.tiempo[n] + (double)0.5f * t.dt) : (float)t.tiempo[n];
+  const float x = t.G[half] * pw_incid(f, t.waves, t.phys, t.pstride, tm, cc) * f.id;
+  t.out[w] = f.sign > 0.0f ? x : -x;
+}
+
+__global__ void __launch_bounds__(256) k_pw_terms(PwTerms t, int n, const int *dn) {
+  const long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (dn) n += *dn;
+  if (w < t.total && n >= 0 && n < t.ntime) pw_term_cell(t, w, n);
+}
+
+// the terms of several grids, each at its own step: blockIdx.y picks the grid
+__global__ void __launch_bounds__(256) k_pw_terms_many(const PwTermsGrid *grids) {
+  const PwTermsGrid &g = grids[blockIdx.y];
+  const int n = *g.dn;
+  if (n < 0 || n >= g.t.ntime) return;
+  for (long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x; w < g.t.total;
+       w += (long long)gridDim.x * blockDim.x)
+    pw_term_cell(g.t, w, n);
+}
+
+int launch_pw_terms(const PwTerms &t, int n, const int *dn, void *stream) {
+  if (t.total <= 0) return 0;
+  hipLaunchKernelGGL(k_pw_terms, dim3((unsigned)((t.total + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, t, n, dn);
+  return (int)hipGetLastError();
+}
+
+int launch_pw_terms_many(const PwTermsGrid *grids, int n, long long maxcells, void *stream) {
+  if (n <= 0 || maxcells <= 0) return 0;
+  const long long b = std::min<long long>((maxcells + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_pw_terms_many, dim3((unsigned)b, (unsigned)n), dim3(256), 0,
+                     (hipStream_t)stream, grids);
+  return (int)hipGetLastError();
+}
+
 // UpdateObservation (observation.F90:2620-2672 point probes, :3553-3600
 // frequency-domain sums) of one grid after a step.  Block 0 samples the
 // probes: one row per call, *count advancing on the device so that a recorded
 // step can be replayed.  The other blocks take one (point, frequency) pair of
 // a frequency-domain box per thread: the three components of the point are
 // read once and multiplied by the complex(8) phase factor of the step (each
-// part scaled by the real sample).  Both only read the fields, and no block
-// reads what another writes.  One launch, not one each: a launch of a few
+// part scaled by the real sample).  The last blocks write the TF/SF terms of
+// the next step, one cell per thread, for the passes that apply them inline.
+// All only read the fields, and no block reads what another writes.  One launch, not one each: a launch of a few
 // hundred threads costs 4.4 us here whatever it does, half the time of a pass
 // over a 64^3 grid.
 __device__ __forceinline__ void observe_block(const DevGrid &g, const Observe &o, int n, int blk,
-                                              bool probes, bool dft) {
+                                              bool probes, bool dft, bool pw) {
+  const int bd = 1 + (int)((o.total + 255) / 256);
+  if (blk >= bd) {
+    const long long w = (long long)(blk - bd) * blockDim.x + threadIdx.x;
+    n += 1 + (o.dn ? *o.dn : 0);
+    if (pw && w < o.pw.total && n < o.pw.ntime) pw_term_cell(o.pw, w, n);
+    return;
+  }
   if (blk == 0) {
     if (!probes || o.np <= 0) return;
     __shared__ int row;
@@ -416,8 +478,9 @@ __device__ __forceinline__ void observe_block(const DevGrid &g, const Observe &o
   }
 }
 
-__global__ void __launch_bounds__(256) k_observe(DevGrid g, Observe o, int n, int probes, int dft) {
-  observe_block(g, o, n, blockIdx.x, probes != 0, dft != 0);
+__global__ void __launch_bounds__(256) k_observe(DevGrid g, Observe o, int n, int probes, int dft,
+                                                 int pw) {
+  observe_block(g, o, n, blockIdx.x, probes != 0, dft != 0, pw != 0);
 }
 
 __global__ void __launch_bounds__(256) k_observe_many(const DevGrid *grids, const ObserveGrid *obs,
@@ -428,16 +491,21 @@ __global__ void __launch_bounds__(256) k_observe_many(const DevGrid *grids, cons
     if (start[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
   }
   const ObserveGrid &s = obs[lo];
-  observe_block(grids[s.grid], s.o, 0, (int)blockIdx.x - start[lo], true, true);
+  observe_block(grids[s.grid], s.o, 0, (int)blockIdx.x - start[lo], true, true, true);
 }
 
-int observe_blocks(const Observe &o) { return 1 + (int)((o.total + 255) / 256); }
+int observe_blocks(const Observe &o) {
+  return 1 + (int)((o.total + 255) / 256) + (int)((o.pw.total + 255) / 256);
+}
 
-int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, void *stream) {
-  const bool p = probes && o.np > 0, d = dft && o.total > 0;
-  if (!p && !d) return 0;
-  hipLaunchKernelGGL(k_observe, dim3(d ? (unsigned)observe_blocks(o) : 1u), dim3(256), 0,
-                     (hipStream_t)stream, g, o, n, p ? 1 : 0, d ? 1 : 0);
+int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, int pw,
+                   void *stream) {
+  const bool p = probes && o.np > 0, d = dft && o.total > 0, w = pw && o.pw.total > 0;
+  if (!p && !d && !w) return 0;
+  const unsigned blocks = w ? (unsigned)observe_blocks(o)
+                            : d ? 1u + (unsigned)((o.total + 255) / 256) : 1u;
+  hipLaunchKernelGGL(k_observe, dim3(blocks), dim3(256), 0, (hipStream_t)stream, g, o, n,
+                     p ? 1 : 0, d ? 1 : 0, w ? 1 : 0);
   return (int)hipGetLastError();
 }
 

@@ -5,11 +5,14 @@
 // copying.  One step of the batch runs, for every grid at its own step:
 //   E face pass of all grids          one persistent launch (k_pass_batch)
 //   pole stage                        one launch for the grids with poles
-//   plane-wave E faces                one launch per (wave, face axis) group
-//   nodal E                           one launch per grid with E sources
+//   plane-wave E faces                inside the pass, or one launch per (wave,
+//                                     face axis) group of the grids that cannot
+//   nodal E                           inside the pass, or one launch per grid
+//                                     that cannot
 //   H face pass of all grids          one persistent launch
 //   plane-wave H faces, nodal H       as above
-//   probes, frequency-domain sums     one launch for all grids
+//   probes, frequency-domain sums,
+//   the next step's TF/SF terms       one launch for all grids
 //   step counters                     one launch for all grids
 // captured once per membership in a HIP graph and replayed.  Each grid keeps
 // its own step counter (its dstep), so grids admitted at different times
@@ -81,6 +84,12 @@ struct fdtd_batch {
   ObserveGrid *dobs = nullptr;
   int *dobstart = nullptr;
   int nobs = 0, obs_blocks = 0;
+  // per slot and half: the sources the grid's passes apply inline, and the
+  // grids whose TF/SF terms a call refreshes before its first step
+  std::vector<char> inl[2];
+  PwTermsGrid *dterms = nullptr;
+  int nterms = 0;
+  long long maxterms = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   // one launch per step: rows per block (0: two passes) and planes per chunk
@@ -237,6 +246,49 @@ int build_descriptors(fdtd_batch *b) {
   }
   b->ncounters = (int)counters.size();
   b->lds = lds;
+  // the sources the one-cell passes apply inline
+  {
+    std::vector<PwTermsGrid> terms;
+    std::vector<PassSrc> src[2];
+    b->maxterms = 0;
+    for (int half = 0; half < 2; ++half) {
+      b->inl[half].assign(b->slots.size(), 0);
+      b->bd.src[half] = nullptr;
+    }
+    int gi = 0;
+    for (size_t s = 0; s < b->slots.size() && b->xcells == 1; ++s) {
+      fdtd_handle *h = b->slots[s];
+      if (!h) continue;
+      bool faces = false;
+      for (int half = 0; half < 2; ++half) {
+        PassSrc ps;
+        bool on = false;
+        if ((rc = make_pass_src(h, tms[(size_t)gi], half, &ps, &on, &b->allocs, nullptr)))
+          return bfail(b, rc, "slot %zu: %s", s, h->err.c_str());
+        ps.dn = h->dstep;
+        b->inl[half][s] = on ? 1 : 0;
+        faces = faces || (on && ps.nface);
+        src[half].push_back(on ? ps : PassSrc{});
+      }
+      if (faces) {
+        terms.push_back(PwTermsGrid{h->pw_terms, h->dstep});
+        b->maxterms = std::max(b->maxterms, h->pw_terms.total);
+      }
+      ++gi;
+    }
+    for (int half = 0; half < 2; ++half) {
+      bool any = false;
+      for (char on : b->inl[half]) any = any || on;
+      PassSrc *d = nullptr;
+      if (any && (rc = bupload(b, &d, src[half].data(), src[half].size()))) return rc;
+      b->bd.src[half] = d;
+    }
+    b->nterms = (int)terms.size();
+    b->dterms = nullptr;
+    if (!terms.empty() && (rc = bupload(b, &b->dterms, terms.data(), terms.size()))) return rc;
+    // (the uploads read these vectors until the stream has run them)
+    BCHK(b, hipStreamSynchronize(b->stream));
+  }
   // pole stage and probes: one launch each for the whole batch
   {
     const bool exact = b->mode == FDTD_MODE_EXACT;
@@ -264,9 +316,11 @@ int build_descriptors(fdtd_batch *b) {
         b->ade_lds[side] = std::max(b->ade_lds[side], la);
         if (h->g.nmedia + 1 > 4096) b->ade_tbl[side] = 0;
       }
-      if (h->nprobe || !h->dfts.empty()) {
+      const bool terms = (b->inl[0][s] || b->inl[1][s]) && h->pw_terms.total > 0;
+      if (h->nprobe || !h->dfts.empty() || terms) {
         ObserveGrid og{};
         og.o = observe_desc(h, h->dstep);
+        if (!terms) og.o.pw = PwTerms{};
         og.grid = gi;
         sets.push_back(og);
         obstart.push_back(obstart.back() + observe_blocks(og.o));
@@ -296,8 +350,9 @@ int build_descriptors(fdtd_batch *b) {
         BatchPwGroup grp;
         grp.half = half;
         grp.start.push_back(0);
-        for (fdtd_handle *h : b->slots) {
-          if (!h) continue;
+        for (size_t s = 0; s < b->slots.size(); ++s) {
+          fdtd_handle *h = b->slots[s];
+          if (!h || b->inl[half][s]) continue;
           for (const PwGroup &g : h->pw_groups) {
             if (g.half != half || g.runs.empty() || g.runs[0].f.wave != w ||
                 g.runs[0].f.axis != axis)
@@ -473,9 +528,11 @@ int launch_step(fdtd_batch *b) {
       e = launch_tfsf_list(g.druns, g.dstart, (int)g.runs.size(), g.start.back(), 0, b->stream);
       if (e) return bfail(b, FDTD_ERR_HIP, "batch plane-wave launch failed");
     }
-    for (fdtd_handle *h : b->slots)
-      if (h && (rc = run_nodal(h, half, 0, h->dstep)))
+    for (size_t s = 0; s < b->slots.size(); ++s) {
+      fdtd_handle *h = b->slots[s];
+      if (h && !b->inl[half][s] && (rc = run_nodal(h, half, 0, h->dstep)))
         return bfail(b, rc, "grid: %s", h->err.c_str());
+    }
   }
   for (fdtd_handle *h : b->slots)
     if (h && (rc = run_mur(h))) return bfail(b, rc, "grid: %s", h->err.c_str());
@@ -570,6 +627,7 @@ int fdtd_batch_admit(fdtd_batch *b, fdtd_handle *h, int32_t n0, int32_t *slot) {
   }
   b->slots[s] = h;
   h->batch = b;
+  h->pw_terms_n = -1;   // the batch's steps refill the grid's TF/SF terms
   b->step[s] = n0;
   b->ready = false;
   *slot = s;
@@ -685,6 +743,10 @@ int fdtd_batch_step(fdtd_batch *b, int32_t nsteps) {
     }
     for (int q = p0; q < pairs; ++q) BCHK(b, hipGraphLaunch(b->pexec, b->stream));
   }
+  // the first two-pass step's TF/SF terms; each step's observation leaves the
+  // next one's
+  if (singles > 0 && launch_pw_terms_many(b->dterms, b->nterms, b->maxterms, b->stream))
+    return bfail(b, FDTD_ERR_HIP, "batch incident-field launch failed");
   if (singles > 0 && !b->gexec) {
     BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     int r2 = launch_step(b);

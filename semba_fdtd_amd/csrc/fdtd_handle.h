@@ -115,6 +115,19 @@ struct fdtd_handle {
   float *dphys = nullptr;
   int pstride = 0;
   double *dtiempo = nullptr;
+  // the faces of each half as the face passes apply them inline (pw_masks:
+  // at most kPassFaces, all inside their components' sweeps), and the buffer
+  // of both halves' terms, which holds those of step pw_terms_n (-1: none)
+  bool pw_masks[2] = {false, false};
+  sfd::PassSrc pw_src[2] = {};
+  std::vector<unsigned> pw_bits[2][3];  // host copy of the faces' index masks
+  sfd::PwTerms pw_terms{};
+  int pw_terms_n = -1;
+  // per half, under the pass tiling tm: the sources the one-cell pass applies
+  // (valid while tmed_ready)
+  bool psrc_on[2] = {false, false};
+  sfd::PassSrc psrc[2] = {};
+  std::vector<void *> psrc_allocs;
   // frequency-domain observation
   std::vector<sfd_host::DftIn> dftin;
   std::vector<sfd::DftDev> dfts;
@@ -209,11 +222,17 @@ int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);
 int run_nodal(fdtd_handle *h, int half, int n, const int *dn);
+// the sources of a half as a one-cell pass over tile map tm applies them:
+// *on tells whether it can (else run_pw and run_nodal follow the pass); flags
+// (null: not wanted): per block of tm, what its tile meets is added
+int make_pass_src(fdtd_handle *h, const sfd::TileMap &tm, int half, sfd::PassSrc *out, bool *on,
+                  std::vector<void *> *list, std::vector<int> *flags);
 // UpdateObservation of grid g (h->g or the written copy of a one-launch step)
 // at step n (or *dn + n): point probes and frequency-domain sums
 sfd::Observe observe_desc(const fdtd_handle *h, const int *dn);
+// (pw: and the TF/SF terms of the next step)
 int run_observe(fdtd_handle *h, const sfd::DevGrid &g, int n, const int *dn, bool probes,
-                bool dft);
+                bool dft, bool pw);
 int run_mur(fdtd_handle *h);
 int run_ade(fdtd_handle *h, int side);
 void invalidate_graph(fdtd_handle *h);

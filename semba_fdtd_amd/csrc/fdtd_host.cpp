@@ -50,6 +50,32 @@ int dzero(fdtd_handle *h, void *p, size_t bytes) {
   return FDTD_OK;
 }
 
+// Many small tables in one device allocation and one copy: add() reserves,
+// alloc() allocates, at() gives the device address, put() fills the host
+// image, send() copies it.  (An upload of its own costs an allocation, a copy
+// and a wait, some 30 us each.)
+struct Pack {
+  std::vector<char> img;
+  char *dev = nullptr;
+  size_t add(size_t bytes) {
+    const size_t off = img.size();
+    img.resize(off + ((bytes + 63) & ~(size_t)63));
+    return off;
+  }
+  int alloc(fdtd_handle *h, std::vector<void *> *list) {
+    return dalloc(h, (void **)&dev, std::max<size_t>(img.size(), 64), list);
+  }
+  template <class T> T *at(size_t off) const { return reinterpret_cast<T *>(dev + off); }
+  template <class T> void put(size_t off, const std::vector<T> &v) {
+    if (!v.empty()) std::memcpy(&img[off], v.data(), v.size() * sizeof(T));
+  }
+  int send(fdtd_handle *h) {
+    HIPCHK(h, hipMemcpyAsync(dev, img.data(), img.size(), hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return FDTD_OK;
+  }
+};
+
 template <class T>
 int upload(fdtd_handle *h, T **dst, const T *src, size_t n,
            std::vector<void *> *list = nullptr) {
@@ -206,8 +232,9 @@ void invalidate_graph(fdtd_handle *h) {
 }
 
 // the medium of each tile of the one-cell pass map (or -1): the passes then
-// skip the media loads of single-medium tiles.  Built outside any capture,
-// before the passes it serves are launched or recorded.
+// skip the media loads of single-medium tiles; and the sources the passes
+// apply inline.  Built outside any capture, before the passes it serves are
+// launched or recorded.
 int build_tile_media(fdtd_handle *h) {
   if (h->tmed_ready) return FDTD_OK;
   if (h->tm.nblk > h->tmed_cap) {
@@ -217,6 +244,16 @@ int build_tile_media(fdtd_handle *h) {
     HIPCHK(h, hipMalloc(&h->tmed, (size_t)h->tm.nblk * sizeof(int)));
     h->tmed_cap = h->tm.nblk;
   }
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  for (void *p : h->psrc_allocs) hipFree(p);
+  h->psrc_allocs.clear();
+  std::vector<int> flags((size_t)h->tm.nblk, 0);
+  for (int half = 0; half < 2; ++half)
+    if (int rc = make_pass_src(h, h->tm, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, &flags))
+      return rc;
+  HIPCHK(h, hipMemcpyAsync(h->tmed, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
+                           h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
   const int e = h->mode == FDTD_MODE_EXACT ? exact::launch_pass_tile_media(h->g, h->tm, h->tmed, h->stream)
                                            : fast::launch_pass_tile_media(h->g, h->tm, h->tmed, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
@@ -823,7 +860,7 @@ static int run_step(fdtd_handle *h, int dir, bool exact_prev = false) {
       launch_mur(sd.go, h->dmur, (int)h->mur_runs.size(), h->mur_total,
                  h->mode == FDTD_MODE_EXACT, h->stream))
     return fail(h, FDTD_ERR_HIP, "Mur launch failed");
-  if ((e = run_observe(h, sd.go, 0, h->dstep, true, true))) return e;
+  if ((e = run_observe(h, sd.go, 0, h->dstep, true, true, false))) return e;
   if (launch_tick(h->dstep, 1, h->stream)) return fail(h, FDTD_ERR_HIP, "tick failed");
   return FDTD_OK;
 }
@@ -923,6 +960,220 @@ int sweep_last(const fdtd_handle *h, int c, int a) {
 int sin_lo(const fdtd_handle *h, int, int a) { return h->g.L[a][0]; }
 int sin_hi(const fdtd_handle *h, int c, int a) { return sweep_last(h, c, a) - h->g.L[a][1]; }
 
+// The faces of both halves for the passes that apply them inline: per half
+// and axis, bit q of entry i says that face q's range holds index i.
+struct PwMasks {
+  std::vector<PwFace> all;           // E faces, then H faces
+  std::vector<long long> start;      // prefix of their cells
+  std::vector<unsigned> m[2][3];
+  std::vector<FaceAddr> fa[2];
+  size_t om[2][3], ofa[2], oall, ostart;   // places in the pack
+};
+static void build_pw_masks(fdtd_handle *h, PwMasks &w, Pack &pk) {
+  const int n3[3] = {h->g.nx, h->g.ny, h->g.nz};
+  w.start.assign(1, 0);
+  for (int half = 0; half < 2; ++half) {
+    const std::vector<PwFace> &F = h->pw_faces[half];
+    PassSrc &s = h->pw_src[half];
+    s = PassSrc{};
+    bool ok = !F.empty() && (int)F.size() <= kPassFaces;
+    for (int a = 0; a < 3; ++a) w.m[half][a].assign((size_t)n3[a] + 1, 0u);
+    for (size_t q = 0; q < F.size(); ++q) {
+      const PwFace &f = F[q];
+      int lo[3], hi[3];
+      for (int a = 0; a < 3; ++a) { lo[a] = f.lo[a]; hi[a] = f.hi[a]; }
+      lo[f.axis] = hi[f.axis] = f.fixed;
+      const int ua = f.axis == 0 ? 1 : 0, va = f.axis == 2 ? 1 : 2;
+      const long long nu = hi[ua] - lo[ua] + 1, nv = hi[va] - lo[va] + 1;
+      const long long cells = nu > 0 && nv > 0 ? nu * nv : 0;
+      FaceAddr A{};
+      if (cells) {
+        // the passes run the components' sweeps: a face outside (a box on
+        // the grid's edge) keeps its own launch
+        for (int a = 0; a < 3; ++a) ok = ok && lo[a] >= 0 && hi[a] <= sweep_last(h, f.comp, a);
+        ok = ok && w.start.back() + cells < 0x40000000LL;
+        if (ok) {
+          for (int a = 0; a < 3; ++a)
+            for (int i = lo[a]; i <= hi[a]; ++i) w.m[half][a][(size_t)i] |= 1u << q;
+          int st[3] = {0, 0, 0};
+          st[ua] = 1;
+          st[va] = (int)nu;
+          A = FaceAddr{(int)(w.start.back() - lo[va] * nu - lo[ua]), st[0], st[1], st[2]};
+          s.cm[f.comp % 3] |= 1u << q;
+        }
+      }
+      w.fa[half].push_back(A);
+      w.all.push_back(f);
+      w.start.push_back(w.start.back() + cells);
+    }
+    h->pw_masks[half] = ok;
+    for (int a = 0; a < 3; ++a) w.om[half][a] = pk.add(w.m[half][a].size() * sizeof(unsigned));
+    w.ofa[half] = pk.add(w.fa[half].size() * sizeof(FaceAddr));
+  }
+  w.oall = pk.add(w.all.size() * sizeof(PwFace));
+  w.ostart = pk.add(w.start.size() * sizeof(long long));
+}
+
+// the device side of the masks, once the pack has its addresses
+static int place_pw_masks(fdtd_handle *h, const PwMasks &w, Pack &pk) {
+  PwTerms &t = h->pw_terms;
+  t = PwTerms{};
+  h->pw_terms_n = -1;
+  pk.put(w.oall, w.all);
+  pk.put(w.ostart, w.start);
+  float *terms = nullptr;
+  if (h->pw_masks[0] || h->pw_masks[1]) {
+    if (int rc = dalloc(h, (void **)&terms, (size_t)std::max(w.start.back(), 1LL) * 4, &h->pw_allocs))
+      return rc;
+    t.faces = pk.at<PwFace>(w.oall);
+    t.start = pk.at<long long>(w.ostart);
+    t.nf0 = (int)h->pw_faces[0].size();
+    t.nf = (int)w.all.size();
+    t.total = w.start.back();
+    t.waves = h->dwaves;
+    t.phys = h->dphys;
+    t.pstride = h->pstride;
+    t.tiempo = h->dtiempo;
+    t.ntime = (int)h->tiempo.size();
+    t.dt = h->dt;
+    t.G[0] = h->g2h[1];
+    t.G[1] = h->gm2h[1];
+    t.out = terms;
+  }
+  for (int half = 0; half < 2; ++half) {
+    PassSrc &s = h->pw_src[half];
+    for (int a = 0; a < 3; ++a) {
+      pk.put(w.om[half][a], w.m[half][a]);
+      h->pw_bits[half][a] = w.m[half][a];
+    }
+    pk.put(w.ofa[half], w.fa[half]);
+    if (!h->pw_masks[half]) { s = PassSrc{}; continue; }
+    s.nface = (int)h->pw_faces[half].size();
+    s.mx = pk.at<unsigned>(w.om[half][0]);
+    s.my = pk.at<unsigned>(w.om[half][1]);
+    s.mz = pk.at<unsigned>(w.om[half][2]);
+    s.fa = pk.at<FaceAddr>(w.ofa[half]);
+    s.terms = terms;
+  }
+  return FDTD_OK;
+}
+
+// A pass applies the sources before the pole stage that follows it, so they
+// move into the pass only where no source cell lies in a pole-state box (the
+// two then act on different cells, in any order), every nodal cell lies in
+// the passes' domain, and the faces fit the masks.  Grids up to kInlineCells:
+// a pass with sources carries more state (63 registers and 35 scalar spills
+// against 51 and 13) and runs 12 % longer at 256^3, the separate launches cost
+// 4.6-9 us each whatever the grid.  A plane wave on 48^3, 100^3, 160^3, 200^3
+// runs 1.64, 1.48, 1.14, 1.02 times as fast inline, on 320^3 0.98 times; a
+// point source on 64^3, 128^3, 200^3 1.16, 1.03, 1.04 times, on 320^3 0.99.
+constexpr long long kInlineCells = 12000000;
+int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, bool *on,
+                  std::vector<void *> *list, std::vector<int> *flags) {
+  *on = false;
+  *out = PassSrc{};
+  const std::vector<PwFace> &F = h->pw_faces[half];
+  const std::vector<NodalCell> &C = h->hcells[half];
+  if (F.empty() && C.empty()) return FDTD_OK;
+  if ((long long)h->g.nx * h->g.ny * h->g.nz > kInlineCells) return FDTD_OK;
+  if (!F.empty() && !h->pw_masks[half]) return FDTD_OK;
+  const AdeSet &A = h->g.ade[half];
+  auto in_poles = [&](int comp, const int lo[3], const int hi[3]) {
+    if (!A.has) return false;
+    const int *b = A.abox[comp % 3];
+    for (int a = 0; a < 3; ++a)
+      if (b[3 + a] <= 0 || hi[a] < b[a] || lo[a] >= b[a] + b[3 + a]) return false;
+    return true;
+  };
+  for (const PwFace &f : F) {
+    int lo[3], hi[3];
+    for (int a = 0; a < 3; ++a) { lo[a] = f.lo[a]; hi[a] = f.hi[a]; }
+    lo[f.axis] = hi[f.axis] = f.fixed;
+    if (in_poles(f.comp, lo, hi)) return FDTD_OK;
+  }
+  const DevGrid &g = h->g;
+  std::vector<int> tile(C.size()), nstart;
+  std::vector<NodalCell> cells(C.size());
+  if (!C.empty()) {
+    nstart.assign((size_t)tm.nblk + 1, 0);
+    for (size_t q = 0; q < C.size(); ++q) {
+      const long long k = C[q].p / g.pxy - 1, r = C[q].p % g.pxy;
+      const long long j = r / g.px - 1, i = r % g.px - g.xoff;
+      if (i < 0 || i > g.nx || j < 0 || j > g.ny || k < 0 || k > g.nz) return FDTD_OK;
+      const int c[3] = {(int)i, (int)j, (int)k};
+      if (in_poles(C[q].comp, c, c)) return FDTD_OK;
+      // the tile of the cell, as tile_column lays the tiles out
+      const long long bz = k / tm.kc;
+      const long long bxy = tm.flat ? (j * (g.nx + 1) + i) / (kWave * tm.bdy)
+                                    : (j / tm.bdy) * tm.tx + i / kWave;
+      tile[q] = (int)(bz * tm.ty * tm.tx + bxy);
+      ++nstart[(size_t)tile[q] + 1];
+    }
+    for (int t = 0; t < tm.nblk; ++t) nstart[(size_t)t + 1] += nstart[(size_t)t];
+    std::vector<int> at(nstart.begin(), nstart.end() - 1);
+    for (size_t q = 0; q < C.size(); ++q) cells[(size_t)at[(size_t)tile[q]]++] = C[q];
+  }
+  *out = h->pw_masks[half] && !F.empty() ? h->pw_src[half] : PassSrc{};
+  int rc;
+  if (!C.empty()) {
+    int *dst = nullptr;
+    NodalCell *dc = nullptr;
+    if ((rc = upload(h, &dst, nstart.data(), nstart.size(), list)) ||
+        (rc = upload(h, &dc, cells.data(), cells.size(), list)))
+      return rc;
+    out->nstart = dst;
+    out->cells = dc;
+    out->values = h->dvalues;
+    out->nsrc = (int)h->srcs.size();
+    out->serial = h->serial[half];
+  }
+  *on = true;
+  if (!flags) return FDTD_OK;
+  // flags are by block: the block that runs tile t
+  auto block_of = [&](int t) {
+    if (!tm.remap) return t;
+    // xcd_remap deals XCD x the tiles x*q + min(x, r) ...
+    const int q = tm.nblk >> 3, r = tm.nblk & 7;
+    const int big = r * (q + 1);
+    const int xcd = t < big ? t / (q + 1) : r + (t - big) / std::max(q, 1);
+    const int loc = t < big ? t % (q + 1) : (t - big) % std::max(q, 1);
+    return loc * 8 + xcd;
+  };
+  if (!C.empty())
+    for (int t = 0; t < tm.nblk; ++t)
+      if (nstart[(size_t)t] < nstart[(size_t)t + 1]) (*flags)[(size_t)block_of(t)] |= kTileNodal[half];
+  if (out->nface) {
+    const std::vector<unsigned> *m = h->pw_bits[half];
+    auto any = [](const std::vector<unsigned> &v, long long a, long long b) {
+      unsigned r = 0;
+      for (long long i = a; i < std::min<long long>(b, (long long)v.size()); ++i) r |= v[(size_t)i];
+      return r;
+    };
+    std::vector<unsigned> xy((size_t)tm.tx * tm.ty);
+    for (int by = 0; by < tm.ty; ++by)
+      for (int bx = 0; bx < tm.tx; ++bx) {
+        unsigned v;
+        if (tm.flat) {
+          const long long f0 = (long long)bx * kWave * tm.bdy, f1 = f0 + (long long)kWave * tm.bdy - 1;
+          const long long j0 = f0 / (g.nx + 1), j1 = f1 / (g.nx + 1);
+          v = any(m[1], j0, j1 + 1) & (j0 == j1 ? any(m[0], f0 % (g.nx + 1), f1 % (g.nx + 1) + 1)
+                                                : any(m[0], 0, g.nx + 1));
+        } else {
+          v = any(m[0], (long long)bx * kWave, (long long)(bx + 1) * kWave) &
+              any(m[1], (long long)by * tm.bdy, (long long)(by + 1) * tm.bdy);
+        }
+        xy[(size_t)by * tm.tx + bx] = v;
+      }
+    for (int bz = 0; bz < tm.tz; ++bz) {
+      const unsigned z = any(m[2], (long long)bz * tm.kc, (long long)(bz + 1) * tm.kc);
+      if (!z) continue;
+      for (int t = 0; t < tm.tx * tm.ty; ++t)
+        if (xy[(size_t)t] & z) (*flags)[(size_t)block_of(bz * tm.tx * tm.ty + t)] |= kTileFaces[half];
+    }
+  }
+  return FDTD_OK;
+}
+
 // InitPlaneWave (planewaves.F90:72-766) and calc_planewaveconstants
 // (:1494-1509) on the host, in real(4) with the reference's expression order;
 // the faces of AdvancePlaneWaveE/H (:878-1475) become one PwFace each, in the
@@ -933,6 +1184,9 @@ int build_planewaves(fdtd_handle *h) {
   h->pw_allocs.clear();
   h->pw_faces[0].clear();
   h->pw_faces[1].clear();
+  h->pw_masks[0] = h->pw_masks[1] = false;
+  h->pw_terms = PwTerms{};
+  h->pw_terms_n = -1;
   h->dwaves = nullptr; h->dphys = nullptr; h->dtiempo = nullptr;
   if (h->pwin.empty()) { h->pw_ready = true; return FDTD_OK; }
   if (h->tiempo.empty()) return fail(h, FDTD_ERR_STATE, "fdtd_set_time not called");
@@ -1035,16 +1289,6 @@ int build_planewaves(fdtd_handle *h) {
     if (il[4]) { face(1, 3, 2, false, 1, 1, -1.f); face(1, 4, 2, false, 0, 1, 1.f); }
     if (il[5]) { face(1, 3, 2, true, 1, 0, 1.f); face(1, 4, 2, true, 0, 0, -1.f); }
   }
-  int rc;
-  for (size_t q = 0; q < waves.size(); ++q) {
-    float *de = nullptr;
-    if ((rc = upload(h, &de, evols[q].data(), evols[q].size(), &h->pw_allocs))) return rc;
-    waves[q].evol = de;
-  }
-  if ((rc = upload(h, &h->dwaves, waves.data(), waves.size(), &h->pw_allocs))) return rc;
-  if ((rc = upload(h, &h->dphys, phys.data(), phys.size(), &h->pw_allocs))) return rc;
-  if ((rc = upload(h, &h->dtiempo, h->tiempo.data(), h->tiempo.size(), &h->pw_allocs))) return rc;
-  h->pstride = S;
   // launch groups: per half, per wave, per face axis (faces of a group are
   // parallel planes, so no two touch the same cell); the group order is the
   // reference's face order
@@ -1069,11 +1313,8 @@ int build_planewaves(fdtd_handle *h) {
           r.px = h->g.px;
           r.xoff = h->g.xoff;
           r.pxy = h->g.pxy;
-          r.wave = h->dwaves;
-          r.phys = h->dphys;
           r.pstride = S;
           r.half = half;
-          r.tiempo = h->dtiempo;
           r.dn = nullptr;
           r.dt = h->dt;
           r.G = half ? h->gm2h[1] : h->g2h[1];
@@ -1081,17 +1322,53 @@ int build_planewaves(fdtd_handle *h) {
           grp.runs.push_back(r);
           grp.start.push_back(grp.start.back() + nu * nv);
         }
-        if (grp.runs.empty()) continue;
-        std::vector<PwRun> counted = grp.runs;
-        for (PwRun &r : counted) r.dn = h->dstep;
-        if ((rc = upload(h, &grp.druns[0], grp.runs.data(), grp.runs.size(), &h->pw_allocs)))
-          return rc;
-        if ((rc = upload(h, &grp.druns[1], counted.data(), counted.size(), &h->pw_allocs)))
-          return rc;
-        if ((rc = upload(h, &grp.dstart, grp.start.data(), grp.start.size(), &h->pw_allocs)))
-          return rc;
-        h->pw_groups.push_back(std::move(grp));
+        if (!grp.runs.empty()) h->pw_groups.push_back(std::move(grp));
       }
+  // every table in one device allocation
+  Pack pk;
+  std::vector<size_t> oev(waves.size());
+  for (size_t q = 0; q < waves.size(); ++q) oev[q] = pk.add(evols[q].size() * 4);
+  const size_t ow = pk.add(waves.size() * sizeof(PwWave)), op = pk.add(phys.size() * 4),
+               ot = pk.add(h->tiempo.size() * 8);
+  std::vector<size_t> og(h->pw_groups.size() * 3);
+  for (size_t q = 0; q < h->pw_groups.size(); ++q) {
+    const PwGroup &grp = h->pw_groups[q];
+    og[3 * q] = pk.add(grp.runs.size() * sizeof(PwRun));
+    og[3 * q + 1] = pk.add(grp.runs.size() * sizeof(PwRun));
+    og[3 * q + 2] = pk.add(grp.start.size() * sizeof(long long));
+  }
+  PwMasks masks;
+  build_pw_masks(h, masks, pk);
+  int rc;
+  if ((rc = pk.alloc(h, &h->pw_allocs))) return rc;
+  for (size_t q = 0; q < waves.size(); ++q) {
+    waves[q].evol = pk.at<float>(oev[q]);
+    pk.put(oev[q], evols[q]);
+  }
+  pk.put(ow, waves);
+  pk.put(op, phys);
+  pk.put(ot, h->tiempo);
+  h->dwaves = pk.at<PwWave>(ow);
+  h->dphys = pk.at<float>(op);
+  h->dtiempo = pk.at<double>(ot);
+  h->pstride = S;
+  for (size_t q = 0; q < h->pw_groups.size(); ++q) {
+    PwGroup &grp = h->pw_groups[q];
+    for (PwRun &r : grp.runs) {
+      r.wave = h->dwaves;
+      r.phys = h->dphys;
+      r.tiempo = h->dtiempo;
+    }
+    std::vector<PwRun> counted = grp.runs;
+    for (PwRun &r : counted) r.dn = h->dstep;
+    pk.put(og[3 * q], grp.runs);
+    pk.put(og[3 * q + 1], counted);
+    pk.put(og[3 * q + 2], grp.start);
+    grp.druns[0] = pk.at<PwRun>(og[3 * q]);
+    grp.druns[1] = pk.at<PwRun>(og[3 * q + 1]);
+    grp.dstart = pk.at<long long>(og[3 * q + 2]);
+  }
+  if ((rc = place_pw_masks(h, masks, pk)) || (rc = pk.send(h))) return rc;
   h->pw_ready = true;
   return FDTD_OK;
 }
@@ -1160,7 +1437,7 @@ int prepare(fdtd_handle *h) {
   return FDTD_OK;
 }
 
-int run_e(fdtd_handle *h, int yee, int cpml, int ade) {
+int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
   // the fused pass (yee and cpml) always runs the CPML kernel: without slab
@@ -1168,20 +1445,20 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade) {
   const int c = cpml && (h->g.has_cpml || yee);
   const int a = ade && h->g.ade[0].has;
   const int *tmed = h->tmed_ready ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, h->stream)
-                                     : fast::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, h->stream);
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "E pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
 
-int run_h(fdtd_handle *h, int yee, int cpml, int ade) {
+int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
   const int c = cpml && (h->g.has_cpml || yee);
   const int a = ade && h->g.ade[1].has;
   const int *tmed = h->tmed_ready ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, h->stream)
-                                     : fast::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, h->stream);
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "H pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1198,12 +1475,14 @@ Observe observe_desc(const fdtd_handle *h, const int *dn) {
   o.dft = h->ddfts;
   o.ndft = (int)h->dfts.size();
   for (const DftDev &d : h->dfts) o.total += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+  o.pw = h->pw_terms;
   o.dn = dn;
   return o;
 }
 
-int run_observe(fdtd_handle *h, const DevGrid &g, int n, const int *dn, bool probes, bool dft) {
-  const int e = launch_observe(g, observe_desc(h, dn), n, probes, dft, h->stream);
+int run_observe(fdtd_handle *h, const DevGrid &g, int n, const int *dn, bool probes, bool dft,
+                bool pw) {
+  const int e = launch_observe(g, observe_desc(h, dn), n, probes, dft, pw, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "observation launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1233,6 +1512,50 @@ int run_nodal(fdtd_handle *h, int half, int n, const int *dn) {
                        n, dn, h->serial[half], h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "nodal launch failed");
   return FDTD_OK;
+}
+
+// is a caller recording the grid's stream
+bool stream_capturing(const fdtd_handle *h) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(h->stream, &st) == hipSuccess && st == hipStreamCaptureStatusActive;
+}
+
+// do the passes of the grid's own steps read the TF/SF terms
+bool inline_faces(const fdtd_handle *h) {
+  return h->tm4.vec != 4 && ((h->psrc_on[0] && h->psrc[0].nface) || (h->psrc_on[1] && h->psrc[1].nface));
+}
+
+// the terms of step n in the buffer, unless the observation of step n - 1
+// left them there
+int need_terms(fdtd_handle *h, int n) {
+  if (!inline_faces(h)) return FDTD_OK;
+  // a caller's own capture replays without this call: it records the launch
+  const bool capturing = stream_capturing(h);
+  if (!capturing && h->pw_terms_n == n) return FDTD_OK;
+  if (n < 0 || n >= (int)h->tiempo.size())
+    return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
+                (int)h->tiempo.size() - 1);
+  h->pw_terms_n = -1;
+  if (launch_pw_terms(h->pw_terms, n, nullptr, h->stream))
+    return fail(h, FDTD_ERR_HIP, "incident-field launch failed");
+  if (!capturing) h->pw_terms_n = n;
+  return FDTD_OK;
+}
+
+// One half step at step n (or *dn + n): the fused face pass with its pole
+// stage, its plane-wave faces and its nodal cells, the sources inside the
+// pass where they can be.
+int run_half(fdtd_handle *h, int half, int n, const int *dn) {
+  const bool in = h->psrc_on[half] && h->tm4.vec != 4;
+  PassSrc s = h->psrc[half];
+  s.dn = dn;
+  s.n = n;
+  if (in && !dn && s.nstart && (n < 0 || n >= h->nvalues_steps))
+    return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n, h->nvalues_steps - 1);
+  int rc = half ? run_h(h, 1, 1, 1, in ? &s : nullptr) : run_e(h, 1, 1, 1, in ? &s : nullptr);
+  if (rc || in) return rc;
+  if ((rc = run_pw(h, half, n, dn))) return rc;
+  return run_nodal(h, half, n, dn);
 }
 
 }  // namespace
@@ -1344,6 +1667,7 @@ int fdtd_destroy(fdtd_handle *h) {
   for (void *p : h->step_allocs) hipFree(p);
   for (void *p : h->step_small) hipFree(p);
   for (void *p : h->pw_allocs) hipFree(p);
+  for (void *p : h->psrc_allocs) hipFree(p);
   for (void *p : h->dft_allocs) hipFree(p);
   for (void *p : h->dft_sums) hipFree(p);
   for (void *p : h->allocs) hipFree(p);
@@ -1701,7 +2025,11 @@ int fdtd_update_observation(fdtd_handle *h, int32_t n) {
   if ((rc = probe_room(h, 1))) return rc;
   // a step outside the time vector still samples the probes
   const bool in = n >= 0 && n < (int)h->tiempo.size();
-  if ((rc = run_observe(h, h->g, n, nullptr, true, in))) return rc;
+  // the terms of the next step ride along when the steps run call by call
+  const bool pw = in && h->tmed_ready && inline_faces(h) && n + 1 < (int)h->tiempo.size() &&
+                  h->pw_terms_n == n && !stream_capturing(h);
+  if ((rc = run_observe(h, h->g, n, nullptr, true, in, pw))) return rc;
+  if (pw) h->pw_terms_n = n + 1;
   h->pbuffered += h->nprobe ? 1 : 0;
   if (!in && !h->dfts.empty())
     return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
@@ -1755,8 +2083,8 @@ int fdtd_advance_e(fdtd_handle *h, int32_t n) {
   h->prev_exact = true;
   hipSetDevice(h->device);
   int rc;
-  if ((rc = prepare(h)) || (rc = build_tile_media(h)) || (rc = run_e(h, 1, 1, 1)) || (rc = run_pw(h, 0, n, nullptr)) ||
-      (rc = run_nodal(h, 0, n, nullptr)))
+  if ((rc = prepare(h)) || (rc = build_tile_media(h)) || (rc = need_terms(h, n)) ||
+      (rc = run_half(h, 0, n, nullptr)))
     return rc;
   return FDTD_OK;
 }
@@ -1767,8 +2095,8 @@ int fdtd_advance_h(fdtd_handle *h, int32_t n) {
   h->prev_exact = true;
   hipSetDevice(h->device);
   int rc;
-  if ((rc = prepare(h)) || (rc = build_tile_media(h)) || (rc = run_h(h, 1, 1, 1)) || (rc = run_pw(h, 1, n, nullptr)) ||
-      (rc = run_nodal(h, 1, n, nullptr)) || (rc = run_mur(h)))
+  if ((rc = prepare(h)) || (rc = build_tile_media(h)) || (rc = need_terms(h, n)) ||
+      (rc = run_half(h, 1, n, nullptr)) || (rc = run_mur(h)))
     return rc;
   return FDTD_OK;
 }
@@ -1846,21 +2174,19 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
     if ((rc = settle_prev(h))) return rc;
   }
   if (singles == 0) return FDTD_OK;
-  if ((rc = build_tile_media(h))) return rc;
+  // the first step's TF/SF terms; each step's observation leaves the next's
+  if ((rc = build_tile_media(h)) || (rc = need_terms(h, n0 + 2 * pairs))) return rc;
+  if (inline_faces(h)) h->pw_terms_n = -1;
   // nrep two-pass steps in one graph: step r of it reads the step number
   // *dstep + r, and the counter advances once, at the end
   auto capture = [h](int nrep, hipGraph_t *gout, hipGraphExec_t *xout) -> int {
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int r2 = 0;
     for (int r = 0; r < nrep && !r2; ++r) {
-      r2 = run_e(h, 1, 1, 1);
-      if (!r2) r2 = run_pw(h, 0, r, h->dstep);
-      if (!r2) r2 = run_nodal(h, 0, r, h->dstep);
-      if (!r2) r2 = run_h(h, 1, 1, 1);
-      if (!r2) r2 = run_pw(h, 1, r, h->dstep);
-      if (!r2) r2 = run_nodal(h, 1, r, h->dstep);
+      r2 = run_half(h, 0, r, h->dstep);
+      if (!r2) r2 = run_half(h, 1, r, h->dstep);
       if (!r2) r2 = run_mur(h);
-      if (!r2) r2 = run_observe(h, h->g, r, h->dstep, true, true);
+      if (!r2) r2 = run_observe(h, h->g, r, h->dstep, true, true, inline_faces(h));
     }
     if (!r2) r2 = launch_tick(h->dstep, nrep, h->stream) ? fail(h, FDTD_ERR_HIP, "tick failed") : 0;
     hipGraph_t graph = nullptr;
@@ -1887,6 +2213,7 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
   }
   for (int32_t s = 0; s < left; ++s) HIPCHK(h, hipGraphLaunch(h->gexec, h->stream));
   h->pbuffered += singles;
+  if (inline_faces(h) && n0 + nsteps < (int)h->tiempo.size()) h->pw_terms_n = n0 + nsteps;
   return FDTD_OK;
 }
 
@@ -2079,7 +2406,7 @@ int fdtd_sample_probes(fdtd_handle *h) {
   if (int rc = refuse_batched(h)) return rc;
   if (int rc = probe_room(h, 1)) return rc;
   hipSetDevice(h->device);
-  if (int rc = run_observe(h, h->g, 0, nullptr, true, false)) return rc;
+  if (int rc = run_observe(h, h->g, 0, nullptr, true, false, false)) return rc;
   h->pbuffered += 1;
   return FDTD_OK;
 }

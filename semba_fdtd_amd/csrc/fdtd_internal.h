@@ -165,6 +165,55 @@ struct PwRun {
   int nu;                     // cells along the first free axis
 };
 
+// The sources of one half step as a one-cell face pass applies them to the
+// cells it updates, after the CPML and before the store.
+// TF/SF: up to 32 faces of the half, in the reference's face order, as bits.
+// A face is a box of cells one cell thick, so the faces crossing cell (i,j,k)
+// are mx[i] & my[j] & mz[k], of which cm[c] act on component c; its term at
+// that cell, +-G * Incid * id, waits at terms[base + i*sx + j*sy + k*sz].
+// Nodal: the cells of tile t (as numbered after the XCD remap) are
+// cells[nstart[t]] .. cells[nstart[t+1]-1], in the reference's order.
+struct FaceAddr {
+  int base, sx, sy, sz;
+};
+constexpr int kPassFaces = 32;
+// What a tile of the one-cell pass map meets, one word per tile: the medium
+// all its cells hold plus one (0: several) in the low 16 bits, and per half
+// whether it meets a TF/SF face or a nodal cell the pass applies inline.
+constexpr int kTileFaces[2] = {1 << 16, 1 << 17}, kTileNodal[2] = {1 << 18, 1 << 19};
+struct PassSrc {
+  int nface;
+  const unsigned *mx, *my, *mz;   // indexed 0 .. n of the axis
+  unsigned cm[3];
+  const FaceAddr *fa;
+  const float *terms;
+  const int *nstart;              // null: no nodal cells
+  const NodalCell *cells;
+  const float *values;
+  int nsrc, serial;               // serial: some field value has two cells
+  const int *dn;                  // device step counter (or null) and offset
+  int n;
+};
+
+// The TF/SF terms of both halves at one step (launch_pw_terms, or the blocks
+// of an observation launch that prepare the next step's): faces[0..nf0) act
+// on E, faces[nf0..nf) on H; face q's cells are out[start[q]] ..
+// out[start[q+1]-1], the face's first free axis fastest.
+struct PwTerms {
+  const PwFace *faces;
+  const long long *start;
+  int nf0, nf;
+  long long total;
+  const PwWave *waves;
+  const float *phys;
+  int pstride;
+  const double *tiempo;
+  int ntime;                  // entries of tiempo
+  double dt;
+  float G[2];                 // G2(1), GM2(1)
+  float *out;
+};
+
 // Frequency-domain observation box (observation.F90:3527-3600): complex(8)
 // running sums acc[pt][comp][freq] += aux[n][freq] * F_comp(pt), the points
 // being the stride multiples of the box (first[a] + t*stride[a], cnt[a] of them).
@@ -193,6 +242,7 @@ struct Observe {
   const DftDev *dft;          // frequency-domain boxes (device), in the order
   int ndft;                   // of their start
   long long total;            // (point, frequency) pairs of all boxes
+  PwTerms pw;                 // the next step's TF/SF terms (pw.total 0: none)
   const int *dn;              // device step counter (null: the launch's n)
 };
 
@@ -315,6 +365,8 @@ struct BatchDev {
   int total;
   const int *tmed;            // per tile: the medium all its cells hold, or -1
                               // (null: every tile loads its media)
+  const PassSrc *src[2];      // per grid: the sources the E and H passes apply
+                              // inline (null: no grid has any)
 };
 
 #ifdef __HIPCC__
@@ -378,15 +430,18 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
 #endif
 
 // launchers, one set per arithmetic mode.  tmed (null: none) holds, per
-// tile of the one-cell map tm, the medium of every cell of the tile or -1,
-// as launch_pass_tile_media writes it; the one-cell passes skip the media
-// loads of the tiles it names.
+// tile of the one-cell map tm, what the tile meets, as
+// launch_pass_tile_media writes it (out holds the flags on entry); the
+// one-cell passes skip the media loads of single-medium tiles.  src (null: none): the sources the fused
+// one-cell pass applies inline.
 #define SFD_DECLARE_LAUNCHERS(NS)                                              \
   namespace NS {                                                             \
   int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4,      \
-               const int *tmed, int yee, int cpml, int ade, void *stream);   \
+               const int *tmed, int yee, int cpml, int ade,                  \
+               const PassSrc *src, void *stream);                            \
   int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4,      \
-               const int *tmed, int yee, int cpml, int ade, void *stream);   \
+               const int *tmed, int yee, int cpml, int ade,                  \
+               const PassSrc *src, void *stream);                            \
   int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out,  \
                              void *stream);                                  \
   size_t step_lds_bytes(const DevGrid &g, int rows, int npw, int kc);       \
@@ -414,9 +469,19 @@ int launch_nodal(const DevGrid &g, const NodalCell *cells, int ncells,
 // *dn += by / *dn = n
 int launch_tick(int *dn, int by, void *stream);
 int launch_set_step(int *dn, int n, void *stream);
-// the observation of a grid at step n: probes sampled (when probes), then
-// frequency-domain sums advanced (when dft)
-int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, void *stream);
+// the observation of a grid at step n: probes sampled (when probes),
+// frequency-domain sums advanced (when dft), the TF/SF terms of step n + 1
+// written (when pw)
+int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, int pw,
+                   void *stream);
+// the TF/SF terms of step n (or *dn + n)
+int launch_pw_terms(const PwTerms &t, int n, const int *dn, void *stream);
+// the terms of many grids, each at its own *dn
+struct PwTermsGrid {
+  PwTerms t;
+  const int *dn;
+};
+int launch_pw_terms_many(const PwTermsGrid *grids, int n, long long maxcells, void *stream);
 // the same for many grids: blocks start[s] .. start[s+1]-1 of the launch
 // serve obs[s] on grids[grid[s]]
 struct ObserveGrid {

@@ -394,6 +394,9 @@ __device__ __forceinline__ void st_at(SFD_GLOBAL T *base, unsigned ob, T v) {
 __device__ __forceinline__ float ro_uniform(const float *t, int idx) {
   return ((const __attribute__((address_space(4))) float *)t)[idx];
 }
+__device__ __forceinline__ unsigned ro_uniform_u(const unsigned *t, int idx) {
+  return ((const __attribute__((address_space(4))) unsigned *)t)[idx];
+}
 
 // Field storage of the face passes: each field array holds fp32 values, or
 // binary16 values with a per-array scale.
@@ -432,6 +435,10 @@ template <> struct Store<float> {
   static __device__ __forceinline__ void sto(SFD_GLOBAL char *b, unsigned ob, float, float v) {
     st_at((SFD_GLOBAL float *)b, ob, v);
   }
+  // a value as it reads back after being stored by a pass, and by a source
+  static __device__ __forceinline__ float trip(float v, float, float) { return v; }
+  static __device__ __forceinline__ float trip_src(float v, float, float) { return v; }
+  static __device__ __forceinline__ void st_src(float *b, long long p, float, float v) { b[p] = v; }
 };
 // binary16 fields with a per-array scale: value = half * s, stored as
 // round(value / s); 8-byte vectors, fp32 arithmetic.  Every scale product is
@@ -442,6 +449,14 @@ template <> struct Store<float> {
 __device__ __forceinline__ float rounded(float x) {
   asm("" : "+v"(x));
   return x;
+}
+// A source launch of its own (fdtd_aux.hip) stores half(value / s) through the
+// mixed-precision FMA, one rounding; a source inside a pass stores the same.
+// (The result is read two cycles later: a partial register write.)
+__device__ __forceinline__ unsigned short half_src(float v, float is) {
+  unsigned r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\ts_nop 1" : "=v"(r) : "v"(is), "v"(v));
+  return (unsigned short)r;
 }
 template <> struct Store<__half> {
   static __device__ __forceinline__ F4 ld4(const float *b, long long p, float s) {
@@ -484,6 +499,15 @@ template <> struct Store<__half> {
   static __device__ __forceinline__ void sto(SFD_GLOBAL char *b, unsigned ob, float is, float v) {
     st_at((SFD_GLOBAL unsigned short *)b, ob, __half_as_ushort(__float2half_rn(rounded(v * is))));
   }
+  static __device__ __forceinline__ float trip(float v, float s, float is) {
+    return cvt(__half_as_ushort(__float2half_rn(rounded(v * is))), s);
+  }
+  static __device__ __forceinline__ float trip_src(float v, float s, float is) {
+    return cvt(half_src(v, is), s);
+  }
+  static __device__ __forceinline__ void st_src(float *b, long long p, float is, float v) {
+    reinterpret_cast<unsigned short *>(b)[p] = half_src(v, is);
+  }
 };
 
 // The column (i, j) of the tile's lane and the tile's z chunk bz.  Tiles are
@@ -506,6 +530,79 @@ __device__ __forceinline__ void tile_column(const TileMap &tm, int blk, int nx, 
   }
 }
 
+// The sources a pass applies inline (PassSrc; CPassSrc read through the
+// constant address space).  They cost a pass two loads per lane and tile and
+// one scalar load, one AND and one branch per plane; as kernels of their own
+// (three per half for a plane wave's face axes, one for nodal cells) they cost
+// a launch each, 4.4-9 us, and a second trip to memory for every face cell.
+typedef __attribute__((address_space(4))) PassSrc CPassSrc;
+
+// the address of face q's term at cell (i, j, k); fal: the faces in LDS
+__device__ __forceinline__ int term_index(const FaceAddr *fal, int q, int i, int j, int k) {
+  const FaceAddr a = fal[q];
+  return a.base + i * a.sx + j * a.sy + k * a.sz;
+}
+// the faces in bits applied to v in the reference's order; first: the first
+// face's term, loaded with the plane.  Binary16 storage rounds before and
+// after each face, as a launch of its own on the stored value would; what
+// comes back is a stored value, which the pass's store leaves as it is.
+template <class S>
+__device__ __forceinline__ float add_faces(unsigned bits, float first, const FaceAddr *fal,
+                                           const float *terms, int i, int j, int k, float v,
+                                           float s, float is) {
+  v = S::trip_src(S::trip(v, s, is) + first, s, is);
+  bits &= bits - 1;
+  while (bits) {
+    const int q = __builtin_ctz(bits);
+    bits &= bits - 1;
+    v = S::trip_src(v + terms[term_index(fal, q, i, j, k)], s, is);
+  }
+  return v;
+}
+// the first face's term of component bits (loaded ahead of its use)
+__device__ __forceinline__ float first_term(unsigned bits, const FaceAddr *fal,
+                                            const float *terms, int i, int j, int k) {
+  return bits ? terms[term_index(fal, __builtin_ctz(bits), i, j, k)] : 0.0f;
+}
+
+// LDS of the face addresses, behind the media table of tab bytes
+static __host__ __device__ __forceinline__ size_t face_lds_offset(size_t tab) {
+  return (tab + 15) & ~(size_t)15;
+}
+template <class PS>
+__device__ __forceinline__ const FaceAddr *stage_faces(const PS &x, float2 *lds, size_t tab) {
+  FaceAddr *f = reinterpret_cast<FaceAddr *>(reinterpret_cast<char *>(lds) + face_lds_offset(tab));
+  const int t = threadIdx.y * blockDim.x + threadIdx.x;
+  const FaceAddr *src = x.fa;
+  if (t < x.nface) f[t] = src[t];
+  return f;
+}
+
+// AdvanceNodalE/H on the cells of one tile, after its march: the block's own
+// stores are visible to it behind the barrier, and no other block writes the
+// tile's cells.  Every thread of the block calls this.
+template <class T, class PS>
+__device__ __forceinline__ void tile_nodal(const DevGrid &g, const TileMap &tm, const PS &x,
+                                           int blk) {
+  if (!x.nstart) return;
+  const int tile = tm.remap ? xcd_remap(blk, tm.nblk) : blk;
+  const int c0 = x.nstart[tile], c1 = x.nstart[tile + 1];
+  if (c0 >= c1) return;
+  __syncthreads();
+  const int t = threadIdx.y * blockDim.x + threadIdx.x, nt = blockDim.x * blockDim.y;
+  const int n = x.n + (x.dn ? *x.dn : 0);
+  // cells that share a field value run in order, on one thread
+  const int step = x.serial ? 1 : nt;
+  for (int c = x.serial ? (t == 0 ? c0 : c1) : c0 + t; c < c1; c += step) {
+    const NodalCell &cell = x.cells[c];
+    if (cell.skip) continue;
+    const float v = x.values[(long long)n * x.nsrc + cell.src];
+    float *f = g.f[cell.comp];
+    const float old = cell.hard ? 0.0f : Store<T>::ld1(f, cell.p, g.fs[cell.comp]);
+    Store<T>::st_src(f, cell.p, g.fi[cell.comp], nodal_apply(old, cell, v));
+  }
+}
+
 // one tile (64 x blockDim.y lanes, one z chunk) of the E face pass; T the
 // field storage (fp32, or binary16 with the arrays' scales).  A lane
 // addresses each z plane by a base the same for every lane (scalar
@@ -513,10 +610,13 @@ __device__ __forceinline__ void tile_column(const TileMap &tm, int blk, int nx, 
 // slabs likewise.  Each plane issues every load it needs (fields, media, the
 // psi values of the CPML slabs) before any arithmetic, so a plane costs one
 // memory round trip; the per-plane spacing and z profile are scalar loads,
-// the x and y profiles fixed for the lane.
-template <bool YEE, bool CPML, bool TBL, class T = float, class G = DevGrid>
+// the x and y profiles fixed for the lane.  X: the TF/SF faces of xs are
+// applied before each store (fal: their addresses in LDS).
+template <bool YEE, bool CPML, bool TBL, class T = float, bool X = false, class G = DevGrid,
+          class PS = PassSrc>
 __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
-                                           const MedTab &tab, int blk, int m0 = -1) {
+                                           const MedTab &tab, int blk, int m0, const PS *xs = nullptr,
+                                           const FaceAddr *fal = nullptr) {
   typedef Store<T> S;
   typedef const SFD_GLOBAL float *cgf;
   constexpr unsigned ES = sizeof(T);
@@ -563,6 +663,9 @@ __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
   float *const pExy = (float *)g.psi[PSI_EXY], *const pExz = (float *)g.psi[PSI_EXZ];
   float *const pEyz = (float *)g.psi[PSI_EYZ], *const pEyx = (float *)g.psi[PSI_EYX];
   float *const pEzy = (float *)g.psi[PSI_EZY], *const pEzx = (float *)g.psi[PSI_EZX];
+  // the faces crossing the lane's column
+  unsigned col = 0;
+  if (X && xs->nface) col = ((const SFD_GLOBAL unsigned *)xs->mx)[i] & ((const SFD_GLOBAL unsigned *)xs->my)[j];
   for (int k = k0; k < k1; ++k) {
     const bool cz = k < nz;
     const long long kb = (long long)(k + 1) * fpb, kmb = (long long)(k + 1) * mpb;
@@ -620,6 +723,17 @@ __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
       if (cz && syn) vzy = ld_at(sEzy, oE);
       if (cz && sxn) vzx = ld_at(sEzx, oD);
     }
+    unsigned fb = 0;
+    float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+    if (X && xs->nface) {
+      fb = col & ro_uniform_u(xs->mz, k);
+      if (fb) {
+        const float *terms = xs->terms;
+        t0 = first_term(fb & xs->cm[0], fal, terms, i, j, k);
+        t1 = first_term(fb & xs->cm[1], fal, terms, i, j, k);
+        t2 = first_term(fb & xs->cm[2], fal, terms, i, j, k);
+      }
+    }
     float hx0 = 0.0f, hy0 = 0.0f, hz0 = 0.0f, hz_jm = 0.0f, hx_jm = 0.0f, hz_im = 0.0f,
           hy_im = 0.0f;
     if (NEEDH) {
@@ -645,6 +759,8 @@ __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
           e = madd(e, -c.y, v);
         }
       }
+      if (X && (fb & xs->cm[0]))
+        e = add_faces<S>(fb & xs->cm[0], t0, fal, xs->terms, i, j, k, e, g.fs[0], g.fi[0]);
       S::sto(exk, of, g.fi[0], e);
     }
     if (cy) {
@@ -663,6 +779,8 @@ __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
           e = madd(e, -c.y, v);
         }
       }
+      if (X && (fb & xs->cm[1]))
+        e = add_faces<S>(fb & xs->cm[1], t1, fal, xs->terms, i, j, k, e, g.fs[1], g.fi[1]);
       S::sto(eyk, of, g.fi[1], e);
     }
     if (cz) {
@@ -681,16 +799,20 @@ __device__ __forceinline__ void epass_tile(const G &g, const TileMap &tm,
           e = madd(e, c.y, v);
         }
       }
+      if (X && (fb & xs->cm[2]))
+        e = add_faces<S>(fb & xs->cm[2], t2, fal, xs->terms, i, j, k, e, g.fs[2], g.fi[2]);
       S::sto(ezk, of, g.fi[2], e);
     }
     if (NEEDH) { hx_km = hx0; hy_km = hy0; }
   }
 }
 
-// one tile of the H face pass (addressing and loads as in the E pass)
-template <bool YEE, bool CPML, bool TBL, class T = float, class G = DevGrid>
+// one tile of the H face pass (addressing, loads and sources as in the E pass)
+template <bool YEE, bool CPML, bool TBL, class T = float, bool X = false, class G = DevGrid,
+          class PS = PassSrc>
 __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
-                                           const MedTab &tab, int blk, int m0 = -1) {
+                                           const MedTab &tab, int blk, int m0, const PS *xs = nullptr,
+                                           const FaceAddr *fal = nullptr) {
   typedef Store<T> S;
   typedef const SFD_GLOBAL float *cgf;
   constexpr unsigned ES = sizeof(T);
@@ -735,6 +857,8 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
   float *const pHxy = (float *)g.psi[PSI_HXY], *const pHxz = (float *)g.psi[PSI_HXZ];
   float *const pHyz = (float *)g.psi[PSI_HYZ], *const pHyx = (float *)g.psi[PSI_HYX];
   float *const pHzy = (float *)g.psi[PSI_HZY], *const pHzx = (float *)g.psi[PSI_HZX];
+  unsigned col = 0;
+  if (X && xs->nface) col = ((const SFD_GLOBAL unsigned *)xs->mx)[i] & ((const SFD_GLOBAL unsigned *)xs->my)[j];
   for (int k = k0; k < k1; ++k) {
     const bool ax = j < ny && k < nz;   // Hx sweep: x[0,nx] y[0,ny-1] z[0,nz-1]
     const bool ay = i < nx && k < nz;   // Hy sweep: x[0,nx-1] y[0,ny] z[0,nz-1]
@@ -788,6 +912,17 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
       if (az && syc) vzy = ld_at(sHzy, oE);
       if (az && sxc) vzx = ld_at(sHzx, oD);
     }
+    unsigned fb = 0;
+    float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+    if (X && xs->nface) {
+      fb = col & ro_uniform_u(xs->mz, k);
+      if (fb) {
+        const float *terms = xs->terms;
+        t0 = first_term(fb & xs->cm[0], fal, terms, i, j, k);
+        t1 = first_term(fb & xs->cm[1], fal, terms, i, j, k);
+        t2 = first_term(fb & xs->cm[2], fal, terms, i, j, k);
+      }
+    }
     const float ex_kp = S::cvt(rex_kp, g.fs[0]), ey_kp = S::cvt(rey_kp, g.fs[1]);
     const float ez_c = S::cvt(rez_c, g.fs[2]);
     const float ez_jp = S::cvt(rez_jp, g.fs[2]), ex_jp = S::cvt(rex_jp, g.fs[0]);
@@ -809,6 +944,8 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
           h = madd(h, c.y, v);
         }
       }
+      if (X && (fb & xs->cm[0]))
+        h = add_faces<S>(fb & xs->cm[0], t0, fal, xs->terms, i, j, k, h, g.fs[3], g.fi[3]);
       S::sto(hxk, of, g.fi[3], h);
     }
     if (ay) {
@@ -827,6 +964,8 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
           h = madd(h, c.y, v);
         }
       }
+      if (X && (fb & xs->cm[1]))
+        h = add_faces<S>(fb & xs->cm[1], t1, fal, xs->terms, i, j, k, h, g.fs[4], g.fi[4]);
       S::sto(hyk, of, g.fi[4], h);
     }
     if (az) {
@@ -845,6 +984,8 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
           h = madd(h, -c.y, v);
         }
       }
+      if (X && (fb & xs->cm[2]))
+        h = add_faces<S>(fb & xs->cm[2], t2, fal, xs->terms, i, j, k, h, g.fs[5], g.fi[5]);
       S::sto(hzk, of, g.fi[5], h);
     }
     ex_c = ex_kp;
@@ -1128,11 +1269,17 @@ __global__ void __launch_bounds__(256) k_hpass4(DevGrid g, TileMap tm) {
   hpass4_tile<true, T>(g, tm, tab, blockIdx.x);
 }
 
+// the tile's word (see kTileFaces) and its medium or -1
+__device__ __forceinline__ int tile_info(const int *tmed) {
+  return tmed ? __builtin_amdgcn_readfirstlane(tmed[blockIdx.x]) : 0;
+}
+__device__ __forceinline__ int tile_medium(int info) { return (info & 0xffff) - 1; }
+
 template <bool YEE, bool CPML, bool TBL, class T = float>
 __global__ void __launch_bounds__(256) k_epass(DevGrid g, TileMap tm, const int *tmed) {
   extern __shared__ float2 lds_tab[];
   const MedTab tab = stage_tables<TBL, false>(g, g.g1, g.g2, lds_tab);
-  const int m0 = tmed ? __builtin_amdgcn_readfirstlane(tmed[blockIdx.x]) : -1;
+  const int m0 = tile_medium(tile_info(tmed));
   epass_tile<YEE, CPML, TBL, T>(g, tm, tab, blockIdx.x, m0);
 }
 
@@ -1140,14 +1287,43 @@ template <bool YEE, bool CPML, bool TBL, class T = float>
 __global__ void __launch_bounds__(256) k_hpass(DevGrid g, TileMap tm, const int *tmed) {
   extern __shared__ float2 lds_tab[];
   const MedTab tab = stage_tables<TBL, false>(g, g.gm1, g.gm2, lds_tab);
-  const int m0 = tmed ? __builtin_amdgcn_readfirstlane(tmed[blockIdx.x]) : -1;
+  const int m0 = tile_medium(tile_info(tmed));
   hpass_tile<YEE, CPML, TBL, T>(g, tm, tab, blockIdx.x, m0);
+}
+
+// the fused passes with the half's sources inline (tab: bytes of the LDS media
+// table)
+template <bool TBL, class T>
+__global__ void __launch_bounds__(256) k_epass_src(DevGrid g, TileMap tm, const int *tmed,
+                                                   PassSrc xs, unsigned tab_bytes) {
+  extern __shared__ float2 lds_tab[];
+  const FaceAddr *fal = stage_faces(xs, lds_tab, tab_bytes);
+  const MedTab tab = stage_tables<TBL, false>(g, g.g1, g.g2, lds_tab);
+  if (!TBL) __syncthreads();
+  const int ti = tile_info(tmed), m0 = tile_medium(ti);
+  if (ti & kTileFaces[0]) epass_tile<true, true, TBL, T, true>(g, tm, tab, blockIdx.x, m0, &xs, fal);
+  else epass_tile<true, true, TBL, T>(g, tm, tab, blockIdx.x, m0);
+  if (ti & kTileNodal[0]) tile_nodal<T>(g, tm, xs, blockIdx.x);
+}
+
+template <bool TBL, class T>
+__global__ void __launch_bounds__(256) k_hpass_src(DevGrid g, TileMap tm, const int *tmed,
+                                                   PassSrc xs, unsigned tab_bytes) {
+  extern __shared__ float2 lds_tab[];
+  const FaceAddr *fal = stage_faces(xs, lds_tab, tab_bytes);
+  const MedTab tab = stage_tables<TBL, false>(g, g.gm1, g.gm2, lds_tab);
+  if (!TBL) __syncthreads();
+  const int ti = tile_info(tmed), m0 = tile_medium(ti);
+  if (ti & kTileFaces[1]) hpass_tile<true, true, TBL, T, true>(g, tm, tab, blockIdx.x, m0, &xs, fal);
+  else hpass_tile<true, true, TBL, T>(g, tm, tab, blockIdx.x, m0);
+  if (ti & kTileNodal[1]) tile_nodal<T>(g, tm, xs, blockIdx.x);
 }
 
 // One block per tile of a one-cell pass map: the medium index that all six
 // media arrays hold on every cell the tile's lanes own (columns i <= nx,
-// j <= ny, the planes of its z chunk), or -1 where they differ.  The tiles
-// are decoded as the passes decode them.
+// j <= ny, the planes of its z chunk), plus one, or 0 where they differ,
+// added to the tile's flags in out.  The tiles are decoded as the passes
+// decode them.
 __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, int *out) {
   int bx, by, bz;
   decode_tile(tm, blockIdx.x, bx, by, bz);
@@ -1167,7 +1343,6 @@ __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, 
     nc = wi > 0 && wj > 0 ? (long long)wi * wj : 0;
   }
   if (nc <= 0 || k1 <= k0) {
-    if (threadIdx.x == 0) out[blockIdx.x] = -1;
     return;
   }
   __shared__ int bad;
@@ -1193,7 +1368,7 @@ __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, 
   }
   if (b) atomicOr(&bad, 1);
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = bad ? -1 : m0;
+  if (threadIdx.x == 0 && !bad) out[blockIdx.x] += m0 + 1;
 }
 
 int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out, void *stream) {
@@ -1228,7 +1403,7 @@ __device__ __forceinline__ int batch_grid(const int *start, int ngrid, int t) {
   return lo;
 }
 
-template <bool H, class T, int VEC>
+template <bool H, class T, int VEC, bool X>
 __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
   extern __shared__ float2 lds_tab[];
   for (int t = blockIdx.x; t < bd.total; t += gridDim.x) {
@@ -1241,6 +1416,10 @@ __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
     const CDevGrid &cg = *(const CDevGrid *)(bd.grids + b);
     const TileMap tm = const_tilemap(bd.tms + b);
     __syncthreads();  // the previous tile is done with the LDS tables
+    // X: the grid's sources, read through the constant address space too
+    const CPassSrc *xs = X ? (const CPassSrc *)(bd.src[H ? 1 : 0] + b) : nullptr;
+    const FaceAddr *fal = nullptr;
+    if (X) fal = stage_faces(*xs, lds_tab, (size_t)(g.nmedia + 1) * 12);
     const MedTab tab = H ? stage_tables<true, false>(g, g.gm1, g.gm2, lds_tab)
                          : stage_tables<true, false>(g, g.g1, g.g2, lds_tab);
     // the CPML variant serves grids without CPML too: with no slab layers
@@ -1252,8 +1431,9 @@ __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
     } else {
       // a tile whose cells all hold one medium skips the media loads
       const int m0 = bd.tmed ? __builtin_amdgcn_readfirstlane(bd.tmed[t]) : -1;
-      if (H) hpass_tile<true, true, true, T, CDevGrid>(cg, tm, tab, blk, m0);
-      else epass_tile<true, true, true, T, CDevGrid>(cg, tm, tab, blk, m0);
+      if (H) hpass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
+      else epass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
+      if (X) tile_nodal<T>(g, tm, *xs, blk);
     }
   }
 }
@@ -1263,19 +1443,20 @@ int launch_pass_batch(const BatchDev &bd, int half, int blocks, int rows, int ve
   if (bd.total <= 0) return 0;
   const dim3 blk(kWave, (unsigned)rows);
   hipStream_t s = (hipStream_t)stream;
-  if (fp16 && vec == 4) {
-    if (half) hipLaunchKernelGGL((k_pass_batch<true, __half, 4>), dim3(blocks), blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_pass_batch<false, __half, 4>), dim3(blocks), blk, lds, s, bd);
-  } else if (fp16) {
-    if (half) hipLaunchKernelGGL((k_pass_batch<true, __half, 1>), dim3(blocks), blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_pass_batch<false, __half, 1>), dim3(blocks), blk, lds, s, bd);
-  } else if (vec == 4) {
-    if (half) hipLaunchKernelGGL((k_pass_batch<true, float, 4>), dim3(blocks), blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_pass_batch<false, float, 4>), dim3(blocks), blk, lds, s, bd);
-  } else {
-    if (half) hipLaunchKernelGGL((k_pass_batch<true, float, 1>), dim3(blocks), blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_pass_batch<false, float, 1>), dim3(blocks), blk, lds, s, bd);
-  }
+  const bool x = vec != 4 && bd.src[half ? 1 : 0];
+  if (x) lds = face_lds_offset(lds) + kPassFaces * sizeof(FaceAddr);
+#define SFD_B(T, V, X)                                                                       \
+  do {                                                                                       \
+    if (half) hipLaunchKernelGGL((k_pass_batch<true, T, V, X>), dim3(blocks), blk, lds, s, bd); \
+    else hipLaunchKernelGGL((k_pass_batch<false, T, V, X>), dim3(blocks), blk, lds, s, bd);  \
+  } while (0)
+  if (fp16 && vec == 4) SFD_B(__half, 4, false);
+  else if (fp16 && x) SFD_B(__half, 1, true);
+  else if (fp16) SFD_B(__half, 1, false);
+  else if (vec == 4) SFD_B(float, 4, false);
+  else if (x) SFD_B(float, 1, true);
+  else SFD_B(float, 1, false);
+#undef SFD_B
   return (int)hipGetLastError();
 }
 
@@ -1330,7 +1511,7 @@ int launch_ade_many(const DevGrid *grids, const int *list, int n, int side, size
 }
 
 int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int *tmed, int yee,
-             int cpml, int ade, void *stream) {
+             int cpml, int ade, const PassSrc *src, void *stream) {
   const dim3 blk(kWave, (unsigned)tm.bdy);
   hipStream_t s = (hipStream_t)stream;
   const int nb = tm.nblk;
@@ -1343,7 +1524,16 @@ int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
     else                                                                       \
       hipLaunchKernelGGL((k_epass<Y, C, false>), dim3(nb), blk, 0, s, g, tm, tmed); \
   } while (0)
-  if (yee && cpml && tbl && tm4.vec == 4) {
+  if (src && yee && cpml && tm4.vec != 4) {
+    // the fused one-cell pass with its sources inline
+    const size_t tb = tbl ? lds : 0, lx = face_lds_offset(tb) + kPassFaces * sizeof(FaceAddr);
+    if (g.fp16)
+      hipLaunchKernelGGL((k_epass_src<true, __half>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
+    else if (tbl)
+      hipLaunchKernelGGL((k_epass_src<true, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
+    else
+      hipLaunchKernelGGL((k_epass_src<false, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, 0u);
+  } else if (yee && cpml && tbl && tm4.vec == 4) {
     // fused pass, four cells per lane (the CPML variant also serves grids
     // without CPML)
     if (g.fp16) hipLaunchKernelGGL(k_epass4<__half>, dim3(tm4.nblk), blk, lds, s, g, tm4);
@@ -1361,7 +1551,7 @@ int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
 }
 
 int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int *tmed, int yee,
-             int cpml, int ade, void *stream) {
+             int cpml, int ade, const PassSrc *src, void *stream) {
   const dim3 blk(kWave, (unsigned)tm.bdy);
   hipStream_t s = (hipStream_t)stream;
   const int nb = tm.nblk;
@@ -1374,7 +1564,16 @@ int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
     else                                                                       \
       hipLaunchKernelGGL((k_hpass<Y, C, false>), dim3(nb), blk, 0, s, g, tm, tmed); \
   } while (0)
-  if (yee && cpml && tbl && tm4.vec == 4) {
+  if (src && yee && cpml && tm4.vec != 4) {
+    // the fused one-cell pass with its sources inline
+    const size_t tb = tbl ? lds : 0, lx = face_lds_offset(tb) + kPassFaces * sizeof(FaceAddr);
+    if (g.fp16)
+      hipLaunchKernelGGL((k_hpass_src<true, __half>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
+    else if (tbl)
+      hipLaunchKernelGGL((k_hpass_src<true, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
+    else
+      hipLaunchKernelGGL((k_hpass_src<false, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, 0u);
+  } else if (yee && cpml && tbl && tm4.vec == 4) {
     if (g.fp16) hipLaunchKernelGGL(k_hpass4<__half>, dim3(tm4.nblk), blk, lds, s, g, tm4);
     else hipLaunchKernelGGL(k_hpass4<float>, dim3(tm4.nblk), blk, lds, s, g, tm4);
   } else if (g.fp16 && yee && cpml && tbl) {
