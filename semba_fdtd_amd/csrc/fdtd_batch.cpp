@@ -66,6 +66,7 @@ struct fdtd_batch {
   std::vector<long long> step;        // host copy of each slot's step counter
   std::vector<unsigned> version;      // each grid's state version at the last build
   int rows = 4, zchunk = 16, xcells = 1, blocks = 0;
+  bool quads = false;                 // the passes run four cells per lane
   // device descriptors, rebuilt when the membership changes
   bool ready = false;
   std::vector<void *> allocs;
@@ -171,25 +172,18 @@ int bupload(fdtd_batch *b, T **dst, const T *src, size_t n, std::vector<void *> 
   return FDTD_OK;
 }
 
-// tile map of one grid under the batch's tiling: four x cells per lane in
-// 256-wide segments, or one cell per lane in flat tiles (runs of 64 * rows
-// columns of the x-y plane, x fastest), which leave no lane idle on grids a
-// few tens of cells wide
+// tile map of one grid under the batch's tiling: runs of 64 * rows columns
+// (one cell per lane) or vectors (four) of the x-y plane, x fastest, which
+// leave no lane idle on grids a few tens of cells wide
 TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
   TileMap tm{};
   tm.bdy = b->rows;
-  if (b->xcells == 4) {
-    const int w = 4 * kWave;
-    tm.vec = 4;
-    tm.tx = (g.nx + 1 + w - 1) / w;
-    tm.ty = (g.ny + 1 + b->rows - 1) / b->rows;
-  } else {
-    const long long cols = (long long)(g.nx + 1) * (g.ny + 1), per = (long long)kWave * b->rows;
-    tm.vec = 1;
-    tm.flat = 1;
-    tm.tx = (int)((cols + per - 1) / per);
-    tm.ty = 1;
-  }
+  const long long cols = (long long)(b->quads ? g.nx / 4 + 1 : g.nx + 1) * (g.ny + 1);
+  const long long per = (long long)kWave * b->rows;
+  tm.vec = b->quads ? 4 : 1;
+  tm.flat = 1;
+  tm.tx = (int)((cols + per - 1) / per);
+  tm.ty = 1;
   tm.kc = std::min(b->zchunk, g.nz + 1);
   tm.tz = (g.nz + 1 + tm.kc - 1) / tm.kc;
   tm.nblk = tm.tx * tm.ty * tm.tz;
@@ -207,6 +201,9 @@ int build_descriptors(fdtd_batch *b) {
   size_t lds = 16;
   int maxwaves = 0;
   int rc;
+  b->quads = b->xcells == 4;
+  for (fdtd_handle *h : b->slots)
+    if (h && !quads_fit(h)) b->quads = false;
   for (size_t s = 0; s < b->slots.size(); ++s) {
     fdtd_handle *h = b->slots[s];
     if (!h) continue;
@@ -237,7 +234,7 @@ int build_descriptors(fdtd_batch *b) {
   b->bd.total = start.back();
   // flat tiles whose cells all hold one medium skip the media loads
   b->bd.tmed = nullptr;
-  if (b->xcells == 1 && b->bd.total > 0) {
+  if (!b->quads && b->bd.total > 0) {
     int *dm = nullptr;
     BCHK(b, hipMalloc((void **)&dm, (size_t)b->bd.total * sizeof(int)));
     b->allocs.push_back(dm);
@@ -256,7 +253,7 @@ int build_descriptors(fdtd_batch *b) {
       b->bd.src[half] = nullptr;
     }
     int gi = 0;
-    for (size_t s = 0; s < b->slots.size() && b->xcells == 1; ++s) {
+    for (size_t s = 0; s < b->slots.size() && !b->quads; ++s) {
       fdtd_handle *h = b->slots[s];
       if (!h) continue;
       bool faces = false;
@@ -507,7 +504,7 @@ int launch_step(fdtd_batch *b) {
   const int blocks = b->blocks > 0 ? b->blocks : 16384;
   int e, rc;
   for (int half = 0; half < 2; ++half) {
-    const int vec = b->xcells == 4 ? 4 : 1;
+    const int vec = b->quads ? 4 : 1;
     e = exact ? exact::launch_pass_batch(b->bd, half, blocks, b->rows, vec, b->lds, 0, b->stream)
               : fast::launch_pass_batch(b->bd, half, blocks, b->rows, vec, b->lds, b->fp16,
                                         b->stream);

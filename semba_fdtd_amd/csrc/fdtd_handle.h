@@ -62,7 +62,8 @@ struct fdtd_handle {
   int storage = FDTD_STORE_FP32;
   sfd::DevGrid g{};
   sfd::TileMap tm{};           // 64-cell x tiles (granular passes)
-  sfd::TileMap tm4{};          // 256-cell x tiles (fused passes, 4 cells per lane)
+  int xcells = 1;              // 4: the fused passes run four cells per lane
+  bool tile_set = false;       // fdtd_set_tiling was called
   int tile_zchunk = 32;        // planes per z chunk as set (tm.kc: clipped to the grid)
   std::vector<void *> allocs;
   int64_t bytes = 0;
@@ -178,6 +179,14 @@ struct fdtd_handle {
   int *tmed = nullptr;
   int tmed_cap = 0;
   bool tmed_ready = false;
+  // the four-cell passes' tiles: boxes, the slabs they meet, rows per block,
+  // planes per chunk, and each tile's word (valid while tmed_ready and the
+  // grid runs these passes)
+  sfd::QuadPlan qplan = {};
+  int qslabs = 0;
+  int qrows = 1, qkc = 1;
+  int *qmed = nullptr;
+  int qmed_cap = 0;
   std::vector<double> step_cells;        // Yee cells owned per class
   std::vector<double> step_bytes;        // compulsory HBM bytes of one launch per class
   uint8_t *mi8[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // step mode
@@ -218,6 +227,7 @@ int refuse_batched(fdtd_handle *h);
 // extents of component comp's Alloc box per axis
 void alloc_extent(const fdtd_handle *h, int comp, long long ext[3]);
 int probe_room(fdtd_handle *h, long long more);
+bool quads_fit(const fdtd_handle *h);
 int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);

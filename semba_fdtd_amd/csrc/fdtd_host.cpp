@@ -194,18 +194,86 @@ int check_ready(fdtd_handle *h) {
 void set_tiles(fdtd_handle *h, int rows, int zchunk, int xcells) {
   const DevGrid &g = h->g;
   h->tile_zchunk = zchunk;
-  for (int v = 0; v < 2; ++v) {
-    TileMap &tm = v ? h->tm4 : h->tm;
-    const int w = v ? 4 * kWave : kWave;
-    tm.bdy = rows;
-    tm.tx = (g.nx + 1 + w - 1) / w;
-    tm.ty = (g.ny + 1 + rows - 1) / rows;
-    tm.kc = std::min(zchunk, g.nz + 1);
-    tm.tz = (g.nz + 1 + tm.kc - 1) / tm.kc;
-    tm.nblk = tm.tx * tm.ty * tm.tz;
-    tm.remap = 1;
-    tm.vec = xcells;
+  h->xcells = xcells;
+  TileMap &tm = h->tm;
+  tm.bdy = rows;
+  tm.tx = (g.nx + 1 + kWave - 1) / kWave;
+  tm.ty = (g.ny + 1 + rows - 1) / rows;
+  tm.kc = std::min(zchunk, g.nz + 1);
+  tm.tz = (g.nz + 1 + tm.kc - 1) / tm.kc;
+  tm.nblk = tm.tx * tm.ty * tm.tz;
+  tm.remap = 1;
+  tm.vec = 1;
+}
+
+static long long cells_of(const fdtd_handle *h) {
+  return (long long)h->g.nx * h->g.ny * h->g.nz;
+}
+// grids up to this apply their sources inside the one-cell passes (see
+// make_pass_src)
+constexpr long long kInlineCells = 12000000;
+
+// Can the four-cell passes run the grid: the media table has to fit in LDS,
+// and a vector may not meet both x slabs.
+bool quads_fit(const fdtd_handle *h) {
+  const DevGrid &g = h->g;
+  const int L = g.L[0][0] + g.L[0][1];
+  return g.nmedia + 1 <= 4096 && (L == 0 || g.nx - L >= 4);
+}
+// ... and do they: unless a tiling of one cell per lane was asked for.  us per
+// step against the one-cell passes at their best tiling: 40^3 16.2 against
+// 15.7, 64^3 18.6 / 24.8, 101x87x65 29.2 / 34.2, 128^3 50.4 / 71.6, 200^3
+// 154 / 205, 256^3 369 / 435, 320^3 680 / 789; without CPML 64^3 13.4 / 20.7,
+// 160^3 58.0 / 77.2, 384^3 1041 / 1085.
+static bool use_quads(const fdtd_handle *h) {
+  return quads_fit(h) && (h->xcells == 4 || !h->tile_set);
+}
+
+// the boxes of the four-cell passes under the handle's tiling
+static void plan_quads(fdtd_handle *h) {
+  const DevGrid &g = h->g;
+  const int Q = g.nx / 4 + 1, J = g.ny + 1, K = g.nz + 1;
+  // rows and planes that touch no y or z slab of E or H
+  auto hi = [&](int a, int n) { return g.L[a][1] ? n - g.L[a][1] : n + 1; };
+  const int ja = g.L[1][0], jb = hi(1, g.ny), ka = g.L[2][0], kb = hi(2, g.nz);
+  if (h->tile_set) {
+    h->qrows = h->tm.bdy;
+    h->qkc = h->tm.kc;
+  } else {
+    // One plane per block: nothing is carried from plane to plane, but twice
+    // the blocks hide the load latency better, and small tiles more often hold
+    // one medium.  Two planes pay where a block moves little per plane: binary16,
+    // and rows packed to 16 bytes on grids that fill the chip.  us per step,
+    // one / two planes: 64^3 18.6 / 22.4, 128^3 52.4 / 50.4, 200^3 163.6 /
+    // 153.8, 256^3 369 / 382, 320^3 680 / 714; binary16 64^3 20.1 / 25.8,
+    // 128^3 49.8 / 48.7, 200^3 135 / 115, 256^3 345 / 284.
+    const long long cells = cells_of(h);
+    h->qrows = 1;
+    h->qkc = cells >= 1500000 && (g.fp16 || g.nx < 256) ? 2 : 1;
   }
+  QuadPlan P = {};
+  std::fill(P.start, P.start + kQuadBoxes + 1, 0x7fffffff);
+  auto add = [&](int j0, int j1, int k0, int k1) {
+    if (j1 <= j0 || k1 <= k0) return;
+    QuadBox &b = P.box[P.nbox];
+    P.start[P.nbox++] = P.nblk;
+    b = QuadBox{0, Q, j0, j1 - j0, k0, k1 - k0, 0, 0};
+    const long long per = (long long)kWave * h->qrows;
+    b.tx = (int)(((long long)b.nq * b.nj + per - 1) / per);
+    P.nblk += b.tx * ((b.nk + h->qkc - 1) / h->qkc);
+  };
+  if (ja < jb && ka < kb) {
+    add(ja, jb, ka, kb);
+    add(0, J, 0, ka);
+    add(0, J, kb, K);
+    add(0, ja, ka, kb);
+    add(jb, J, ka, kb);
+    h->qslabs = P.nbox > 1 ? kSlabMix : g.L[0][0] + g.L[0][1] ? kSlabX : 0;
+  } else {
+    add(0, J, 0, K);
+    h->qslabs = kSlabAll;
+  }
+  h->qplan = P;
 }
 
 static void drop_multi_graph(fdtd_handle *h) {
@@ -235,8 +303,37 @@ void invalidate_graph(fdtd_handle *h) {
 // skip the media loads of single-medium tiles; and the sources the passes
 // apply inline.  Built outside any capture, before the passes it serves are
 // launched or recorded.
+static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags);
 int build_tile_media(fdtd_handle *h) {
   if (h->tmed_ready) return FDTD_OK;
+  h->psrc_on[0] = h->psrc_on[1] = false;
+  if (use_quads(h)) {
+    plan_quads(h);
+    const int n = h->qplan.nblk;
+    if (n > h->qmed_cap) {
+      HIPCHK(h, hipStreamSynchronize(h->stream));
+      if (h->qmed) hipFree(h->qmed);
+      h->qmed = nullptr;
+      h->qmed_cap = 0;
+      HIPCHK(h, hipMalloc(&h->qmed, (size_t)n * sizeof(int)));
+      h->qmed_cap = n;
+    }
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    for (void *p : h->psrc_allocs) hipFree(p);
+    h->psrc_allocs.clear();
+    std::vector<int> flags((size_t)n, 0);
+    for (int half = 0; half < 2; ++half)
+      if (int rc = make_quad_src(h, half, &flags)) return rc;
+    HIPCHK(h, hipMemcpyAsync(h->qmed, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
+                             h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const int e = h->mode == FDTD_MODE_EXACT
+                      ? exact::launch_quad_media(h->g, h->qplan, h->qrows, h->qkc, h->qmed, h->stream)
+                      : fast::launch_quad_media(h->g, h->qplan, h->qrows, h->qkc, h->qmed, h->stream);
+    if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
+    h->tmed_ready = true;
+    return FDTD_OK;
+  }
   if (h->tm.nblk > h->tmed_cap) {
     if (h->tmed) hipFree(h->tmed);
     h->tmed = nullptr;
@@ -1058,6 +1155,124 @@ static int place_pw_masks(fdtd_handle *h, const PwMasks &w, Pack &pk) {
   return FDTD_OK;
 }
 
+// does a box of cells of component comp meet its pole-state box
+static bool in_poles(const fdtd_handle *h, int comp, const int lo[3], const int hi[3]) {
+  const AdeSet &A = h->g.ade[comp / 3];
+  if (!A.has) return false;
+  const int *b = A.abox[comp % 3];
+  for (int a = 0; a < 3; ++a)
+    if (b[3 + a] <= 0 || hi[a] < b[a] || lo[a] >= b[a] + b[3 + a]) return false;
+  return true;
+}
+
+// the nodal cells of a pass, grouped by tile: tile(i, j, k) of ntile
+template <class F>
+static int tile_cells(fdtd_handle *h, int half, int ntile, F tile_of, PassSrc *out, bool *on,
+                      std::vector<void *> *list, std::vector<int> *start) {
+  const std::vector<NodalCell> &C = h->hcells[half];
+  const DevGrid &g = h->g;
+  std::vector<int> tile(C.size());
+  std::vector<int> &nstart = *start;
+  std::vector<NodalCell> cells(C.size());
+  nstart.assign((size_t)ntile + 1, 0);
+  for (size_t q = 0; q < C.size(); ++q) {
+    const long long k = C[q].p / g.pxy - 1, r = C[q].p % g.pxy;
+    const long long j = r / g.px - 1, i = r % g.px - g.xoff;
+    if (i < 0 || i > g.nx || j < 0 || j > g.ny || k < 0 || k > g.nz) return FDTD_OK;
+    const int c[3] = {(int)i, (int)j, (int)k};
+    if (in_poles(h, C[q].comp, c, c)) return FDTD_OK;
+    tile[q] = tile_of(c[0], c[1], c[2]);
+    ++nstart[(size_t)tile[q] + 1];
+  }
+  for (int t = 0; t < ntile; ++t) nstart[(size_t)t + 1] += nstart[(size_t)t];
+  std::vector<int> at(nstart.begin(), nstart.end() - 1);
+  for (size_t q = 0; q < C.size(); ++q) cells[(size_t)at[(size_t)tile[q]]++] = C[q];
+  int *dst = nullptr, rc;
+  NodalCell *dc = nullptr;
+  if ((rc = upload(h, &dst, nstart.data(), nstart.size(), list)) ||
+      (rc = upload(h, &dc, cells.data(), cells.size(), list)))
+    return rc;
+  out->nstart = dst;
+  out->cells = dc;
+  out->values = h->dvalues;
+  out->nsrc = (int)h->srcs.size();
+  out->serial = h->serial[half];
+  *on = true;
+  return FDTD_OK;
+}
+
+// does a plane-wave face of the half meet a pole-state box
+static bool face_in_poles(const fdtd_handle *h, int half) {
+  for (const PwFace &f : h->pw_faces[half]) {
+    int lo[3], hi[3];
+    for (int a = 0; a < 3; ++a) { lo[a] = f.lo[a]; hi[a] = f.hi[a]; }
+    lo[f.axis] = hi[f.axis] = f.fixed;
+    if (in_poles(h, f.comp, lo, hi)) return true;
+  }
+  return false;
+}
+
+// The sources of a half in the four-cell passes, where make_pass_src's rule on
+// places allows it; the passes apply no faces in tiles of the y and z slabs (a
+// box that touches them keeps its own launches).  Grids of every size: the
+// tiles without faces run code without them.  us per step, separate / inline:
+// 64^3 38.4 / 18.6, 128^3 80.2 / 52.4, 256^3 429 / 369, 384^3 1558 / 1431.
+static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags) {
+  h->psrc[half] = PassSrc{};
+  const bool faces = !h->pw_faces[half].empty();
+  if (!faces && h->hcells[half].empty()) return FDTD_OK;
+  if (faces && (!h->pw_masks[half] || face_in_poles(h, half))) return FDTD_OK;
+  const QuadPlan &p = h->qplan;
+  PassSrc x = faces ? h->pw_src[half] : PassSrc{};
+  if (x.nface) {
+    const std::vector<unsigned> *m = h->pw_bits[half];
+    auto any = [](const std::vector<unsigned> &v, int a, int b) {
+      unsigned r = 0;
+      for (int i = a; i < std::min(b, (int)v.size()); ++i) r |= v[(size_t)i];
+      return r;
+    };
+    const int run = kWave * h->qrows;
+    int t = 0;
+    for (int q = 0; q < p.nbox; ++q) {
+      const QuadBox &o = p.box[q];
+      const bool slabs = h->qslabs == kSlabAll || (h->qslabs == kSlabMix && q > 0);
+      std::vector<unsigned> xy((size_t)o.tx);
+      for (int r = 0; r < o.tx; ++r) {
+        const int f0 = r * run, f1 = std::min(f0 + run, o.nq * o.nj) - 1;
+        const int j0 = f0 / o.nq, j1 = f1 / o.nq;
+        xy[(size_t)r] = any(m[1], o.j0 + j0, o.j0 + j1 + 1) &
+                        (j0 == j1 ? any(m[0], 4 * (f0 % o.nq), 4 * (f1 % o.nq) + 4)
+                                  : any(m[0], 0, h->g.nx + 1));
+      }
+      for (int k = o.k0; k < o.k0 + o.nk; k += h->qkc) {
+        const unsigned z = any(m[2], k, std::min(k + h->qkc, o.k0 + o.nk));
+        for (int r = 0; r < o.tx; ++r, ++t) {
+          if (!(xy[(size_t)r] & z)) continue;
+          if (slabs) return FDTD_OK;
+          (*flags)[(size_t)t] |= kTileFaces[half];
+        }
+      }
+    }
+  }
+  if (!h->hcells[half].empty()) {
+    std::vector<int> start;
+    bool on = false;
+    const int rc = tile_cells(h, half, p.nblk, [&](int i, int j, int k) {
+      for (int b = 0; b < p.nbox; ++b) {
+        const QuadBox &o = p.box[b];
+        if (j < o.j0 || j >= o.j0 + o.nj || k < o.k0 || k >= o.k0 + o.nk) continue;
+        const int f = (j - o.j0) * o.nq + i / 4;
+        return p.start[b] + (k - o.k0) / h->qkc * o.tx + f / (kWave * h->qrows);
+      }
+      return 0;   // (the boxes hold every swept cell)
+    }, &x, &on, &h->psrc_allocs, &start);
+    if (rc || !on) return rc;
+  }
+  h->psrc[half] = x;
+  h->psrc_on[half] = true;
+  return FDTD_OK;
+}
+
 // A pass applies the sources before the pole stage that follows it, so they
 // move into the pass only where no source cell lies in a pole-state box (the
 // two then act on different cells, in any order), every nodal cell lies in
@@ -1067,7 +1282,6 @@ static int place_pw_masks(fdtd_handle *h, const PwMasks &w, Pack &pk) {
 // 4.6-9 us each whatever the grid.  A plane wave on 48^3, 100^3, 160^3, 200^3
 // runs 1.64, 1.48, 1.14, 1.02 times as fast inline, on 320^3 0.98 times; a
 // point source on 64^3, 128^3, 200^3 1.16, 1.03, 1.04 times, on 320^3 0.99.
-constexpr long long kInlineCells = 12000000;
 int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, bool *on,
                   std::vector<void *> *list, std::vector<int> *flags) {
   *on = false;
@@ -1075,57 +1289,21 @@ int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, boo
   const std::vector<PwFace> &F = h->pw_faces[half];
   const std::vector<NodalCell> &C = h->hcells[half];
   if (F.empty() && C.empty()) return FDTD_OK;
-  if ((long long)h->g.nx * h->g.ny * h->g.nz > kInlineCells) return FDTD_OK;
+  if (cells_of(h) > kInlineCells) return FDTD_OK;
   if (!F.empty() && !h->pw_masks[half]) return FDTD_OK;
-  const AdeSet &A = h->g.ade[half];
-  auto in_poles = [&](int comp, const int lo[3], const int hi[3]) {
-    if (!A.has) return false;
-    const int *b = A.abox[comp % 3];
-    for (int a = 0; a < 3; ++a)
-      if (b[3 + a] <= 0 || hi[a] < b[a] || lo[a] >= b[a] + b[3 + a]) return false;
-    return true;
-  };
-  for (const PwFace &f : F) {
-    int lo[3], hi[3];
-    for (int a = 0; a < 3; ++a) { lo[a] = f.lo[a]; hi[a] = f.hi[a]; }
-    lo[f.axis] = hi[f.axis] = f.fixed;
-    if (in_poles(f.comp, lo, hi)) return FDTD_OK;
-  }
+  if (face_in_poles(h, half)) return FDTD_OK;
   const DevGrid &g = h->g;
-  std::vector<int> tile(C.size()), nstart;
-  std::vector<NodalCell> cells(C.size());
-  if (!C.empty()) {
-    nstart.assign((size_t)tm.nblk + 1, 0);
-    for (size_t q = 0; q < C.size(); ++q) {
-      const long long k = C[q].p / g.pxy - 1, r = C[q].p % g.pxy;
-      const long long j = r / g.px - 1, i = r % g.px - g.xoff;
-      if (i < 0 || i > g.nx || j < 0 || j > g.ny || k < 0 || k > g.nz) return FDTD_OK;
-      const int c[3] = {(int)i, (int)j, (int)k};
-      if (in_poles(C[q].comp, c, c)) return FDTD_OK;
-      // the tile of the cell, as tile_column lays the tiles out
-      const long long bz = k / tm.kc;
-      const long long bxy = tm.flat ? (j * (g.nx + 1) + i) / (kWave * tm.bdy)
-                                    : (j / tm.bdy) * tm.tx + i / kWave;
-      tile[q] = (int)(bz * tm.ty * tm.tx + bxy);
-      ++nstart[(size_t)tile[q] + 1];
-    }
-    for (int t = 0; t < tm.nblk; ++t) nstart[(size_t)t + 1] += nstart[(size_t)t];
-    std::vector<int> at(nstart.begin(), nstart.end() - 1);
-    for (size_t q = 0; q < C.size(); ++q) cells[(size_t)at[(size_t)tile[q]]++] = C[q];
-  }
+  std::vector<int> nstart;
   *out = h->pw_masks[half] && !F.empty() ? h->pw_src[half] : PassSrc{};
-  int rc;
   if (!C.empty()) {
-    int *dst = nullptr;
-    NodalCell *dc = nullptr;
-    if ((rc = upload(h, &dst, nstart.data(), nstart.size(), list)) ||
-        (rc = upload(h, &dc, cells.data(), cells.size(), list)))
-      return rc;
-    out->nstart = dst;
-    out->cells = dc;
-    out->values = h->dvalues;
-    out->nsrc = (int)h->srcs.size();
-    out->serial = h->serial[half];
+    // the tile of a cell, as tile_column lays the tiles out
+    const int rc = tile_cells(h, half, tm.nblk, [&](int i, int j, int k) {
+      const long long bxy = tm.flat ? ((long long)j * (g.nx + 1) + i) / (kWave * tm.bdy)
+                                    : (long long)(j / tm.bdy) * tm.tx + i / kWave;
+      return (int)((long long)(k / tm.kc) * tm.ty * tm.tx + bxy);
+    }, out, on, list, &nstart);
+    if (rc) return rc;
+    if (!*on) { *out = PassSrc{}; return FDTD_OK; }
   }
   *on = true;
   if (!flags) return FDTD_OK;
@@ -1437,16 +1615,34 @@ int prepare(fdtd_handle *h) {
   return FDTD_OK;
 }
 
+// the fused face pass of a half, four cells per lane (build_tile_media laid
+// its tiles out)
+int run_quads(fdtd_handle *h, int half, const PassSrc *src) {
+  const PassSrc x = src ? *src : PassSrc{};
+  const int e = h->mode == FDTD_MODE_EXACT
+                    ? exact::launch_quad(h->g, h->qplan, h->qslabs, h->qrows, h->qkc, h->qmed, half, x, h->stream)
+                    : fast::launch_quad(h->g, h->qplan, h->qslabs, h->qrows, h->qkc, h->qmed, half, x, h->stream);
+  if (e) return fail(h, FDTD_ERR_HIP, "%s pass launch failed: %s", half ? "H" : "E",
+                     hipGetErrorString((hipError_t)e));
+  return FDTD_OK;
+}
+
 int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
   // the fused pass (yee and cpml) always runs the CPML kernel: without slab
   // layers it updates no psi
-  const int c = cpml && (h->g.has_cpml || yee);
+  int c = cpml && (h->g.has_cpml || yee);
   const int a = ade && h->g.ade[0].has;
-  const int *tmed = h->tmed_ready ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream)
-                                     : fast::launch_e(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream);
+  const bool quads = use_quads(h);
+  if (quads && yee && cpml) {
+    if (int rc = run_quads(h, 0, src)) return rc;
+    if (!a) return FDTD_OK;
+    yee = c = 0;
+  }
+  const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, h->tm, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_e(h->g, h->tm, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "E pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1454,11 +1650,17 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
 int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
-  const int c = cpml && (h->g.has_cpml || yee);
+  int c = cpml && (h->g.has_cpml || yee);
   const int a = ade && h->g.ade[1].has;
-  const int *tmed = h->tmed_ready ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream)
-                                     : fast::launch_h(h->g, h->tm, h->tm4, tmed, yee, c, a, src, h->stream);
+  const bool quads = use_quads(h);
+  if (quads && yee && cpml) {
+    if (int rc = run_quads(h, 1, src)) return rc;
+    if (!a) return FDTD_OK;
+    yee = c = 0;
+  }
+  const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, h->tm, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_h(h->g, h->tm, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "H pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1522,7 +1724,7 @@ bool stream_capturing(const fdtd_handle *h) {
 
 // do the passes of the grid's own steps read the TF/SF terms
 bool inline_faces(const fdtd_handle *h) {
-  return h->tm4.vec != 4 && ((h->psrc_on[0] && h->psrc[0].nface) || (h->psrc_on[1] && h->psrc[1].nface));
+  return ((h->psrc_on[0] && h->psrc[0].nface) || (h->psrc_on[1] && h->psrc[1].nface));
 }
 
 // the terms of step n in the buffer, unless the observation of step n - 1
@@ -1546,7 +1748,7 @@ int need_terms(fdtd_handle *h, int n) {
 // stage, its plane-wave faces and its nodal cells, the sources inside the
 // pass where they can be.
 int run_half(fdtd_handle *h, int half, int n, const int *dn) {
-  const bool in = h->psrc_on[half] && h->tm4.vec != 4;
+  const bool in = h->psrc_on[half];
   PassSrc s = h->psrc[half];
   s.dn = dn;
   s.n = n;
@@ -1673,6 +1875,7 @@ int fdtd_destroy(fdtd_handle *h) {
   for (void *p : h->allocs) hipFree(p);
   if (h->stage) hipFree(h->stage);
   if (h->tmed) hipFree(h->tmed);
+  if (h->qmed) hipFree(h->qmed);
   if (h->solo_stream) h->stream = h->solo_stream;
   if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
   delete h;
@@ -1800,7 +2003,9 @@ int fdtd_set_cpml(fdtd_handle *h, const int32_t layers[6], const float *pbe_x,
     int rc;
     if (len[s] != h->psilen[s]) g.psi[s] = nullptr;  // a different layout: fresh array
     if (!g.psi[s] && len[s] > 0) {
-      if ((rc = dalloc(h, (void **)&g.psi[s], (size_t)len[s] * 4))) return rc;
+      // (the four-cell passes read up to four values past either end)
+      if ((rc = dalloc(h, (void **)&g.psi[s], (size_t)(len[s] + 8) * 4))) return rc;
+      g.psi[s] += 4;
     }
     h->psilen[s] = len[s];
     if (len[s] > 0 && (rc = dzero(h, g.psi[s], (size_t)len[s] * 4))) return rc;
@@ -1908,6 +2113,7 @@ int fdtd_set_tiling(fdtd_handle *h, int32_t rows, int32_t zchunk, int32_t xcells
                          ((h->g.nz + zchunk) / zchunk);
   if (nblk > 0x7fffffffLL) return fail(h, FDTD_ERR_ARG, "tiling gives too many blocks");
   set_tiles(h, rows, zchunk, xcells);
+  h->tile_set = true;
   invalidate_graph(h);
   return FDTD_OK;
 }
@@ -1916,7 +2122,7 @@ int fdtd_get_tiling(const fdtd_handle *h, int32_t *rows, int32_t *zchunk, int32_
   if (!h || !rows || !zchunk || !xcells) return FDTD_ERR_ARG;
   *rows = h->tm.bdy;
   *zchunk = h->tile_zchunk;
-  *xcells = h->tm4.vec;
+  *xcells = h->xcells;
   return FDTD_OK;
 }
 

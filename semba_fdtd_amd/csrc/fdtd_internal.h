@@ -89,10 +89,29 @@ struct TileMap {
   int nblk;
   int remap;
   int bdy;          // rows per block (block = 64 x bdy threads, <= 256)
-  int vec;          // x cells per lane of the fused passes (1 or 4)
+  int vec;          // x cells per lane of the fused passes as asked (1 or 4)
   int flat;         // 1: tiles are runs of 64 * bdy columns of the x-y plane
                     // (one cell per lane), tx per plane, ty = 1
 };
+
+// The boxes of one launch of the four-cell passes (fdtd_quad.h): vectors of
+// four x cells q0 .. q0 + nq - 1, rows j0 .. , planes k0 ..; tx runs of
+// vectors per plane.
+// Box b holds tiles start[b] .. start[b+1] - 1 (unused entries: past any tile).
+struct QuadBox {
+  int q0, nq, j0, nj, k0, nk;
+  int tx, pad;
+};
+constexpr int kQuadBoxes = 5;
+// the slabs the tiles of a launch may meet: bits for x, y, z, or kSlabMix: the
+// first box's at most x, the others' all
+constexpr int kSlabX = 1, kSlabY = 2, kSlabZ = 4, kSlabAll = 7, kSlabMix = 8;
+struct QuadPlan {
+  int nbox, nblk;
+  int start[kQuadBoxes + 1];
+  QuadBox box[kQuadBoxes];
+};
+
 
 // First-order Mur (bordersmur.F90): one tangential H component on one
 // absorbing face.  The plane just outside the component's sweep (ghost) is
@@ -436,12 +455,17 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
 // one-cell pass applies inline.
 #define SFD_DECLARE_LAUNCHERS(NS)                                              \
   namespace NS {                                                             \
-  int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4,      \
-               const int *tmed, int yee, int cpml, int ade,                  \
-               const PassSrc *src, void *stream);                            \
-  int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4,      \
-               const int *tmed, int yee, int cpml, int ade,                  \
-               const PassSrc *src, void *stream);                            \
+  int launch_e(const DevGrid &g, const TileMap &tm, const int *tmed,        \
+               int yee, int cpml, int ade, const PassSrc *src, void *stream); \
+  int launch_h(const DevGrid &g, const TileMap &tm, const int *tmed,        \
+               int yee, int cpml, int ade, const PassSrc *src, void *stream); \
+  int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, \
+                  int kc, const int *tmed, int half, const PassSrc &src,    \
+                  void *stream);                                             \
+  int launch_quad_batch(const BatchDev &bd, int half, int blocks, int rows, \
+                        size_t lds, int fp16, void *stream);                 \
+  int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows,      \
+                        int kc, int *out, void *stream);                     \
   int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out,  \
                              void *stream);                                  \
   size_t step_lds_bytes(const DevGrid &g, int rows, int npw, int kc);       \

@@ -27,169 +27,10 @@
 // state of dispersive edges) and only then computes, so the pole state's
 // HBM latency overlaps the curl arithmetic.  The thread domain covers
 // [0,nx]x[0,ny]x[0,nz]; each component updates the part inside its sweep.
-#include <hip/hip_fp16.h>
-#include <hip/hip_runtime.h>
-#include "fdtd_internal.h"
-
-#ifndef SFD_NS
-#error "compile with -DSFD_NS=fast or -DSFD_NS=exact"
-#endif
-#ifndef SFD_EXACT
-#define SFD_EXACT 0
-#endif
+#include "fdtd_device.h"
 
 namespace sfd {
 namespace SFD_NS {
-
-// pole states prefetched into registers per edge: one Lorentz pair is two
-// complex(8) states in EXACT and one folded complex64 state in FAST
-#if SFD_EXACT
-typedef double2 jstate_t;  // complex(8) pole state, reference layout
-typedef double coef_t;
-constexpr int kPre = 2;
-#else
-typedef float2 jstate_t;   // complex64 state, conjugate pairs folded
-typedef float coef_t;
-#ifndef SFD_PREFETCH_POLES
-#define SFD_PREFETCH_POLES 1
-#endif
-constexpr int kPre = SFD_PREFETCH_POLES;
-#endif
-
-// hardware dispatches block b to XCD b % 8; give each XCD one contiguous
-// range of tiles so that x/y neighbours share that XCD's L2
-// global memory, spelled out for the pointers the compiler cannot infer it
-// for (those read out of memory rather than passed as kernel arguments)
-#define SFD_GLOBAL __attribute__((address_space(1)))
-
-__device__ __forceinline__ int xcd_remap(int b, int nblk) {
-  const int q = nblk >> 3, r = nblk & 7;
-  const int xcd = b & 7, loc = b >> 3;
-  return (xcd < r) ? xcd * (q + 1) + loc : r * (q + 1) + (xcd - r) * q + loc;
-}
-
-__device__ __forceinline__ void decode_tile(const TileMap &tm, int b, int &bx, int &by,
-                                            int &bz) {
-  if (tm.remap) b = xcd_remap(b, tm.nblk);
-  bx = b % tm.tx;
-  b /= tm.tx;
-  by = b % tm.ty;
-  bz = b / tm.ty;
-}
-
-// slab coordinate along a stretched axis.  "node" axes hold n+1 positions
-// (tangential E, normal H), "cell" axes n.  High slabs start after the
-// interior: node n-Lhi+1, cell n-Lhi (borderscpml.F90:149-193).
-__device__ __forceinline__ bool slab_node(int c, int n, int L0, int L1, int &q) {
-  if (c < L0) { q = c; return true; }
-  const int hs = n - L1 + 1;
-  if (c >= hs) { q = L0 + (c - hs); return true; }
-  return false;
-}
-__device__ __forceinline__ bool slab_cell(int c, int n, int L0, int L1, int &q) {
-  if (c < L0) { q = c; return true; }
-  const int hs = n - L1;
-  if (c >= hs) { q = L0 + (c - hs); return true; }
-  return false;
-}
-
-// The update arithmetic.  EXACT: plain products and sums (the file is built
-// without contraction), the reference's order.  FAST: explicit fused
-// multiply-adds, so that every variant of a pass (one or four cells per lane,
-// one grid or a batch) rounds the same way and gives the same bits.
-// a*ia - b*ib
-__device__ __forceinline__ float curl2(float a, float ia, float b, float ib) {
-#if SFD_EXACT
-  return a * ia - b * ib;
-#else
-  return __builtin_fmaf(a, ia, -(b * ib));
-#endif
-}
-// g1*f + g2*cu
-__device__ __forceinline__ float yee_upd(float g1, float f, float g2, float cu) {
-#if SFD_EXACT
-  return g1 * f + g2 * cu;
-#else
-  return __builtin_fmaf(g1, f, g2 * cu);
-#endif
-}
-// x + g*v
-__device__ __forceinline__ float madd(float x, float g, float v) {
-#if SFD_EXACT
-  return x + g * v;
-#else
-  return __builtin_fmaf(g, v, x);
-#endif
-}
-
-// psi <- b*psi + d*c ; returns the new psi
-__device__ __forceinline__ float psi_step(float *psi, long long s, float b,
-                                          float d, float c) {
-  const float v = madd(d * c, b, psi[s]);
-  psi[s] = v;
-  return v;
-}
-
-// per-medium tables staged in LDS (TBL) or read from global memory
-struct MedTab {
-  const float2 *gg;     // {G1,G2} or {GM1,GM2}
-  const int *slot;      // dispersive slot per medium (-1: not dispersive)
-  const int *anp;       // stored poles per slot
-  const coef_t *acf;    // per slot per pole {kr,ki,br,bi,g3r,g3i}
-};
-
-__device__ __forceinline__ const coef_t *ade_coefs(const AdeSet &ad) {
-#if SFD_EXACT
-  return ad.aded;
-#else
-  return ad.adef;
-#endif
-}
-
-// LDS layout: gg[nm+1] | slot[nm+1] | anp[ndisp] | (8-byte aligned) acf.
-// ad: the pole state whose tables are staged (ADE only).
-template <bool TBL, bool ADE>
-__device__ __forceinline__ MedTab stage_tables(const DevGrid &g, const float *a,
-                                               const float *b, float2 *lds,
-                                               const AdeSet *ad = nullptr) {
-  MedTab t;
-  const int nm = g.nmedia;
-  if (TBL) {
-    int *ls = reinterpret_cast<int *>(lds + (nm + 1));
-    int *lnp = ls + (nm + 1);
-    const int nd = ADE ? ad->ndisp : 0;
-    const size_t off = ((size_t)(nm + 1) * 12 + (size_t)nd * 4 + 7) & ~(size_t)7;
-    coef_t *lcf = reinterpret_cast<coef_t *>(reinterpret_cast<char *>(lds) + off);
-    const int tid = threadIdx.y * blockDim.x + threadIdx.x;
-    const int nt = blockDim.x * blockDim.y;
-    for (int m = tid; m <= nm; m += nt) {
-      lds[m] = make_float2(a[m], b[m]);
-      if (ADE) ls[m] = nd ? ad->dslot[m] : -1;
-    }
-    if (ADE) {
-      const coef_t *cf = ade_coefs(*ad);
-      for (int d = tid; d < nd; d += nt) lnp[d] = ad->anp[d];
-      for (int q = tid; q < nd * kPMax * 6; q += nt) lcf[q] = cf[q];
-    }
-    __syncthreads();
-    t.gg = lds;
-    t.slot = ls;
-    t.anp = lnp;
-    t.acf = lcf;
-  } else {
-    t.gg = nullptr;
-    t.slot = ADE ? ad->dslot : nullptr;
-    t.anp = ADE ? ad->anp : nullptr;
-    t.acf = ADE ? ade_coefs(*ad) : nullptr;
-  }
-  return t;
-}
-
-template <bool TBL>
-__device__ __forceinline__ float2 coef(const MedTab &t, const float *a, const float *b, int m) {
-  if (TBL) return t.gg[m];
-  return make_float2(a[m], b[m]);
-}
 
 // ---- pole-residue ADE (electricdispersive.F90:304-362 on E,
 // magneticdispersive.F90:306-362 on H, the same recursion) -----------------
@@ -364,243 +205,6 @@ __global__ void __launch_bounds__(256) k_ade_box(DevGrid g) {
 template <bool TBL, int SIDE>
 __global__ void __launch_bounds__(256) k_ade_many(const DevGrid *grids, const int *list) {
   ade_box_run<TBL, SIDE>(grids[list[blockIdx.z]]);
-}
-
-// Loads and stores of the march address a plane through a base pointer that
-// is the same for every lane (scalar registers) plus the lane's byte offset
-// inside the plane (one 32-bit register).  The plane base is made opaque to
-// the compiler, which otherwise hoists a 64-bit (array base + offset) pair per
-// array and lane out of the march; it stays in the global address space so
-// that the accesses are global, not flat, loads and stores.
-template <class T>
-__device__ __forceinline__ SFD_GLOBAL T *plane_base(T *base, long long P) {
-  SFD_GLOBAL T *q = (SFD_GLOBAL T *)(base + P);
-  asm volatile("" : "+s"(q));
-  return q;
-}
-template <class T>
-__device__ __forceinline__ T ld_at(const SFD_GLOBAL T *base, unsigned ob) {
-  return *reinterpret_cast<const SFD_GLOBAL T *>(reinterpret_cast<const SFD_GLOBAL char *>(base) +
-                                                 ob);
-}
-template <class T>
-__device__ __forceinline__ void st_at(SFD_GLOBAL T *base, unsigned ob, T v) {
-  *reinterpret_cast<SFD_GLOBAL T *>(reinterpret_cast<SFD_GLOBAL char *>(base) + ob) = v;
-}
-
-// an element of a table the kernel never writes, at an index the same for
-// every lane: read through the constant address space, i.e. by a scalar load
-// that does not join the vector-memory counter shared with the stores
-__device__ __forceinline__ float ro_uniform(const float *t, int idx) {
-  return ((const __attribute__((address_space(4))) float *)t)[idx];
-}
-__device__ __forceinline__ unsigned ro_uniform_u(const unsigned *t, int idx) {
-  return ((const __attribute__((address_space(4))) unsigned *)t)[idx];
-}
-
-// Field storage of the face passes: each field array holds fp32 values, or
-// binary16 values with a per-array scale.
-struct F4 {
-  float v[4];
-};
-
-template <class T> struct Store;
-// fp32 fields: plain 16-byte vectors (the scale arguments are unused)
-template <> struct Store<float> {
-  static __device__ __forceinline__ F4 ld4(const float *b, long long p, float) {
-    const float4 t = *reinterpret_cast<const float4 *>(b + p);
-    return {{t.x, t.y, t.z, t.w}};
-  }
-  static __device__ __forceinline__ float ld1(const float *b, long long p, float) { return b[p]; }
-  static __device__ __forceinline__ void st1(float *b, long long p, float, float v) { b[p] = v; }
-  static __device__ __forceinline__ float ld1(const SFD_GLOBAL float *b, long long p, float) {
-    return b[p];
-  }
-  static __device__ __forceinline__ void st1(SFD_GLOBAL float *b, long long p, float, float v) {
-    b[p] = v;
-  }
-  static __device__ __forceinline__ void st4(float *b, long long p, float, const F4 &v) {
-    *reinterpret_cast<float4 *>(b + p) = make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
-  }
-  // a plane base and the lane's byte offset in the plane; ldr/cvt split the
-  // load from the conversion so that a plane's loads all issue first
-  typedef float raw_t;
-  static __device__ __forceinline__ raw_t ldr(const SFD_GLOBAL char *b, unsigned ob) {
-    return ld_at((const SFD_GLOBAL float *)b, ob);
-  }
-  static __device__ __forceinline__ float cvt(raw_t r, float) { return r; }
-  static __device__ __forceinline__ float ldo(const SFD_GLOBAL char *b, unsigned ob, float) {
-    return ld_at((const SFD_GLOBAL float *)b, ob);
-  }
-  static __device__ __forceinline__ void sto(SFD_GLOBAL char *b, unsigned ob, float, float v) {
-    st_at((SFD_GLOBAL float *)b, ob, v);
-  }
-  // a value as it reads back after being stored by a pass, and by a source
-  static __device__ __forceinline__ float trip(float v, float, float) { return v; }
-  static __device__ __forceinline__ float trip_src(float v, float, float) { return v; }
-  static __device__ __forceinline__ void st_src(float *b, long long p, float, float v) { b[p] = v; }
-};
-// binary16 fields with a per-array scale: value = half * s, stored as
-// round(value / s); 8-byte vectors, fp32 arithmetic.  Every scale product is
-// rounded to fp32 on its own (an empty asm barrier keeps the compiler from
-// fusing it into the arithmetic that uses it, or into the conversion to
-// binary16 as a mixed-precision FMA, which would round once instead of
-// twice), so every kernel shape rounds alike.
-__device__ __forceinline__ float rounded(float x) {
-  asm("" : "+v"(x));
-  return x;
-}
-// A source launch of its own (fdtd_aux.hip) stores half(value / s) through the
-// mixed-precision FMA, one rounding; a source inside a pass stores the same.
-// (The result is read two cycles later: a partial register write.)
-__device__ __forceinline__ unsigned short half_src(float v, float is) {
-  unsigned r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\ts_nop 1" : "=v"(r) : "v"(is), "v"(v));
-  return (unsigned short)r;
-}
-template <> struct Store<__half> {
-  static __device__ __forceinline__ F4 ld4(const float *b, long long p, float s) {
-    const uint2 t = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(b) + p);
-    const float2 lo = __half22float2(*reinterpret_cast<const __half2 *>(&t.x));
-    const float2 hi = __half22float2(*reinterpret_cast<const __half2 *>(&t.y));
-    return {{rounded(lo.x * s), rounded(lo.y * s), rounded(hi.x * s), rounded(hi.y * s)}};
-  }
-  static __device__ __forceinline__ float ld1(const float *b, long long p, float s) {
-    return rounded(__half2float(reinterpret_cast<const __half *>(b)[p]) * s);
-  }
-  static __device__ __forceinline__ void st1(float *b, long long p, float is, float v) {
-    reinterpret_cast<__half *>(b)[p] = __float2half_rn(rounded(v * is));
-  }
-  static __device__ __forceinline__ float ld1(const SFD_GLOBAL float *b, long long p, float s) {
-    const unsigned short h = ((const SFD_GLOBAL unsigned short *)b)[p];
-    return rounded(__half2float(__ushort_as_half(h)) * s);
-  }
-  static __device__ __forceinline__ void st1(SFD_GLOBAL float *b, long long p, float is, float v) {
-    ((SFD_GLOBAL unsigned short *)b)[p] = __half_as_ushort(__float2half_rn(rounded(v * is)));
-  }
-  static __device__ __forceinline__ void st4(float *b, long long p, float is, const F4 &v) {
-    const __half2 lo = __floats2half2_rn(rounded(v.v[0] * is), rounded(v.v[1] * is));
-    const __half2 hi = __floats2half2_rn(rounded(v.v[2] * is), rounded(v.v[3] * is));
-    uint2 t;
-    t.x = *reinterpret_cast<const unsigned *>(&lo);
-    t.y = *reinterpret_cast<const unsigned *>(&hi);
-    *reinterpret_cast<uint2 *>(reinterpret_cast<__half *>(b) + p) = t;
-  }
-  typedef unsigned short raw_t;
-  static __device__ __forceinline__ raw_t ldr(const SFD_GLOBAL char *b, unsigned ob) {
-    return ld_at((const SFD_GLOBAL unsigned short *)b, ob);
-  }
-  static __device__ __forceinline__ float cvt(raw_t h, float s) {
-    return rounded(__half2float(__ushort_as_half(h)) * s);
-  }
-  static __device__ __forceinline__ float ldo(const SFD_GLOBAL char *b, unsigned ob, float s) {
-    return cvt(ldr(b, ob), s);
-  }
-  static __device__ __forceinline__ void sto(SFD_GLOBAL char *b, unsigned ob, float is, float v) {
-    st_at((SFD_GLOBAL unsigned short *)b, ob, __half_as_ushort(__float2half_rn(rounded(v * is))));
-  }
-  static __device__ __forceinline__ float trip(float v, float s, float is) {
-    return cvt(__half_as_ushort(__float2half_rn(rounded(v * is))), s);
-  }
-  static __device__ __forceinline__ float trip_src(float v, float s, float is) {
-    return cvt(half_src(v, is), s);
-  }
-  static __device__ __forceinline__ void st_src(float *b, long long p, float is, float v) {
-    reinterpret_cast<unsigned short *>(b)[p] = half_src(v, is);
-  }
-};
-
-// The column (i, j) of the tile's lane and the tile's z chunk bz.  Tiles are
-// 64-wide x segments of blockDim.y rows, or, in flat tile maps, runs of
-// 64 * blockDim.y consecutive columns of the x-y plane in x-fastest order
-// (grids whose nx + 1 is far from a multiple of 64 then leave no lane idle;
-// every neighbour of the face passes comes from memory, so a run may wrap
-// from one row to the next).  j > ny marks a lane past the plane.
-__device__ __forceinline__ void tile_column(const TileMap &tm, int blk, int nx, int &i, int &j,
-                                            int &bz) {
-  int bx, by;
-  decode_tile(tm, blk, bx, by, bz);
-  if (tm.flat) {
-    const int f = bx * kWave * (int)blockDim.y + (int)threadIdx.y * kWave + (int)threadIdx.x;
-    i = f % (nx + 1);
-    j = f / (nx + 1);
-  } else {
-    i = bx * kWave + threadIdx.x;
-    j = by * blockDim.y + threadIdx.y;
-  }
-}
-
-// The sources a pass applies inline (PassSrc; CPassSrc read through the
-// constant address space).  They cost a pass two loads per lane and tile and
-// one scalar load, one AND and one branch per plane; as kernels of their own
-// (three per half for a plane wave's face axes, one for nodal cells) they cost
-// a launch each, 4.4-9 us, and a second trip to memory for every face cell.
-typedef __attribute__((address_space(4))) PassSrc CPassSrc;
-
-// the address of face q's term at cell (i, j, k); fal: the faces in LDS
-__device__ __forceinline__ int term_index(const FaceAddr *fal, int q, int i, int j, int k) {
-  const FaceAddr a = fal[q];
-  return a.base + i * a.sx + j * a.sy + k * a.sz;
-}
-// the faces in bits applied to v in the reference's order; first: the first
-// face's term, loaded with the plane.  Binary16 storage rounds before and
-// after each face, as a launch of its own on the stored value would; what
-// comes back is a stored value, which the pass's store leaves as it is.
-template <class S>
-__device__ __forceinline__ float add_faces(unsigned bits, float first, const FaceAddr *fal,
-                                           const float *terms, int i, int j, int k, float v,
-                                           float s, float is) {
-  v = S::trip_src(S::trip(v, s, is) + first, s, is);
-  bits &= bits - 1;
-  while (bits) {
-    const int q = __builtin_ctz(bits);
-    bits &= bits - 1;
-    v = S::trip_src(v + terms[term_index(fal, q, i, j, k)], s, is);
-  }
-  return v;
-}
-// the first face's term of component bits (loaded ahead of its use)
-__device__ __forceinline__ float first_term(unsigned bits, const FaceAddr *fal,
-                                            const float *terms, int i, int j, int k) {
-  return bits ? terms[term_index(fal, __builtin_ctz(bits), i, j, k)] : 0.0f;
-}
-
-// LDS of the face addresses, behind the media table of tab bytes
-static __host__ __device__ __forceinline__ size_t face_lds_offset(size_t tab) {
-  return (tab + 15) & ~(size_t)15;
-}
-template <class PS>
-__device__ __forceinline__ const FaceAddr *stage_faces(const PS &x, float2 *lds, size_t tab) {
-  FaceAddr *f = reinterpret_cast<FaceAddr *>(reinterpret_cast<char *>(lds) + face_lds_offset(tab));
-  const int t = threadIdx.y * blockDim.x + threadIdx.x;
-  const FaceAddr *src = x.fa;
-  if (t < x.nface) f[t] = src[t];
-  return f;
-}
-
-// AdvanceNodalE/H on the cells of one tile, after its march: the block's own
-// stores are visible to it behind the barrier, and no other block writes the
-// tile's cells.  Every thread of the block calls this.
-template <class T, class PS>
-__device__ __forceinline__ void tile_nodal(const DevGrid &g, const TileMap &tm, const PS &x,
-                                           int blk) {
-  if (!x.nstart) return;
-  const int tile = tm.remap ? xcd_remap(blk, tm.nblk) : blk;
-  const int c0 = x.nstart[tile], c1 = x.nstart[tile + 1];
-  if (c0 >= c1) return;
-  __syncthreads();
-  const int t = threadIdx.y * blockDim.x + threadIdx.x, nt = blockDim.x * blockDim.y;
-  const int n = x.n + (x.dn ? *x.dn : 0);
-  // cells that share a field value run in order, on one thread
-  const int step = x.serial ? 1 : nt;
-  for (int c = x.serial ? (t == 0 ? c0 : c1) : c0 + t; c < c1; c += step) {
-    const NodalCell &cell = x.cells[c];
-    if (cell.skip) continue;
-    const float v = x.values[(long long)n * x.nsrc + cell.src];
-    float *f = g.f[cell.comp];
-    const float old = cell.hard ? 0.0f : Store<T>::ld1(f, cell.p, g.fs[cell.comp]);
-    Store<T>::st_src(f, cell.p, g.fi[cell.comp], nodal_apply(old, cell, v));
-  }
 }
 
 // one tile (64 x blockDim.y lanes, one z chunk) of the E face pass; T the
@@ -993,288 +597,6 @@ __device__ __forceinline__ void hpass_tile(const G &g, const TileMap &tm,
   }
 }
 
-// ---- four consecutive x cells per lane ------------------------------------
-// The fused passes move each field value with 16-byte (fp32) accesses: lane l
-// of a wave owns cells 4l..4l+3 of a 256-cell x segment.  The x neighbour one
-// cell down (E pass) or up (H pass) comes from the next lane by a cross-lane
-// shuffle, and from one extra load at the wave's edge.  The row pitch leaves
-// room for the last vector of a row, whose cells beyond the sweep are written
-// back unchanged.
-__device__ __forceinline__ void ld_mi4(const int16_t *m, long long p, int (&o)[4]) {
-  const short4 t = *reinterpret_cast<const short4 *>(m + p);
-  o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
-}
-
-// E face pass (Yee E + CPML E), four cells per lane
-template <bool TBL, class T>
-__device__ __forceinline__ void epass4_tile(const DevGrid &g, const TileMap &tm,
-                                            const MedTab &tab, int blk) {
-  int bx, by, bz;
-  decode_tile(tm, blk, bx, by, bz);
-  const int lane = threadIdx.x;
-  const int i0 = bx * (kWave * 4) + 4 * lane;
-  const int j = by * blockDim.y + threadIdx.y;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  if (j > ny) return;                       // whole wave: one row per wave
-  const bool live = i0 <= nx;               // lanes past the sweep only shuffle
-  const int k0 = bz * tm.kc;
-  const int k1 = min(k0 + tm.kc, nz + 1);
-  const long long px = g.px, pxy = g.pxy;
-  long long p = (long long)(k0 + 1) * pxy + (long long)(j + 1) * px + g.xoff + i0;
-  float *__restrict__ Ex = g.f[0];
-  float *__restrict__ Ey = g.f[1];
-  float *__restrict__ Ez = g.f[2];
-  const float *__restrict__ Hx = g.f[3];
-  const float *__restrict__ Hy = g.f[4];
-  const float *__restrict__ Hz = g.f[5];
-  F4 hx_km = {}, hy_km = {};
-  if (live) {
-    hx_km = Store<T>::ld4(Hx, p - pxy, g.fs[3]);
-    hy_km = Store<T>::ld4(Hy, p - pxy, g.fs[4]);
-  }
-  const float idyh = g.id[4][j + 1];
-  float idxh[4];
-  int qxn[4];
-  bool sxn[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int i = min(i0 + c, nx + 1);
-    idxh[c] = g.id[3][i + 1];
-    sxn[c] = slab_node(i0 + c, nx, g.L[0][0], g.L[0][1], qxn[c]);
-  }
-  int qyn = 0;
-  const bool syn = slab_node(j, ny, g.L[1][0], g.L[1][1], qyn);
-  const bool cy = j < ny;
-  const int Lx = g.L[0][0] + g.L[0][1], Ly = g.L[1][0] + g.L[1][1];
-  for (int k = k0; k < k1; ++k, p += pxy) {
-    const bool cz = k < nz;
-    const float idzh = g.id[5][k + 1];
-    F4 hx0 = {}, hy0 = {}, hz0 = {}, hz_jm = {}, hx_jm = {}, ex = {}, ey = {}, ez = {};
-    int mx[4] = {}, my[4] = {}, mz[4] = {};
-    float hz_edge = 0.0f, hy_edge = 0.0f;
-    if (live) {
-      hx0 = Store<T>::ld4(Hx, p, g.fs[3]); hy0 = Store<T>::ld4(Hy, p, g.fs[4]); hz0 = Store<T>::ld4(Hz, p, g.fs[5]);
-      hz_jm = Store<T>::ld4(Hz, p - px, g.fs[5]); hx_jm = Store<T>::ld4(Hx, p - px, g.fs[3]);
-      ex = Store<T>::ld4(Ex, p, g.fs[0]); ld_mi4(g.mi[0], p, mx);
-      if (cy) { ey = Store<T>::ld4(Ey, p, g.fs[1]); ld_mi4(g.mi[1], p, my); }
-      if (cz) { ez = Store<T>::ld4(Ez, p, g.fs[2]); ld_mi4(g.mi[2], p, mz); }
-      if (lane == 0) { hz_edge = Store<T>::ld1(Hz, p - 1, g.fs[5]); hy_edge = Store<T>::ld1(Hy, p - 1, g.fs[4]); }
-    }
-    // x - 1 neighbours: the previous lane's last cell
-    float hz_im[4], hy_im[4];
-    const float hz_up = __shfl_up(hz0.v[3], 1), hy_up = __shfl_up(hy0.v[3], 1);
-    hz_im[0] = lane == 0 ? hz_edge : hz_up;
-    hy_im[0] = lane == 0 ? hy_edge : hy_up;
-#pragma unroll
-    for (int c = 1; c < 4; ++c) { hz_im[c] = hz0.v[c - 1]; hy_im[c] = hy0.v[c - 1]; }
-    int qzn = 0;
-    const bool szn = slab_node(k, nz, g.L[2][0], g.L[2][1], qzn);
-    if (live) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int i = i0 + c;
-        if (i < nx) {  // Ex sweep x[0,nx-1]
-          float e = ex.v[c];
-          const float2 cf = coef<TBL>(tab, g.g1, g.g2, mx[c]);
-          e = yee_upd(cf.x, e, cf.y, curl2(hz0.v[c] - hz_jm.v[c], idyh, hy0.v[c] - hy_km.v[c], idzh));
-          if (syn) {  // psi_Exy, left/right (borderscpml.F90:609-623)
-            const long long s = ((long long)k * Ly + qyn) * nx + i;
-            e = madd(e, cf.y, psi_step(g.psi[PSI_EXY], s, g.pbe[1][j + 1], hz0.v[c] - hz_jm.v[c],
-                                    g.pce[1][j + 1]));
-          }
-          if (szn) {  // psi_Exz, down/up (:699-712)
-            const long long s = ((long long)qzn * (ny + 1) + j) * nx + i;
-            e = madd(e, -cf.y, psi_step(g.psi[PSI_EXZ], s, g.pbe[2][k + 1], hy0.v[c] - hy_km.v[c],
-                                    g.pce[2][k + 1]));
-          }
-          ex.v[c] = e;
-        }
-        if (cy && i <= nx) {  // Ey sweep x[0,nx] y[0,ny-1]
-          float e = ey.v[c];
-          const float2 cf = coef<TBL>(tab, g.g1, g.g2, my[c]);
-          e = yee_upd(cf.x, e, cf.y, curl2(hx0.v[c] - hx_km.v[c], idzh, hz0.v[c] - hz_im[c], idxh[c]));
-          if (szn) {  // psi_Eyz, down/up (:680-693)
-            const long long s = ((long long)qzn * ny + j) * (nx + 1) + i;
-            e = madd(e, cf.y, psi_step(g.psi[PSI_EYZ], s, g.pbe[2][k + 1], hx0.v[c] - hx_km.v[c],
-                                    g.pce[2][k + 1]));
-          }
-          if (sxn[c]) {  // psi_Eyx, back/front (:790-802)
-            const long long s = ((long long)k * ny + j) * Lx + qxn[c];
-            e = madd(e, -cf.y, psi_step(g.psi[PSI_EYX], s, g.pbe[0][i + 1], hz0.v[c] - hz_im[c],
-                                    g.pce[0][i + 1]));
-          }
-          ey.v[c] = e;
-        }
-        if (cz && i <= nx) {  // Ez sweep x[0,nx] z[0,nz-1]
-          float e = ez.v[c];
-          const float2 cf = coef<TBL>(tab, g.g1, g.g2, mz[c]);
-          e = yee_upd(cf.x, e, cf.y, curl2(hy0.v[c] - hy_im[c], idxh[c], hx0.v[c] - hx_jm.v[c], idyh));
-          if (syn) {  // psi_Ezy, left/right (:630-642)
-            const long long s = ((long long)k * Ly + qyn) * (nx + 1) + i;
-            e = madd(e, -cf.y, psi_step(g.psi[PSI_EZY], s, g.pbe[1][j + 1], hx0.v[c] - hx_jm.v[c],
-                                    g.pce[1][j + 1]));
-          }
-          if (sxn[c]) {  // psi_Ezx, back/front (:771-783)
-            const long long s = ((long long)k * (ny + 1) + j) * Lx + qxn[c];
-            e = madd(e, cf.y, psi_step(g.psi[PSI_EZX], s, g.pbe[0][i + 1], hy0.v[c] - hy_im[c],
-                                    g.pce[0][i + 1]));
-          }
-          ez.v[c] = e;
-        }
-      }
-      Store<T>::st4(Ex, p, g.fi[0], ex);
-      if (cy) Store<T>::st4(Ey, p, g.fi[1], ey);
-      if (cz) Store<T>::st4(Ez, p, g.fi[2], ez);
-    }
-    hx_km = hx0;
-    hy_km = hy0;
-  }
-}
-
-// H face pass (Yee H + CPML H), four cells per lane
-template <bool TBL, class T>
-__device__ __forceinline__ void hpass4_tile(const DevGrid &g, const TileMap &tm,
-                                            const MedTab &tab, int blk) {
-  int bx, by, bz;
-  decode_tile(tm, blk, bx, by, bz);
-  const int lane = threadIdx.x;
-  const int i0 = bx * (kWave * 4) + 4 * lane;
-  const int j = by * blockDim.y + threadIdx.y;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  if (j > ny) return;
-  const bool live = i0 <= nx;
-  const int k0 = bz * tm.kc;
-  const int k1 = min(k0 + tm.kc, nz + 1);
-  const long long px = g.px, pxy = g.pxy;
-  long long p = (long long)(k0 + 1) * pxy + (long long)(j + 1) * px + g.xoff + i0;
-  const float *__restrict__ Ex = g.f[0];
-  const float *__restrict__ Ey = g.f[1];
-  const float *__restrict__ Ez = g.f[2];
-  float *__restrict__ Hx = g.f[3];
-  float *__restrict__ Hy = g.f[4];
-  float *__restrict__ Hz = g.f[5];
-  const float idye = g.id[1][j + 1];
-  float idxe[4];
-  int qxc[4];
-  bool sxc[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int i = min(i0 + c, nx + 1);
-    idxe[c] = g.id[0][i + 1];
-    sxc[c] = slab_cell(i0 + c, nx, g.L[0][0], g.L[0][1], qxc[c]);
-  }
-  int qyc = 0;
-  const bool syc = slab_cell(j, ny, g.L[1][0], g.L[1][1], qyc);
-  const bool cy = j < ny;
-  const int Lx = g.L[0][0] + g.L[0][1], Ly = g.L[1][0] + g.L[1][1];
-  F4 ex_c = {}, ey_c = {};
-  if (live) { ex_c = Store<T>::ld4(Ex, p, g.fs[0]); ey_c = Store<T>::ld4(Ey, p, g.fs[1]); }
-  for (int k = k0; k < k1; ++k, p += pxy) {
-    const float idze = g.id[2][k + 1];
-    const bool cz = k < nz;
-    F4 ex_kp = {}, ey_kp = {}, ez_c = {}, ez_jp = {}, ex_jp = {}, hx = {}, hy = {}, hz = {};
-    int mx[4] = {}, my[4] = {}, mz[4] = {};
-    float ez_edge = 0.0f, ey_edge = 0.0f;
-    if (live) {
-      ex_kp = Store<T>::ld4(Ex, p + pxy, g.fs[0]); ey_kp = Store<T>::ld4(Ey, p + pxy, g.fs[1]);
-      ez_c = Store<T>::ld4(Ez, p, g.fs[2]);
-      ez_jp = Store<T>::ld4(Ez, p + px, g.fs[2]); ex_jp = Store<T>::ld4(Ex, p + px, g.fs[0]);
-      if (cy && cz) { hx = Store<T>::ld4(Hx, p, g.fs[3]); ld_mi4(g.mi[3], p, mx); }
-      if (cz) { hy = Store<T>::ld4(Hy, p, g.fs[4]); ld_mi4(g.mi[4], p, my); }
-      if (cy) { hz = Store<T>::ld4(Hz, p, g.fs[5]); ld_mi4(g.mi[5], p, mz); }
-      if (lane == kWave - 1) { ez_edge = Store<T>::ld1(Ez, p + 4, g.fs[2]); ey_edge = Store<T>::ld1(Ey, p + 4, g.fs[1]); }
-    }
-    // x + 1 neighbours: the next lane's first cell
-    float ez_ip[4], ey_ip[4];
-    const float ez_dn = __shfl_down(ez_c.v[0], 1), ey_dn = __shfl_down(ey_c.v[0], 1);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) { ez_ip[c] = ez_c.v[c + 1]; ey_ip[c] = ey_c.v[c + 1]; }
-    ez_ip[3] = lane == kWave - 1 ? ez_edge : ez_dn;
-    ey_ip[3] = lane == kWave - 1 ? ey_edge : ey_dn;
-    int qzc = 0;
-    const bool szc = slab_cell(k, nz, g.L[2][0], g.L[2][1], qzc);
-    if (live) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int i = i0 + c;
-        if (cy && cz && i <= nx) {  // Hx sweep: x[0,nx] y[0,ny-1] z[0,nz-1]
-          const float2 cf = coef<TBL>(tab, g.gm1, g.gm2, mx[c]);
-          float h = hx.v[c];
-          h = yee_upd(cf.x, h, cf.y, curl2(ey_kp.v[c] - ey_c.v[c], idze, ez_jp.v[c] - ez_c.v[c], idye));
-          if (syc) {  // psi_Hxy (borderscpml.F90:911-921)
-            const long long s = ((long long)k * Ly + qyc) * (nx + 1) + i;
-            h = madd(h, -cf.y, psi_step(g.psi[PSI_HXY], s, g.pbm[1][j + 1], ez_jp.v[c] - ez_c.v[c],
-                                    g.pcm[1][j + 1]));
-          }
-          if (szc) {  // psi_Hxz (:1021-1031)
-            const long long s = ((long long)qzc * ny + j) * (nx + 1) + i;
-            h = madd(h, cf.y, psi_step(g.psi[PSI_HXZ], s, g.pbm[2][k + 1], ey_kp.v[c] - ey_c.v[c],
-                                    g.pcm[2][k + 1]));
-          }
-          hx.v[c] = h;
-        }
-        if (cz && i < nx) {  // Hy sweep: x[0,nx-1] y[0,ny] z[0,nz-1]
-          const float2 cf = coef<TBL>(tab, g.gm1, g.gm2, my[c]);
-          float h = hy.v[c];
-          h = yee_upd(cf.x, h, cf.y, curl2(ez_ip[c] - ez_c.v[c], idxe[c], ex_kp.v[c] - ex_c.v[c], idze));
-          if (szc) {  // psi_Hyz (:1001-1011)
-            const long long s = ((long long)qzc * (ny + 1) + j) * nx + i;
-            h = madd(h, -cf.y, psi_step(g.psi[PSI_HYZ], s, g.pbm[2][k + 1], ex_kp.v[c] - ex_c.v[c],
-                                    g.pcm[2][k + 1]));
-          }
-          if (sxc[c]) {  // psi_Hyx (:1111-1121)
-            const long long s = ((long long)k * (ny + 1) + j) * Lx + qxc[c];
-            h = madd(h, cf.y, psi_step(g.psi[PSI_HYX], s, g.pbm[0][i + 1], ez_ip[c] - ez_c.v[c],
-                                    g.pcm[0][i + 1]));
-          }
-          hy.v[c] = h;
-        }
-        if (cy && i < nx) {  // Hz sweep: x[0,nx-1] y[0,ny-1] z[0,nz]
-          const float2 cf = coef<TBL>(tab, g.gm1, g.gm2, mz[c]);
-          float h = hz.v[c];
-          h = yee_upd(cf.x, h, cf.y, curl2(ex_jp.v[c] - ex_c.v[c], idye, ey_ip[c] - ey_c.v[c], idxe[c]));
-          if (syc) {  // psi_Hzy (:931-941)
-            const long long s = ((long long)k * Ly + qyc) * nx + i;
-            h = madd(h, cf.y, psi_step(g.psi[PSI_HZY], s, g.pbm[1][j + 1], ex_jp.v[c] - ex_c.v[c],
-                                    g.pcm[1][j + 1]));
-          }
-          if (sxc[c]) {  // psi_Hzx (:1091-1101)
-            const long long s = ((long long)k * ny + j) * Lx + qxc[c];
-            h = madd(h, -cf.y, psi_step(g.psi[PSI_HZX], s, g.pbm[0][i + 1], ey_ip[c] - ey_c.v[c],
-                                    g.pcm[0][i + 1]));
-          }
-          hz.v[c] = h;
-        }
-      }
-      if (cy && cz) Store<T>::st4(Hx, p, g.fi[3], hx);
-      if (cz) Store<T>::st4(Hy, p, g.fi[4], hy);
-      if (cy) Store<T>::st4(Hz, p, g.fi[5], hz);
-    }
-    ex_c = ex_kp;
-    ey_c = ey_kp;
-  }
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_epass4(DevGrid g, TileMap tm) {
-  extern __shared__ float2 lds_tab[];
-  const MedTab tab = stage_tables<true, false>(g, g.g1, g.g2, lds_tab);
-  epass4_tile<true, T>(g, tm, tab, blockIdx.x);
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_hpass4(DevGrid g, TileMap tm) {
-  extern __shared__ float2 lds_tab[];
-  const MedTab tab = stage_tables<true, false>(g, g.gm1, g.gm2, lds_tab);
-  hpass4_tile<true, T>(g, tm, tab, blockIdx.x);
-}
-
-// the tile's word (see kTileFaces) and its medium or -1
-__device__ __forceinline__ int tile_info(const int *tmed) {
-  return tmed ? __builtin_amdgcn_readfirstlane(tmed[blockIdx.x]) : 0;
-}
-__device__ __forceinline__ int tile_medium(int info) { return (info & 0xffff) - 1; }
-
 template <bool YEE, bool CPML, bool TBL, class T = float>
 __global__ void __launch_bounds__(256) k_epass(DevGrid g, TileMap tm, const int *tmed) {
   extern __shared__ float2 lds_tab[];
@@ -1383,27 +705,7 @@ int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out, void *
 // batch: block b takes tiles b, b + gridDim.x, ...; the grid of a tile is
 // found by binary search in the prefix of tile counts, its media tables are
 // staged in LDS before the tile runs.
-// a tile map read word by word through the constant address space (scalar
-// loads; the maps never change during a launch)
-__device__ __forceinline__ TileMap const_tilemap(const TileMap *t) {
-  static_assert(sizeof(TileMap) % sizeof(int) == 0, "TileMap holds ints only");
-  typedef const __attribute__((address_space(4))) int CInt;
-  TileMap m;
-  int *o = reinterpret_cast<int *>(&m);
-  for (int q = 0; q < (int)(sizeof(TileMap) / sizeof(int)); ++q) o[q] = ((CInt *)t)[q];
-  return m;
-}
-
-__device__ __forceinline__ int batch_grid(const int *start, int ngrid, int t) {
-  int lo = 0, hi = ngrid - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] <= t) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-template <bool H, class T, int VEC, bool X>
+template <bool H, class T, bool X>
 __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
   extern __shared__ float2 lds_tab[];
   for (int t = blockIdx.x; t < bd.total; t += gridDim.x) {
@@ -1425,37 +727,31 @@ __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
     // the CPML variant serves grids without CPML too: with no slab layers
     // no cell of the sweep falls in a slab
     const int blk = t - bd.start[b];
-    if (VEC == 4) {
-      if (H) hpass4_tile<true, T>(g, tm, tab, blk);
-      else epass4_tile<true, T>(g, tm, tab, blk);
-    } else {
-      // a tile whose cells all hold one medium skips the media loads
-      const int m0 = bd.tmed ? __builtin_amdgcn_readfirstlane(bd.tmed[t]) : -1;
-      if (H) hpass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
-      else epass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
-      if (X) tile_nodal<T>(g, tm, *xs, blk);
-    }
+    // a tile whose cells all hold one medium skips the media loads
+    const int m0 = bd.tmed ? __builtin_amdgcn_readfirstlane(bd.tmed[t]) : -1;
+    if (H) hpass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
+    else epass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
+    if (X) tile_nodal<T>(g, tm, *xs, blk);
   }
 }
 
 int launch_pass_batch(const BatchDev &bd, int half, int blocks, int rows, int vec, size_t lds,
                       int fp16, void *stream) {
   if (bd.total <= 0) return 0;
+  if (vec == 4) return launch_quad_batch(bd, half, blocks, rows, lds, fp16, stream);
   const dim3 blk(kWave, (unsigned)rows);
   hipStream_t s = (hipStream_t)stream;
-  const bool x = vec != 4 && bd.src[half ? 1 : 0];
+  const bool x = bd.src[half ? 1 : 0];
   if (x) lds = face_lds_offset(lds) + kPassFaces * sizeof(FaceAddr);
-#define SFD_B(T, V, X)                                                                       \
-  do {                                                                                       \
-    if (half) hipLaunchKernelGGL((k_pass_batch<true, T, V, X>), dim3(blocks), blk, lds, s, bd); \
-    else hipLaunchKernelGGL((k_pass_batch<false, T, V, X>), dim3(blocks), blk, lds, s, bd);  \
+#define SFD_B(T, X)                                                                       \
+  do {                                                                                    \
+    if (half) hipLaunchKernelGGL((k_pass_batch<true, T, X>), dim3(blocks), blk, lds, s, bd); \
+    else hipLaunchKernelGGL((k_pass_batch<false, T, X>), dim3(blocks), blk, lds, s, bd);  \
   } while (0)
-  if (fp16 && vec == 4) SFD_B(__half, 4, false);
-  else if (fp16 && x) SFD_B(__half, 1, true);
-  else if (fp16) SFD_B(__half, 1, false);
-  else if (vec == 4) SFD_B(float, 4, false);
-  else if (x) SFD_B(float, 1, true);
-  else SFD_B(float, 1, false);
+  if (fp16 && x) SFD_B(__half, true);
+  else if (fp16) SFD_B(__half, false);
+  else if (x) SFD_B(float, true);
+  else SFD_B(float, false);
 #undef SFD_B
   return (int)hipGetLastError();
 }
@@ -1510,7 +806,7 @@ int launch_ade_many(const DevGrid *grids, const int *list, int n, int side, size
   return (int)hipGetLastError();
 }
 
-int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int *tmed, int yee,
+int launch_e(const DevGrid &g, const TileMap &tm, const int *tmed, int yee,
              int cpml, int ade, const PassSrc *src, void *stream) {
   const dim3 blk(kWave, (unsigned)tm.bdy);
   hipStream_t s = (hipStream_t)stream;
@@ -1524,7 +820,7 @@ int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
     else                                                                       \
       hipLaunchKernelGGL((k_epass<Y, C, false>), dim3(nb), blk, 0, s, g, tm, tmed); \
   } while (0)
-  if (src && yee && cpml && tm4.vec != 4) {
+  if (src && yee && cpml) {
     // the fused one-cell pass with its sources inline
     const size_t tb = tbl ? lds : 0, lx = face_lds_offset(tb) + kPassFaces * sizeof(FaceAddr);
     if (g.fp16)
@@ -1533,11 +829,6 @@ int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
       hipLaunchKernelGGL((k_epass_src<true, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
     else
       hipLaunchKernelGGL((k_epass_src<false, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, 0u);
-  } else if (yee && cpml && tbl && tm4.vec == 4) {
-    // fused pass, four cells per lane (the CPML variant also serves grids
-    // without CPML)
-    if (g.fp16) hipLaunchKernelGGL(k_epass4<__half>, dim3(tm4.nblk), blk, lds, s, g, tm4);
-    else hipLaunchKernelGGL(k_epass4<float>, dim3(tm4.nblk), blk, lds, s, g, tm4);
   } else if (g.fp16 && yee && cpml && tbl) {
     // binary16 storage, one cell per lane (the set-up admits binary16 only
     // with the fused Yee + CPML pass and LDS tables)
@@ -1550,7 +841,7 @@ int launch_e(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
   return (int)hipGetLastError();
 }
 
-int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int *tmed, int yee,
+int launch_h(const DevGrid &g, const TileMap &tm, const int *tmed, int yee,
              int cpml, int ade, const PassSrc *src, void *stream) {
   const dim3 blk(kWave, (unsigned)tm.bdy);
   hipStream_t s = (hipStream_t)stream;
@@ -1564,7 +855,7 @@ int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
     else                                                                       \
       hipLaunchKernelGGL((k_hpass<Y, C, false>), dim3(nb), blk, 0, s, g, tm, tmed); \
   } while (0)
-  if (src && yee && cpml && tm4.vec != 4) {
+  if (src && yee && cpml) {
     // the fused one-cell pass with its sources inline
     const size_t tb = tbl ? lds : 0, lx = face_lds_offset(tb) + kPassFaces * sizeof(FaceAddr);
     if (g.fp16)
@@ -1573,9 +864,6 @@ int launch_h(const DevGrid &g, const TileMap &tm, const TileMap &tm4, const int 
       hipLaunchKernelGGL((k_hpass_src<true, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, (unsigned)tb);
     else
       hipLaunchKernelGGL((k_hpass_src<false, float>), dim3(nb), blk, lx, s, g, tm, tmed, *src, 0u);
-  } else if (yee && cpml && tbl && tm4.vec == 4) {
-    if (g.fp16) hipLaunchKernelGGL(k_hpass4<__half>, dim3(tm4.nblk), blk, lds, s, g, tm4);
-    else hipLaunchKernelGGL(k_hpass4<float>, dim3(tm4.nblk), blk, lds, s, g, tm4);
   } else if (g.fp16 && yee && cpml && tbl) {
     hipLaunchKernelGGL((k_hpass<true, true, true, __half>), dim3(nb), blk, lds, s, g, tm, tmed);
   } else if (yee && cpml) SFD_H(true, true);
@@ -2273,28 +1561,6 @@ __global__ void __launch_bounds__(64 * R) k_step_many(const StepDev *__restrict_
 // wave shifts, lane 0's H at x0 - 1 is a scalar load.  Rows exchange E
 // through LDS as in k_step.  Per cell the arithmetic and its order are
 // k_step's, so the results are the same bits.
-
-// 16-byte and 8-byte vectors as the compiler's own vector types (these load
-// and store through global-address-space pointers)
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ f32x4 v4(float a, float b, float c, float d) {
-  f32x4 r;
-  r.x = a; r.y = b; r.z = c; r.w = d;
-  return r;
-}
-
-// lane l receives lane l - 1's v (wave_shr:1); lane 0 receives first
-__device__ __forceinline__ float from_left(float v, float first) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, first),
-                                                               __builtin_bit_cast(int, v), 0x138,
-                                                               0xf, 0xf, false));
-}
-// lane l receives lane l + 1's v (wave_shl:1); lane 63 receives 0
-__device__ __forceinline__ float from_right(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                               0x130, 0xf, 0xf, false));
-}
 
 // the four media indices of a lane's cells, from the 8-bit copies (one
 // dword) or the int16 arrays (two dwords)
