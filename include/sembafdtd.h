@@ -160,8 +160,12 @@ int fdtd_add_planewave(fdtd_handle *h, const int32_t box[6], int32_t nmodes, con
  * reference (its loops are OpenMP over k); chosen by the autotuner
  * (semba_fdtd_amd.tuning) or left at the default by grid depth: 2 rows x 4
  * planes up to 160 planes (nz + 1), 4 x 8 up to 640, 4 x 16 beyond; 1 cell.
- * Either storage runs either.  fdtd_get_tiling returns the
- * values as set (a chunk longer than the grid runs as the whole grid). */
+ * Until fdtd_set_tiling is called the fused passes choose by themselves: four
+ * cells per lane and 1 row x 1 or 2 planes by the grid's size wherever the
+ * media fit LDS and the x slabs leave four cells between them; the default
+ * values above are the other passes'.  Either storage runs either.
+ * fdtd_get_tiling returns the values as set (a chunk longer than the grid runs
+ * as the whole grid). */
 int fdtd_set_tiling(fdtd_handle *h, int32_t rows, int32_t zchunk, int32_t xcells);
 int fdtd_get_tiling(const fdtd_handle *h, int32_t *rows, int32_t *zchunk, int32_t *xcells);
 
@@ -394,11 +398,13 @@ int fdtd_batch_admit(fdtd_batch *b, fdtd_handle *h, int32_t n0, int32_t *slot);
 int fdtd_batch_retire(fdtd_batch *b, int32_t slot);
 /* Step the grid of slot will run next (-1 for an empty slot). */
 int64_t fdtd_batch_step_of(const fdtd_batch *b, int32_t slot);
-/* Tiling of the batched face passes (rows 1, 2 or 4; zchunk planes; xcells 1:
- * one cell per lane, each block taking a run of 64 * rows consecutive columns
- * of a grid's x-y plane, x fastest, so that narrow grids leave no lane idle;
- * xcells 4: four x cells per lane over 256-cell x segments) and the
- * persistent launch's block count (0: 16384).  Either storage runs either. */
+/* Tiling of the batched face passes (rows 1, 2 or 4; zchunk planes).  xcells 4:
+ * four x cells per lane, each block taking a run of 64 * rows consecutive
+ * four-cell vectors of a grid's x-y plane.  xcells 1: the passes choose rows
+ * and planes by the batch's size and run four cells per lane where every grid
+ * can; else one cell per lane, each block taking a run of 64 * rows consecutive
+ * columns, x fastest, with the persistent launch's block count (0: 16384).
+ * Either storage runs either. */
 int fdtd_batch_set_tiling(fdtd_batch *b, int32_t rows, int32_t zchunk, int32_t xcells,
                           int32_t blocks);
 /* One launch per step for the batch (rows 4, 8 or 16; 0: the face passes

@@ -37,9 +37,11 @@ class Batch:
 
     def set_tiling(self, rows: int, zchunk: int, blocks: int = 0, xcells: int = 1):
         """Blocks of 64 x rows threads marching zchunk z planes, xcells x
-        cells per lane (1: each block takes a run of 64 * rows consecutive
-        columns of a grid's x-y plane; 4: 256-cell x segments), and the
-        persistent launch's block count (0: 16384)."""
+        cells per lane (4: each block takes a run of 64 * rows consecutive
+        four-cell vectors of a grid's x-y plane; 1: the passes choose rows and
+        planes by the batch's size and run four cells per lane where every
+        grid can, else runs of 64 * rows columns), and the one-cell passes'
+        persistent block count (0: 16384)."""
         self._ck(self.lib.fdtd_batch_set_tiling(self.b, rows, zchunk, xcells, blocks),
                  "fdtd_batch_set_tiling")
 

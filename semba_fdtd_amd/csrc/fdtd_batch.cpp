@@ -67,6 +67,7 @@ struct fdtd_batch {
   std::vector<unsigned> version;      // each grid's state version at the last build
   int rows = 4, zchunk = 16, xcells = 1, blocks = 0;
   bool quads = false;                 // the passes run four cells per lane
+  int prows = 4;                      // rows per block of the passes
   // device descriptors, rebuilt when the membership changes
   bool ready = false;
   std::vector<void *> allocs;
@@ -172,15 +173,15 @@ int bupload(fdtd_batch *b, T **dst, const T *src, size_t n, std::vector<void *> 
   return FDTD_OK;
 }
 
-// tile map of one grid under the batch's tiling: runs of 64 * rows columns
-// (one cell per lane) or vectors (four) of the x-y plane, x fastest, which
-// leave no lane idle on grids a few tens of cells wide
+// one-cell tile map of one grid under the batch's tiling: runs of 64 * rows
+// columns of the x-y plane, x fastest, which leave no lane idle on grids a few
+// tens of cells wide
 TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
   TileMap tm{};
   tm.bdy = b->rows;
-  const long long cols = (long long)(b->quads ? g.nx / 4 + 1 : g.nx + 1) * (g.ny + 1);
+  const long long cols = (long long)(g.nx + 1) * (g.ny + 1);
   const long long per = (long long)kWave * b->rows;
-  tm.vec = b->quads ? 4 : 1;
+  tm.vec = 1;
   tm.flat = 1;
   tm.tx = (int)((cols + per - 1) / per);
   tm.ty = 1;
@@ -189,6 +190,16 @@ TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
   tm.nblk = tm.tx * tm.ty * tm.tz;
   tm.remap = 0;
   return tm;
+}
+
+// The four-cell tiles of one grid, under the batch's tiling if it was set with
+// xcells 4.  Else one row per block, and as many planes as still leave the chip
+// enough blocks, by the cells of all grids: 256 grids of 95 M cells run 2318,
+// 2212, 2276 us a step with 1, 2, 4 planes, 64 binary16 ones of 24 M cells 571,
+// 489, 459 us; six grids of 1.5 M cells fill it with one plane only.
+QuadLayout batch_quads(const fdtd_batch *b, const fdtd_handle *h, double cells) {
+  if (b->xcells == 4) return plan_quads(h, b->rows, b->zchunk);
+  return plan_quads(h, 1, cells < 1.5e6 ? 1 : b->fp16 && cells > 1e7 ? 4 : 2);
 }
 
 int build_descriptors(fdtd_batch *b) {
@@ -201,9 +212,16 @@ int build_descriptors(fdtd_batch *b) {
   size_t lds = 16;
   int maxwaves = 0;
   int rc;
-  b->quads = b->xcells == 4;
+  // four cells per lane where every grid can (256 uneven grids 2570 -> 2212 us
+  // a step); a tiling with xcells 4 sets their rows and planes, with xcells 1
+  // those of the one-cell passes
+  b->quads = true;
   for (fdtd_handle *h : b->slots)
     if (h && !quads_fit(h)) b->quads = false;
+  std::vector<QuadLayout> quad;
+  double cells = 0.0;
+  for (fdtd_handle *h : b->slots)
+    if (h) cells += (double)h->g.nx * h->g.ny * h->g.nz;
   for (size_t s = 0; s < b->slots.size(); ++s) {
     fdtd_handle *h = b->slots[s];
     if (!h) continue;
@@ -212,9 +230,11 @@ int build_descriptors(fdtd_batch *b) {
     b->version[s] = h->version;
     grids.push_back(h->g);
     tms.push_back(batch_tiles(b, h->g));
-    if ((long long)start.back() + tms.back().nblk > 0x7fffffffLL)
+    if (b->quads) quad.push_back(batch_quads(b, h, cells));
+    const int nblk = b->quads ? quad.back().p.nblk : tms.back().nblk;
+    if ((long long)start.back() + nblk > 0x7fffffffLL)
       return bfail(b, FDTD_ERR_ARG, "batch holds too many tiles");
-    start.push_back(start.back() + tms.back().nblk);
+    start.push_back(start.back() + nblk);
     counters.push_back(h->dstep);
     lds = std::max(lds, (size_t)(h->g.nmedia + 1) * 12);
     maxwaves = std::max(maxwaves, (int)h->pwin.size());
@@ -243,7 +263,10 @@ int build_descriptors(fdtd_batch *b) {
   }
   b->ncounters = (int)counters.size();
   b->lds = lds;
-  // the sources the one-cell passes apply inline
+  b->prows = b->quads ? (quad.empty() ? 1 : quad[0].rows) : b->rows;
+  b->bd.qtiles = nullptr;
+  std::vector<int> words(b->quads ? (size_t)b->bd.total : 0, 0);
+  // the sources the passes apply inline
   {
     std::vector<PwTermsGrid> terms;
     std::vector<PassSrc> src[2];
@@ -253,14 +276,16 @@ int build_descriptors(fdtd_batch *b) {
       b->bd.src[half] = nullptr;
     }
     int gi = 0;
-    for (size_t s = 0; s < b->slots.size() && !b->quads; ++s) {
+    for (size_t s = 0; s < b->slots.size(); ++s) {
       fdtd_handle *h = b->slots[s];
       if (!h) continue;
       bool faces = false;
       for (int half = 0; half < 2; ++half) {
         PassSrc ps;
         bool on = false;
-        if ((rc = make_pass_src(h, tms[(size_t)gi], half, &ps, &on, &b->allocs, nullptr)))
+        rc = b->quads ? make_quad_src(h, quad[(size_t)gi], half, &ps, &on, &b->allocs, &words[(size_t)start[(size_t)gi]])
+                      : make_pass_src(h, tms[(size_t)gi], half, &ps, &on, &b->allocs, nullptr);
+        if (rc)
           return bfail(b, rc, "slot %zu: %s", s, h->err.c_str());
         ps.dn = h->dstep;
         b->inl[half][s] = on ? 1 : 0;
@@ -284,6 +309,37 @@ int build_descriptors(fdtd_batch *b) {
     b->dterms = nullptr;
     if (!terms.empty() && (rc = bupload(b, &b->dterms, terms.data(), terms.size()))) return rc;
     // (the uploads read these vectors until the stream has run them)
+    BCHK(b, hipStreamSynchronize(b->stream));
+  }
+  // the four-cell passes' tiles: grid after grid, a grid's boxes in order
+  if (b->quads && b->bd.total > 0) {
+    std::vector<QuadTile> tiles((size_t)b->bd.total);
+    std::vector<QuadBox> boxes(quad.size() * kQuadBoxes);
+    int q = 0;
+    for (size_t g = 0; g < quad.size(); ++g) {
+      const QuadPlan &p = quad[g].p;
+      int x = 0;
+      for (int t = 0; t < p.nblk; ++t, ++q) {
+        while (x + 1 < p.nbox && t >= p.start[x + 1]) ++x;
+        const bool slabs = quad[g].slabs == kSlabAll || (quad[g].slabs == kSlabMix && x > 0);
+        QuadTile &o = tiles[(size_t)q];
+        o = QuadTile{};
+        o.grid = (int)g;
+        o.box = (int)g * kQuadBoxes + x;
+        o.t = t - p.start[x];
+        o.tg = t;
+        o.info = words[(size_t)q] | (slabs ? kTileSlabs : 0);
+      }
+      std::copy(p.box, p.box + kQuadBoxes, boxes.begin() + (long)g * kQuadBoxes);
+    }
+    QuadBox *db = nullptr;
+    if ((rc = bupload(b, &b->bd.qtiles, tiles.data(), tiles.size())) ||
+        (rc = bupload(b, &db, boxes.data(), boxes.size())))
+      return rc;
+    b->bd.qboxes = db;
+    const int e = b->mode == FDTD_MODE_EXACT ? exact::launch_quad_media_batch(b->bd, b->prows, b->stream)
+                                             : fast::launch_quad_media_batch(b->bd, b->prows, b->stream);
+    if (e) return bfail(b, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
     BCHK(b, hipStreamSynchronize(b->stream));
   }
   // pole stage and probes: one launch each for the whole batch
@@ -504,9 +560,8 @@ int launch_step(fdtd_batch *b) {
   const int blocks = b->blocks > 0 ? b->blocks : 16384;
   int e, rc;
   for (int half = 0; half < 2; ++half) {
-    const int vec = b->quads ? 4 : 1;
-    e = exact ? exact::launch_pass_batch(b->bd, half, blocks, b->rows, vec, b->lds, 0, b->stream)
-              : fast::launch_pass_batch(b->bd, half, blocks, b->rows, vec, b->lds, b->fp16,
+    e = exact ? exact::launch_pass_batch(b->bd, half, blocks, b->prows, b->lds, 0, b->stream)
+              : fast::launch_pass_batch(b->bd, half, blocks, b->prows, b->lds, b->fp16,
                                         b->stream);
     if (e) return bfail(b, FDTD_ERR_HIP, "batch face pass failed: %s", hipGetErrorString((hipError_t)e));
     // the pole stage of every grid with poles on this field follows the face

@@ -42,6 +42,13 @@ struct PwGroup {
   long long *dstart = nullptr;
 };
 
+// the tiles of the four-cell passes: boxes, the slabs they meet (launch_quad),
+// rows per block, planes per tile
+struct QuadLayout {
+  QuadPlan p = {};
+  int slabs = 0, rows = 1, kc = 1;
+};
+
 struct PlaneWaveIn {     // sgg%PlaneWave(j) (planeonde_t, fdetypes.F90:458-465)
   int esq[6];            // esqx1, esqx2, esqy1, esqy2, esqz1, esqz2
   int nmodes;
@@ -179,12 +186,9 @@ struct fdtd_handle {
   int *tmed = nullptr;
   int tmed_cap = 0;
   bool tmed_ready = false;
-  // the four-cell passes' tiles: boxes, the slabs they meet, rows per block,
-  // planes per chunk, and each tile's word (valid while tmed_ready and the
-  // grid runs these passes)
-  sfd::QuadPlan qplan = {};
-  int qslabs = 0;
-  int qrows = 1, qkc = 1;
+  // the four-cell passes' tiles and their words (valid while tmed_ready and
+  // the grid runs these passes)
+  sfd_host::QuadLayout quad;
   int *qmed = nullptr;
   int qmed_cap = 0;
   std::vector<double> step_cells;        // Yee cells owned per class
@@ -228,6 +232,7 @@ int refuse_batched(fdtd_handle *h);
 void alloc_extent(const fdtd_handle *h, int comp, long long ext[3]);
 int probe_room(fdtd_handle *h, long long more);
 bool quads_fit(const fdtd_handle *h);
+QuadLayout plan_quads(const fdtd_handle *h, int rows, int kc);
 int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);
@@ -237,6 +242,9 @@ int run_nodal(fdtd_handle *h, int half, int n, const int *dn);
 // (null: not wanted): per block of tm, what its tile meets is added
 int make_pass_src(fdtd_handle *h, const sfd::TileMap &tm, int half, sfd::PassSrc *out, bool *on,
                   std::vector<void *> *list, std::vector<int> *flags);
+// the same for the four-cell passes (flags: the words of the layout's tiles)
+int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, sfd::PassSrc *out, bool *on,
+                  std::vector<void *> *list, int *flags);
 // UpdateObservation of grid g (h->g or the written copy of a one-launch step)
 // at step n (or *dn + n): point probes and frequency-domain sums
 sfd::Observe observe_desc(const fdtd_handle *h, const int *dn);

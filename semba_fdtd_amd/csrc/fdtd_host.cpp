@@ -229,17 +229,18 @@ static bool use_quads(const fdtd_handle *h) {
   return quads_fit(h) && (h->xcells == 4 || !h->tile_set);
 }
 
-// the boxes of the four-cell passes under the handle's tiling
-static void plan_quads(fdtd_handle *h) {
+// the tiles of the four-cell passes: rows per block and planes per chunk as
+// given, or (rows 0) the default of the grid's size
+QuadLayout plan_quads(const fdtd_handle *h, int rows, int kc) {
   const DevGrid &g = h->g;
+  QuadLayout l;
   const int Q = g.nx / 4 + 1, J = g.ny + 1, K = g.nz + 1;
   // rows and planes that touch no y or z slab of E or H
   auto hi = [&](int a, int n) { return g.L[a][1] ? n - g.L[a][1] : n + 1; };
   const int ja = g.L[1][0], jb = hi(1, g.ny), ka = g.L[2][0], kb = hi(2, g.nz);
-  if (h->tile_set) {
-    h->qrows = h->tm.bdy;
-    h->qkc = h->tm.kc;
-  } else {
+  l.rows = rows;
+  l.kc = std::min(kc, K);
+  if (!rows) {
     // One plane per block: nothing is carried from plane to plane, but twice
     // the blocks hide the load latency better, and small tiles more often hold
     // one medium.  Two planes pay where a block moves little per plane: binary16,
@@ -248,19 +249,19 @@ static void plan_quads(fdtd_handle *h) {
     // 153.8, 256^3 369 / 382, 320^3 680 / 714; binary16 64^3 20.1 / 25.8,
     // 128^3 49.8 / 48.7, 200^3 135 / 115, 256^3 345 / 284.
     const long long cells = cells_of(h);
-    h->qrows = 1;
-    h->qkc = cells >= 1500000 && (g.fp16 || g.nx < 256) ? 2 : 1;
+    l.rows = 1;
+    l.kc = cells >= 1500000 && (g.fp16 || g.nx < 256) ? 2 : 1;
   }
-  QuadPlan P = {};
+  QuadPlan &P = l.p;
   std::fill(P.start, P.start + kQuadBoxes + 1, 0x7fffffff);
   auto add = [&](int j0, int j1, int k0, int k1) {
     if (j1 <= j0 || k1 <= k0) return;
     QuadBox &b = P.box[P.nbox];
     P.start[P.nbox++] = P.nblk;
-    b = QuadBox{0, Q, j0, j1 - j0, k0, k1 - k0, 0, 0};
-    const long long per = (long long)kWave * h->qrows;
+    b = QuadBox{0, Q, j0, j1 - j0, k0, k1 - k0, 0, l.kc};
+    const long long per = (long long)kWave * l.rows;
     b.tx = (int)(((long long)b.nq * b.nj + per - 1) / per);
-    P.nblk += b.tx * ((b.nk + h->qkc - 1) / h->qkc);
+    P.nblk += b.tx * ((b.nk + l.kc - 1) / l.kc);
   };
   if (ja < jb && ka < kb) {
     add(ja, jb, ka, kb);
@@ -268,12 +269,12 @@ static void plan_quads(fdtd_handle *h) {
     add(0, J, kb, K);
     add(0, ja, ka, kb);
     add(jb, J, ka, kb);
-    h->qslabs = P.nbox > 1 ? kSlabMix : g.L[0][0] + g.L[0][1] ? kSlabX : 0;
+    l.slabs = P.nbox > 1 ? kSlabMix : g.L[0][0] + g.L[0][1] ? kSlabX : 0;
   } else {
     add(0, J, 0, K);
-    h->qslabs = kSlabAll;
+    l.slabs = kSlabAll;
   }
-  h->qplan = P;
+  return l;
 }
 
 static void drop_multi_graph(fdtd_handle *h) {
@@ -303,13 +304,12 @@ void invalidate_graph(fdtd_handle *h) {
 // skip the media loads of single-medium tiles; and the sources the passes
 // apply inline.  Built outside any capture, before the passes it serves are
 // launched or recorded.
-static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags);
 int build_tile_media(fdtd_handle *h) {
   if (h->tmed_ready) return FDTD_OK;
   h->psrc_on[0] = h->psrc_on[1] = false;
   if (use_quads(h)) {
-    plan_quads(h);
-    const int n = h->qplan.nblk;
+    h->quad = plan_quads(h, h->tile_set ? h->tm.bdy : 0, h->tm.kc);
+    const int n = h->quad.p.nblk;
     if (n > h->qmed_cap) {
       HIPCHK(h, hipStreamSynchronize(h->stream));
       if (h->qmed) hipFree(h->qmed);
@@ -323,13 +323,14 @@ int build_tile_media(fdtd_handle *h) {
     h->psrc_allocs.clear();
     std::vector<int> flags((size_t)n, 0);
     for (int half = 0; half < 2; ++half)
-      if (int rc = make_quad_src(h, half, &flags)) return rc;
+      if (int rc = make_quad_src(h, h->quad, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, flags.data()))
+        return rc;
     HIPCHK(h, hipMemcpyAsync(h->qmed, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
                              h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     const int e = h->mode == FDTD_MODE_EXACT
-                      ? exact::launch_quad_media(h->g, h->qplan, h->qrows, h->qkc, h->qmed, h->stream)
-                      : fast::launch_quad_media(h->g, h->qplan, h->qrows, h->qkc, h->qmed, h->stream);
+                      ? exact::launch_quad_media(h->g, h->quad.p, h->quad.rows, h->qmed, h->stream)
+                      : fast::launch_quad_media(h->g, h->quad.p, h->quad.rows, h->qmed, h->stream);
     if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
     h->tmed_ready = true;
     return FDTD_OK;
@@ -1217,12 +1218,15 @@ static bool face_in_poles(const fdtd_handle *h, int half) {
 // box that touches them keeps its own launches).  Grids of every size: the
 // tiles without faces run code without them.  us per step, separate / inline:
 // 64^3 38.4 / 18.6, 128^3 80.2 / 52.4, 256^3 429 / 369, 384^3 1558 / 1431.
-static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags) {
-  h->psrc[half] = PassSrc{};
+int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, PassSrc *out, bool *on,
+                  std::vector<void *> *list, int *flags) {
+  *out = PassSrc{};
+  *on = false;
+  std::vector<int> word((size_t)l.p.nblk, 0);
   const bool faces = !h->pw_faces[half].empty();
   if (!faces && h->hcells[half].empty()) return FDTD_OK;
   if (faces && (!h->pw_masks[half] || face_in_poles(h, half))) return FDTD_OK;
-  const QuadPlan &p = h->qplan;
+  const QuadPlan &p = l.p;
   PassSrc x = faces ? h->pw_src[half] : PassSrc{};
   if (x.nface) {
     const std::vector<unsigned> *m = h->pw_bits[half];
@@ -1231,11 +1235,11 @@ static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags) {
       for (int i = a; i < std::min(b, (int)v.size()); ++i) r |= v[(size_t)i];
       return r;
     };
-    const int run = kWave * h->qrows;
+    const int run = kWave * l.rows;
     int t = 0;
     for (int q = 0; q < p.nbox; ++q) {
       const QuadBox &o = p.box[q];
-      const bool slabs = h->qslabs == kSlabAll || (h->qslabs == kSlabMix && q > 0);
+      const bool slabs = l.slabs == kSlabAll || (l.slabs == kSlabMix && q > 0);
       std::vector<unsigned> xy((size_t)o.tx);
       for (int r = 0; r < o.tx; ++r) {
         const int f0 = r * run, f1 = std::min(f0 + run, o.nq * o.nj) - 1;
@@ -1244,32 +1248,35 @@ static int make_quad_src(fdtd_handle *h, int half, std::vector<int> *flags) {
                         (j0 == j1 ? any(m[0], 4 * (f0 % o.nq), 4 * (f1 % o.nq) + 4)
                                   : any(m[0], 0, h->g.nx + 1));
       }
-      for (int k = o.k0; k < o.k0 + o.nk; k += h->qkc) {
-        const unsigned z = any(m[2], k, std::min(k + h->qkc, o.k0 + o.nk));
+      for (int k = o.k0; k < o.k0 + o.nk; k += l.kc) {
+        const unsigned z = any(m[2], k, std::min(k + l.kc, o.k0 + o.nk));
         for (int r = 0; r < o.tx; ++r, ++t) {
           if (!(xy[(size_t)r] & z)) continue;
           if (slabs) return FDTD_OK;
-          (*flags)[(size_t)t] |= kTileFaces[half];
+          word[(size_t)t] |= kTileFaces[half];
         }
       }
     }
   }
   if (!h->hcells[half].empty()) {
     std::vector<int> start;
-    bool on = false;
+    bool ok = false;
     const int rc = tile_cells(h, half, p.nblk, [&](int i, int j, int k) {
       for (int b = 0; b < p.nbox; ++b) {
         const QuadBox &o = p.box[b];
         if (j < o.j0 || j >= o.j0 + o.nj || k < o.k0 || k >= o.k0 + o.nk) continue;
         const int f = (j - o.j0) * o.nq + i / 4;
-        return p.start[b] + (k - o.k0) / h->qkc * o.tx + f / (kWave * h->qrows);
+        return p.start[b] + (k - o.k0) / l.kc * o.tx + f / (kWave * l.rows);
       }
       return 0;   // (the boxes hold every swept cell)
-    }, &x, &on, &h->psrc_allocs, &start);
-    if (rc || !on) return rc;
+    }, &x, &ok, list, &start);
+    if (rc || !ok) return rc;
+    for (int t = 0; t < p.nblk; ++t)
+      if (start[(size_t)t] < start[(size_t)t + 1]) word[(size_t)t] |= kTileNodal[half];
   }
-  h->psrc[half] = x;
-  h->psrc_on[half] = true;
+  for (int t = 0; t < p.nblk; ++t) flags[t] |= word[(size_t)t];
+  *out = x;
+  *on = true;
   return FDTD_OK;
 }
 
@@ -1620,8 +1627,8 @@ int prepare(fdtd_handle *h) {
 int run_quads(fdtd_handle *h, int half, const PassSrc *src) {
   const PassSrc x = src ? *src : PassSrc{};
   const int e = h->mode == FDTD_MODE_EXACT
-                    ? exact::launch_quad(h->g, h->qplan, h->qslabs, h->qrows, h->qkc, h->qmed, half, x, h->stream)
-                    : fast::launch_quad(h->g, h->qplan, h->qslabs, h->qrows, h->qkc, h->qmed, half, x, h->stream);
+                    ? exact::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, h->stream)
+                    : fast::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "%s pass launch failed: %s", half ? "H" : "E",
                      hipGetErrorString((hipError_t)e));
   return FDTD_OK;

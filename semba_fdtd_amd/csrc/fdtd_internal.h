@@ -96,11 +96,11 @@ struct TileMap {
 
 // The boxes of one launch of the four-cell passes (fdtd_quad.h): vectors of
 // four x cells q0 .. q0 + nq - 1, rows j0 .. , planes k0 ..; tx runs of
-// vectors per plane.
+// vectors per plane, kc planes per tile.
 // Box b holds tiles start[b] .. start[b+1] - 1 (unused entries: past any tile).
 struct QuadBox {
   int q0, nq, j0, nj, k0, nk;
-  int tx, pad;
+  int tx, kc;
 };
 constexpr int kQuadBoxes = 5;
 // the slabs the tiles of a launch may meet: bits for x, y, z, or kSlabMix: the
@@ -112,6 +112,12 @@ struct QuadPlan {
   QuadBox box[kQuadBoxes];
 };
 
+
+// One tile of a batch: grid, box, the tile's place in the box and in the grid,
+// and its word.
+struct QuadTile {
+  int grid, box, t, tg, info, pad[3];
+};
 
 // First-order Mur (bordersmur.F90): one tangential H component on one
 // absorbing face.  The plane just outside the component's sweep (ghost) is
@@ -199,6 +205,8 @@ constexpr int kPassFaces = 32;
 // What a tile of the one-cell pass map meets, one word per tile: the medium
 // all its cells hold plus one (0: several) in the low 16 bits, and per half
 // whether it meets a TF/SF face or a nodal cell the pass applies inline.
+// kTileSlabs: a four-cell tile in the y or z slabs.
+constexpr int kTileSlabs = 1 << 20;
 constexpr int kTileFaces[2] = {1 << 16, 1 << 17}, kTileNodal[2] = {1 << 18, 1 << 19};
 struct PassSrc {
   int nface;
@@ -386,6 +394,10 @@ struct BatchDev {
                               // (null: every tile loads its media)
   const PassSrc *src[2];      // per grid: the sources the E and H passes apply
                               // inline (null: no grid has any)
+  // the four-cell passes (null: the one-cell passes run): tile t of the batch
+  // is qtiles[t], box b of grid g is qboxes[g * kQuadBoxes + b]
+  QuadTile *qtiles;
+  const QuadBox *qboxes;
 };
 
 #ifdef __HIPCC__
@@ -460,12 +472,12 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
   int launch_h(const DevGrid &g, const TileMap &tm, const int *tmed,        \
                int yee, int cpml, int ade, const PassSrc *src, void *stream); \
   int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, \
-                  int kc, const int *tmed, int half, const PassSrc &src,    \
-                  void *stream);                                             \
-  int launch_quad_batch(const BatchDev &bd, int half, int blocks, int rows, \
-                        size_t lds, int fp16, void *stream);                 \
+                  const int *tmed, int half, const PassSrc &src, void *stream); \
+  int launch_quad_batch(const BatchDev &bd, int half, int rows, size_t lds, \
+                        int fp16, void *stream);                             \
   int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows,      \
-                        int kc, int *out, void *stream);                     \
+                        int *out, void *stream);                             \
+  int launch_quad_media_batch(const BatchDev &bd, int rows, void *stream);  \
   int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out,  \
                              void *stream);                                  \
   size_t step_lds_bytes(const DevGrid &g, int rows, int npw, int kc);       \
@@ -478,7 +490,7 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
   int launch_ade_many(const DevGrid *grids, const int *list, int n, int side, \
                       size_t lds, int tbl, long long nmax, void *stream);     \
   int launch_pass_batch(const BatchDev &bd, int half, int blocks, int rows,  \
-                        int vec, size_t lds, int fp16, void *stream);        \
+                        size_t lds, int fp16, void *stream);                 \
   }
 SFD_DECLARE_LAUNCHERS(fast)
 SFD_DECLARE_LAUNCHERS(exact)

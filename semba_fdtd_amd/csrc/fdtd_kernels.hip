@@ -735,10 +735,10 @@ __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
   }
 }
 
-int launch_pass_batch(const BatchDev &bd, int half, int blocks, int rows, int vec, size_t lds,
-                      int fp16, void *stream) {
+int launch_pass_batch(const BatchDev &bd, int half, int blocks, int rows, size_t lds, int fp16,
+                      void *stream) {
   if (bd.total <= 0) return 0;
-  if (vec == 4) return launch_quad_batch(bd, half, blocks, rows, lds, fp16, stream);
+  if (bd.qtiles) return launch_quad_batch(bd, half, rows, lds, fp16, stream);
   const dim3 blk(kWave, (unsigned)rows);
   hipStream_t s = (hipStream_t)stream;
   const bool x = bd.src[half ? 1 : 0];

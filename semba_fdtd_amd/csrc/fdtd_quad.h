@@ -162,7 +162,7 @@ __device__ __forceinline__ void plane_wait() {
 
 #define SFD_ALL4(x) {(x), (x), (x), (x)}
 
-// the lane's vector in tile t of the plan: its row j and first cell i0, the
+// the lane's vector in tile t of box x: its row j and first cell i0, the
 // tile's planes k0 .. k1 - 1, and whether the vector is the first or the last
 // of its box's row; false for a lane past the box (these are the last lanes
 // of the tile: no other lane's wave shift needs them)
@@ -170,41 +170,31 @@ struct QuadPos {
   int i0, j, k0, k1;
   bool first, last;
 };
-template <class P>
-__device__ __forceinline__ bool quad_pos(const P &p, int t, int kc, QuadPos &o) {
-  int b = 0, start = 0;
-#pragma unroll
-  for (int i = 1; i < kQuadBoxes; ++i)
-    if (t >= p.start[i]) { b = i; start = p.start[i]; }
-  const auto &q0 = p.box[b];
-  const QuadBox x{q0.q0, q0.nq, q0.j0, q0.nj, q0.k0, q0.nk, q0.tx, 0};
-  t -= start;
+__device__ __forceinline__ bool quad_pos(const QuadBox &x, int t, QuadPos &o) {
   const int bz = t / x.tx, run = t - bz * x.tx;
   const int f = (run * (int)blockDim.y + (int)threadIdx.y) * kWave + (int)threadIdx.x;
   const int r = f / x.nq, q = f - r * x.nq;
   o.i0 = 4 * (x.q0 + q);
   o.j = x.j0 + r;
-  o.k0 = x.k0 + bz * kc;
-  o.k1 = min(o.k0 + kc, x.k0 + x.nk);
+  o.k0 = x.k0 + bz * x.kc;
+  o.k1 = min(o.k0 + x.kc, x.k0 + x.nk);
   o.first = q == 0;
   o.last = q == x.nq - 1;
   return r < x.nj;
 }
-
-// the same in tile blk of a batch's map: runs of the whole x-y plane
-__device__ __forceinline__ bool quad_pos(const TileMap &tm, int blk, int nx, int ny, int nz,
-                                         QuadPos &o) {
-  const int Q = (nx >> 2) + 1;
-  const int bz = blk / tm.tx, run = blk - bz * tm.tx;
-  const int f = (run * (int)blockDim.y + (int)threadIdx.y) * kWave + (int)threadIdx.x;
-  o.j = f / Q;
-  const int q = f - o.j * Q;
-  o.i0 = 4 * q;
-  o.k0 = bz * tm.kc;
-  o.k1 = min(o.k0 + tm.kc, nz + 1);
-  o.first = q == 0;
-  o.last = q == Q - 1;
-  return o.j <= ny;
+// a box read through whatever address space holds it
+template <class B>
+__device__ __forceinline__ QuadBox load_box(const B &b) {
+  return QuadBox{b.q0, b.nq, b.j0, b.nj, b.k0, b.nk, b.tx, b.kc};
+}
+// tile t of a plan
+template <class P>
+__device__ __forceinline__ bool quad_pos(const P &p, int t, QuadPos &o) {
+  int b = 0, start = 0;
+#pragma unroll
+  for (int i = 1; i < kQuadBoxes; ++i)
+    if (t >= p.start[i]) { b = i; start = p.start[i]; }
+  return quad_pos(load_box(p.box[b]), t - start, o);
 }
 
 // a descriptor whose members are read anew where this is called: held across

@@ -9,7 +9,6 @@ namespace SFD_NS {
 struct QuadArgs {
   DevGrid g;
   QuadPlan p;
-  int kc;
   const int *tmed;
   PassSrc x;      // the half's sources
 };
@@ -59,7 +58,7 @@ __global__ void __launch_bounds__(256) k_quad(QuadArgs) {
   const int t = xcd_remap(blockIdx.x, a.p.nblk);
   const int info = ro_uniform_i(a.tmed, t);
   QuadPos at;
-  const bool live = quad_pos(a.p, t, a.kc, at);
+  const bool live = quad_pos(a.p, t, at);
   int c0 = 0, c1 = 0;   // the tile's nodal cells
   if (a.x.nstart) {
     c0 = ro_uniform_i(a.x.nstart, t);
@@ -70,46 +69,52 @@ __global__ void __launch_bounds__(256) k_quad(QuadArgs) {
   if (c0 < c1) nodal_cells<T>(a.g, a.x, c0, c1);
 }
 
-// One persistent launch over the tiles of every grid of a batch: block b runs
-// tiles b, b + gridDim.x, ...
-template <bool H, class T>
+// The tiles of every grid of a batch, one block each, descriptors read through
+// the constant address space.  X: some grid's passes apply sources inline.
+template <bool H, bool X, class T>
 __global__ void __launch_bounds__(256) k_quad_batch(BatchDev bd) {
   extern __shared__ float2 lds_tab[];
   typedef __attribute__((address_space(4))) DevGrid CDevGrid;
-  for (int t = blockIdx.x; t < bd.total; t += gridDim.x) {
-    const int b = __builtin_amdgcn_readfirstlane(batch_grid(bd.start, bd.ngrid, t));
-    const CDevGrid &g = *(const CDevGrid *)(bd.grids + b);
-    const TileMap tm = const_tilemap(bd.tms + b);
-    __syncthreads();  // the previous tile is done with the LDS table
-    QuadPos at;
-    const bool live = quad_pos(tm, t - bd.start[b], g.nx, g.ny, g.nz, at);
-    run_quad<H, kSlabAll, false, T>(g, lds_tab, 0, at, live, PassSrc{});
-  }
+  typedef __attribute__((address_space(4))) QuadTile CQuadTile;
+  typedef __attribute__((address_space(4))) QuadBox CQuadBox;
+  const CQuadTile &qt = ((const CQuadTile *)bd.qtiles)[blockIdx.x];
+  const int b = qt.grid, info = qt.info;
+  const CDevGrid &g = *(const CDevGrid *)(bd.grids + b);
+  const CPassSrc &x = *((const CPassSrc *)bd.src[H ? 1 : 0] + (X ? b : 0));
+  QuadPos at;
+  const bool live = quad_pos(load_box(((const CQuadBox *)bd.qboxes)[qt.box]), qt.t, at);
+  if (info & kTileSlabs) run_quad<H, kSlabAll, false, T>(g, lds_tab, info, at, live, x);
+  else run_quad<H, kSlabX, X, T>(g, lds_tab, info, at, live, x);
+  if (X && (info & kTileNodal[H ? 1 : 0]))
+    nodal_cells<T>(g, x, ro_uniform_i(x.nstart, qt.tg), ro_uniform_i(x.nstart, qt.tg + 1));
 }
 
-int launch_quad_batch(const BatchDev &bd, int half, int blocks, int rows, size_t lds, int fp16,
-                      void *stream) {
-  const dim3 grid((unsigned)blocks), blk(kWave, (unsigned)rows);
+int launch_quad_batch(const BatchDev &bd, int half, int rows, size_t lds, int fp16, void *stream) {
+  const dim3 grid((unsigned)bd.total), blk(kWave, (unsigned)rows);
   hipStream_t s = (hipStream_t)stream;
-  if (fp16) {
-    if (half) hipLaunchKernelGGL((k_quad_batch<true, __half>), grid, blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_quad_batch<false, __half>), grid, blk, lds, s, bd);
-  } else {
-    if (half) hipLaunchKernelGGL((k_quad_batch<true, float>), grid, blk, lds, s, bd);
-    else hipLaunchKernelGGL((k_quad_batch<false, float>), grid, blk, lds, s, bd);
-  }
+  const bool x = bd.src[half ? 1 : 0];
+  if (x) lds = face_lds_offset(lds) + kPassFaces * sizeof(FaceAddr);
+#define SFD_QB(X, T)                                                                        \
+  do {                                                                                      \
+    if (half) hipLaunchKernelGGL((k_quad_batch<true, X, T>), grid, blk, lds, s, bd);        \
+    else hipLaunchKernelGGL((k_quad_batch<false, X, T>), grid, blk, lds, s, bd);            \
+  } while (0)
+  if (fp16 && x) SFD_QB(true, __half);
+  else if (fp16) SFD_QB(false, __half);
+  else if (x) SFD_QB(true, float);
+  else SFD_QB(false, float);
+#undef SFD_QB
   return (int)hipGetLastError();
 }
 
-// Adds to out[t], the tile's flags, the medium that all six media arrays hold
-// on every swept cell of tile t plus one (0: they hold several).  The tiles are laid out as the passes lay them out.
-__global__ void __launch_bounds__(256) k_quad_media(DevGrid g, QuadPlan p, int kc, int *out) {
+// The medium that all six media arrays hold on every swept cell of a tile plus
+// one, or 0 (they hold several), from every thread of its block.
+__device__ __forceinline__ int tile_one_medium(const DevGrid &g, const QuadPos &at, bool live) {
   __shared__ int lo, hi;
   if (threadIdx.x == 0 && threadIdx.y == 0) { lo = 0x7fffffff; hi = -0x7fffffff; }
   __syncthreads();
-  QuadPos at;
   int a = 0x7fffffff, b = -0x7fffffff;
-  if (quad_pos(p, blockIdx.x, kc, at))
+  if (live)
     for (int k = at.k0; k < at.k1; ++k) {
       const long long q = (long long)(k + 1) * g.pxy + (long long)(at.j + 1) * g.px + g.xoff + at.i0;
       for (int c = 0; c < 6; ++c)
@@ -122,20 +127,42 @@ __global__ void __launch_bounds__(256) k_quad_media(DevGrid g, QuadPlan p, int k
   atomicMin(&lo, a);
   atomicMax(&hi, b);
   __syncthreads();
-  if (threadIdx.x == 0 && threadIdx.y == 0) out[blockIdx.x] += lo == hi ? lo + 1 : 0;
+  return lo == hi ? lo + 1 : 0;
 }
 
-int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows, int kc, int *out, void *stream) {
+// adds it to the word of each tile: out[t], or the batch's qtiles[t].info
+__global__ void __launch_bounds__(256) k_quad_media(DevGrid g, QuadPlan p, int *out) {
+  QuadPos at;
+  const bool live = quad_pos(p, (int)blockIdx.x, at);
+  const int m = tile_one_medium(g, at, live);
+  if (threadIdx.x == 0 && threadIdx.y == 0) out[blockIdx.x] += m;
+}
+__global__ void __launch_bounds__(256) k_quad_media_batch(BatchDev bd) {
+  QuadTile &qt = bd.qtiles[blockIdx.x];
+  QuadPos at;
+  const bool live = quad_pos(bd.qboxes[qt.box], qt.t, at);
+  const int m = tile_one_medium(bd.grids[qt.grid], at, live);
+  if (threadIdx.x == 0 && threadIdx.y == 0) qt.info += m;
+}
+
+int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows, int *out, void *stream) {
   if (p.nblk <= 0) return 0;
   hipLaunchKernelGGL(k_quad_media, dim3((unsigned)p.nblk), dim3(kWave, (unsigned)rows), 0,
-                     (hipStream_t)stream, g, p, kc, out);
+                     (hipStream_t)stream, g, p, out);
   return (int)hipGetLastError();
 }
 
-int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, int kc, const int *tmed,
+int launch_quad_media_batch(const BatchDev &bd, int rows, void *stream) {
+  if (bd.total <= 0) return 0;
+  hipLaunchKernelGGL(k_quad_media_batch, dim3((unsigned)bd.total), dim3(kWave, (unsigned)rows), 0,
+                     (hipStream_t)stream, bd);
+  return (int)hipGetLastError();
+}
+
+int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, const int *tmed,
                 int half, const PassSrc &src, void *stream) {
   if (p.nblk <= 0) return 0;
-  const QuadArgs a{g, p, kc, tmed, src};
+  const QuadArgs a{g, p, tmed, src};
   const dim3 grid((unsigned)p.nblk), blk(kWave, (unsigned)rows);
   const size_t tab = (size_t)(g.nmedia + 1) * sizeof(float2);
   const size_t lds = src.nface ? face_lds_offset(tab) + kPassFaces * sizeof(FaceAddr) : tab;

@@ -31,10 +31,12 @@ from ._lib import FdtdError
 Tiling = Tuple[int, int, int]          # rows, zchunk, xcells
 StepShape = Tuple[int, int]            # rows, zchunk (rows 0: two passes)
 
-# short z chunks give small grids more blocks: a 64^3 cavity steps in 22 us
-# with 4-plane chunks against 41 us with 16
+# short z chunks give small grids more blocks (64^3 cavity, one cell per lane:
+# 22 us per step with 4-plane chunks against 41 us with 16); four cells per lane
+# run best on one or two planes a block, whatever the grid's size
 DEFAULT_CANDIDATES: Tuple[Tiling, ...] = tuple(
-    (r, k, x) for x in (1, 4) for r in (1, 2, 4) for k in (4, 8, 16, 32, 64))
+    [(r, k, 1) for r in (1, 2, 4) for k in (4, 8, 16, 32, 64)] +
+    [(r, k, 4) for r in (1, 2, 4) for k in (1, 2, 4, 8, 16)])
 STEP_CANDIDATES: Tuple[StepShape, ...] = ((4, 16), (8, 16), (8, 32), (16, 16), (16, 32))
 
 NCLASS = 17                            # tile classes of the one-launch step

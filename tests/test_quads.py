@@ -108,3 +108,28 @@ def test_grids_without_interior(n, L):
     want = split(pb, "fast")
     assert same(fused(pb, "fast"), want)
     assert same(fused(pb, "fast", tiling=(2, 4, 4)), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["fp32", "fp16"])
+@pytest.mark.parametrize("narrow", [False, True])
+def test_batch_quads_equal_alone(storage, narrow):
+    """Grids of every layout in one batch; with a grid the four-cell passes
+    cannot run (narrow) the whole batch runs one cell per lane."""
+    from semba_fdtd_amd.batch import Batch
+    pbs = [build(*CASES[q]) for q in (2, 9, 12, 15, 16, 17, 18, 20, 21)]
+    if narrow:
+        pbs.append(build((9, 20, 19), NONE))
+        pbs[-1].cpml_layers = [[3, 3], [0, 0], [0, 0]]
+    want = [fused(pb, "fast", storage, (2, 4, 1)) for pb in pbs]
+    for tiling in ((4, 16, 0, 1), (2, 5, 0, 4)):
+        b = Batch()
+        b.set_tiling(*tiling)
+        sol = [sf.Solver(pb, storage=storage) for pb in pbs]
+        for s, pb in zip(sol, pbs):
+            start(s, pb)
+            b.admit(s)
+        b.step(STEPS)
+        for q, s in enumerate(sol):
+            assert same([s.field(c) for c in range(6)], want[q]), (tiling, q)
+        b.close()
