@@ -6,7 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 
-#include "fdtd_internal.h"
+#include "fdtd_observe.h"
 
 namespace sfd {
 
@@ -356,39 +356,16 @@ int launch_pw_incident_many(const PwIncJob *jobs, int njobs, int maxnf, long lon
   return (int)hipGetLastError();
 }
 
-__global__ void k_tick_many(int *const *counters, int n) {
+__global__ void k_tick_many(int *const *counters, int n, int by) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) *counters[t] += 1;
+  if (t < n) *counters[t] += by;
 }
 
-int launch_tick_many(int *const *counters, int n, void *stream) {
+int launch_tick_many(int *const *counters, int n, int by, void *stream) {
   if (n <= 0) return 0;
   hipLaunchKernelGGL(k_tick_many, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream,
-                     counters, n);
+                     counters, n, by);
   return (int)hipGetLastError();
-}
-
-// The TF/SF term +-G * Incid * id (AdvancePlaneWaveE/H, planewaves.F90:878-1475)
-// of cell w of the faces' cells at step n: what pw_apply adds to the field,
-// with the same roundings.
-__device__ __forceinline__ void pw_term_cell(const PwTerms &t, long long w, int n) {
-#pragma clang fp contract(off)
-  int lo = 0, hi = t.nf - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (t.start[mid] <= w) lo = mid; else hi = mid - 1;
-  }
-  const PwFace &f = t.faces[lo];
-  const int half = lo >= t.nf0 ? 1 : 0;
-  const int ua = f.axis == 0 ? 1 : 0, va = f.axis == 2 ? 1 : 2;
-  const int c = (int)(w - t.start[lo]), nu = f.hi[ua] - f.lo[ua] + 1;
-  int cc[3];
-  cc[f.axis] = f.fixed;
-  cc[ua] = f.lo[ua] + c % nu;
-  cc[va] = f.lo[va] + c / nu;
-  const float tm = half ? (float)(t.tiempo[n] + (double)0.5f * t.dt) : (float)t.tiempo[n];
-  const float x = t.G[half] * pw_incid(f, t.waves, t.phys, t.pstride, tm, cc) * f.id;
-  t.out[w] = f.sign > 0.0f ? x : -x;
 }
 
 __global__ void __launch_bounds__(256) k_pw_terms(PwTerms t, int n, const int *dn) {
@@ -422,98 +399,38 @@ int launch_pw_terms_many(const PwTermsGrid *grids, int n, long long maxcells, vo
   return (int)hipGetLastError();
 }
 
-// UpdateObservation (observation.F90:2620-2672 point probes, :3553-3600
-// frequency-domain sums) of one grid after a step.  Block 0 samples the
-// probes: one row per call, *count advancing on the device so that a recorded
-// step can be replayed.  The other blocks take one (point, frequency) pair of
-// a frequency-domain box per thread: the three components of the point are
-// read once and multiplied by the complex(8) phase factor of the step (each
-// part scaled by the real sample).  The last blocks write the TF/SF terms of
-// the next step, one cell per thread, for the passes that apply them inline.
-// All only read the fields, and no block reads what another writes.  One launch, not one each: a launch of a few
-// hundred threads costs 4.4 us here whatever it does, half the time of a pass
-// over a 64^3 grid.
-__device__ __forceinline__ void observe_block(const DevGrid &g, const Observe &o, int n, int blk,
-                                              bool probes, bool dft, bool pw) {
-  const int bd = 1 + (int)((o.total + 255) / 256);
-  if (blk >= bd) {
-    const long long w = (long long)(blk - bd) * blockDim.x + threadIdx.x;
-    n += 1 + (o.dn ? *o.dn : 0);
-    if (pw && w < o.pw.total && n < o.pw.ntime) pw_term_cell(o.pw, w, n);
-    return;
-  }
-  if (blk == 0) {
-    if (!probes || o.np <= 0) return;
-    __shared__ int row;
-    if (threadIdx.x == 0) row = *o.count;
-    __syncthreads();
-    if (row < o.cap) {
-      for (int t = threadIdx.x; t < o.np; t += blockDim.x)
-        o.buf[(long long)row * o.np + t] = field_ld(g, o.pr[t].comp, o.pr[t].p);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && row < o.cap) *o.count = row + 1;
-    return;
-  }
-  const long long w = (long long)(blk - 1) * blockDim.x + threadIdx.x;
-  if (!dft || w >= o.total) return;
-  if (o.dn) n += *o.dn;
-  int q = 0;
-  while (q + 1 < o.ndft && o.dft[q + 1].start <= w) ++q;
-  const DftDev &d = o.dft[q];
-  const long long t = w - d.start;
-  const long long pt = t / d.nfreq;
-  const int f = (int)(t - pt * d.nfreq);
-  const int it = (int)(pt % d.cnt[0]);
-  const int jt = (int)((pt / d.cnt[0]) % d.cnt[1]);
-  const int kt = (int)(pt / ((long long)d.cnt[0] * d.cnt[1]));
-  const long long p = fidx(g, d.first[0] + it * d.stride[0], d.first[1] + jt * d.stride[1],
-                           d.first[2] + kt * d.stride[2]);
-  const double2 a = d.aux[(long long)n * d.nfreq + f];
-  for (int c = 0; c < 3; ++c) {
-    const double v = (double)field_ld(g, 3 * d.kind + c, p);
-    double2 *acc = d.acc + (pt * 3 + c) * d.nfreq + f;
-    const double2 o2 = *acc;
-    *acc = make_double2(o2.x + a.x * v, o2.y + a.y * v);
-  }
-}
-
-__global__ void __launch_bounds__(256) k_observe(DevGrid g, Observe o, int n, int probes, int dft,
-                                                 int pw) {
-  observe_block(g, o, n, blockIdx.x, probes != 0, dft != 0, pw != 0);
+__global__ void __launch_bounds__(256) k_observe(DevGrid g, ObservePart p) {
+  observe_block(g, p, p.n, blockIdx.x, 256);
 }
 
 __global__ void __launch_bounds__(256) k_observe_many(const DevGrid *grids, const ObserveGrid *obs,
-                                                      const int *start, int nobs) {
+                                                      const int *start, int nobs, int n) {
   int lo = 0, hi = nobs - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (start[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
   }
   const ObserveGrid &s = obs[lo];
-  observe_block(grids[s.grid], s.o, 0, (int)blockIdx.x - start[lo], true, true, true);
+  observe_block(grids[s.grid], s.p, n, (int)blockIdx.x - start[lo], 256);
 }
 
-int observe_blocks(const Observe &o) {
-  return 1 + (int)((o.total + 255) / 256) + (int)((o.pw.total + 255) / 256);
+int observe_blocks(const ObservePart &p, int nt) {
+  if (!p.sample && p.d1 <= p.d0 && p.w1 <= p.w0) return 0;
+  return 1 + (int)((p.d1 - p.d0 + nt - 1) / nt) + (int)((p.w1 - p.w0 + nt - 1) / nt);
 }
 
-int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, int pw,
-                   void *stream) {
-  const bool p = probes && o.np > 0, d = dft && o.total > 0, w = pw && o.pw.total > 0;
-  if (!p && !d && !w) return 0;
-  const unsigned blocks = w ? (unsigned)observe_blocks(o)
-                            : d ? 1u + (unsigned)((o.total + 255) / 256) : 1u;
-  hipLaunchKernelGGL(k_observe, dim3(blocks), dim3(256), 0, (hipStream_t)stream, g, o, n,
-                     p ? 1 : 0, d ? 1 : 0, w ? 1 : 0);
+int launch_observe(const DevGrid &g, const ObservePart &p, void *stream) {
+  const int blocks = observe_blocks(p, 256);
+  if (blocks <= 0) return 0;
+  hipLaunchKernelGGL(k_observe, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, g, p);
   return (int)hipGetLastError();
 }
 
 int launch_observe_many(const DevGrid *grids, const ObserveGrid *obs, const int *start, int nobs,
-                        int blocks, void *stream) {
+                        int blocks, int n, void *stream) {
   if (nobs <= 0 || blocks <= 0) return 0;
   hipLaunchKernelGGL(k_observe_many, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
-                     grids, obs, start, nobs);
+                     grids, obs, start, nobs, n);
   return (int)hipGetLastError();
 }
 

@@ -44,6 +44,8 @@ using namespace sfd_host;
 
 namespace {
 thread_local std::string g_batch_error;
+// two-pass steps per recorded graph of a batch
+constexpr int kBatchGraphSteps = 8;
 
 // the plane-wave groups of one (half, wave, axis) key across the batch
 struct BatchPwGroup {
@@ -92,8 +94,10 @@ struct fdtd_batch {
   PwTermsGrid *dterms = nullptr;
   int nterms = 0;
   long long maxterms = 0;
-  hipGraph_t graph = nullptr;
+  hipGraph_t graph = nullptr;         // one two-pass step
   hipGraphExec_t gexec = nullptr;
+  hipGraph_t mgraph = nullptr;        // kBatchGraphSteps of them
+  hipGraphExec_t mexec = nullptr;
   // one launch per step: rows per block (0: two passes) and planes per chunk
   int step_rows = 0, step_kc = 16;
   bool sready = false;
@@ -139,8 +143,10 @@ int bfail(fdtd_batch *b, int code, const char *fmt, ...) {
 void drop_graph(fdtd_batch *b) {
   if (b->gexec) hipGraphExecDestroy(b->gexec);
   if (b->graph) hipGraphDestroy(b->graph);
-  b->gexec = nullptr;
-  b->graph = nullptr;
+  if (b->mexec) hipGraphExecDestroy(b->mexec);
+  if (b->mgraph) hipGraphDestroy(b->mgraph);
+  b->gexec = b->mexec = nullptr;
+  b->graph = b->mgraph = nullptr;
 }
 
 void drop_step(fdtd_batch *b) {
@@ -372,11 +378,10 @@ int build_descriptors(fdtd_batch *b) {
       const bool terms = (b->inl[0][s] || b->inl[1][s]) && h->pw_terms.total > 0;
       if (h->nprobe || !h->dfts.empty() || terms) {
         ObserveGrid og{};
-        og.o = observe_desc(h, h->dstep);
-        if (!terms) og.o.pw = PwTerms{};
+        og.p = observe_part(h, 2, 0, h->dstep, true, true, terms);
         og.grid = gi;
         sets.push_back(og);
-        obstart.push_back(obstart.back() + observe_blocks(og.o));
+        obstart.push_back(obstart.back() + observe_blocks(og.p, 256));
       }
       ++gi;
     }
@@ -546,19 +551,21 @@ int launch_step_dir(fdtd_batch *b, int d, bool exact_prev) {
     if (launch_mur(h->sd[d].go, h->dmur, (int)h->mur_runs.size(), h->mur_total, exact, b->stream))
       return bfail(b, FDTD_ERR_HIP, "batch Mur launch failed");
   }
-  if (launch_observe_many(b->dgo[d], b->dobs, b->dobstart, b->nobs, b->obs_blocks, b->stream))
+  if (launch_observe_many(b->dgo[d], b->dobs, b->dobstart, b->nobs, b->obs_blocks, 0, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
-  if (launch_tick_many(b->dcounters, b->ncounters, b->stream))
+  if (launch_tick_many(b->dcounters, b->ncounters, 1, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
   return FDTD_OK;
 }
 
-int launch_step(fdtd_batch *b) {
+// one two-pass step of every grid, step r of a recorded sequence
+int launch_step(fdtd_batch *b, int r) {
   const bool exact = b->mode == FDTD_MODE_EXACT;
   // persistent blocks: 16384 measured fastest on the 256 uneven instances
   // (flat tiles of 64 x 4 threads, 16-plane chunks)
   const int blocks = b->blocks > 0 ? b->blocks : 16384;
   int e, rc;
+  b->bd.n = r;
   for (int half = 0; half < 2; ++half) {
     e = exact ? exact::launch_pass_batch(b->bd, half, blocks, b->prows, b->lds, 0, b->stream)
               : fast::launch_pass_batch(b->bd, half, blocks, b->prows, b->lds, b->fp16,
@@ -577,21 +584,19 @@ int launch_step(fdtd_batch *b) {
     }
     for (const BatchPwGroup &g : b->pw) {
       if (g.half != half) continue;
-      e = launch_tfsf_list(g.druns, g.dstart, (int)g.runs.size(), g.start.back(), 0, b->stream);
+      e = launch_tfsf_list(g.druns, g.dstart, (int)g.runs.size(), g.start.back(), r, b->stream);
       if (e) return bfail(b, FDTD_ERR_HIP, "batch plane-wave launch failed");
     }
     for (size_t s = 0; s < b->slots.size(); ++s) {
       fdtd_handle *h = b->slots[s];
-      if (h && !b->inl[half][s] && (rc = run_nodal(h, half, 0, h->dstep)))
+      if (h && !b->inl[half][s] && (rc = run_nodal(h, half, r, h->dstep)))
         return bfail(b, rc, "grid: %s", h->err.c_str());
     }
   }
   for (fdtd_handle *h : b->slots)
     if (h && (rc = run_mur(h))) return bfail(b, rc, "grid: %s", h->err.c_str());
-  if (launch_observe_many(b->bd.grids, b->dobs, b->dobstart, b->nobs, b->obs_blocks, b->stream))
+  if (launch_observe_many(b->bd.grids, b->dobs, b->dobstart, b->nobs, b->obs_blocks, r, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
-  if (launch_tick_many(b->dcounters, b->ncounters, b->stream))
-    return bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
   return FDTD_OK;
 }
 
@@ -799,17 +804,29 @@ int fdtd_batch_step(fdtd_batch *b, int32_t nsteps) {
   // next one's
   if (singles > 0 && launch_pw_terms_many(b->dterms, b->nterms, b->maxterms, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch incident-field launch failed");
-  if (singles > 0 && !b->gexec) {
+  // k steps in one graph: step r reads the step number *counter + r, and the
+  // counters move once, at the end (a launch of 3.8 us a step otherwise)
+  auto record = [b](int k, hipGraph_t *gout, hipGraphExec_t *xout) -> int {
     BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int r2 = launch_step(b);
+    int r2 = 0;
+    for (int r = 0; r < k && !r2; ++r) r2 = launch_step(b, r);
+    if (!r2 && launch_tick_many(b->dcounters, b->ncounters, k, b->stream))
+      r2 = bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
     hipGraph_t graph = nullptr;
     hipError_t ec = hipStreamEndCapture(b->stream, &graph);
     if (r2) { if (graph) hipGraphDestroy(graph); return r2; }
     if (ec != hipSuccess) return bfail(b, FDTD_ERR_HIP, "batch capture failed: %s", hipGetErrorString(ec));
-    b->graph = graph;
-    BCHK(b, hipGraphInstantiate(&b->gexec, graph, nullptr, nullptr, 0));
+    *gout = graph;
+    BCHK(b, hipGraphInstantiate(xout, graph, nullptr, nullptr, 0));
+    return FDTD_OK;
+  };
+  int left = singles;
+  if (left >= kBatchGraphSteps) {
+    if (!b->mexec && (rc = record(kBatchGraphSteps, &b->mgraph, &b->mexec))) return rc;
+    for (; left >= kBatchGraphSteps; left -= kBatchGraphSteps) BCHK(b, hipGraphLaunch(b->mexec, b->stream));
   }
-  for (int32_t s = 0; s < singles; ++s) BCHK(b, hipGraphLaunch(b->gexec, b->stream));
+  if (left > 0 && !b->gexec && (rc = record(1, &b->graph, &b->gexec))) return rc;
+  for (; left > 0; --left) BCHK(b, hipGraphLaunch(b->gexec, b->stream));
   for (size_t s = 0; s < b->slots.size(); ++s)
     if (b->slots[s]) {
       b->step[s] += nsteps;

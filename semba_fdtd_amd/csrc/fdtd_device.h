@@ -406,10 +406,10 @@ __device__ __forceinline__ const FaceAddr *stage_faces(const PS &x, float2 *lds,
 // stores are visible to it behind the barrier, and no other block writes the
 // tile's cells.  Every thread of the block calls this.
 template <class T, class G, class PS>
-__device__ __forceinline__ void nodal_cells(const G &g, const PS &x, int c0, int c1) {
+__device__ __forceinline__ void nodal_cells(const G &g, const PS &x, int c0, int c1, int off = 0) {
   __syncthreads();
   const int t = threadIdx.y * blockDim.x + threadIdx.x, nt = blockDim.x * blockDim.y;
-  const int n = x.n + (x.dn ? *x.dn : 0);
+  const int n = x.n + off + (x.dn ? *x.dn : 0);
   // cells that share a field value run in order, on one thread
   const int step = x.serial ? 1 : nt;
   for (int c = x.serial ? (t == 0 ? c0 : c1) : c0 + t; c < c1; c += step) {
@@ -423,11 +423,11 @@ __device__ __forceinline__ void nodal_cells(const G &g, const PS &x, int c0, int
 }
 template <class T, class PS>
 __device__ __forceinline__ void tile_nodal(const DevGrid &g, const TileMap &tm, const PS &x,
-                                           int blk) {
+                                           int blk, int off = 0) {
   if (!x.nstart) return;
   const int tile = tm.remap ? xcd_remap(blk, tm.nblk) : blk;
   const int c0 = x.nstart[tile], c1 = x.nstart[tile + 1];
-  if (c0 < c1) nodal_cells<T>(g, x, c0, c1);
+  if (c0 < c1) nodal_cells<T>(g, x, c0, c1, off);
 }
 
 // the tile's word (see kTileFaces) and its medium or -1

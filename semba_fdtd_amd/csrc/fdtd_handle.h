@@ -131,6 +131,7 @@ struct fdtd_handle {
   std::vector<unsigned> pw_bits[2][3];  // host copy of the faces' index masks
   sfd::PwTerms pw_terms{};
   int pw_terms_n = -1;
+  long long pw_split = 0;          // terms of the E faces
   // per half, under the pass tiling tm: the sources the one-cell pass applies
   // (valid while tmed_ready)
   bool psrc_on[2] = {false, false};
@@ -139,7 +140,8 @@ struct fdtd_handle {
   // frequency-domain observation
   std::vector<sfd_host::DftIn> dftin;
   std::vector<sfd::DftDev> dfts;
-  sfd::DftDev *ddfts = nullptr;       // device copy of dfts
+  sfd::DftDev *ddfts = nullptr;       // device copy of dfts, the boxes of E first
+  long long dft_end[2] = {0, 0};      // pairs of E's boxes, of all boxes
   bool dft_ready = false;
   std::vector<void *> dft_allocs;     // phase tables (rebuilt with the time vector)
   std::vector<void *> dft_sums;       // running sums (kept across rebuilds)
@@ -245,12 +247,13 @@ int make_pass_src(fdtd_handle *h, const sfd::TileMap &tm, int half, sfd::PassSrc
 // the same for the four-cell passes (flags: the words of the layout's tiles)
 int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, sfd::PassSrc *out, bool *on,
                   std::vector<void *> *list, int *flags);
-// UpdateObservation of grid g (h->g or the written copy of a one-launch step)
-// at step n (or *dn + n): point probes and frequency-domain sums
-sfd::Observe observe_desc(const fdtd_handle *h, const int *dn);
-// (pw: and the TF/SF terms of the next step)
-int run_observe(fdtd_handle *h, const sfd::DevGrid &g, int n, const int *dn, bool probes,
-                bool dft, bool pw);
+// UpdateObservation at step n (or *dn + n): point probes, frequency-domain
+// sums, and (pw) the TF/SF terms of the next step; half 0, 1: the E, the H
+// quantities alone (the H part moves the sample count), 2: all.  run_observe
+// launches it on grid g (h->g or the written copy of a one-launch step).
+sfd::ObservePart observe_part(const fdtd_handle *h, int half, int n, const int *dn, bool probes,
+                              bool dft, bool pw);
+int run_observe(fdtd_handle *h, const sfd::DevGrid &g, const sfd::ObservePart &p);
 int run_mur(fdtd_handle *h);
 int run_ade(fdtd_handle *h, int side);
 void invalidate_graph(fdtd_handle *h);

@@ -958,7 +958,7 @@ static int run_step(fdtd_handle *h, int dir, bool exact_prev = false) {
       launch_mur(sd.go, h->dmur, (int)h->mur_runs.size(), h->mur_total,
                  h->mode == FDTD_MODE_EXACT, h->stream))
     return fail(h, FDTD_ERR_HIP, "Mur launch failed");
-  if ((e = run_observe(h, sd.go, 0, h->dstep, true, true, false))) return e;
+  if ((e = run_observe(h, sd.go, observe_part(h, 2, 0, h->dstep, true, true, false)))) return e;
   if (launch_tick(h->dstep, 1, h->stream)) return fail(h, FDTD_ERR_HIP, "tick failed");
   return FDTD_OK;
 }
@@ -1067,7 +1067,7 @@ struct PwMasks {
   std::vector<FaceAddr> fa[2];
   size_t om[2][3], ofa[2], oall, ostart;   // places in the pack
 };
-static void build_pw_masks(fdtd_handle *h, PwMasks &w, Pack &pk) {
+static void build_pw_masks(fdtd_handle *h, const std::vector<PwWave> &waves, PwMasks &w, Pack &pk) {
   const int n3[3] = {h->g.nx, h->g.ny, h->g.nz};
   w.start.assign(1, 0);
   for (int half = 0; half < 2; ++half) {
@@ -1082,8 +1082,25 @@ static void build_pw_masks(fdtd_handle *h, PwMasks &w, Pack &pk) {
       for (int a = 0; a < 3; ++a) { lo[a] = f.lo[a]; hi[a] = f.hi[a]; }
       lo[f.axis] = hi[f.axis] = f.fixed;
       const int ua = f.axis == 0 ? 1 : 0, va = f.axis == 2 ? 1 : 2;
-      const long long nu = hi[ua] - lo[ua] + 1, nv = hi[va] - lo[va] + 1;
-      const long long cells = nu > 0 && nv > 0 ? nu * nv : 0;
+      long long nu = hi[ua] - lo[ua] + 1, nv = hi[va] - lo[va] + 1;
+      // One term serves every index of an axis that no mode of the wave moves
+      // along: x * 0 adds a zero to the retarded distance, which changes no
+      // bit of it (256 grids with waves along z: 22 M terms and 219 us a step
+      // otherwise).
+      PwFace ft = f;
+      int st[3] = {0, 0, 0};
+      auto one_term = [&](int a, long long &n) {
+        const PwWave &v = waves[(size_t)f.wave];
+        for (int m = 0; m < v.nmodes; ++m)
+          if (v.pn[m][a] != 0.0f) return false;
+        ft.hi[a] = ft.lo[a];
+        n = 1;
+        return true;
+      };
+      const bool any = nu > 0 && nv > 0;
+      if (any && !one_term(ua, nu)) st[ua] = 1;
+      if (any && !one_term(va, nv)) st[va] = (int)nu;
+      const long long cells = any ? nu * nv : 0;
       FaceAddr A{};
       if (cells) {
         // the passes run the components' sweeps: a face outside (a box on
@@ -1093,15 +1110,13 @@ static void build_pw_masks(fdtd_handle *h, PwMasks &w, Pack &pk) {
         if (ok) {
           for (int a = 0; a < 3; ++a)
             for (int i = lo[a]; i <= hi[a]; ++i) w.m[half][a][(size_t)i] |= 1u << q;
-          int st[3] = {0, 0, 0};
-          st[ua] = 1;
-          st[va] = (int)nu;
-          A = FaceAddr{(int)(w.start.back() - lo[va] * nu - lo[ua]), st[0], st[1], st[2]};
+          A = FaceAddr{(int)(w.start.back() - (long long)lo[va] * st[va] - (long long)lo[ua] * st[ua]),
+                       st[0], st[1], st[2]};
           s.cm[f.comp % 3] |= 1u << q;
         }
       }
       w.fa[half].push_back(A);
-      w.all.push_back(f);
+      w.all.push_back(ft);
       w.start.push_back(w.start.back() + cells);
     }
     h->pw_masks[half] = ok;
@@ -1128,6 +1143,7 @@ static int place_pw_masks(fdtd_handle *h, const PwMasks &w, Pack &pk) {
     t.nf0 = (int)h->pw_faces[0].size();
     t.nf = (int)w.all.size();
     t.total = w.start.back();
+    h->pw_split = w.start[h->pw_faces[0].size()];
     t.waves = h->dwaves;
     t.phys = h->dphys;
     t.pstride = h->pstride;
@@ -1523,7 +1539,7 @@ int build_planewaves(fdtd_handle *h) {
     og[3 * q + 2] = pk.add(grp.start.size() * sizeof(long long));
   }
   PwMasks masks;
-  build_pw_masks(h, masks, pk);
+  build_pw_masks(h, waves, masks, pk);
   int rc;
   if ((rc = pk.alloc(h, &h->pw_allocs))) return rc;
   for (size_t q = 0; q < waves.size(); ++q) {
@@ -1600,13 +1616,20 @@ int build_dfts(fdtd_handle *h) {
     if ((rc = upload(h, &da, aux.data(), aux.size(), &h->dft_allocs))) return rc;
     h->dfts[q].aux = da;
   }
+  // on the device the boxes of E come first
+  std::vector<DftDev> order;
   long long start = 0;
-  for (DftDev &d : h->dfts) {
-    d.start = start;
-    start += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+  for (int kind = 0; kind < 2; ++kind) {
+    for (DftDev d : h->dfts)
+      if (d.kind == kind) {
+        d.start = start;
+        start += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+        order.push_back(d);
+      }
+    h->dft_end[kind] = start;
   }
   h->ddfts = nullptr;
-  if ((rc = upload(h, &h->ddfts, h->dfts.data(), h->dfts.size(), &h->dft_allocs))) return rc;
+  if ((rc = upload(h, &h->ddfts, order.data(), order.size(), &h->dft_allocs))) return rc;
   h->dft_ready = true;
   return FDTD_OK;
 }
@@ -1624,17 +1647,18 @@ int prepare(fdtd_handle *h) {
 
 // the fused face pass of a half, four cells per lane (build_tile_media laid
 // its tiles out)
-int run_quads(fdtd_handle *h, int half, const PassSrc *src) {
+int run_quads(fdtd_handle *h, int half, const PassSrc *src, const ObservePart *obs) {
   const PassSrc x = src ? *src : PassSrc{};
   const int e = h->mode == FDTD_MODE_EXACT
-                    ? exact::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, h->stream)
-                    : fast::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, h->stream);
+                    ? exact::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, obs, h->stream)
+                    : fast::launch_quad(h->g, h->quad.p, h->quad.slabs, h->quad.rows, h->qmed, half, x, obs, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "%s pass launch failed: %s", half ? "H" : "E",
                      hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
 
-int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
+int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr,
+          const ObservePart *obs = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
   // the fused pass (yee and cpml) always runs the CPML kernel: without slab
@@ -1643,7 +1667,7 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
   const int a = ade && h->g.ade[0].has;
   const bool quads = use_quads(h);
   if (quads && yee && cpml) {
-    if (int rc = run_quads(h, 0, src)) return rc;
+    if (int rc = run_quads(h, 0, src, obs)) return rc;
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
@@ -1654,14 +1678,15 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
   return FDTD_OK;
 }
 
-int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr) {
+int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullptr,
+          const ObservePart *obs = nullptr) {
   if (h->g.fp16 && (yee != cpml || h->g.nmedia + 1 > 4096))
     return fail(h, FDTD_ERR_STATE, "binary16 storage runs the fused passes only (<= 4095 media)");
   int c = cpml && (h->g.has_cpml || yee);
   const int a = ade && h->g.ade[1].has;
   const bool quads = use_quads(h);
   if (quads && yee && cpml) {
-    if (int rc = run_quads(h, 1, src)) return rc;
+    if (int rc = run_quads(h, 1, src, obs)) return rc;
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
@@ -1674,8 +1699,10 @@ int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
 
 int run_ade(fdtd_handle *h, int side) { return side ? run_h(h, 0, 0, 1) : run_e(h, 0, 0, 1); }
 
-Observe observe_desc(const fdtd_handle *h, const int *dn) {
-  Observe o{};
+ObservePart observe_part(const fdtd_handle *h, int half, int n, const int *dn, bool probes, bool dft,
+                         bool pw) {
+  ObservePart x{};
+  Observe &o = x.o;
   o.pr = h->dprobes;
   o.buf = h->dpbuf;
   o.count = h->dpcount;
@@ -1683,15 +1710,26 @@ Observe observe_desc(const fdtd_handle *h, const int *dn) {
   o.cap = h->pcap;
   o.dft = h->ddfts;
   o.ndft = (int)h->dfts.size();
-  for (const DftDev &d : h->dfts) o.total += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
   o.pw = h->pw_terms;
   o.dn = dn;
-  return o;
+  x.half = half;
+  x.n = n;
+  x.sample = probes && h->nprobe > 0;
+  x.advance = half == 0 ? 0 : 1;
+  const int first = half == 1 ? 1 : 0, last = half == 0 ? 0 : 1;
+  if (dft && !h->dfts.empty()) {
+    x.d0 = first ? h->dft_end[0] : 0;
+    x.d1 = h->dft_end[last];
+  }
+  if (pw && h->pw_terms.total > 0) {
+    x.w0 = first ? h->pw_split : 0;
+    x.w1 = last ? h->pw_terms.total : h->pw_split;
+  }
+  return x;
 }
 
-int run_observe(fdtd_handle *h, const DevGrid &g, int n, const int *dn, bool probes, bool dft,
-                bool pw) {
-  const int e = launch_observe(g, observe_desc(h, dn), n, probes, dft, pw, h->stream);
+int run_observe(fdtd_handle *h, const DevGrid &g, const ObservePart &p) {
+  const int e = launch_observe(g, p, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "observation launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1754,14 +1792,14 @@ int need_terms(fdtd_handle *h, int n) {
 // One half step at step n (or *dn + n): the fused face pass with its pole
 // stage, its plane-wave faces and its nodal cells, the sources inside the
 // pass where they can be.
-int run_half(fdtd_handle *h, int half, int n, const int *dn) {
+int run_half(fdtd_handle *h, int half, int n, const int *dn, const ObservePart *obs = nullptr) {
   const bool in = h->psrc_on[half];
   PassSrc s = h->psrc[half];
   s.dn = dn;
   s.n = n;
   if (in && !dn && s.nstart && (n < 0 || n >= h->nvalues_steps))
     return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n, h->nvalues_steps - 1);
-  int rc = half ? run_h(h, 1, 1, 1, in ? &s : nullptr) : run_e(h, 1, 1, 1, in ? &s : nullptr);
+  int rc = half ? run_h(h, 1, 1, 1, in ? &s : nullptr, obs) : run_e(h, 1, 1, 1, in ? &s : nullptr, obs);
   if (rc || in) return rc;
   if ((rc = run_pw(h, half, n, dn))) return rc;
   return run_nodal(h, half, n, dn);
@@ -2241,7 +2279,7 @@ int fdtd_update_observation(fdtd_handle *h, int32_t n) {
   // the terms of the next step ride along when the steps run call by call
   const bool pw = in && h->tmed_ready && inline_faces(h) && n + 1 < (int)h->tiempo.size() &&
                   h->pw_terms_n == n && !stream_capturing(h);
-  if ((rc = run_observe(h, h->g, n, nullptr, true, in, pw))) return rc;
+  if ((rc = run_observe(h, h->g, observe_part(h, 2, n, nullptr, true, in, pw)))) return rc;
   if (pw) h->pw_terms_n = n + 1;
   h->pbuffered += h->nprobe ? 1 : 0;
   if (!in && !h->dfts.empty())
@@ -2396,10 +2434,24 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int r2 = 0;
     for (int r = 0; r < nrep && !r2; ++r) {
-      r2 = run_half(h, 0, r, h->dstep);
-      if (!r2) r2 = run_half(h, 1, r, h->dstep);
+      // The four-cell passes carry the observation in blocks of their own: the
+      // H pass of a step its E quantities, the next E pass its H quantities (the
+      // first of these follow the last pass), and each the TF/SF terms of that
+      // half's next step.  A launch of its own, 4.7 us, is a third of a step of
+      // a 64^3 cavity.
+      const bool pw = inline_faces(h), ride = use_quads(h);
+      ObservePart e = observe_part(h, 0, r, h->dstep, true, true, pw),
+                  hp = observe_part(h, 1, r - 1, h->dstep, true, true, pw);
+      e.row = r;
+      hp.row = r - 1;
+      hp.advance = 0;
+      r2 = run_half(h, 0, r, h->dstep, ride && r > 0 ? &hp : nullptr);
+      if (!r2) r2 = run_half(h, 1, r, h->dstep, ride ? &e : nullptr);
       if (!r2) r2 = run_mur(h);
-      if (!r2) r2 = run_observe(h, h->g, r, h->dstep, true, true, inline_faces(h));
+      if (r2 || (ride && r + 1 < nrep)) continue;
+      hp = observe_part(h, ride ? 1 : 2, r, h->dstep, true, true, pw);
+      if (ride) { hp.row = r; hp.advance = nrep; }
+      r2 = run_observe(h, h->g, hp);
     }
     if (!r2) r2 = launch_tick(h->dstep, nrep, h->stream) ? fail(h, FDTD_ERR_HIP, "tick failed") : 0;
     hipGraph_t graph = nullptr;
@@ -2602,8 +2654,9 @@ int fdtd_set_probes(fdtd_handle *h, int32_t nprobe, const int32_t *comp, const i
   int rc;
   h->dprobes = nullptr; h->dpbuf = nullptr; h->dpcount = nullptr;
   if ((rc = dalloc(h, (void **)&h->dprobes, sizeof(ProbeDev) * std::max(nprobe, 1)))) return rc;
-  if ((rc = dalloc(h, (void **)&h->dpbuf, (size_t)bufsteps * std::max(nprobe, 1) * 4))) return rc;
-  if ((rc = dalloc(h, (void **)&h->dpcount, 16))) return rc;
+  // the sample count leads the samples: one copy reads both
+  if ((rc = dalloc(h, (void **)&h->dpcount, 16 + (size_t)bufsteps * std::max(nprobe, 1) * 4))) return rc;
+  h->dpbuf = (float *)h->dpcount + 4;
   if (nprobe) HIPCHK(h, hipMemcpy(h->dprobes, pr.data(), sizeof(ProbeDev) * nprobe, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemset(h->dpcount, 0, 16));
   h->nprobe = nprobe;
@@ -2619,7 +2672,7 @@ int fdtd_sample_probes(fdtd_handle *h) {
   if (int rc = refuse_batched(h)) return rc;
   if (int rc = probe_room(h, 1)) return rc;
   hipSetDevice(h->device);
-  if (int rc = run_observe(h, h->g, 0, nullptr, true, false, false)) return rc;
+  if (int rc = run_observe(h, h->g, observe_part(h, 2, 0, nullptr, true, false, false))) return rc;
   h->pbuffered += 1;
   return FDTD_OK;
 }
@@ -2629,14 +2682,25 @@ int fdtd_read_probes(fdtd_handle *h, float *out, int32_t max_samples, int32_t *n
   hipSetDevice(h->device);
   *nsamples = 0;
   if (!h->nprobe) return FDTD_OK;
-  int cnt = 0;
-  HIPCHK(h, hipMemcpyAsync(&cnt, h->dpcount, 4, hipMemcpyDeviceToHost, h->stream));
+  // One copy of the count and the samples this handle counted (a caller's own
+  // recorded steps may have taken more: a second copy), and the count cleared
+  // on the stream: 54 us a read with four transfers and their waits, 28 us so
+  // (both with the Python around it).
+  const size_t row = (size_t)h->nprobe * 4;
+  const int known = (int)std::min<long long>(std::min<long long>(h->pbuffered, h->pcap), std::max(max_samples, 0));
+  std::vector<char> img(16 + (size_t)known * row);
+  HIPCHK(h, hipMemcpyAsync(img.data(), h->dpcount, img.size(), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  int cnt;
+  std::memcpy(&cnt, img.data(), 4);
   if (cnt > max_samples) return fail(h, FDTD_ERR_ARG, "%d samples buffered, room for %d", cnt, max_samples);
-  if (cnt) HIPCHK(h, hipMemcpy(out, h->dpbuf, (size_t)cnt * h->nprobe * 4, hipMemcpyDeviceToHost));
-  const int zero = 0;
-  HIPCHK(h, hipMemcpyAsync(h->dpcount, &zero, 4, hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  std::memcpy(out, img.data() + 16, (size_t)std::min(cnt, known) * row);
+  if (cnt > known) {
+    HIPCHK(h, hipMemcpyAsync(out + (size_t)known * h->nprobe, h->dpbuf + (size_t)known * h->nprobe,
+                             (size_t)(cnt - known) * row, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+  }
+  HIPCHK(h, (hipError_t)launch_set_step(h->dpcount, 0, h->stream));
   h->pbuffered = 0;
   *nsamples = cnt;
   return FDTD_OK;

@@ -226,6 +226,8 @@ struct PassSrc {
 // of an observation launch that prepare the next step's): faces[0..nf0) act
 // on E, faces[nf0..nf) on H; face q's cells are out[start[q]] ..
 // out[start[q+1]-1], the face's first free axis fastest.
+// A face's terms do not depend on an axis its wave's directions have no
+// component along: its ranges here then hold one index of that axis.
 struct PwTerms {
   const PwFace *faces;
   const long long *start;
@@ -268,9 +270,22 @@ struct Observe {
   int np, cap;
   const DftDev *dft;          // frequency-domain boxes (device), in the order
   int ndft;                   // of their start
-  long long total;            // (point, frequency) pairs of all boxes
-  PwTerms pw;                 // the next step's TF/SF terms (pw.total 0: none)
+  PwTerms pw;                 // the next step's TF/SF terms
   const int *dn;              // device step counter (null: the launch's n)
+};
+
+// What one launch does of it, at step n (or *dn + n).  The E quantities may be
+// taken while the H pass of the step runs (it only reads E), the H quantities
+// while the E pass of the next step does; either part adds its probes to row
+// *count + row.
+struct ObservePart {
+  Observe o;
+  int half;                   // 0: the E quantities, 1: H, 2: both
+  int sample;                 // sample the half's probes,
+  int row, advance;           // ... and then move *count
+  int n;
+  long long d0, d1;           // its (point, frequency) pairs
+  long long w0, w1;           // its cells of pw
 };
 
 // TF/SF faces per half that a one-launch step handles (one bit each in the
@@ -398,6 +413,7 @@ struct BatchDev {
   // is qtiles[t], box b of grid g is qboxes[g * kQuadBoxes + b]
   QuadTile *qtiles;
   const QuadBox *qboxes;
+  int n;                      // the step's place in the recorded sequence
 };
 
 #ifdef __HIPCC__
@@ -472,7 +488,8 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
   int launch_h(const DevGrid &g, const TileMap &tm, const int *tmed,        \
                int yee, int cpml, int ade, const PassSrc *src, void *stream); \
   int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, \
-                  const int *tmed, int half, const PassSrc &src, void *stream); \
+                  const int *tmed, int half, const PassSrc &src,            \
+                  const ObservePart *obs, void *stream);                     \
   int launch_quad_batch(const BatchDev &bd, int half, int rows, size_t lds, \
                         int fp16, void *stream);                             \
   int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows,      \
@@ -505,11 +522,8 @@ int launch_nodal(const DevGrid &g, const NodalCell *cells, int ncells,
 // *dn += by / *dn = n
 int launch_tick(int *dn, int by, void *stream);
 int launch_set_step(int *dn, int n, void *stream);
-// the observation of a grid at step n: probes sampled (when probes),
-// frequency-domain sums advanced (when dft), the TF/SF terms of step n + 1
-// written (when pw)
-int launch_observe(const DevGrid &g, const Observe &o, int n, int probes, int dft, int pw,
-                   void *stream);
+// (a part of) the observation of a grid
+int launch_observe(const DevGrid &g, const ObservePart &p, void *stream);
 // the TF/SF terms of step n (or *dn + n)
 int launch_pw_terms(const PwTerms &t, int n, const int *dn, void *stream);
 // the terms of many grids, each at its own *dn
@@ -519,14 +533,15 @@ struct PwTermsGrid {
 };
 int launch_pw_terms_many(const PwTermsGrid *grids, int n, long long maxcells, void *stream);
 // the same for many grids: blocks start[s] .. start[s+1]-1 of the launch
-// serve obs[s] on grids[grid[s]]
+// serve obs[s] on its grid, at step n of each
 struct ObserveGrid {
-  Observe o;
+  ObservePart p;
   int grid;
 };
 int launch_observe_many(const DevGrid *grids, const ObserveGrid *obs, const int *start, int nobs,
-                        int blocks, void *stream);
-int observe_blocks(const Observe &o);
+                        int blocks, int n, void *stream);
+// blocks of nt threads of a part
+int observe_blocks(const ObservePart &p, int nt);
 // a group of TF/SF faces at step n (or each run's *dn): F += sign * G *
 // Incid(t) * id, t the real(4) time stamp of the half step (E: tiempo(n), H:
 // tiempo(n) + dt/2); runs[r] covers cells start[r] .. start[r+1]-1 of total
@@ -563,8 +578,8 @@ int launch_pw_incident(const PwFace *faces, int nf0, int nf, long long maxcells,
 // maxcells: the most cells of a face)
 int launch_pw_incident_many(const PwIncJob *jobs, int njobs, int maxnf, long long maxcells,
                             void *stream);
-// increments every counter of the list (per-grid step counters of a batch)
-int launch_tick_many(int *const *counters, int n, void *stream);
+// adds by to every counter of the list (per-grid step counters of a batch)
+int launch_tick_many(int *const *counters, int n, int by, void *stream);
 // bounding box {xmin,ymin,zmin,xmax,ymax,zmax} of the dispersive edges of
 // component comp; out must hold {INT_MAX x3, INT_MIN x3} on entry
 int launch_disp_bbox(const DevGrid &g, int side, int c, int32_t *out, void *stream);

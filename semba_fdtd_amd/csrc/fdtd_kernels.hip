@@ -731,7 +731,7 @@ __global__ void __launch_bounds__(256) k_pass_batch(BatchDev bd) {
     const int m0 = bd.tmed ? __builtin_amdgcn_readfirstlane(bd.tmed[t]) : -1;
     if (H) hpass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
     else epass_tile<true, true, true, T, X, CDevGrid, CPassSrc>(cg, tm, tab, blk, m0, xs, fal);
-    if (X) tile_nodal<T>(g, tm, *xs, blk);
+    if (X) tile_nodal<T>(g, tm, *xs, blk, bd.n);
   }
 }
 

@@ -1,4 +1,5 @@
 // fdtd_quad.hip -- kernels of the four-cell face passes of one grid (fdtd_quad.h).
+#include "fdtd_observe.h"
 #include "fdtd_quad.h"
 
 namespace sfd {
@@ -11,6 +12,9 @@ struct QuadArgs {
   QuadPlan p;
   const int *tmed;
   PassSrc x;      // the half's sources
+  int nobs;       // blocks ahead of the tiles' that observe (a multiple of 8:
+                  // the tiles keep their XCDs)
+  ObservePart obs;
 };
 typedef __attribute__((address_space(4))) QuadArgs CQuadArgs;
 
@@ -52,10 +56,14 @@ __device__ __forceinline__ void run_quad(const G &g, float2 *lds, int info, cons
 
 // SLABS, X: what the launch's tiles may meet
 template <bool H, int SLABS, bool X, class T>
-__global__ void __launch_bounds__(256) k_quad(QuadArgs) {
+__global__ void __launch_bounds__(256, SLABS == 0 && !X ? 6 : 1) k_quad(QuadArgs) {
   extern __shared__ float2 lds_tab[];
   const CQuadArgs &a = *(const CQuadArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-  const int t = xcd_remap(blockIdx.x, a.p.nblk);
+  if ((int)blockIdx.x < a.nobs) {
+    observe_block(a.g, a.obs, a.obs.n, (int)blockIdx.x, (int)(blockDim.x * blockDim.y));
+    return;
+  }
+  const int t = xcd_remap((int)blockIdx.x - a.nobs, a.p.nblk);
   const int info = ro_uniform_i(a.tmed, t);
   QuadPos at;
   const bool live = quad_pos(a.p, t, at);
@@ -86,7 +94,8 @@ __global__ void __launch_bounds__(256) k_quad_batch(BatchDev bd) {
   if (info & kTileSlabs) run_quad<H, kSlabAll, false, T>(g, lds_tab, info, at, live, x);
   else run_quad<H, kSlabX, X, T>(g, lds_tab, info, at, live, x);
   if (X && (info & kTileNodal[H ? 1 : 0]))
-    nodal_cells<T>(g, x, ro_uniform_i(x.nstart, qt.tg), ro_uniform_i(x.nstart, qt.tg + 1));
+    nodal_cells<T>(g, x, ro_uniform_i(x.nstart, qt.tg), ro_uniform_i(x.nstart, qt.tg + 1),
+                   bd.n);
 }
 
 int launch_quad_batch(const BatchDev &bd, int half, int rows, size_t lds, int fp16, void *stream) {
@@ -160,10 +169,14 @@ int launch_quad_media_batch(const BatchDev &bd, int rows, void *stream) {
 }
 
 int launch_quad(const DevGrid &g, const QuadPlan &p, int slabs, int rows, const int *tmed,
-                int half, const PassSrc &src, void *stream) {
+                int half, const PassSrc &src, const ObservePart *obs, void *stream) {
   if (p.nblk <= 0) return 0;
-  const QuadArgs a{g, p, tmed, src};
-  const dim3 grid((unsigned)p.nblk), blk(kWave, (unsigned)rows);
+  QuadArgs a{g, p, tmed, src, 0, {}};
+  if (obs) {
+    a.obs = *obs;
+    a.nobs = (observe_blocks(*obs, kWave * rows) + 7) & ~7;
+  }
+  const dim3 grid((unsigned)(p.nblk + a.nobs)), blk(kWave, (unsigned)rows);
   const size_t tab = (size_t)(g.nmedia + 1) * sizeof(float2);
   const size_t lds = src.nface ? face_lds_offset(tab) + kPassFaces * sizeof(FaceAddr) : tab;
   hipStream_t s = (hipStream_t)stream;

@@ -8,7 +8,7 @@ import pytest
 import semba_fdtd_amd as sf
 from semba_fdtd_amd import problem as P
 
-STEPS = 12
+STEPS = 24
 SPLIT = ("advance_e_yee", "advance_e_cpml", "advance_e_dispersive", "advance_planewave_e",
          "advance_nodal_e", "advance_h_yee", "advance_h_cpml", "advance_h_dispersive",
          "advance_planewave_h", "advance_nodal_h", "advance_mur")
@@ -133,3 +133,26 @@ def test_batch_quads_equal_alone(storage, narrow):
         for q, s in enumerate(sol):
             assert same([s.field(c) for c in range(6)], want[q]), (tiling, q)
         b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wave", [False, True])
+def test_observation_in_the_passes(wave):
+    """Probes of all components and frequency-domain boxes of H before E, in
+    runs of the 16-step and the one-step graph, against call by call."""
+    pb = build((67, 15, 14), ((8, 8), (3, 2), (2, 3)), wave)
+    pb.dfts = [P.DftBox(1, (0, 66, 3, 6, 4, 6), (3, 1, 1), [0.7e9, 1.9e9]),
+               P.DftBox(0, (1, 60, 2, 9, 3, 3), (2, 2, 1), [1.1e9])]
+    a, b = sf.Solver(pb), sf.Solver(pb)
+    for n in (1, 5, 6):
+        a.run(n)
+    for _ in range(12):
+        b.step()
+    assert np.array_equal(a.probes().view(np.uint32), b.probes().view(np.uint32))
+    for x, y in zip(a.dft_sums(), b.dft_sums()):
+        assert np.abs(x).max() > 0 and np.array_equal(x.view(np.uint64), y.view(np.uint64))
+    a.set_graph_steps(4)
+    a.run(9)
+    for _ in range(9):
+        b.step()
+    assert np.array_equal(a.probes().view(np.uint32), b.probes().view(np.uint32))
