@@ -169,6 +169,10 @@ struct fdtd_handle {
                                   // rows than step_rows runs the step's tiles cut
                                   // into row bands
   bool step_vec = true;           // plain tiles run four x cells per lane (k_step4)
+  // the branches of a recorded one-launch step
+  hipStream_t side[2] = {};
+  hipEvent_t forked = nullptr, joined[2] = {};
+  int cus = 256;                  // compute units of the device
   int lds_max = 65536;            // LDS bytes a block may use on the device
   bool step_ready = false;
   bool step_stale = true;         // B's fields must be refreshed from A

@@ -762,6 +762,14 @@ int build_step(fdtd_handle *h) {
     StepPlan plan;
     std::string perr;
     if (plan_step(pg, &plan, &perr)) return fail(h, FDTD_ERR_ARG, "%s", perr.c_str());
+    // The plain tiles run one block a compute unit: merged over 64 planes those
+    // of a mid-size grid are a wave and a bit of blocks, the second of it nearly
+    // empty.  Unmerged below eight blocks a unit: 256^3 1018 -> 624 us per step
+    // (64 tiles), 320^3 1038 -> 890 (200), 500x444x390 2452 -> 2339 (336).
+    if (plan.tiles[0].size() + plan.tiles[kPlanVec].size() < 8u * (unsigned)h->cus) {
+      pg.zrun = pg.kc;
+      if (plan_step(pg, &plan, &perr)) return fail(h, FDTD_ERR_ARG, "%s", perr.c_str());
+    }
     std::vector<StepTile> all;
     h->step_cls.clear(); h->step_cnt.clear(); h->step_off.clear(); h->step_cells.clear();
     h->step_bytes.clear();
@@ -912,25 +920,82 @@ static StepDev class_sd(const fdtd_handle *h, int dir, size_t q) {
   return sd;
 }
 
-static int launch_class(const fdtd_handle *h, const StepDev &sd, size_t q) {
+static int launch_class(const fdtd_handle *h, const StepDev &sd, size_t q, hipStream_t s) {
   const int nuni = h->step_uni[q];
   return h->mode == FDTD_MODE_EXACT
-             ? exact::launch_step(sd, h->step_crows[q], h->step_cls[q], nuni, h->stream)
-             : fast::launch_step(sd, h->step_crows[q], h->step_cls[q], nuni, h->stream);
+             ? exact::launch_step(sd, h->step_crows[q], h->step_cls[q], nuni, s)
+             : fast::launch_step(sd, h->step_crows[q], h->step_cls[q], nuni, s);
 }
 
-static int launch_step_kernels(fdtd_handle *h, int dir, bool exact_prev = false) {
+// The branches of a recorded step: its classes write cells of their own and
+// read the other state copy, so they may run side by side.  Each ends in a wave
+// of blocks that leaves most of the chip idle, which on grids up to kForkCells
+// is a large part of it: us per step, one branch / three, 256^3 626 / 515,
+// 400^3 1414 / 1322, 500x444x390 2339 / 2067, 600^3 4186 / 4024, 800x640x640
+// 5654 / 5560.  1024^3 loses more to the classes competing for memory: 20.4 /
+// 21.4 ms.
+constexpr int kBranches = 3;
+constexpr double kForkCells = 5e8;
+
+// the branch of each class: the heaviest first, each to the least loaded
+// (boundary classes take about four times their bytes)
+static std::vector<int> class_branches(const fdtd_handle *h) {
+  const size_t n = h->step_cls.size();
+  std::vector<size_t> by(n);
+  std::vector<double> w(n);
+  for (size_t q = 0; q < n; ++q) {
+    by[q] = q;
+    const int c = h->step_cls[q] >= kPlanHalf ? h->step_cls[q] - kPlanHalf : h->step_cls[q];
+    w[q] = h->step_bytes[q] * (h->step_cls[q] != kPlanVec && (c & 5) ? 4.0 : 1.0);
+  }
+  std::stable_sort(by.begin(), by.end(), [&](size_t a, size_t b) { return w[a] > w[b]; });
+  double load[kBranches] = {};
+  std::vector<int> at(n);
+  for (size_t q : by) {
+    const int b = (int)(std::min_element(load, load + kBranches) - load);
+    at[q] = b;
+    load[b] += w[q];
+  }
+  return at;
+}
+
+// the side streams and events of the branches (default priority), kept for
+// the life of the handle
+static int make_branches(fdtd_handle *h) {
+  for (int b = 0; b + 1 < kBranches; ++b) {
+    if (!h->side[b]) HIPCHK(h, hipStreamCreateWithFlags(&h->side[b], hipStreamNonBlocking));
+    if (!h->joined[b]) HIPCHK(h, hipEventCreateWithFlags(&h->joined[b], hipEventDisableTiming));
+  }
+  if (!h->forked) HIPCHK(h, hipEventCreateWithFlags(&h->forked, hipEventDisableTiming));
+  return FDTD_OK;
+}
+
+// fork: into branches (while recording, after make_branches)
+static int launch_step_kernels(fdtd_handle *h, int dir, bool exact_prev, bool fork) {
   if (h->step_nf > 0 &&
       launch_pw_incident(h->dsfaces, h->step_nf0, h->step_nf, h->step_maxcells, h->dstepsrc,
                          h->dstep, h->dinc, h->stream))
     return fail(h, FDTD_ERR_HIP, "incident-field launch failed");
-  for (size_t q = 0; q < h->step_cls.size(); ++q) {
+  std::vector<int> at(h->step_cls.size(), 0);
+  if (fork) {
+    at = class_branches(h);
+    HIPCHK(h, hipEventRecord(h->forked, h->stream));
+    for (int b = 0; b + 1 < kBranches; ++b) HIPCHK(h, hipStreamWaitEvent(h->side[b], h->forked, 0));
+  }
+  int e = 0;
+  for (size_t q = 0; q < h->step_cls.size() && !e; ++q) {
     StepDev sd = class_sd(h, dir, q);
     sd.prev_from_field = exact_prev ? 0 : 1;
     sd.lazy_prev = 1;
-    const int e = launch_class(h, sd, q);
-    if (e) return fail(h, FDTD_ERR_HIP, "step launch failed: %s", hipGetErrorString((hipError_t)e));
+    e = launch_class(h, sd, q, at[q] ? h->side[at[q] - 1] : h->stream);
   }
+  // (the branches join whatever failed: a recording may not end with one open)
+  if (fork)
+    for (int b = 0; b + 1 < kBranches; ++b) {
+      HIPCHK(h, hipEventRecord(h->joined[b], h->side[b]));
+      HIPCHK(h, hipStreamWaitEvent(h->stream, h->joined[b], 0));
+    }
+  if (e) return fail(h, FDTD_ERR_HIP, "step launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
 
@@ -950,9 +1015,9 @@ static int settle_prev(fdtd_handle *h) {
   return FDTD_OK;
 }
 
-static int run_step(fdtd_handle *h, int dir, bool exact_prev = false) {
+static int run_step(fdtd_handle *h, int dir, bool exact_prev = false, bool fork = false) {
   const StepDev &sd = h->sd[dir];
-  int e = launch_step_kernels(h, dir, exact_prev);
+  int e = launch_step_kernels(h, dir, exact_prev, fork);
   if (e) return e;
   if (!h->mur_runs.empty() &&
       launch_mur(sd.go, h->dmur, (int)h->mur_runs.size(), h->mur_total,
@@ -1842,6 +1907,7 @@ int fdtd_create(const fdtd_grid_desc *d, fdtd_handle **out) {
   h->mode = d->mode;
   h->storage = d->storage;
   h->lds_max = (int)std::min<size_t>(prop.sharedMemPerBlock, 1u << 30);
+  h->cus = prop.multiProcessorCount;
   if (hipSetDevice(d->device) != hipSuccess) { delete h; return fail(nullptr, FDTD_ERR_DEVICE, "hipSetDevice failed"); }
   if (d->stream) {
     h->stream = (hipStream_t)d->stream;
@@ -1920,6 +1986,10 @@ int fdtd_destroy(fdtd_handle *h) {
   for (void *p : h->allocs) hipFree(p);
   if (h->stage) hipFree(h->stage);
   if (h->tmed) hipFree(h->tmed);
+  for (hipStream_t q : h->side)
+    if (q) hipStreamDestroy(q);
+  for (hipEvent_t q : {h->forked, h->joined[0], h->joined[1]})
+    if (q) hipEventDestroy(q);
   if (h->qmed) hipFree(h->qmed);
   if (h->solo_stream) h->stream = h->solo_stream;
   if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
@@ -2398,10 +2468,11 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
   const int pairs = paired ? nsteps / 2 : 0;
   const int singles = paired ? nsteps % 2 : nsteps;
   if (pairs > 0 && !h->pexec) {
-    if ((rc = build_step(h))) return rc;
+    const bool fork = (double)cells_of(h) <= kForkCells;
+    if ((rc = build_step(h)) || (fork && (rc = make_branches(h)))) return rc;
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    int r2 = run_step(h, 0);
-    if (!r2) r2 = run_step(h, 1);
+    int r2 = run_step(h, 0, false, fork);
+    if (!r2) r2 = run_step(h, 1, false, fork);
     hipGraph_t graph = nullptr;
     hipError_t ec = hipStreamEndCapture(h->stream, &graph);
     if (r2) { if (graph) hipGraphDestroy(graph); return r2; }
@@ -2555,7 +2626,7 @@ int fdtd_time_step(fdtd_handle *h, int32_t reps, float *ms) {
   // the step kernels alone, in pairs so that the state ends in A
   auto pair = [&]() -> int {
     for (int dir = 0; dir < 2; ++dir) {
-      const int e = launch_step_kernels(h, dir);
+      const int e = launch_step_kernels(h, dir, false, false);
       if (e) return e;
     }
     return FDTD_OK;
@@ -2615,7 +2686,7 @@ int fdtd_step_classes(fdtd_handle *h, int32_t reps, int32_t cls[FDTD_STEP_CLASSE
     StepDev sd = class_sd(h, 0, (size_t)q);
     sd.prev_from_field = 1;
     sd.lazy_prev = 1;
-    auto one = [&]() { return launch_class(h, sd, (size_t)q); };
+    auto one = [&]() { return launch_class(h, sd, (size_t)q, h->stream); };
     if (one()) { rc = fail(h, FDTD_ERR_HIP, "step launch failed"); break; }
     hipEventRecord(ev[0], h->stream);
     for (int r = 0; r < reps && !rc; ++r)

@@ -190,7 +190,7 @@ int plan_step(const PlanGeom &g, StepPlan *out, std::string *err) {
   for (const Seg &s : sy) split(s.lo, s.hi, Wy, 1, &yt);
   for (const Seg &s : sz) split(s.lo, s.hi, kc, 1, &zt);
   // tiles in z order of chunks, rows, columns (x fastest); plain tiles merge
-  // with the plain tiles above them into runs of up to 64 planes
+  // with the plain tiles above them into runs of up to zrun planes
   for (int c = 0; c < kPlanClasses; ++c) {
     out->tiles[c].clear();
     out->owned[c] = out->psi[c] = out->disp[c][0] = out->disp[c][1] = 0.0;
@@ -314,7 +314,7 @@ int plan_step(const PlanGeom &g, StepPlan *out, std::string *err) {
           const Seg &s = pieces[q];
           const bool mergeable = cls == 0 || cls == 8;
           if (p.open && mergeable && p.cls == cls && p.x0 == s.lo && p.wx == s.hi - s.lo &&
-              p.k1 == z.lo && z.hi - p.k0 <= 64) {
+              p.k1 == z.lo && z.hi - p.k0 <= g.zrun) {
             p.k1 = z.hi;
             continue;
           }

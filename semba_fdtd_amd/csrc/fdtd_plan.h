@@ -34,6 +34,7 @@ struct PlanGeom {
                      // owns up to 2 hrows - 1 rows)
   int vrows;         // rows per block of the four-cell kernel (<= R)
   bool vec;          // plain tiles may run four x cells per lane
+  int zrun = 64;     // planes that plain tiles above each other merge up to
   std::vector<PlanBox> boxes;
 };
 
