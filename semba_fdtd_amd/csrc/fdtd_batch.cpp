@@ -3,18 +3,21 @@
 // A batch holds grids that were set up as single grids (fdtd_create and the
 // set-up calls); admitting one hands its device state to the batch without
 // copying.  One step of the batch runs, for every grid at its own step:
-//   E face pass of all grids          one persistent launch (k_pass_batch)
+//   E face pass of all grids          one launch over a list of all grids'
+//                                     tiles (k_quad_batch), or a persistent
+//                                     one (k_pass_batch) where some grid
+//                                     cannot run four cells per lane
 //   pole stage                        one launch for the grids with poles
 //   plane-wave E faces                inside the pass, or one launch per (wave,
 //                                     face axis) group of the grids that cannot
 //   nodal E                           inside the pass, or one launch per grid
 //                                     that cannot
-//   H face pass of all grids          one persistent launch
+//   H face pass of all grids          as the E pass
 //   plane-wave H faces, nodal H       as above
 //   probes, frequency-domain sums,
 //   the next step's TF/SF terms       one launch for all grids
-//   step counters                     one launch for all grids
-// captured once per membership in a HIP graph and replayed.  Each grid keeps
+//   step counters                     one launch for all grids per graph
+// captured once per membership in HIP graphs of eight steps and of one.  Each grid keeps
 // its own step counter (its dstep), so grids admitted at different times
 // advance in lock-step from different n.
 //
