@@ -125,12 +125,14 @@ struct fdtd_handle {
   double *dtiempo = nullptr;
   // the faces of each half as the face passes apply them inline (pw_masks:
   // at most kPassFaces, all inside their components' sweeps), and the buffer
-  // of both halves' terms, which holds those of step pw_terms_n (-1: none)
+  // of both halves' terms, which holds those of step pw_terms_n (-1: none) until
+  // a caller has recorded a step that writes it (pw_recorded)
   bool pw_masks[2] = {false, false};
   sfd::PassSrc pw_src[2] = {};
   std::vector<unsigned> pw_bits[2][3];  // host copy of the faces' index masks
   sfd::PwTerms pw_terms{};
   int pw_terms_n = -1;
+  bool pw_recorded = false;
   long long pw_split = 0;          // terms of the E faces
   // per half, under the pass tiling tm: the sources the one-cell pass applies
   // (valid while tmed_ready)

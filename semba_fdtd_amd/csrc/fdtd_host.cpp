@@ -1837,20 +1837,25 @@ bool inline_faces(const fdtd_handle *h) {
   return ((h->psrc_on[0] && h->psrc[0].nface) || (h->psrc_on[1] && h->psrc[1].nface));
 }
 
+// Does the terms' buffer hold step n's.  A caller's own capture replays without
+// these calls: it records the launch, and from then on any replay may have
+// written the buffer, so every call writes the terms it needs.
+bool have_terms(fdtd_handle *h, int n) {
+  h->pw_recorded = h->pw_recorded || stream_capturing(h);
+  return !h->pw_recorded && h->pw_terms_n == n;
+}
+
 // the terms of step n in the buffer, unless the observation of step n - 1
 // left them there
 int need_terms(fdtd_handle *h, int n) {
-  if (!inline_faces(h)) return FDTD_OK;
-  // a caller's own capture replays without this call: it records the launch
-  const bool capturing = stream_capturing(h);
-  if (!capturing && h->pw_terms_n == n) return FDTD_OK;
+  if (!inline_faces(h) || have_terms(h, n)) return FDTD_OK;
   if (n < 0 || n >= (int)h->tiempo.size())
     return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
                 (int)h->tiempo.size() - 1);
   h->pw_terms_n = -1;
   if (launch_pw_terms(h->pw_terms, n, nullptr, h->stream))
     return fail(h, FDTD_ERR_HIP, "incident-field launch failed");
-  if (!capturing) h->pw_terms_n = n;
+  h->pw_terms_n = n;
   return FDTD_OK;
 }
 
@@ -2348,7 +2353,7 @@ int fdtd_update_observation(fdtd_handle *h, int32_t n) {
   const bool in = n >= 0 && n < (int)h->tiempo.size();
   // the terms of the next step ride along when the steps run call by call
   const bool pw = in && h->tmed_ready && inline_faces(h) && n + 1 < (int)h->tiempo.size() &&
-                  h->pw_terms_n == n && !stream_capturing(h);
+                  have_terms(h, n);
   if ((rc = run_observe(h, h->g, observe_part(h, 2, n, nullptr, true, in, pw)))) return rc;
   if (pw) h->pw_terms_n = n + 1;
   h->pbuffered += h->nprobe ? 1 : 0;

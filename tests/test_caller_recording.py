@@ -1,0 +1,146 @@
+"""Steps that a caller records on the grid's stream (hipStreamBeginCapture
+around the step calls) and replays, mixed with direct calls and runs: the same
+bits as the same steps called directly.  A recorded call has to do by itself
+what it does when called, whatever ran or was replayed in between."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import semba_fdtd_amd as sf
+from semba_fdtd_amd import problem as P
+
+pytestmark = pytest.mark.gpu
+
+STEPS = 30
+
+
+class Recorder:
+    """A stream of the library's own HIP runtime, and recordings of it."""
+
+    def __init__(self):
+        self.hip = sf.load_library()     # its dependencies resolve through it
+        self.stream = C.c_void_p()
+        self._do("hipStreamCreateWithFlags", C.byref(self.stream), 1)
+        self.graphs = []
+
+    def _do(self, name, *args):
+        f = getattr(self.hip, name)
+        f.restype = C.c_int
+        rc = f(*args)
+        assert rc == 0, (name, rc)
+
+    def record(self, calls):
+        graph, ex = C.c_void_p(), C.c_void_p()
+        self._do("hipStreamBeginCapture", self.stream, 1)
+        try:
+            calls()
+        finally:
+            self._do("hipStreamEndCapture", self.stream, C.byref(graph))
+        self._do("hipGraphInstantiate", C.byref(ex), graph, None, None, C.c_size_t(0))
+        self.graphs.append((graph, ex))
+        return ex
+
+    def replay(self, ex):
+        self._do("hipGraphLaunch", ex, self.stream)
+
+    def close(self):
+        self._do("hipStreamSynchronize", self.stream)
+        for graph, ex in self.graphs:
+            self._do("hipGraphExecDestroy", ex)
+            self._do("hipGraphDestroy", graph)
+        self._do("hipStreamDestroy", self.stream)
+
+
+@pytest.fixture
+def rec():
+    r = Recorder()
+    yield r
+    r.close()
+
+
+def step(s, n):
+    for name in ("advance_e", "advance_h", "update_observation"):
+        assert getattr(s.lib, "fdtd_" + name)(s.h, n) == 0, s.lib.fdtd_last_error(s.h)
+
+
+def fields(s):
+    return [s.field(c) for c in range(6)]
+
+
+def same(a, b):
+    return all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(a, b))
+
+
+def wave_problem(nodal=False):
+    pb = P.scatterer_problem(n=(40, 30, 28), L=((4, 5), (3, 4), (5, 3)), nsteps=4 * STEPS, disp=False)
+    if not nodal:
+        pb.nodal = []
+    q = np.arange(STEPS + 5)
+    ev = (np.sin(q / 3.0) * (1 - np.exp(-q / 2.0))).astype(np.float32)
+    pb.planewaves = [P.PlaneWave((6, 33, 5, 24, 7, 23), [(0.48, 0.64, 0.6)], [(0.8, -0.6, 0.0)], ev,
+                                 float(np.float32(pb.dt)))]
+    pb.probes = []
+    return pb
+
+
+@pytest.mark.parametrize("tiling", [None, (2, 4, 1)])
+@pytest.mark.parametrize("then", ["advance", "run"])
+def test_direct_steps_after_a_replay(rec, tiling, then):
+    """Ten steps called directly leave the plane wave's next terms behind; a
+    replay of recorded steps writes the terms of its own.  The steps that
+    follow need theirs."""
+    pb = wave_problem()
+
+    def grid(**kw):
+        s = sf.Solver(pb, **kw)
+        if tiling:
+            s.set_tiling(*tiling)
+        return s
+
+    ref = grid()
+    for n in range(16):
+        step(ref, n)
+    want = fields(ref)
+    s = grid(stream=rec.stream)
+    start = s.save_state()
+    for n in range(10):
+        step(s, n)
+    s.load_state(start)
+    ten = rec.record(lambda: [step(s, n) for n in range(10)])
+    for _ in range(3):
+        s.load_state(start)
+        for n in range(10):
+            step(s, n)
+        s.load_state(start)
+        rec.replay(ten)
+        if then == "run":
+            assert s.lib.fdtd_run(s.h, 10, 6) == 0
+        else:
+            for n in range(10, 16):
+                step(s, n)
+        assert np.abs(want[0]).max() > 0
+        assert same(fields(s), want)
+    s.close()
+
+
+def test_half_steps_after_a_replay(rec):
+    """A recorded step replayed between the halves of a direct one (on a
+    saved state of its own) leaves the second half its terms."""
+    pb = wave_problem()
+    ref = sf.Solver(pb)
+    for n in range(12):
+        step(ref, n)
+    want = fields(ref)
+    s = sf.Solver(pb, stream=rec.stream)
+    for n in range(10):
+        step(s, n)
+    three = rec.record(lambda: step(s, 3))
+    assert s.lib.fdtd_advance_e(s.h, 10) == 0
+    mid = s.save_state()
+    rec.replay(three)
+    s.load_state(mid)
+    assert s.lib.fdtd_advance_h(s.h, 10) == 0
+    step(s, 11)
+    assert same(fields(s), want)
+    s.close()
