@@ -134,8 +134,10 @@ struct fdtd_handle {
   int pw_terms_n = -1;
   bool pw_recorded = false;
   long long pw_split = 0;          // terms of the E faces
-  // per half, under the pass tiling tm: the sources the one-cell pass applies
-  // (valid while tmed_ready)
+  // per half: the sources the pass applies inline under the tiling (valid while
+  // psrc_gen == src_gen).  src_gen counts the changes of the tiling, the sources
+  // and the pole-state boxes.
+  unsigned src_gen = 1, psrc_gen = 0;
   bool psrc_on[2] = {false, false};
   sfd::PassSrc psrc[2] = {};
   std::vector<void *> psrc_allocs;
@@ -189,13 +191,13 @@ struct fdtd_handle {
   std::vector<int> step_cls, step_cnt, step_off;
   std::vector<int> step_crows;           // rows per block of each class launch
   std::vector<int> step_uni;             // leading single-medium tiles of each class launch
-  // per tile of the one-cell pass map tm: the medium filling it, or -1
-  // (valid while tmed_ready; tiling and media changes clear it)
+  // the words of the tiles of the one-cell pass map tm (valid while tmed_ready;
+  // tiling and media changes clear it), tmed_cap of them, then their flags
   int *tmed = nullptr;
   int tmed_cap = 0;
   bool tmed_ready = false;
-  // the four-cell passes' tiles and their words (valid while tmed_ready and
-  // the grid runs these passes)
+  // the four-cell passes' tiles and their words and flags (valid while
+  // tmed_ready and the grid runs these passes)
   sfd_host::QuadLayout quad;
   int *qmed = nullptr;
   int qmed_cap = 0;

@@ -195,6 +195,7 @@ void set_tiles(fdtd_handle *h, int rows, int zchunk, int xcells) {
   const DevGrid &g = h->g;
   h->tile_zchunk = zchunk;
   h->xcells = xcells;
+  ++h->src_gen;
   TileMap &tm = h->tm;
   tm.bdy = rows;
   tm.tx = (g.nx + 1 + kWave - 1) / kWave;
@@ -300,60 +301,59 @@ void invalidate_graph(fdtd_handle *h) {
   h->tmed_ready = false;
 }
 
-// the medium of each tile of the one-cell pass map (or -1): the passes then
-// skip the media loads of single-medium tiles; and the sources the passes
-// apply inline.  Built outside any capture, before the passes it serves are
-// launched or recorded.
+// a device array of at least n words and n flags behind them
+static int tile_words(fdtd_handle *h, int **words, int *cap, int n) {
+  if (n <= *cap) return FDTD_OK;
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (*words) hipFree(*words);
+  *words = nullptr;
+  *cap = 0;
+  HIPCHK(h, hipMalloc(words, (size_t)n * 2 * sizeof(int)));
+  *cap = n;
+  return FDTD_OK;
+}
+
+// The words of the passes' tiles (kTileFaces): the flags say which sources a
+// tile meets, a launch over the media arrays adds the medium that fills it (the
+// passes skip the media loads of such tiles).  Built outside any capture the
+// library makes, before the passes it serves are launched or recorded.  The
+// flags and the sources' tables follow the tiling, the sources and the
+// pole-state boxes (src_gen); where only the media or the recorded graphs
+// changed the launch is all, and a caller may be recording it.
 int build_tile_media(fdtd_handle *h) {
   if (h->tmed_ready) return FDTD_OK;
-  h->psrc_on[0] = h->psrc_on[1] = false;
-  if (use_quads(h)) {
-    h->quad = plan_quads(h, h->tile_set ? h->tm.bdy : 0, h->tm.kc);
-    const int n = h->quad.p.nblk;
-    if (n > h->qmed_cap) {
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-      if (h->qmed) hipFree(h->qmed);
-      h->qmed = nullptr;
-      h->qmed_cap = 0;
-      HIPCHK(h, hipMalloc(&h->qmed, (size_t)n * sizeof(int)));
-      h->qmed_cap = n;
-    }
+  const bool quads = use_quads(h);
+  int **words = quads ? &h->qmed : &h->tmed, *cap = quads ? &h->qmed_cap : &h->tmed_cap;
+  int rc;
+  if (h->psrc_gen != h->src_gen) {
+    h->psrc_gen = 0;
+    h->psrc_on[0] = h->psrc_on[1] = false;
+    if (quads) h->quad = plan_quads(h, h->tile_set ? h->tm.bdy : 0, h->tm.kc);
+    const int n = quads ? h->quad.p.nblk : h->tm.nblk;
+    if ((rc = tile_words(h, words, cap, n))) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     for (void *p : h->psrc_allocs) hipFree(p);
     h->psrc_allocs.clear();
     std::vector<int> flags((size_t)n, 0);
-    for (int half = 0; half < 2; ++half)
-      if (int rc = make_quad_src(h, h->quad, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, flags.data()))
-        return rc;
-    HIPCHK(h, hipMemcpyAsync(h->qmed, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
+    for (int half = 0; half < 2; ++half) {
+      rc = quads ? make_quad_src(h, h->quad, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, flags.data())
+                 : make_pass_src(h, h->tm, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, &flags);
+      if (rc) return rc;
+    }
+    HIPCHK(h, hipMemcpyAsync(*words + *cap, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
                              h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    const int e = h->mode == FDTD_MODE_EXACT
-                      ? exact::launch_quad_media(h->g, h->quad.p, h->quad.rows, h->qmed, h->stream)
-                      : fast::launch_quad_media(h->g, h->quad.p, h->quad.rows, h->qmed, h->stream);
-    if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
-    h->tmed_ready = true;
-    return FDTD_OK;
+    h->psrc_gen = h->src_gen;
   }
-  if (h->tm.nblk > h->tmed_cap) {
-    if (h->tmed) hipFree(h->tmed);
-    h->tmed = nullptr;
-    h->tmed_cap = 0;
-    HIPCHK(h, hipMalloc(&h->tmed, (size_t)h->tm.nblk * sizeof(int)));
-    h->tmed_cap = h->tm.nblk;
-  }
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  for (void *p : h->psrc_allocs) hipFree(p);
-  h->psrc_allocs.clear();
-  std::vector<int> flags((size_t)h->tm.nblk, 0);
-  for (int half = 0; half < 2; ++half)
-    if (int rc = make_pass_src(h, h->tm, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, &flags))
-      return rc;
-  HIPCHK(h, hipMemcpyAsync(h->tmed, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
-                           h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  const int e = h->mode == FDTD_MODE_EXACT ? exact::launch_pass_tile_media(h->g, h->tm, h->tmed, h->stream)
-                                           : fast::launch_pass_tile_media(h->g, h->tm, h->tmed, h->stream);
+  int *const out = *words, *const flags = *words + *cap;
+  const bool exact = h->mode == FDTD_MODE_EXACT;
+  int e;
+  if (quads)
+    e = exact ? exact::launch_quad_media(h->g, h->quad.p, h->quad.rows, flags, out, h->stream)
+              : fast::launch_quad_media(h->g, h->quad.p, h->quad.rows, flags, out, h->stream);
+  else
+    e = exact ? exact::launch_pass_tile_media(h->g, h->tm, flags, out, h->stream)
+              : fast::launch_pass_tile_media(h->g, h->tm, flags, out, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
   h->tmed_ready = true;
   return FDTD_OK;
@@ -478,12 +478,14 @@ static int build_ade_side(fdtd_handle *h, int side) {
 
 int build_ade(fdtd_handle *h) {
   if (h->ade_ready) return FDTD_OK;
+  if (h->g.ade[0].has || h->g.ade[1].has) ++h->src_gen;
   for (void *p : h->ade_allocs) hipFree(p);
   h->ade_allocs.clear();
   for (int side = 0; side < 2; ++side) {
     const int rc = build_ade_side(h, side);
     if (rc) return rc;
   }
+  if (h->g.ade[0].has || h->g.ade[1].has) ++h->src_gen;
   h->ade_ready = true;
   return FDTD_OK;
 }
@@ -1032,6 +1034,7 @@ static int run_step(fdtd_handle *h, int dir, bool exact_prev = false, bool fork 
 int build_nodal(fdtd_handle *h) {
   if (h->nodal_ready) return FDTD_OK;
   if (h->srcs.empty()) { h->nodal_ready = true; return FDTD_OK; }
+  ++h->src_gen;
   if (h->tiempo.empty()) return fail(h, FDTD_ERR_STATE, "fdtd_set_time not called");
   std::vector<NodalCell> cells[2];
   for (int half = 0; half < 2; ++half) {
@@ -1446,6 +1449,7 @@ int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, boo
 // order the reference applies them.
 int build_planewaves(fdtd_handle *h) {
   if (h->pw_ready) return FDTD_OK;
+  if (!h->pwin.empty()) ++h->src_gen;
   for (void *p : h->pw_allocs) hipFree(p);
   h->pw_allocs.clear();
   h->pw_faces[0].clear();
@@ -2026,6 +2030,7 @@ int fdtd_set_media(fdtd_handle *h, int32_t nmedia, const float *g1, const float 
   h->mur_ready = false;
   h->nodal_ready = false;
   h->pw_ready = false;
+  ++h->src_gen;
   invalidate_graph(h);
   return FDTD_OK;
 }
@@ -2133,6 +2138,7 @@ int fdtd_set_cpml(fdtd_handle *h, const int32_t layers[6], const float *pbe_x,
   HIPCHK(h, hipStreamSynchronize(h->stream));
   g.has_cpml = any ? 1 : 0;
   h->pw_ready = false;
+  ++h->src_gen;
   invalidate_graph(h);
   return FDTD_OK;
 }

@@ -478,7 +478,7 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
 
 // launchers, one set per arithmetic mode.  tmed (null: none) holds, per
 // tile of the one-cell map tm, what the tile meets, as
-// launch_pass_tile_media writes it (out holds the flags on entry); the
+// launch_pass_tile_media writes it (its flags, plus its medium); the
 // one-cell passes skip the media loads of single-medium tiles.  src (null: none): the sources the fused
 // one-cell pass applies inline.
 #define SFD_DECLARE_LAUNCHERS(NS)                                              \
@@ -493,10 +493,10 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
   int launch_quad_batch(const BatchDev &bd, int half, int rows, size_t lds, \
                         int fp16, void *stream);                             \
   int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows,      \
-                        int *out, void *stream);                             \
+                        const int *flags, int *out, void *stream);           \
   int launch_quad_media_batch(const BatchDev &bd, int rows, void *stream);  \
-  int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, int *out,  \
-                             void *stream);                                  \
+  int launch_pass_tile_media(const DevGrid &g, const TileMap &tm,            \
+                             const int *flags, int *out, void *stream);      \
   size_t step_lds_bytes(const DevGrid &g, int rows, int npw, int kc);       \
   int launch_step(const StepDev &sd, int rows, int cls, int nuni, void *stream); \
   int launch_step_many(const StepDev *sds, const GridTile *tiles, int n, int narrow, int rows, \

@@ -139,12 +139,13 @@ __device__ __forceinline__ int tile_one_medium(const DevGrid &g, const QuadPos &
   return lo == hi ? lo + 1 : 0;
 }
 
-// adds it to the word of each tile: out[t], or the batch's qtiles[t].info
-__global__ void __launch_bounds__(256) k_quad_media(DevGrid g, QuadPlan p, int *out) {
+// the word of each tile: out[t] = flags[t] plus it, or added to the batch's
+// qtiles[t].info
+__global__ void __launch_bounds__(256) k_quad_media(DevGrid g, QuadPlan p, const int *flags, int *out) {
   QuadPos at;
   const bool live = quad_pos(p, (int)blockIdx.x, at);
   const int m = tile_one_medium(g, at, live);
-  if (threadIdx.x == 0 && threadIdx.y == 0) out[blockIdx.x] += m;
+  if (threadIdx.x == 0 && threadIdx.y == 0) out[blockIdx.x] = flags[blockIdx.x] + m;
 }
 __global__ void __launch_bounds__(256) k_quad_media_batch(BatchDev bd) {
   QuadTile &qt = bd.qtiles[blockIdx.x];
@@ -154,10 +155,11 @@ __global__ void __launch_bounds__(256) k_quad_media_batch(BatchDev bd) {
   if (threadIdx.x == 0 && threadIdx.y == 0) qt.info += m;
 }
 
-int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows, int *out, void *stream) {
+int launch_quad_media(const DevGrid &g, const QuadPlan &p, int rows, const int *flags, int *out,
+                      void *stream) {
   if (p.nblk <= 0) return 0;
   hipLaunchKernelGGL(k_quad_media, dim3((unsigned)p.nblk), dim3(kWave, (unsigned)rows), 0,
-                     (hipStream_t)stream, g, p, out);
+                     (hipStream_t)stream, g, p, flags, out);
   return (int)hipGetLastError();
 }
 

@@ -9,10 +9,12 @@ import pytest
 
 import semba_fdtd_amd as sf
 from semba_fdtd_amd import problem as P
+from semba_fdtd_amd._lib import i32p, ptr
 
 pytestmark = pytest.mark.gpu
 
 STEPS = 30
+PRIO = np.array([1000, 0, 20], np.int32)
 
 
 class Recorder:
@@ -143,4 +145,63 @@ def test_half_steps_after_a_replay(rec):
     assert s.lib.fdtd_advance_h(s.h, 10) == 0
     step(s, 11)
     assert same(fields(s), want)
+    s.close()
+
+
+@pytest.mark.parametrize("tiling", [None, (2, 4, 1)])
+def test_recording_after_a_media_change(rec, tiling):
+    """Media written since the last step, the sources as they were: the step
+    calls can be recorded at once."""
+    pb = wave_problem()
+    s = sf.Solver(pb, stream=rec.stream)
+    ref = sf.Solver(pb)
+    if tiling:
+        s.set_tiling(*tiling)
+    for q in (s, ref):
+        for n in range(12):
+            step(q, n)
+        assert q.lib.fdtd_media_paint_box(q.h, 12, 20, 10, 16, 9, 15, 2, 3, ptr(PRIO, i32p)) == 0
+    two = rec.record(lambda: [step(s, n) for n in (12, 13)])
+    rec.replay(two)
+    for n in (12, 13):
+        step(ref, n)
+    got, want = fields(s), fields(ref)
+    assert np.abs(want[0]).max() > 0 and same(got, want), tiling
+    s.close()
+
+
+@pytest.mark.parametrize("tiling", [None, (2, 4, 1)])
+def test_recording_outlives_what_drops_the_graphs(rec, tiling):
+    """Calls that only drop the library's own recorded steps (here the step
+    mode set again) leave a caller's recording what it reads: the sources'
+    tables stay where they are."""
+    pb = wave_problem(nodal=True)
+
+    def grid(**kw):
+        s = sf.Solver(pb, **kw)
+        if tiling:
+            s.set_tiling(*tiling)
+        return s
+
+    ref = grid()
+    for n in range(16):
+        step(ref, n)
+    want = fields(ref)
+    s = grid(stream=rec.stream)
+    start = s.save_state()
+    for n in range(10):
+        step(s, n)
+    s.load_state(start)
+    ten = rec.record(lambda: [step(s, n) for n in range(10)])
+    s.set_step_mode(0, 16)
+    step(s, 0)
+    others = [sf.Solver(P.scatterer_problem(nsteps=20)) for _ in range(3)]
+    for q in others:
+        q.run(5)
+    for _ in range(2):
+        s.load_state(start)
+        rec.replay(ten)
+        for n in range(10, 16):
+            step(s, n)
+        assert same(fields(s), want)
     s.close()
