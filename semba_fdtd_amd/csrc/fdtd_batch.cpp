@@ -290,16 +290,23 @@ int build_descriptors(fdtd_batch *b) {
       if (!h) continue;
       bool faces = false;
       for (int half = 0; half < 2; ++half) {
-        PassSrc ps;
-        bool on = false;
-        rc = b->quads ? make_quad_src(h, quad[(size_t)gi], half, &ps, &on, &b->allocs, &words[(size_t)start[(size_t)gi]])
-                      : make_pass_src(h, tms[(size_t)gi], half, &ps, &on, &b->allocs, nullptr);
-        if (rc)
-          return bfail(b, rc, "slot %zu: %s", s, h->err.c_str());
-        ps.dn = h->dstep;
-        b->inl[half][s] = on ? 1 : 0;
-        faces = faces || (on && ps.nface);
-        src[half].push_back(on ? ps : PassSrc{});
+        SrcTables t;
+        if (b->quads) make_quad_src(h, quad[(size_t)gi], half, &t, &words[(size_t)start[(size_t)gi]]);
+        else make_pass_src(h, tms[(size_t)gi], half, &t, nullptr);
+        if (!t.cells.empty()) {
+          int *ns = nullptr;
+          NodalCell *cells = nullptr;
+          if ((rc = bupload(b, &ns, t.nstart.data(), t.nstart.size())) ||
+              (rc = bupload(b, &cells, t.cells.data(), t.cells.size())))
+            return rc;
+          BCHK(b, hipStreamSynchronize(b->stream));   // (the copies read t)
+          t.src.nstart = ns;
+          t.src.cells = cells;
+        }
+        t.src.dn = h->dstep;
+        b->inl[half][s] = t.on ? 1 : 0;
+        faces = faces || t.src.nface;
+        src[half].push_back(t.on ? t.src : PassSrc{});
       }
       if (faces) {
         terms.push_back(PwTermsGrid{h->pw_terms, h->dstep});

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "fdtd_internal.h"
@@ -49,6 +50,15 @@ struct QuadLayout {
   int slabs = 0, rows = 1, kc = 1;
 };
 
+// the sources of a half that a pass applies inline, and its nodal cells' tables
+// (src.nstart and src.cells: their device copies, once placed)
+struct SrcTables {
+  bool on = false;
+  PassSrc src = {};
+  std::vector<int> nstart;
+  std::vector<NodalCell> cells;
+};
+
 struct PlaneWaveIn {     // sgg%PlaneWave(j) (planeonde_t, fdetypes.F90:458-465)
   int esq[6];            // esqx1, esqx2, esqy1, esqy2, esqz1, esqz2
   int nmodes;
@@ -73,6 +83,7 @@ struct fdtd_handle {
   bool tile_set = false;       // fdtd_set_tiling was called
   int tile_zchunk = 32;        // planes per z chunk as set (tm.kc: clipped to the grid)
   std::vector<void *> allocs;
+  std::unordered_map<void *, size_t> sizes;   // of each allocation
   int64_t bytes = 0;
   float *fld[6] = {};
   int16_t *mi[6] = {};
@@ -247,14 +258,13 @@ int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);
 int run_nodal(fdtd_handle *h, int half, int n, const int *dn);
-// the sources of a half as a one-cell pass over tile map tm applies them:
-// *on tells whether it can (else run_pw and run_nodal follow the pass); flags
-// (null: not wanted): per block of tm, what its tile meets is added
-int make_pass_src(fdtd_handle *h, const sfd::TileMap &tm, int half, sfd::PassSrc *out, bool *on,
-                  std::vector<void *> *list, std::vector<int> *flags);
+// the sources of a half as a one-cell pass over tile map tm applies them, on
+// only where it can (else run_pw and run_nodal follow the pass); flags (null:
+// not wanted): per block of tm, what its tile meets is added
+void make_pass_src(const fdtd_handle *h, const sfd::TileMap &tm, int half, SrcTables *out,
+                   std::vector<int> *flags);
 // the same for the four-cell passes (flags: the words of the layout's tiles)
-int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, sfd::PassSrc *out, bool *on,
-                  std::vector<void *> *list, int *flags);
+void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTables *out, int *flags);
 // UpdateObservation at step n (or *dn + n): point probes, frequency-domain
 // sums, and (pw) the TF/SF terms of the next step; half 0, 1: the E, the H
 // quantities alone (the H part moves the sample count), 2: all.  run_observe

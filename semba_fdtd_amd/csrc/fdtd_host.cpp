@@ -41,8 +41,20 @@ int dalloc(fdtd_handle *h, void **p, size_t bytes, std::vector<void *> *list) {
   if (e != hipSuccess)
     return fail(h, FDTD_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   (list ? list : &h->allocs)->push_back(*p);
+  h->sizes[*p] = bytes;
   h->bytes += (int64_t)bytes;
   return FDTD_OK;
+}
+
+// what dalloc allocated into list, given back
+static void dfree(fdtd_handle *h, std::vector<void *> *list) {
+  for (void *p : *list) {
+    hipFree(p);
+    const auto at = h->sizes.find(p);
+    h->bytes -= (int64_t)at->second;
+    h->sizes.erase(at);
+  }
+  list->clear();
 }
 
 int dzero(fdtd_handle *h, void *p, size_t bytes) {
@@ -332,13 +344,23 @@ int build_tile_media(fdtd_handle *h) {
     const int n = quads ? h->quad.p.nblk : h->tm.nblk;
     if ((rc = tile_words(h, words, cap, n))) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (void *p : h->psrc_allocs) hipFree(p);
-    h->psrc_allocs.clear();
+    dfree(h, &h->psrc_allocs);
     std::vector<int> flags((size_t)n, 0);
     for (int half = 0; half < 2; ++half) {
-      rc = quads ? make_quad_src(h, h->quad, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, flags.data())
-                 : make_pass_src(h, h->tm, half, &h->psrc[half], &h->psrc_on[half], &h->psrc_allocs, &flags);
-      if (rc) return rc;
+      SrcTables t;
+      if (quads) make_quad_src(h, h->quad, half, &t, flags.data());
+      else make_pass_src(h, h->tm, half, &t, &flags);
+      if (!t.cells.empty()) {
+        int *start = nullptr;
+        NodalCell *cells = nullptr;
+        if ((rc = upload(h, &start, t.nstart.data(), t.nstart.size(), &h->psrc_allocs)) ||
+            (rc = upload(h, &cells, t.cells.data(), t.cells.size(), &h->psrc_allocs)))
+          return rc;
+        t.src.nstart = start;
+        t.src.cells = cells;
+      }
+      h->psrc[half] = t.src;
+      h->psrc_on[half] = t.on;
     }
     HIPCHK(h, hipMemcpyAsync(*words + *cap, flags.data(), flags.size() * sizeof(int), hipMemcpyHostToDevice,
                              h->stream));
@@ -479,8 +501,7 @@ static int build_ade_side(fdtd_handle *h, int side) {
 int build_ade(fdtd_handle *h) {
   if (h->ade_ready) return FDTD_OK;
   if (h->g.ade[0].has || h->g.ade[1].has) ++h->src_gen;
-  for (void *p : h->ade_allocs) hipFree(p);
-  h->ade_allocs.clear();
+  dfree(h, &h->ade_allocs);
   for (int side = 0; side < 2; ++side) {
     const int rc = build_ade_side(h, side);
     if (rc) return rc;
@@ -496,8 +517,7 @@ int build_ade(fdtd_handle *h) {
 // components' sweeps give the face extents (InitMURBorders, :113-160).
 static int build_mur(fdtd_handle *h) {
   if (h->mur_ready) return FDTD_OK;
-  for (void *p : h->mur_allocs) hipFree(p);
-  h->mur_allocs.clear();
+  dfree(h, &h->mur_allocs);
   h->mur_runs.clear();
   h->dmur = nullptr;
   h->mur_total = 0;
@@ -624,8 +644,7 @@ int build_step(fdtd_handle *h) {
   int rc;
   std::vector<void *> ptr(sizes.size(), nullptr);
   if (sizes != h->step_sizes) {
-    for (void *p : h->step_allocs) { hipFree(p); }
-    h->step_allocs.clear();
+    dfree(h, &h->step_allocs);
     h->step_sizes.clear();
     for (size_t q = 0; q < sizes.size(); ++q) {
       if (!sizes[q]) continue;
@@ -662,8 +681,7 @@ int build_step(fdtd_handle *h) {
       gb.ade[side].jst[c] = h->gB.ade[side].jst[c];
     }
   h->gB = gb;
-  for (void *p : h->step_small) hipFree(p);
-  h->step_small.clear();
+  dfree(h, &h->step_small);
   StepDev sd{};
   TileMap &tm = sd.tm;
   tm.bdy = R;
@@ -1089,8 +1107,7 @@ int build_nodal(fdtd_handle *h) {
       vals[(size_t)n * ns + s] = fdtd_evolucion(t, S.deltaevol, S.numus, S.evol.data());
     }
   int rc;
-  for (void *p : h->nodal_allocs) hipFree(p);
-  h->nodal_allocs.clear();
+  dfree(h, &h->nodal_allocs);
   h->dvalues = nullptr;
   h->dcells[0] = h->dcells[1] = nullptr;
   if ((rc = dalloc(h, (void **)&h->dvalues, vals.size() * 4, &h->nodal_allocs))) return rc;
@@ -1250,40 +1267,32 @@ static bool in_poles(const fdtd_handle *h, int comp, const int lo[3], const int 
   return true;
 }
 
-// the nodal cells of a pass, grouped by tile: tile(i, j, k) of ntile
+// the nodal cells of a pass, grouped by tile: tile(i, j, k) of ntile; false
+// where a cell cannot go inline
 template <class F>
-static int tile_cells(fdtd_handle *h, int half, int ntile, F tile_of, PassSrc *out, bool *on,
-                      std::vector<void *> *list, std::vector<int> *start) {
+static bool tile_cells(const fdtd_handle *h, int half, int ntile, F tile_of, SrcTables *out) {
   const std::vector<NodalCell> &C = h->hcells[half];
   const DevGrid &g = h->g;
   std::vector<int> tile(C.size());
-  std::vector<int> &nstart = *start;
-  std::vector<NodalCell> cells(C.size());
+  std::vector<int> &nstart = out->nstart;
   nstart.assign((size_t)ntile + 1, 0);
   for (size_t q = 0; q < C.size(); ++q) {
     const long long k = C[q].p / g.pxy - 1, r = C[q].p % g.pxy;
     const long long j = r / g.px - 1, i = r % g.px - g.xoff;
-    if (i < 0 || i > g.nx || j < 0 || j > g.ny || k < 0 || k > g.nz) return FDTD_OK;
+    if (i < 0 || i > g.nx || j < 0 || j > g.ny || k < 0 || k > g.nz) return false;
     const int c[3] = {(int)i, (int)j, (int)k};
-    if (in_poles(h, C[q].comp, c, c)) return FDTD_OK;
+    if (in_poles(h, C[q].comp, c, c)) return false;
     tile[q] = tile_of(c[0], c[1], c[2]);
     ++nstart[(size_t)tile[q] + 1];
   }
   for (int t = 0; t < ntile; ++t) nstart[(size_t)t + 1] += nstart[(size_t)t];
   std::vector<int> at(nstart.begin(), nstart.end() - 1);
-  for (size_t q = 0; q < C.size(); ++q) cells[(size_t)at[(size_t)tile[q]]++] = C[q];
-  int *dst = nullptr, rc;
-  NodalCell *dc = nullptr;
-  if ((rc = upload(h, &dst, nstart.data(), nstart.size(), list)) ||
-      (rc = upload(h, &dc, cells.data(), cells.size(), list)))
-    return rc;
-  out->nstart = dst;
-  out->cells = dc;
-  out->values = h->dvalues;
-  out->nsrc = (int)h->srcs.size();
-  out->serial = h->serial[half];
-  *on = true;
-  return FDTD_OK;
+  out->cells.resize(C.size());
+  for (size_t q = 0; q < C.size(); ++q) out->cells[(size_t)at[(size_t)tile[q]]++] = C[q];
+  out->src.values = h->dvalues;
+  out->src.nsrc = (int)h->srcs.size();
+  out->src.serial = h->serial[half];
+  return true;
 }
 
 // does a plane-wave face of the half meet a pole-state box
@@ -1302,17 +1311,16 @@ static bool face_in_poles(const fdtd_handle *h, int half) {
 // box that touches them keeps its own launches).  Grids of every size: the
 // tiles without faces run code without them.  us per step, separate / inline:
 // 64^3 38.4 / 18.6, 128^3 80.2 / 52.4, 256^3 429 / 369, 384^3 1558 / 1431.
-int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, PassSrc *out, bool *on,
-                  std::vector<void *> *list, int *flags) {
-  *out = PassSrc{};
-  *on = false;
+void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTables *out, int *flags) {
+  *out = SrcTables{};
   std::vector<int> word((size_t)l.p.nblk, 0);
   const bool faces = !h->pw_faces[half].empty();
-  if (!faces && h->hcells[half].empty()) return FDTD_OK;
-  if (faces && (!h->pw_masks[half] || face_in_poles(h, half))) return FDTD_OK;
+  if (!faces && h->hcells[half].empty()) return;
+  if (faces && (!h->pw_masks[half] || face_in_poles(h, half))) return;
   const QuadPlan &p = l.p;
-  PassSrc x = faces ? h->pw_src[half] : PassSrc{};
-  if (x.nface) {
+  SrcTables x;
+  if (faces) x.src = h->pw_src[half];
+  if (x.src.nface) {
     const std::vector<unsigned> *m = h->pw_bits[half];
     auto any = [](const std::vector<unsigned> &v, int a, int b) {
       unsigned r = 0;
@@ -1336,16 +1344,14 @@ int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, PassSrc *out, b
         const unsigned z = any(m[2], k, std::min(k + l.kc, o.k0 + o.nk));
         for (int r = 0; r < o.tx; ++r, ++t) {
           if (!(xy[(size_t)r] & z)) continue;
-          if (slabs) return FDTD_OK;
+          if (slabs) return;
           word[(size_t)t] |= kTileFaces[half];
         }
       }
     }
   }
   if (!h->hcells[half].empty()) {
-    std::vector<int> start;
-    bool ok = false;
-    const int rc = tile_cells(h, half, p.nblk, [&](int i, int j, int k) {
+    const bool ok = tile_cells(h, half, p.nblk, [&](int i, int j, int k) {
       for (int b = 0; b < p.nbox; ++b) {
         const QuadBox &o = p.box[b];
         if (j < o.j0 || j >= o.j0 + o.nj || k < o.k0 || k >= o.k0 + o.nk) continue;
@@ -1353,15 +1359,14 @@ int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, PassSrc *out, b
         return p.start[b] + (k - o.k0) / l.kc * o.tx + f / (kWave * l.rows);
       }
       return 0;   // (the boxes hold every swept cell)
-    }, &x, &ok, list, &start);
-    if (rc || !ok) return rc;
+    }, &x);
+    if (!ok) return;
     for (int t = 0; t < p.nblk; ++t)
-      if (start[(size_t)t] < start[(size_t)t + 1]) word[(size_t)t] |= kTileNodal[half];
+      if (x.nstart[(size_t)t] < x.nstart[(size_t)t + 1]) word[(size_t)t] |= kTileNodal[half];
   }
   for (int t = 0; t < p.nblk; ++t) flags[t] |= word[(size_t)t];
-  *out = x;
-  *on = true;
-  return FDTD_OK;
+  x.on = true;
+  *out = std::move(x);
 }
 
 // A pass applies the sources before the pole stage that follows it, so they
@@ -1373,31 +1378,31 @@ int make_quad_src(fdtd_handle *h, const QuadLayout &l, int half, PassSrc *out, b
 // 4.6-9 us each whatever the grid.  A plane wave on 48^3, 100^3, 160^3, 200^3
 // runs 1.64, 1.48, 1.14, 1.02 times as fast inline, on 320^3 0.98 times; a
 // point source on 64^3, 128^3, 200^3 1.16, 1.03, 1.04 times, on 320^3 0.99.
-int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, bool *on,
-                  std::vector<void *> *list, std::vector<int> *flags) {
-  *on = false;
-  *out = PassSrc{};
+void make_pass_src(const fdtd_handle *h, const TileMap &tm, int half, SrcTables *out,
+                   std::vector<int> *flags) {
+  *out = SrcTables{};
   const std::vector<PwFace> &F = h->pw_faces[half];
   const std::vector<NodalCell> &C = h->hcells[half];
-  if (F.empty() && C.empty()) return FDTD_OK;
-  if (cells_of(h) > kInlineCells) return FDTD_OK;
-  if (!F.empty() && !h->pw_masks[half]) return FDTD_OK;
-  if (face_in_poles(h, half)) return FDTD_OK;
+  if (F.empty() && C.empty()) return;
+  if (cells_of(h) > kInlineCells) return;
+  if (!F.empty() && !h->pw_masks[half]) return;
+  if (face_in_poles(h, half)) return;
   const DevGrid &g = h->g;
-  std::vector<int> nstart;
-  *out = h->pw_masks[half] && !F.empty() ? h->pw_src[half] : PassSrc{};
+  SrcTables x;
+  if (!F.empty()) x.src = h->pw_src[half];
   if (!C.empty()) {
     // the tile of a cell, as tile_column lays the tiles out
-    const int rc = tile_cells(h, half, tm.nblk, [&](int i, int j, int k) {
+    const bool ok = tile_cells(h, half, tm.nblk, [&](int i, int j, int k) {
       const long long bxy = tm.flat ? ((long long)j * (g.nx + 1) + i) / (kWave * tm.bdy)
                                     : (long long)(j / tm.bdy) * tm.tx + i / kWave;
       return (int)((long long)(k / tm.kc) * tm.ty * tm.tx + bxy);
-    }, out, on, list, &nstart);
-    if (rc) return rc;
-    if (!*on) { *out = PassSrc{}; return FDTD_OK; }
+    }, &x);
+    if (!ok) return;
   }
-  *on = true;
-  if (!flags) return FDTD_OK;
+  x.on = true;
+  *out = std::move(x);
+  if (!flags) return;
+  const std::vector<int> &nstart = out->nstart;
   // flags are by block: the block that runs tile t
   auto block_of = [&](int t) {
     if (!tm.remap) return t;
@@ -1411,7 +1416,7 @@ int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, boo
   if (!C.empty())
     for (int t = 0; t < tm.nblk; ++t)
       if (nstart[(size_t)t] < nstart[(size_t)t + 1]) (*flags)[(size_t)block_of(t)] |= kTileNodal[half];
-  if (out->nface) {
+  if (out->src.nface) {
     const std::vector<unsigned> *m = h->pw_bits[half];
     auto any = [](const std::vector<unsigned> &v, long long a, long long b) {
       unsigned r = 0;
@@ -1440,7 +1445,6 @@ int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, boo
         if (xy[(size_t)t] & z) (*flags)[(size_t)block_of(bz * tm.tx * tm.ty + t)] |= kTileFaces[half];
     }
   }
-  return FDTD_OK;
 }
 
 // InitPlaneWave (planewaves.F90:72-766) and calc_planewaveconstants
@@ -1450,8 +1454,7 @@ int make_pass_src(fdtd_handle *h, const TileMap &tm, int half, PassSrc *out, boo
 int build_planewaves(fdtd_handle *h) {
   if (h->pw_ready) return FDTD_OK;
   if (!h->pwin.empty()) ++h->src_gen;
-  for (void *p : h->pw_allocs) hipFree(p);
-  h->pw_allocs.clear();
+  dfree(h, &h->pw_allocs);
   h->pw_faces[0].clear();
   h->pw_faces[1].clear();
   h->pw_masks[0] = h->pw_masks[1] = false;
@@ -1673,8 +1676,7 @@ void dft_phases(const DftIn &d, const std::vector<double> &tiempo, double dt,
 
 int build_dfts(fdtd_handle *h) {
   if (h->dft_ready) return FDTD_OK;
-  for (void *p : h->dft_allocs) hipFree(p);
-  h->dft_allocs.clear();
+  dfree(h, &h->dft_allocs);
   if (h->dftin.empty()) { h->dft_ready = true; return FDTD_OK; }
   if (h->tiempo.empty()) return fail(h, FDTD_ERR_STATE, "fdtd_set_time not called");
   int rc;
