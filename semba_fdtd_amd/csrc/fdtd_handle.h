@@ -149,6 +149,7 @@ struct fdtd_handle {
   // psrc_gen == src_gen).  src_gen counts the changes of the tiling, the sources
   // and the pole-state boxes.
   unsigned src_gen = 1, psrc_gen = 0;
+  bool inline_ok = true;           // (sfd_set_inline_sources)
   bool psrc_on[2] = {false, false};
   sfd::PassSrc psrc[2] = {};
   std::vector<void *> psrc_allocs;

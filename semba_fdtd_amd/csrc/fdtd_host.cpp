@@ -1313,6 +1313,7 @@ static bool face_in_poles(const fdtd_handle *h, int half) {
 // 64^3 38.4 / 18.6, 128^3 80.2 / 52.4, 256^3 429 / 369, 384^3 1558 / 1431.
 void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTables *out, int *flags) {
   *out = SrcTables{};
+  if (!h->inline_ok) return;
   std::vector<int> word((size_t)l.p.nblk, 0);
   const bool faces = !h->pw_faces[half].empty();
   if (!faces && h->hcells[half].empty()) return;
@@ -1381,6 +1382,7 @@ void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTable
 void make_pass_src(const fdtd_handle *h, const TileMap &tm, int half, SrcTables *out,
                    std::vector<int> *flags) {
   *out = SrcTables{};
+  if (!h->inline_ok) return;
   const std::vector<PwFace> &F = h->pw_faces[half];
   const std::vector<NodalCell> &C = h->hcells[half];
   if (F.empty() && C.empty()) return;
@@ -3110,3 +3112,21 @@ int fdtd_load_state(fdtd_handle *h, const void *buf, int64_t size, int32_t *n) {
 }
 
 }  // extern "C"
+
+// The tests' view of the inline sources: whether the passes may apply them (on
+// = 0: every face and nodal cell in launches of its own, as the granular calls
+// run them), and per half, in bits 0 and 1, whether the grid's passes do.
+extern "C" int sfd_set_inline_sources(fdtd_handle *h, int32_t on) {
+  if (!h) return FDTD_ERR_ARG;
+  h->inline_ok = on != 0;
+  ++h->src_gen;
+  invalidate_graph(h);
+  return FDTD_OK;
+}
+extern "C" int sfd_inline_sources(fdtd_handle *h) {
+  if (!h) return FDTD_ERR_ARG;
+  hipSetDevice(h->device);
+  int rc = prepare(h);
+  if (!rc) rc = build_tile_media(h);
+  return rc ? rc : (h->psrc_on[0] ? 1 : 0) | (h->psrc_on[1] ? 2 : 0);
+}
