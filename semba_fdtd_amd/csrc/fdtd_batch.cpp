@@ -853,3 +853,14 @@ int fdtd_batch_synchronize(fdtd_batch *b) {
 }
 
 }  // extern "C"
+
+// The tests' view of a batch: whether its passes run four cells per lane, their
+// tiles, and the observation's blocks in a two-pass and in a one-launch step
+// (as last built).
+extern "C" int sfd_batch_plan(const fdtd_batch *b, int32_t out[4]) {
+  if (!b || !out) return FDTD_ERR_ARG;
+  out[0] = b->quads ? 1 : 0;
+  out[1] = b->bd.total;
+  out[2] = out[3] = b->obs_blocks;
+  return FDTD_OK;
+}

@@ -185,6 +185,7 @@ struct fdtd_handle {
                                   // rows than step_rows runs the step's tiles cut
                                   // into row bands
   bool step_vec = true;           // plain tiles run four x cells per lane (k_step4)
+  int step_merge = -1, step_fork = -1;   // (sfd_set_step_plan)
   // the branches of a recorded one-launch step
   hipStream_t side[2] = {};
   hipEvent_t forked = nullptr, joined[2] = {};

@@ -786,7 +786,8 @@ int build_step(fdtd_handle *h) {
     // of a mid-size grid are a wave and a bit of blocks, the second of it nearly
     // empty.  Unmerged below eight blocks a unit: 256^3 1018 -> 624 us per step
     // (64 tiles), 320^3 1038 -> 890 (200), 500x444x390 2452 -> 2339 (336).
-    if (plan.tiles[0].size() + plan.tiles[kPlanVec].size() < 8u * (unsigned)h->cus) {
+    const bool merge = plan.tiles[0].size() + plan.tiles[kPlanVec].size() >= 8u * (unsigned)h->cus;
+    if (!(h->step_merge < 0 ? merge : h->step_merge > 0)) {
       pg.zrun = pg.kc;
       if (plan_step(pg, &plan, &perr)) return fail(h, FDTD_ERR_ARG, "%s", perr.c_str());
     }
@@ -2483,7 +2484,7 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
   const int pairs = paired ? nsteps / 2 : 0;
   const int singles = paired ? nsteps % 2 : nsteps;
   if (pairs > 0 && !h->pexec) {
-    const bool fork = (double)cells_of(h) <= kForkCells;
+    const bool fork = h->step_fork < 0 ? (double)cells_of(h) <= kForkCells : h->step_fork > 0;
     if ((rc = build_step(h)) || (fork && (rc = make_branches(h)))) return rc;
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int r2 = run_step(h, 0, false, fork);
@@ -3129,4 +3130,22 @@ extern "C" int sfd_inline_sources(fdtd_handle *h) {
   int rc = prepare(h);
   if (!rc) rc = build_tile_media(h);
   return rc ? rc : (h->psrc_on[0] ? 1 : 0) | (h->psrc_on[1] ? 2 : 0);
+}
+
+// The tests' view of the one-launch step: merge (1: plain tiles merged, 0:
+// not, -1: by their number), fork (1: class kernels in branches, 0: one after
+// another, -1: by the grid's size), whatever the grid; and the tiles of each
+// class (by the class numbers of FDTD_STEP_CLASSES) as last planned.
+extern "C" int sfd_set_step_plan(fdtd_handle *h, int32_t merge, int32_t fork) {
+  if (!h) return FDTD_ERR_ARG;
+  h->step_merge = merge;
+  h->step_fork = fork;
+  invalidate_graph(h);
+  return FDTD_OK;
+}
+extern "C" int sfd_step_tiles(const fdtd_handle *h, int32_t count[FDTD_STEP_CLASSES]) {
+  if (!h || !count) return FDTD_ERR_ARG;
+  std::fill(count, count + FDTD_STEP_CLASSES, 0);
+  for (size_t q = 0; q < h->step_cls.size(); ++q) count[h->step_cls[q]] = h->step_cnt[q];
+  return FDTD_OK;
 }
