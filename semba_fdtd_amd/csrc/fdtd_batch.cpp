@@ -88,9 +88,13 @@ struct fdtd_batch {
   size_t ade_lds[2] = {0, 0};
   int ade_tbl[2] = {1, 1};
   long long ade_nmax[2] = {0, 0};
-  ObserveGrid *dobs = nullptr;
-  int *dobstart = nullptr;
-  int nobs = 0, obs_blocks = 0;
+  // the observation after a two-pass step (with the next step's TF/SF terms)
+  // and after a one-launch step (whose incident field has a launch of its own)
+  struct Observation {
+    ObserveGrid *obs = nullptr;
+    int *start = nullptr;
+    int n = 0, blocks = 0;
+  } obs[2];
   // per slot and half: the sources the grid's passes apply inline, and the
   // grids whose TF/SF terms a call refreshes before its first step
   std::vector<char> inl[2];
@@ -361,8 +365,8 @@ int build_descriptors(fdtd_batch *b) {
   // pole stage and probes: one launch each for the whole batch
   {
     const bool exact = b->mode == FDTD_MODE_EXACT;
-    std::vector<ObserveGrid> sets;
-    std::vector<int> obstart(1, 0);
+    std::vector<ObserveGrid> sets[2];
+    std::vector<int> obstart[2] = {{0}, {0}};
     std::vector<int> al[2];
     for (int side = 0; side < 2; ++side) {
       b->ade_lds[side] = 0;
@@ -386,12 +390,14 @@ int build_descriptors(fdtd_batch *b) {
         if (h->g.nmedia + 1 > 4096) b->ade_tbl[side] = 0;
       }
       const bool terms = (b->inl[0][s] || b->inl[1][s]) && h->pw_terms.total > 0;
-      if (h->nprobe || !h->dfts.empty() || terms) {
+      for (int one = 0; one < 2; ++one) {
         ObserveGrid og{};
-        og.p = observe_part(h, 2, 0, h->dstep, true, true, terms);
+        og.p = observe_part(h, 2, 0, h->dstep, true, true, terms && !one);
         og.grid = gi;
-        sets.push_back(og);
-        obstart.push_back(obstart.back() + observe_blocks(og.p, 256));
+        const int blocks = observe_blocks(og.p, 256);
+        if (!blocks) continue;
+        sets[one].push_back(og);
+        obstart[one].push_back(obstart[one].back() + blocks);
       }
       ++gi;
     }
@@ -402,13 +408,16 @@ int build_descriptors(fdtd_batch *b) {
       if (!al[side].empty() && (rc = bupload(b, &b->dade[side], al[side].data(), al[side].size())))
         return rc;
     }
-    b->nobs = (int)sets.size();
-    b->obs_blocks = obstart.back();
-    b->dobs = nullptr;
-    b->dobstart = nullptr;
-    if (!sets.empty() && ((rc = bupload(b, &b->dobs, sets.data(), sets.size())) ||
-                          (rc = bupload(b, &b->dobstart, obstart.data(), obstart.size()))))
-      return rc;
+    for (int one = 0; one < 2; ++one) {
+      fdtd_batch::Observation &o = b->obs[one];
+      o = fdtd_batch::Observation{};
+      o.n = (int)sets[one].size();
+      o.blocks = obstart[one].back();
+      if (o.n && ((rc = bupload(b, &o.obs, sets[one].data(), sets[one].size())) ||
+                  (rc = bupload(b, &o.start, obstart[one].data(), obstart[one].size()))))
+        return rc;
+    }
+    BCHK(b, hipStreamSynchronize(b->stream));   // (the copies read these vectors)
   }
   // plane-wave groups across the batch, in each grid's face order: per half,
   // per wave index, per face axis (the runs read each grid's own counter)
@@ -561,7 +570,8 @@ int launch_step_dir(fdtd_batch *b, int d, bool exact_prev) {
     if (launch_mur(h->sd[d].go, h->dmur, (int)h->mur_runs.size(), h->mur_total, exact, b->stream))
       return bfail(b, FDTD_ERR_HIP, "batch Mur launch failed");
   }
-  if (launch_observe_many(b->dgo[d], b->dobs, b->dobstart, b->nobs, b->obs_blocks, 0, b->stream))
+  const fdtd_batch::Observation &o = b->obs[1];
+  if (launch_observe_many(b->dgo[d], o.obs, o.start, o.n, o.blocks, 0, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
   if (launch_tick_many(b->dcounters, b->ncounters, 1, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch step counter launch failed");
@@ -605,7 +615,8 @@ int launch_step(fdtd_batch *b, int r) {
   }
   for (fdtd_handle *h : b->slots)
     if (h && (rc = run_mur(h))) return bfail(b, rc, "grid: %s", h->err.c_str());
-  if (launch_observe_many(b->bd.grids, b->dobs, b->dobstart, b->nobs, b->obs_blocks, r, b->stream))
+  const fdtd_batch::Observation &o = b->obs[0];
+  if (launch_observe_many(b->bd.grids, o.obs, o.start, o.n, o.blocks, r, b->stream))
     return bfail(b, FDTD_ERR_HIP, "batch observation launch failed");
   return FDTD_OK;
 }
@@ -861,6 +872,7 @@ extern "C" int sfd_batch_plan(const fdtd_batch *b, int32_t out[4]) {
   if (!b || !out) return FDTD_ERR_ARG;
   out[0] = b->quads ? 1 : 0;
   out[1] = b->bd.total;
-  out[2] = out[3] = b->obs_blocks;
+  out[2] = b->obs[0].blocks;
+  out[3] = b->obs[1].blocks;
   return FDTD_OK;
 }
