@@ -399,11 +399,12 @@ int fdtd_batch_retire(fdtd_batch *b, int32_t slot);
 /* Step the grid of slot will run next (-1 for an empty slot). */
 int64_t fdtd_batch_step_of(const fdtd_batch *b, int32_t slot);
 /* Tiling of the batched face passes (rows 1, 2 or 4; zchunk planes).  xcells 4:
- * four x cells per lane, each block taking a run of 64 * rows consecutive
- * four-cell vectors of a grid's x-y plane.  xcells 1: the passes choose rows
- * and planes by the batch's size and run four cells per lane where every grid
- * can; else one cell per lane, each block taking a run of 64 * rows consecutive
- * columns, x fastest, with the persistent launch's block count (0: 16384).
+ * four x cells per lane where every grid can, each block taking a run of
+ * 64 * rows consecutive four-cell vectors of a grid's x-y plane.  xcells 1: one
+ * cell per lane, each block taking a run of 64 * rows consecutive columns, x
+ * fastest, with the persistent launch's block count (0: 16384).  Until this is
+ * called the passes choose: four cells per lane where every grid can, rows and
+ * planes by the batch's size, else one cell per lane in 4 rows x 16 planes.
  * Either storage runs either. */
 int fdtd_batch_set_tiling(fdtd_batch *b, int32_t rows, int32_t zchunk, int32_t xcells,
                           int32_t blocks);

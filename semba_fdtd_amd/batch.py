@@ -11,14 +11,19 @@ alone.
 from __future__ import annotations
 
 import ctypes as C
+from typing import Optional
 
 from . import _lib
 from ._lib import FdtdError
 
 
 class Batch:
-    def __init__(self, device: int = 0, stream=None, rows: int = 4, zchunk: int = 16,
-                 blocks: int = 0, xcells: int = 1, step_rows: int = 0, step_zchunk: int = 16):
+    """rows, zchunk, blocks, xcells: a tiling (``set_tiling``; those left out
+    are 4, 16, 0 and 1).  With none of them the passes choose their own."""
+
+    def __init__(self, device: int = 0, stream=None, rows: Optional[int] = None,
+                 zchunk: Optional[int] = None, blocks: Optional[int] = None,
+                 xcells: Optional[int] = None, step_rows: int = 0, step_zchunk: int = 16):
         self.lib = lib = _lib.load()
         b = C.c_void_p()
         rc = lib.fdtd_batch_create(device, stream, C.byref(b))
@@ -27,7 +32,9 @@ class Batch:
                             f"{lib.fdtd_batch_last_error(None).decode()}")
         self.b = b
         self.members = {}          # slot -> Solver
-        self.set_tiling(rows, zchunk, blocks, xcells)
+        given = (rows, zchunk, blocks, xcells)
+        if any(v is not None for v in given):
+            self.set_tiling(*(d if v is None else v for v, d in zip(given, (4, 16, 0, 1))))
         self.set_step_mode(step_rows, step_zchunk)
 
     def _ck(self, rc, what):
@@ -37,11 +44,10 @@ class Batch:
 
     def set_tiling(self, rows: int, zchunk: int, blocks: int = 0, xcells: int = 1):
         """Blocks of 64 x rows threads marching zchunk z planes, xcells x
-        cells per lane (4: each block takes a run of 64 * rows consecutive
-        four-cell vectors of a grid's x-y plane; 1: the passes choose rows and
-        planes by the batch's size and run four cells per lane where every
-        grid can, else runs of 64 * rows columns), and the one-cell passes'
-        persistent block count (0: 16384)."""
+        cells per lane (4, where every grid can: each block takes a run of
+        64 * rows consecutive four-cell vectors of a grid's x-y plane; 1: runs
+        of 64 * rows columns), and the one-cell passes' persistent block count
+        (0: 16384)."""
         self._ck(self.lib.fdtd_batch_set_tiling(self.b, rows, zchunk, xcells, blocks),
                  "fdtd_batch_set_tiling")
 

@@ -71,6 +71,7 @@ struct fdtd_batch {
   std::vector<long long> step;        // host copy of each slot's step counter
   std::vector<unsigned> version;      // each grid's state version at the last build
   int rows = 4, zchunk = 16, xcells = 1, blocks = 0;
+  bool tile_set = false;              // fdtd_batch_set_tiling was called
   bool quads = false;                 // the passes run four cells per lane
   int prows = 4;                      // rows per block of the passes
   // device descriptors, rebuilt when the membership changes
@@ -205,13 +206,13 @@ TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
   return tm;
 }
 
-// The four-cell tiles of one grid, under the batch's tiling if it was set with
-// xcells 4.  Else one row per block, and as many planes as still leave the chip
+// The four-cell tiles of one grid, under the batch's tiling if it was set.  Else
+// one row per block, and as many planes as still leave the chip
 // enough blocks, by the cells of all grids: 256 grids of 95 M cells run 2318,
 // 2212, 2276 us a step with 1, 2, 4 planes, 64 binary16 ones of 24 M cells 571,
 // 489, 459 us; six grids of 1.5 M cells fill it with one plane only.
 QuadLayout batch_quads(const fdtd_batch *b, const fdtd_handle *h, double cells) {
-  if (b->xcells == 4) return plan_quads(h, b->rows, b->zchunk);
+  if (b->tile_set) return plan_quads(h, b->rows, b->zchunk);
   return plan_quads(h, 1, cells < 1.5e6 ? 1 : b->fp16 && cells > 1e7 ? 4 : 2);
 }
 
@@ -226,9 +227,8 @@ int build_descriptors(fdtd_batch *b) {
   int maxwaves = 0;
   int rc;
   // four cells per lane where every grid can (256 uneven grids 2570 -> 2212 us
-  // a step); a tiling with xcells 4 sets their rows and planes, with xcells 1
-  // those of the one-cell passes
-  b->quads = true;
+  // a step), unless a tiling of one cell per lane was asked for
+  b->quads = !b->tile_set || b->xcells == 4;
   for (fdtd_handle *h : b->slots)
     if (h && !quads_fit(h)) b->quads = false;
   std::vector<QuadLayout> quad;
@@ -747,6 +747,7 @@ int fdtd_batch_set_tiling(fdtd_batch *b, int32_t rows, int32_t zchunk, int32_t x
   b->zchunk = zchunk;
   b->xcells = xcells;
   b->blocks = blocks;
+  b->tile_set = true;
   b->ready = false;
   return FDTD_OK;
 }

@@ -90,8 +90,9 @@ def serve_plain(requests, mode: str = "fast", storage: str = "fp32") -> List[Res
 
 
 def serve_batched(requests, mode: str = "fast", storage: str = "fp32",
-                  reserve: int = 8 << 30, max_chunk: int = 250, rows: int = 4,
-                  zchunk: int = 16, blocks: int = 0, xcells: int = 1, step_rows: int = 0,
+                  reserve: int = 8 << 30, max_chunk: int = 250, rows: Optional[int] = None,
+                  zchunk: Optional[int] = None, blocks: Optional[int] = None,
+                  xcells: Optional[int] = None, step_rows: int = 0,
                   max_cells: Optional[int] = None, device: int = 0,
                   cancel: Optional[Callable[[str], bool]] = None,
                   check_finite: bool = True) -> List[Result]:
@@ -102,7 +103,8 @@ def serve_batched(requests, mode: str = "fast", storage: str = "fp32",
     admitted grid finishes (or after max_chunk steps), retire finished grids.
     max_cells trades latency for throughput: once the batch holds enough
     cells to fill the device, admitting more only stretches every admitted
-    request's time.  step_rows > 0 runs the batch one launch per step
+    request's time.  rows, zchunk, blocks, xcells: a tiling of the batch's
+    passes (``Batch``).  step_rows > 0 runs the batch one launch per step
     (``Batch.set_step_mode``).  At each chunk boundary, requests with non-finite probe
     samples (check_finite) or cancelled by the caller leave the batch early
     with status "diverged" / "cancelled"."""
