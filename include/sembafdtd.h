@@ -154,18 +154,18 @@ int fdtd_add_planewave(fdtd_handle *h, const int32_t box[6], int32_t nmodes, con
                        const float *e, const float *incert, float deltaevol, int32_t numus,
                        const float *evol, float eps0, float mu0);
 
-/* Work decomposition of the face passes: blocks of 64 x rows threads (rows =
- * 1, 2 or 4) that march zchunk z planes each, every lane owning xcells (1 or
- * 4) consecutive x cells of the fused passes.  No counterpart in the
- * reference (its loops are OpenMP over k); chosen by the autotuner
- * (semba_fdtd_amd.tuning) or left at the default by grid depth: 2 rows x 4
- * planes up to 160 planes (nz + 1), 4 x 8 up to 640, 4 x 16 beyond; 1 cell.
- * Until fdtd_set_tiling is called the fused passes choose by themselves: four
- * cells per lane and 1 row x 1 or 2 planes by the grid's size wherever the
- * media fit LDS and the x slabs leave four cells between them; the default
- * values above are the other passes'.  Either storage runs either.
- * fdtd_get_tiling returns the values as set (a chunk longer than the grid runs
- * as the whole grid). */
+/* Work decomposition of the fused face passes: blocks of 64 x rows threads (rows
+ * = 1, 2 or 4) that march zchunk z planes each, every lane owning xcells (1 or
+ * 4) consecutive x cells.  No counterpart in the reference (its loops are
+ * OpenMP over k); chosen by the autotuner (semba_fdtd_amd.tuning) or left to
+ * the passes: four cells per lane and 1 row x 1 or 2 planes by the grid's size
+ * wherever the media fit LDS and the x slabs leave four cells between them,
+ * else one cell per lane and a default by grid depth: 2 rows x 4 planes up to
+ * 160 planes (nz + 1), 4 x 8 up to 640, 4 x 16 beyond.  The granular calls run
+ * one cell per lane, on the tiling set with xcells 1 or that default.  Either
+ * storage runs either.  fdtd_get_tiling returns the values as set (a chunk
+ * longer than the grid runs as the whole grid), and until any are set those the
+ * fused passes run. */
 int fdtd_set_tiling(fdtd_handle *h, int32_t rows, int32_t zchunk, int32_t xcells);
 int fdtd_get_tiling(const fdtd_handle *h, int32_t *rows, int32_t *zchunk, int32_t *xcells);
 

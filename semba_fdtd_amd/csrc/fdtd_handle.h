@@ -78,7 +78,9 @@ struct fdtd_handle {
   int mode = FDTD_MODE_FAST;
   int storage = FDTD_STORE_FP32;
   sfd::DevGrid g{};
-  sfd::TileMap tm{};           // 64-cell x tiles (granular passes)
+  // 64-cell x tiles of the one-cell passes: as set, and the default by depth,
+  // which the granular calls keep where the fused passes run four cells per lane
+  sfd::TileMap tm{}, tm_default{};
   int xcells = 1;              // 4: the fused passes run four cells per lane
   bool tile_set = false;       // fdtd_set_tiling was called
   int tile_zchunk = 32;        // planes per z chunk as set (tm.kc: clipped to the grid)

@@ -203,12 +203,9 @@ int check_ready(fdtd_handle *h) {
 }
 
 // blocks of 64 x rows threads march z in chunks of zchunk planes
-void set_tiles(fdtd_handle *h, int rows, int zchunk, int xcells) {
+static TileMap tile_map(const fdtd_handle *h, int rows, int zchunk) {
   const DevGrid &g = h->g;
-  h->tile_zchunk = zchunk;
-  h->xcells = xcells;
-  ++h->src_gen;
-  TileMap &tm = h->tm;
+  TileMap tm{};
   tm.bdy = rows;
   tm.tx = (g.nx + 1 + kWave - 1) / kWave;
   tm.ty = (g.ny + 1 + rows - 1) / rows;
@@ -217,6 +214,7 @@ void set_tiles(fdtd_handle *h, int rows, int zchunk, int xcells) {
   tm.nblk = tm.tx * tm.ty * tm.tz;
   tm.remap = 1;
   tm.vec = 1;
+  return tm;
 }
 
 static long long cells_of(const fdtd_handle *h) {
@@ -242,8 +240,22 @@ static bool use_quads(const fdtd_handle *h) {
   return quads_fit(h) && (h->xcells == 4 || !h->tile_set);
 }
 
+// Rows per block and planes per chunk of the four-cell passes left to choose.
+// One plane per block: nothing is carried from plane to plane, but twice the
+// blocks hide the load latency better, and small tiles more often hold one
+// medium.  Two planes pay where a block moves little per plane: binary16, and
+// rows packed to 16 bytes on grids that fill the chip.  us per step, one / two
+// planes: 64^3 18.6 / 22.4, 128^3 52.4 / 50.4, 200^3 163.6 / 153.8, 256^3 369 /
+// 382, 320^3 680 / 714; binary16 64^3 20.1 / 25.8, 128^3 49.8 / 48.7, 200^3 135 /
+// 115, 256^3 345 / 284.
+static void quad_default(const fdtd_handle *h, int *rows, int *kc) {
+  const long long cells = cells_of(h);
+  *rows = 1;
+  *kc = cells >= 1500000 && (h->g.fp16 || h->g.nx < 256) ? 2 : 1;
+}
+
 // the tiles of the four-cell passes: rows per block and planes per chunk as
-// given, or (rows 0) the default of the grid's size
+// given, or (rows 0) the default
 QuadLayout plan_quads(const fdtd_handle *h, int rows, int kc) {
   const DevGrid &g = h->g;
   QuadLayout l;
@@ -251,20 +263,9 @@ QuadLayout plan_quads(const fdtd_handle *h, int rows, int kc) {
   // rows and planes that touch no y or z slab of E or H
   auto hi = [&](int a, int n) { return g.L[a][1] ? n - g.L[a][1] : n + 1; };
   const int ja = g.L[1][0], jb = hi(1, g.ny), ka = g.L[2][0], kb = hi(2, g.nz);
+  if (!rows) quad_default(h, &rows, &kc);
   l.rows = rows;
   l.kc = std::min(kc, K);
-  if (!rows) {
-    // One plane per block: nothing is carried from plane to plane, but twice
-    // the blocks hide the load latency better, and small tiles more often hold
-    // one medium.  Two planes pay where a block moves little per plane: binary16,
-    // and rows packed to 16 bytes on grids that fill the chip.  us per step,
-    // one / two planes: 64^3 18.6 / 22.4, 128^3 52.4 / 50.4, 200^3 163.6 /
-    // 153.8, 256^3 369 / 382, 320^3 680 / 714; binary16 64^3 20.1 / 25.8,
-    // 128^3 49.8 / 48.7, 200^3 135 / 115, 256^3 345 / 284.
-    const long long cells = cells_of(h);
-    l.rows = 1;
-    l.kc = cells >= 1500000 && (g.fp16 || g.nx < 256) ? 2 : 1;
-  }
   QuadPlan &P = l.p;
   std::fill(P.start, P.start + kQuadBoxes + 1, 0x7fffffff);
   auto add = [&](int j0, int j1, int k0, int k1) {
@@ -1746,8 +1747,9 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     yee = c = 0;
   }
   const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, h->tm, tmed, yee, c, a, src, h->stream)
-                                     : fast::launch_e(h->g, h->tm, tmed, yee, c, a, src, h->stream);
+  const TileMap &tm = quads ? h->tm_default : h->tm;
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "E pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1765,8 +1767,9 @@ int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     yee = c = 0;
   }
   const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
-  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, h->tm, tmed, yee, c, a, src, h->stream)
-                                     : fast::launch_h(h->g, h->tm, tmed, yee, c, a, src, h->stream);
+  const TileMap &tm = quads ? h->tm_default : h->tm;
+  int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream)
+                                     : fast::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "H pass launch failed: %s", hipGetErrorString((hipError_t)e));
   return FDTD_OK;
 }
@@ -1974,9 +1977,8 @@ int fdtd_create(const fdtd_grid_desc *d, fdtd_handle **out) {
   // small grids enough blocks (64^3: 22 us per step with 4-plane chunks
   // against 41 us with 16 and 70 us with 32; 256^3: 8 planes best)
   const int planes = g.nz + 1;
-  if (planes <= 160) set_tiles(h, 2, 4, 1);
-  else if (planes <= 640) set_tiles(h, 4, 8, 1);
-  else set_tiles(h, 4, 16, 1);
+  h->tile_zchunk = planes <= 160 ? 4 : planes <= 640 ? 8 : 16;
+  h->tm = h->tm_default = tile_map(h, planes <= 160 ? 2 : 4, h->tile_zchunk);
   hipStreamSynchronize(h->stream);
   *out = h;
   return FDTD_OK;
@@ -2243,8 +2245,11 @@ int fdtd_set_tiling(fdtd_handle *h, int32_t rows, int32_t zchunk, int32_t xcells
   const long long nblk = (long long)((h->g.nx + kWave) / kWave) * ((h->g.ny + rows) / rows) *
                          ((h->g.nz + zchunk) / zchunk);
   if (nblk > 0x7fffffffLL) return fail(h, FDTD_ERR_ARG, "tiling gives too many blocks");
-  set_tiles(h, rows, zchunk, xcells);
+  h->tm = tile_map(h, rows, zchunk);
+  h->tile_zchunk = zchunk;
+  h->xcells = xcells;
   h->tile_set = true;
+  ++h->src_gen;
   invalidate_graph(h);
   return FDTD_OK;
 }
@@ -2254,6 +2259,11 @@ int fdtd_get_tiling(const fdtd_handle *h, int32_t *rows, int32_t *zchunk, int32_
   *rows = h->tm.bdy;
   *zchunk = h->tile_zchunk;
   *xcells = h->xcells;
+  // (before any is set: what the fused passes run)
+  if (!h->tile_set && use_quads(h)) {
+    quad_default(h, rows, zchunk);
+    *xcells = 4;
+  }
   return FDTD_OK;
 }
 

@@ -44,9 +44,14 @@ NCLASS = 17                            # tile classes of the one-launch step
 _cache: Dict[str, tuple] = {}
 
 
+# the passes a choice was timed on: raised when they change, so that a choice
+# kept from others is timed again
+_PASSES = "p2"
+
+
 def _key(solver) -> str:
     nx, ny, nz = solver.n3
-    return f"{nx}x{ny}x{nz}:{solver.mode}:{getattr(solver, 'storage', 'fp32')}"
+    return f"{nx}x{ny}x{nz}:{solver.mode}:{getattr(solver, 'storage', 'fp32')}:{_PASSES}"
 
 
 def _load(path: Optional[str]) -> None:
@@ -158,7 +163,9 @@ def autotune(solver, candidates: Iterable[Tiling] = DEFAULT_CANDIDATES, reps: in
         if state is not None:
             solver.load_state(state)
     if not table:
-        _apply(solver, before)
+        # no tiling was tried, so the one in use (or the passes' own choice) stays
+        solver.set_step_mode(*before[3:])
+        solver.set_step_class_rows(0)
         return {"tiling": before[:3], "step": before[3:], "class_rows": None, "ms": None,
                 "table": [], "step_table": step_table, "cached": False}
     best = min(table, key=lambda r: r[1] + r[2])
