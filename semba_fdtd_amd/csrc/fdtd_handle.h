@@ -211,6 +211,7 @@ struct fdtd_handle {
   int *tmed = nullptr;
   int tmed_cap = 0;
   bool tmed_ready = false;
+  bool gmed_ready = false;     // tmed holds the granular calls' (tm_default) instead
   // the four-cell passes' tiles and their words and flags (valid while
   // tmed_ready and the grid runs these passes)
   sfd_host::QuadLayout quad;
@@ -260,6 +261,7 @@ bool quads_fit(const fdtd_handle *h);
 QuadLayout plan_quads(const fdtd_handle *h, int rows, int kc);
 int prepare(fdtd_handle *h);
 int build_tile_media(fdtd_handle *h);
+int build_granular_media(fdtd_handle *h);
 int run_pw(fdtd_handle *h, int half, int n, const int *dn);
 int run_nodal(fdtd_handle *h, int half, int n, const int *dn);
 // the sources of a half as a one-cell pass over tile map tm applies them, on

@@ -312,6 +312,7 @@ void invalidate_graph(fdtd_handle *h) {
   h->graph_ok = false;
   h->step_ready = false;
   h->tmed_ready = false;
+  h->gmed_ready = false;
 }
 
 // a device array of at least n words and n flags behind them
@@ -379,6 +380,21 @@ int build_tile_media(fdtd_handle *h) {
               : fast::launch_pass_tile_media(h->g, h->tm, flags, out, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
   h->tmed_ready = true;
+  return FDTD_OK;
+}
+
+// The media of the granular calls' tiles where the fused passes run four cells
+// per lane (else build_tile_media's words serve both).  320^3, all the granular
+// calls of a step: 1583 us reading every index, 1457 skipping those of
+// single-medium tiles.
+int build_granular_media(fdtd_handle *h) {
+  if (h->gmed_ready || !use_quads(h)) return FDTD_OK;
+  if (int rc = tile_words(h, &h->tmed, &h->tmed_cap, h->tm_default.nblk)) return rc;
+  const int e = h->mode == FDTD_MODE_EXACT
+                    ? exact::launch_pass_tile_media(h->g, h->tm_default, nullptr, h->tmed, h->stream)
+                    : fast::launch_pass_tile_media(h->g, h->tm_default, nullptr, h->tmed, h->stream);
+  if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
+  h->gmed_ready = true;
   return FDTD_OK;
 }
 
@@ -1746,7 +1762,7 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
-  const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
+  const int *tmed = (quads ? h->gmed_ready : h->tmed_ready) ? h->tmed : nullptr;
   const TileMap &tm = quads ? h->tm_default : h->tm;
   int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream)
                                      : fast::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream);
@@ -1766,7 +1782,7 @@ int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
-  const int *tmed = h->tmed_ready && !quads ? h->tmed : nullptr;
+  const int *tmed = (quads ? h->gmed_ready : h->tmed_ready) ? h->tmed : nullptr;
   const TileMap &tm = quads ? h->tm_default : h->tm;
   int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream)
                                      : fast::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream);
@@ -2456,6 +2472,7 @@ int fdtd_advance_h(fdtd_handle *h, int32_t n) {
     hipSetDevice(h->device);                                                   \
     int rc = prepare(h);                                                       \
     if (!rc) rc = build_tile_media(h);                                         \
+    if (!rc) rc = build_granular_media(h);                                     \
     if (rc) return rc;                                                         \
     return body;                                                               \
   }

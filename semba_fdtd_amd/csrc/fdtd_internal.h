@@ -478,7 +478,7 @@ __device__ __forceinline__ float nodal_apply(float v, const NodalCell &c, float 
 
 // launchers, one set per arithmetic mode.  tmed (null: none) holds, per
 // tile of the one-cell map tm, what the tile meets, as
-// launch_pass_tile_media writes it (its flags, plus its medium); the
+// launch_pass_tile_media writes it (its flags, null: none, plus its medium); the
 // one-cell passes skip the media loads of single-medium tiles.  src (null: none): the sources the fused
 // one-cell pass applies inline.
 #define SFD_DECLARE_LAUNCHERS(NS)                                              \

@@ -644,7 +644,8 @@ __global__ void __launch_bounds__(256) k_hpass_src(DevGrid g, TileMap tm, const 
 // One block per tile of a one-cell pass map: the medium index that all six
 // media arrays hold on every cell the tile's lanes own (columns i <= nx,
 // j <= ny, the planes of its z chunk), plus one, or 0 where they differ,
-// added to the tile's flags.  The tiles are decoded as the passes decode them.
+// added to the tile's flags (null: none).  The tiles are decoded as the passes
+// decode them.
 __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, const int *flags,
                                                          int *out) {
   int bx, by, bz;
@@ -665,7 +666,7 @@ __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, 
     nc = wi > 0 && wj > 0 ? (long long)wi * wj : 0;
   }
   if (nc <= 0 || k1 <= k0) {
-    if (threadIdx.x == 0) out[blockIdx.x] = flags[blockIdx.x];
+    if (threadIdx.x == 0) out[blockIdx.x] = flags ? flags[blockIdx.x] : 0;
     return;
   }
   __shared__ int bad;
@@ -691,7 +692,7 @@ __global__ void __launch_bounds__(256) k_pass_tile_media(DevGrid g, TileMap tm, 
   }
   if (b) atomicOr(&bad, 1);
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = flags[blockIdx.x] + (bad ? 0 : m0 + 1);
+  if (threadIdx.x == 0) out[blockIdx.x] = (flags ? flags[blockIdx.x] : 0) + (bad ? 0 : m0 + 1);
 }
 
 int launch_pass_tile_media(const DevGrid &g, const TileMap &tm, const int *flags, int *out,
