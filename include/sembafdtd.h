@@ -159,7 +159,8 @@ int fdtd_add_planewave(fdtd_handle *h, const int32_t box[6], int32_t nmodes, con
  * 4) consecutive x cells.  No counterpart in the reference (its loops are
  * OpenMP over k); chosen by the autotuner (semba_fdtd_amd.tuning) or left to
  * the passes: four cells per lane and 1 row x 1 or 2 planes by the grid's size
- * wherever the media fit LDS and the x slabs leave four cells between them,
+ * (4 rows x 1 or 4 planes beyond 255 media) wherever the media fit LDS and the
+ * x slabs leave four cells between them,
  * else one cell per lane and a default by grid depth: 2 rows x 4 planes up to
  * 160 planes (nz + 1), 4 x 8 up to 640, 4 x 16 beyond.  The granular calls run
  * one cell per lane, on the tiling set with xcells 1 or that default.  Either

@@ -207,13 +207,15 @@ TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
 }
 
 // The four-cell tiles of one grid, under the batch's tiling if it was set.  Else
-// one row per block, and as many planes as still leave the chip
-// enough blocks, by the cells of all grids: 256 grids of 95 M cells run 2318,
-// 2212, 2276 us a step with 1, 2, 4 planes, 64 binary16 ones of 24 M cells 571,
-// 489, 459 us; six grids of 1.5 M cells fill it with one plane only.
-QuadLayout batch_quads(const fdtd_batch *b, const fdtd_handle *h, double cells) {
+// one row per block, and as many planes as still leave the chip enough blocks,
+// by the cells of all grids: 256 grids of 95 M cells run 2318, 2212, 2276 us a
+// step with 1, 2, 4 planes, 64 binary16 ones of 24 M cells 571, 489, 459 us, six
+// of 48^3 29.9, 30.2 us with 1, 2, of 63^3 49.0, 47.1, of 100^3 137, 131.  With a
+// large media table four rows share it (quad_default): 12 grids of random media
+// and 2 M cells, 300 media 127 / 120 us, 4000 media 508 / 134.
+QuadLayout batch_quads(const fdtd_batch *b, const fdtd_handle *h, double cells, bool many) {
   if (b->tile_set) return plan_quads(h, b->rows, b->zchunk);
-  return plan_quads(h, 1, cells < 1.5e6 ? 1 : b->fp16 && cells > 1e7 ? 4 : 2);
+  return plan_quads(h, many ? 4 : 1, cells < 1.5e6 ? 1 : many || (b->fp16 && cells > 1e7) ? 4 : 2);
 }
 
 int build_descriptors(fdtd_batch *b) {
@@ -233,8 +235,12 @@ int build_descriptors(fdtd_batch *b) {
     if (h && !quads_fit(h)) b->quads = false;
   std::vector<QuadLayout> quad;
   double cells = 0.0;
+  bool many = false;   // some grid has a large media table
   for (fdtd_handle *h : b->slots)
-    if (h) cells += (double)h->g.nx * h->g.ny * h->g.nz;
+    if (h) {
+      cells += (double)h->g.nx * h->g.ny * h->g.nz;
+      many = many || h->g.nmedia + 1 > kManyMedia;
+    }
   for (size_t s = 0; s < b->slots.size(); ++s) {
     fdtd_handle *h = b->slots[s];
     if (!h) continue;
@@ -243,7 +249,7 @@ int build_descriptors(fdtd_batch *b) {
     b->version[s] = h->version;
     grids.push_back(h->g);
     tms.push_back(batch_tiles(b, h->g));
-    if (b->quads) quad.push_back(batch_quads(b, h, cells));
+    if (b->quads) quad.push_back(batch_quads(b, h, cells, many));
     const int nblk = b->quads ? quad.back().p.nblk : tms.back().nblk;
     if ((long long)start.back() + nblk > 0x7fffffffLL)
       return bfail(b, FDTD_ERR_ARG, "batch holds too many tiles");

@@ -43,6 +43,10 @@ struct PwGroup {
   long long *dstart = nullptr;
 };
 
+// a media table past this many entries is shared by four rows of the four-cell
+// passes (quad_default)
+constexpr int kManyMedia = 256;
+
 // the tiles of the four-cell passes: boxes, the slabs they meet (launch_quad),
 // rows per block, planes per tile
 struct QuadLayout {

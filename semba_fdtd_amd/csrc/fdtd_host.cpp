@@ -248,10 +248,21 @@ static bool use_quads(const fdtd_handle *h) {
 // planes: 64^3 18.6 / 22.4, 128^3 52.4 / 50.4, 200^3 163.6 / 153.8, 256^3 369 /
 // 382, 320^3 680 / 714; binary16 64^3 20.1 / 25.8, 128^3 49.8 / 48.7, 200^3 135 /
 // 115, 256^3 345 / 284.
+// A tile of several media stages the media table, 8 bytes a medium: with many
+// the table outweighs a small block's cells and holds its LDS, so four rows
+// share one, over four planes on grids that fill the chip.  us per step of
+// grids of random media, as above / so: 300 media 64^3 14.4 / 14.2, 96^3 32.2 /
+// 28.6, 200^3 172 / 160, 320^3 752 / 763; 1000 media 96^3 44.8 / 30.7, 200^3 200 /
+// 162; 4000 media 96^3 115 / 42, 200^3 525 / 180, 320^3 3186 / 778; binary16 1000
+// media 200^3 151 / 114.
 static void quad_default(const fdtd_handle *h, int *rows, int *kc) {
-  const long long cells = cells_of(h);
+  const bool large = cells_of(h) >= 1500000;
   *rows = 1;
-  *kc = cells >= 1500000 && (h->g.fp16 || h->g.nx < 256) ? 2 : 1;
+  *kc = large && (h->g.fp16 || h->g.nx < 256) ? 2 : 1;
+  if (h->g.nmedia + 1 > kManyMedia) {
+    *rows = 4;
+    *kc = large ? 4 : 1;
+  }
 }
 
 // the tiles of the four-cell passes: rows per block and planes per chunk as
