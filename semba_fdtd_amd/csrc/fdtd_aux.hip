@@ -416,7 +416,7 @@ __global__ void __launch_bounds__(256) k_observe_many(const DevGrid *grids, cons
 
 int observe_blocks(const ObservePart &p, int nt) {
   if (!p.sample && p.d1 <= p.d0 && p.w1 <= p.w0) return 0;
-  return 1 + (int)((p.d1 - p.d0 + nt - 1) / nt) + (int)((p.w1 - p.w0 + nt - 1) / nt);
+  return probe_blocks(p, nt) + (int)((p.d1 - p.d0 + nt - 1) / nt) + (int)((p.w1 - p.w0 + nt - 1) / nt);
 }
 
 int launch_observe(const DevGrid &g, const ObservePart &p, void *stream) {

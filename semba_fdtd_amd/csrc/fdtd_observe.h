@@ -32,11 +32,20 @@ __device__ __forceinline__ void pw_term_cell(const P &t, long long w, int n) {
   t.out[w] = f.sign > 0.0f ? x : -x;
 }
 
+// Blocks of nt threads that sample a part's probes, at least one.  A part that
+// moves the sample count has one block, which reads it before it moves it; the
+// others, of as few as 64 threads inside a face pass, take one probe a thread:
+// 10000 probes of a 64^3 cavity 162 us a step with one block, 11.2 so.
+template <class P>
+__host__ __device__ __forceinline__ int probe_blocks(const P &x, int nt) {
+  return x.sample && !x.advance && x.o.np > nt ? (x.o.np + nt - 1) / nt : 1;
+}
+
 // UpdateObservation (observation.F90:2620-2672 point probes, :3553-3600
-// frequency-domain sums), block blk of nt threads.  Block 0 samples the
+// frequency-domain sums), block blk of nt threads.  The first blocks sample the
 // probes: row *count + row of their buffer, *count moving where the part says
 // so, on the device so that a recorded step can be replayed.  The blocks after
-// it take one (point, frequency) pair of a frequency-domain box per thread:
+// them take one (point, frequency) pair of a frequency-domain box per thread:
 // the three components of the point are read once and multiplied by the
 // complex(8) phase factor of the step (each part scaled by the real sample).
 // The last blocks write the TF/SF terms of the next step, one cell per thread,
@@ -50,14 +59,15 @@ __device__ __forceinline__ void observe_block(const G &g, const P &x, int n, int
   auto field = [&](int c, long long p) {
     return g.fp16 ? __half2float(reinterpret_cast<const __half *>(g.f[c])[p]) * g.fs[c] : g.f[c][p];
   };
-  if (blk == 0) {
+  const int bp = probe_blocks(x, nt);
+  if (blk < bp) {
     if (!x.sample || o.np <= 0) return;
     __shared__ int first;
     if (t == 0) first = *o.count;
     __syncthreads();
     const int row = first + x.row;
     if (row < o.cap)
-      for (int q = t; q < o.np; q += nt) {
+      for (int q = blk * nt + t; q < o.np; q += bp * nt) {
         const ProbeDev &pr = o.pr[q];
         if (x.half == 2 || pr.comp / 3 == x.half)
           o.buf[(long long)row * o.np + q] = field(pr.comp, pr.p);
@@ -67,13 +77,13 @@ __device__ __forceinline__ void observe_block(const G &g, const P &x, int n, int
     return;
   }
   const int dn = o.dn ? *o.dn : 0;
-  const int bd = 1 + (int)((x.d1 - x.d0 + nt - 1) / nt);
+  const int bd = bp + (int)((x.d1 - x.d0 + nt - 1) / nt);
   if (blk >= bd) {
     const long long w = x.w0 + (long long)(blk - bd) * nt + t;
     if (w < x.w1 && n + 1 + dn < o.pw.ntime) pw_term_cell(o.pw, w, n + 1 + dn);
     return;
   }
-  const long long w = x.d0 + (long long)(blk - 1) * nt + t;
+  const long long w = x.d0 + (long long)(blk - bp) * nt + t;
   if (w >= x.d1) return;
   int q = 0;
   while (q + 1 < o.ndft && o.dft[q + 1].start <= w) ++q;
