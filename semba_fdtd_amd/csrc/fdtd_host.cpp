@@ -1725,7 +1725,8 @@ int build_dfts(fdtd_handle *h) {
     for (DftDev d : h->dfts)
       if (d.kind == kind) {
         d.start = start;
-        start += (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+        const long long n = (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq;
+        start += (n + kDftAlign - 1) / kDftAlign * kDftAlign;
         order.push_back(d);
       }
     h->dft_end[kind] = start;

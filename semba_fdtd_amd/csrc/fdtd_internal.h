@@ -246,12 +246,14 @@ struct PwTerms {
 // Frequency-domain observation box (observation.F90:3527-3600): complex(8)
 // running sums acc[pt][comp][freq] += aux[n][freq] * F_comp(pt), the points
 // being the stride multiples of the box (first[a] + t*stride[a], cnt[a] of them).
+constexpr int kDftAlign = 256;
 struct DftDev {
   int kind;                   // 0: Ex,Ey,Ez  1: Hx,Hy,Hz
   int first[3], stride[3], cnt[3];
   int nfreq;
   long long start;            // first (point, frequency) pair of the box in the
-                              // observation launch of its grid
+                              // observation launch of its grid, a multiple of
+                              // kDftAlign (so of any block's threads)
   const double2 *aux;         // [step][freq]
   double2 *acc;               // [pt][3][freq], pt = (kt*cnt1 + jt)*cnt0 + it
 };

@@ -83,12 +83,18 @@ __device__ __forceinline__ void observe_block(const G &g, const P &x, int n, int
     if (w < x.w1 && n + 1 + dn < o.pw.ntime) pw_term_cell(o.pw, w, n + 1 + dn);
     return;
   }
-  const long long w = x.d0 + (long long)(blk - bp) * nt + t;
-  if (w >= x.d1) return;
+  // A box starts at a multiple of every block's size: the block's threads share
+  // it, and its descriptor comes by scalar loads.  (Read by each lane it was most
+  // of the work: E and H boxes of 1.8 M pairs on 64^3 45.8 against 37.4 us a
+  // step, of 6.6 M on 96^3 216 against 157.)
+  const long long w = x.d0 + (long long)(blk - bp) * nt;
+  typedef __attribute__((address_space(4))) DftDev CDft;
+  const CDft *box = (const CDft *)o.dft;
   int q = 0;
-  while (q + 1 < o.ndft && o.dft[q + 1].start <= w) ++q;
-  const DftDev &d = o.dft[q];
-  const long long u = w - d.start;
+  while (q + 1 < o.ndft && box[q + 1].start <= w) ++q;
+  const CDft &d = box[q];
+  const long long u = w + t - d.start;
+  if (u >= (long long)d.cnt[0] * d.cnt[1] * d.cnt[2] * d.nfreq) return;
   const long long pt = u / d.nfreq;
   const int f = (int)(u - pt * d.nfreq);
   const int it = (int)(pt % d.cnt[0]);
