@@ -1343,43 +1343,23 @@ static bool face_in_poles(const fdtd_handle *h, int half) {
 void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTables *out, int *flags) {
   *out = SrcTables{};
   if (!h->inline_ok) return;
-  std::vector<int> word((size_t)l.p.nblk, 0);
   const bool faces = !h->pw_faces[half].empty();
   if (!faces && h->hcells[half].empty()) return;
   if (faces && (!h->pw_masks[half] || face_in_poles(h, half))) return;
   const QuadPlan &p = l.p;
+  const std::vector<unsigned> *m = h->pw_bits[half];
+  auto any = [](const std::vector<unsigned> &v, int a, int b) {
+    unsigned r = 0;
+    for (int i = a; i < std::min(b, (int)v.size()); ++i) r |= v[(size_t)i];
+    return r;
+  };
   SrcTables x;
   if (faces) x.src = h->pw_src[half];
-  if (x.src.nface) {
-    const std::vector<unsigned> *m = h->pw_bits[half];
-    auto any = [](const std::vector<unsigned> &v, int a, int b) {
-      unsigned r = 0;
-      for (int i = a; i < std::min(b, (int)v.size()); ++i) r |= v[(size_t)i];
-      return r;
-    };
-    const int run = kWave * l.rows;
-    int t = 0;
-    for (int q = 0; q < p.nbox; ++q) {
+  if (x.src.nface)
+    for (int q = l.slabs == kSlabAll ? 0 : l.slabs == kSlabMix ? 1 : p.nbox; q < p.nbox; ++q) {
       const QuadBox &o = p.box[q];
-      const bool slabs = l.slabs == kSlabAll || (l.slabs == kSlabMix && q > 0);
-      std::vector<unsigned> xy((size_t)o.tx);
-      for (int r = 0; r < o.tx; ++r) {
-        const int f0 = r * run, f1 = std::min(f0 + run, o.nq * o.nj) - 1;
-        const int j0 = f0 / o.nq, j1 = f1 / o.nq;
-        xy[(size_t)r] = any(m[1], o.j0 + j0, o.j0 + j1 + 1) &
-                        (j0 == j1 ? any(m[0], 4 * (f0 % o.nq), 4 * (f1 % o.nq) + 4)
-                                  : any(m[0], 0, h->g.nx + 1));
-      }
-      for (int k = o.k0; k < o.k0 + o.nk; k += l.kc) {
-        const unsigned z = any(m[2], k, std::min(k + l.kc, o.k0 + o.nk));
-        for (int r = 0; r < o.tx; ++r, ++t) {
-          if (!(xy[(size_t)r] & z)) continue;
-          if (slabs) return;
-          word[(size_t)t] |= kTileFaces[half];
-        }
-      }
+      if (any(m[1], o.j0, o.j0 + o.nj) & any(m[2], o.k0, o.k0 + o.nk)) return;
     }
-  }
   if (!h->hcells[half].empty()) {
     const bool ok = tile_cells(h, half, p.nblk, [&](int i, int j, int k) {
       for (int b = 0; b < p.nbox; ++b) {
@@ -1392,9 +1372,28 @@ void make_quad_src(const fdtd_handle *h, const QuadLayout &l, int half, SrcTable
     }, &x);
     if (!ok) return;
     for (int t = 0; t < p.nblk; ++t)
-      if (x.nstart[(size_t)t] < x.nstart[(size_t)t + 1]) word[(size_t)t] |= kTileNodal[half];
+      if (x.nstart[(size_t)t] < x.nstart[(size_t)t + 1]) flags[t] |= kTileNodal[half];
   }
-  for (int t = 0; t < p.nblk; ++t) flags[t] |= word[(size_t)t];
+  // (faces lie in the first box alone: the slabs were looked at above)
+  if (x.src.nface) {
+    const QuadBox &o = p.box[0];
+    const int run = kWave * l.rows;
+    std::vector<unsigned> xy((size_t)o.tx);
+    for (int r = 0; r < o.tx; ++r) {
+      const int f0 = r * run, f1 = std::min(f0 + run, o.nq * o.nj) - 1;
+      const int j0 = f0 / o.nq, j1 = f1 / o.nq;
+      xy[(size_t)r] = any(m[1], o.j0 + j0, o.j0 + j1 + 1) &
+                      (j0 == j1 ? any(m[0], 4 * (f0 % o.nq), 4 * (f1 % o.nq) + 4)
+                                : any(m[0], 0, h->g.nx + 1));
+    }
+    int *row = flags;
+    for (int k = o.k0; k < o.k0 + o.nk; k += l.kc, row += o.tx) {
+      const unsigned z = any(m[2], k, std::min(k + l.kc, o.k0 + o.nk));
+      if (!z) continue;
+      for (int r = 0; r < o.tx; ++r)
+        if (xy[(size_t)r] & z) row[r] |= kTileFaces[half];
+    }
+  }
   x.on = true;
   *out = std::move(x);
 }

@@ -123,15 +123,19 @@ __device__ __forceinline__ int tile_one_medium(const DevGrid &g, const QuadPos &
   if (threadIdx.x == 0 && threadIdx.y == 0) { lo = 0x7fffffff; hi = -0x7fffffff; }
   __syncthreads();
   int a = 0x7fffffff, b = -0x7fffffff;
+  const int n = g.nx + 1 - at.i0;   // cells inside the sweeps
   if (live)
     for (int k = at.k0; k < at.k1; ++k) {
       const long long q = (long long)(k + 1) * g.pxy + (long long)(at.j + 1) * g.px + g.xoff + at.i0;
-      for (int c = 0; c < 6; ++c)
-        for (int x = 0; x < 4 && at.i0 + x <= g.nx; ++x) {
-          const int m = g.mi[c][q + x];
-          a = min(a, m);
-          b = max(b, m);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        const u32x2 v = *reinterpret_cast<const u32x2 *>(g.mi[c] + q);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int m = (int)(((x < 2 ? v.x : v.y) >> (16 * (x & 1))) & 0xffffu);
+          if (x < n) { a = min(a, m); b = max(b, m); }
         }
+      }
     }
   atomicMin(&lo, a);
   atomicMax(&hi, b);
