@@ -368,9 +368,8 @@ int launch_tick_many(int *const *counters, int n, int by, void *stream) {
   return (int)hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) k_pw_terms(PwTerms t, int n, const int *dn) {
+__global__ void __launch_bounds__(256) k_pw_terms(PwTerms t, int n) {
   const long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (dn) n += *dn;
   if (w < t.total && n >= 0 && n < t.ntime) pw_term_cell(t, w, n);
 }
 
@@ -384,10 +383,10 @@ __global__ void __launch_bounds__(256) k_pw_terms_many(const PwTermsGrid *grids)
     pw_term_cell(g.t, w, n);
 }
 
-int launch_pw_terms(const PwTerms &t, int n, const int *dn, void *stream) {
+int launch_pw_terms(const PwTerms &t, int n, void *stream) {
   if (t.total <= 0) return 0;
   hipLaunchKernelGGL(k_pw_terms, dim3((unsigned)((t.total + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, t, n, dn);
+                     (hipStream_t)stream, t, n);
   return (int)hipGetLastError();
 }
 

@@ -6,7 +6,8 @@
 //   E face pass of all grids          one launch over a list of all grids'
 //                                     tiles (k_quad_batch), or a persistent
 //                                     one (k_pass_batch) where some grid
-//                                     cannot run four cells per lane
+//                                     cannot run four cells per lane or one
+//                                     was asked for
 //   pole stage                        one launch for the grids with poles
 //   plane-wave E faces                inside the pass, or one launch per (wave,
 //                                     face axis) group of the grids that cannot
@@ -195,7 +196,6 @@ TileMap batch_tiles(const fdtd_batch *b, const DevGrid &g) {
   tm.bdy = b->rows;
   const long long cols = (long long)(g.nx + 1) * (g.ny + 1);
   const long long per = (long long)kWave * b->rows;
-  tm.vec = 1;
   tm.flat = 1;
   tm.tx = (int)((cols + per - 1) / per);
   tm.ty = 1;

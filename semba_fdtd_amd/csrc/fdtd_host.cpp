@@ -213,7 +213,6 @@ static TileMap tile_map(const fdtd_handle *h, int rows, int zchunk) {
   tm.tz = (g.nz + 1 + tm.kc - 1) / tm.kc;
   tm.nblk = tm.tx * tm.ty * tm.tz;
   tm.remap = 1;
-  tm.vec = 1;
   return tm;
 }
 
@@ -713,7 +712,6 @@ int build_step(fdtd_handle *h) {
   StepDev sd{};
   TileMap &tm = sd.tm;
   tm.bdy = R;
-  tm.vec = 1;
   tm.kc = std::min(h->step_kc, h->g.nz + 1);
   tm.remap = 1;
   StepSrc src{};
@@ -954,14 +952,8 @@ int sync_b(fdtd_handle *h) {
   return FDTD_OK;
 }
 
-// one step of the pair, from sd[dir].gi to sd[dir].go, then the H-side
-// boundary, observation and step counter on the written copy
-// the step kernels of one direction: one launch per tile class
-// The class kernels of one step direction, one after another on the
-// handle's stream.  (They read the same state and write disjoint cells, but
-// running the small classes on side streams beside the interior one was
-// measured slower: they compete for the same bandwidth and caches.)
-// the descriptor of class launch q in direction dir
+// The class kernels of one step direction, one launch per tile class: the
+// descriptor of class launch q in direction dir, and its launch
 static StepDev class_sd(const fdtd_handle *h, int dir, size_t q) {
   StepDev sd = h->sd[dir];
   sd.tiles = h->dtiles + h->step_off[q];
@@ -1019,7 +1011,8 @@ static int make_branches(fdtd_handle *h) {
   return FDTD_OK;
 }
 
-// fork: into branches (while recording, after make_branches)
+// the class kernels of a step, from sd[dir].gi to sd[dir].go; fork: into
+// branches (while recording, after make_branches)
 static int launch_step_kernels(fdtd_handle *h, int dir, bool exact_prev, bool fork) {
   if (h->step_nf > 0 &&
       launch_pw_incident(h->dsfaces, h->step_nf0, h->step_nf, h->step_maxcells, h->dstepsrc,
@@ -1892,7 +1885,7 @@ int need_terms(fdtd_handle *h, int n) {
     return fail(h, FDTD_ERR_ARG, "step %d outside the time vector (0..%d)", n,
                 (int)h->tiempo.size() - 1);
   h->pw_terms_n = -1;
-  if (launch_pw_terms(h->pw_terms, n, nullptr, h->stream))
+  if (launch_pw_terms(h->pw_terms, n, h->stream))
     return fail(h, FDTD_ERR_HIP, "incident-field launch failed");
   h->pw_terms_n = n;
   return FDTD_OK;

@@ -89,9 +89,8 @@ struct TileMap {
   int nblk;
   int remap;
   int bdy;          // rows per block (block = 64 x bdy threads, <= 256)
-  int vec;          // x cells per lane of the fused passes as asked (1 or 4)
-  int flat;         // 1: tiles are runs of 64 * bdy columns of the x-y plane
-                    // (one cell per lane), tx per plane, ty = 1
+  int flat;         // 1: tiles are runs of 64 * bdy columns of the x-y plane, tx
+                    // per plane, ty = 1
 };
 
 // The boxes of one launch of the four-cell passes (fdtd_quad.h): vectors of
@@ -526,8 +525,8 @@ int launch_tick(int *dn, int by, void *stream);
 int launch_set_step(int *dn, int n, void *stream);
 // (a part of) the observation of a grid
 int launch_observe(const DevGrid &g, const ObservePart &p, void *stream);
-// the TF/SF terms of step n (or *dn + n)
-int launch_pw_terms(const PwTerms &t, int n, const int *dn, void *stream);
+// the TF/SF terms of step n
+int launch_pw_terms(const PwTerms &t, int n, void *stream);
 // the terms of many grids, each at its own *dn
 struct PwTermsGrid {
   PwTerms t;
