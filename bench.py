@@ -13,7 +13,7 @@ graph.  Prints one JSON line.
                     [--no-serve] [--serve-requests N] [--serve-rate R]
 
 Besides the 1024^3 line it measures the batched-instances workload (256
-uneven grids, one persistent launch per half step, against the plain
+uneven grids, one launch per half step, against the plain
 one-at-a-time path) and a serving stream (continuous batching against the
 plain path: p50/p99 latency and aggregate Mcell-updates/s), reported in the
 "batch" and "serve" objects of the same JSON line.
@@ -244,7 +244,7 @@ def batch_leg(count, steps, plain_sample, mode, storage="fp32"):
             "plain_mcell_updates_per_s": round(plain, 1),
             "plain_sample_instances": len(pick),
             "speedup": round(batched / plain, 2), "probes_finite": finite,
-            "note": "batched: one persistent face-pass launch per half step for all instances, "
+            "note": "batched: one face-pass launch per half step for all instances, "
                     "graph-replayed; plain: a seeded random sample (numpy default_rng(1004)) "
                     "of the same instances, each alone on its own graph; both timed after "
                     "set-up and 2 warm-up steps"}

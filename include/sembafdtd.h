@@ -268,8 +268,8 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps);
 /* Steps per replay of fdtd_run's captured two-pass step (1..64; default
  * 16): one graph records that many steps back to back and is replayed while
  * that many steps remain, the rest one step per replay.  Fewer replays cost
- * less launch time on small grids (64^3 cavity: 76.7 -> 72.2 us per step
- * from 1 to 16); the results do not depend on it.  No counterpart in the
+ * less launch time on small grids (64^3 cavity: 18.0, 10.9, 9.2, 8.9 us per
+ * step with 1, 4, 16, 64); the results do not depend on it.  No counterpart in the
  * reference. */
 int fdtd_set_graph_steps(fdtd_handle *h, int32_t steps);
 
@@ -380,8 +380,8 @@ float fdtd_evolucion(float t, float deltaevol, int32_t numus, const float *evol)
 
 /* ---- batches of independent grids ---------------------------------------
  * No counterpart in the reference (one solve per process there).  A batch
- * advances many grids, each set up as above, together: one persistent launch
- * per half step covers the face passes of every grid, the rest of the step
+ * advances many grids, each set up as above, together: one launch per
+ * half step covers the face passes of every grid, the rest of the step
  * is grouped across grids, and the step is replayed from a HIP graph.  Each
  * grid keeps its own step counter, so grids join (admit) and leave (retire)
  * between steps: continuous batching.  Results equal the grid advanced

@@ -3,7 +3,7 @@
 
 A grid is set up as a ``Solver`` and then admitted; from then on
 ``Batch.step`` advances every admitted grid, each from its own step, with one
-persistent face-pass launch per half step for the whole batch and the step
+face-pass launch per half step for the whole batch and the step
 replayed from a HIP graph.  Grids can be admitted and retired between steps
 (continuous batching).  A grid's results are the same as when it is advanced
 alone.
