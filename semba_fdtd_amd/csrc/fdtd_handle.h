@@ -43,6 +43,17 @@ struct PwGroup {
   long long *dstart = nullptr;
 };
 
+// Has a device table been built: by launches that ran, or by launches that a
+// caller is recording, for the other calls of that recording alone (rec: the
+// recording's id plus one, 0: none).
+struct BuiltIn {
+  bool now = false;
+  unsigned long long rec = 0;
+  bool ok(unsigned long long id) const { return now || (id && id == rec); }
+  void set(unsigned long long id) { if (id) rec = id; else now = true; }
+  void drop() { now = false; rec = 0; }
+};
+
 // a media table past this many entries is shared by four rows of the four-cell
 // passes (quad_default)
 constexpr int kManyMedia = 256;
@@ -210,14 +221,14 @@ struct fdtd_handle {
   std::vector<int> step_cls, step_cnt, step_off;
   std::vector<int> step_crows;           // rows per block of each class launch
   std::vector<int> step_uni;             // leading single-medium tiles of each class launch
-  // the words of the tiles of the one-cell pass map tm (valid while tmed_ready;
-  // tiling and media changes clear it), tmed_cap of them, then their flags
+  // the words of the tiles of the one-cell pass map tm (while tmed_on; tiling and
+  // media changes drop it), tmed_cap of them, then their flags
   int *tmed = nullptr;
   int tmed_cap = 0;
-  bool tmed_ready = false;
-  bool gmed_ready = false;     // tmed holds the granular calls' (tm_default) instead
-  // the four-cell passes' tiles and their words and flags (valid while
-  // tmed_ready and the grid runs these passes)
+  sfd_host::BuiltIn tmed_on;
+  sfd_host::BuiltIn gmed_on;   // tmed holds the granular calls' (tm_default) instead
+  // the four-cell passes' tiles and their words and flags (while tmed_on and the
+  // grid runs these passes)
   sfd_host::QuadLayout quad;
   int *qmed = nullptr;
   int qmed_cap = 0;

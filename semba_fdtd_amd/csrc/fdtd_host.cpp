@@ -321,8 +321,16 @@ void invalidate_graph(fdtd_handle *h) {
   h->pgraph = nullptr;
   h->graph_ok = false;
   h->step_ready = false;
-  h->tmed_ready = false;
-  h->gmed_ready = false;
+  h->tmed_on.drop();
+  h->gmed_on.drop();
+}
+
+// the recording that a caller is making of the grid's stream (0: none)
+static unsigned long long recording(const fdtd_handle *h) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  return hipStreamGetCaptureInfo(h->stream, &st, &id) == hipSuccess && st == hipStreamCaptureStatusActive
+             ? id + 1 : 0;
 }
 
 // a device array of at least n words and n flags behind them
@@ -345,7 +353,9 @@ static int tile_words(fdtd_handle *h, int **words, int *cap, int n) {
 // pole-state boxes (src_gen); where only the media or the recorded graphs
 // changed the launch is all, and a caller may be recording it.
 int build_tile_media(fdtd_handle *h) {
-  if (h->tmed_ready) return FDTD_OK;
+  if (h->tmed_on.now) return FDTD_OK;
+  const unsigned long long rec = recording(h);
+  if (h->tmed_on.ok(rec)) return FDTD_OK;
   const bool quads = use_quads(h);
   int **words = quads ? &h->qmed : &h->tmed, *cap = quads ? &h->qmed_cap : &h->tmed_cap;
   int rc;
@@ -389,7 +399,7 @@ int build_tile_media(fdtd_handle *h) {
     e = exact ? exact::launch_pass_tile_media(h->g, h->tm, flags, out, h->stream)
               : fast::launch_pass_tile_media(h->g, h->tm, flags, out, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
-  h->tmed_ready = true;
+  h->tmed_on.set(rec);
   return FDTD_OK;
 }
 
@@ -398,13 +408,16 @@ int build_tile_media(fdtd_handle *h) {
 // calls of a step: 1583 us reading every index, 1457 skipping those of
 // single-medium tiles.
 int build_granular_media(fdtd_handle *h) {
-  if (h->gmed_ready || !use_quads(h)) return FDTD_OK;
+  if (h->gmed_on.now || !use_quads(h)) return FDTD_OK;
+  const unsigned long long rec = recording(h);
+  // (without words the passes read every index: a recording cannot allocate)
+  if (h->gmed_on.ok(rec) || (rec && h->tm_default.nblk > h->tmed_cap)) return FDTD_OK;
   if (int rc = tile_words(h, &h->tmed, &h->tmed_cap, h->tm_default.nblk)) return rc;
   const int e = h->mode == FDTD_MODE_EXACT
                     ? exact::launch_pass_tile_media(h->g, h->tm_default, nullptr, h->tmed, h->stream)
                     : fast::launch_pass_tile_media(h->g, h->tm_default, nullptr, h->tmed, h->stream);
   if (e) return fail(h, FDTD_ERR_HIP, "tile media launch failed: %s", hipGetErrorString((hipError_t)e));
-  h->gmed_ready = true;
+  h->gmed_on.set(rec);
   return FDTD_OK;
 }
 
@@ -1766,7 +1779,8 @@ int run_e(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
-  const int *tmed = (quads ? h->gmed_ready : h->tmed_ready) ? h->tmed : nullptr;
+  const BuiltIn &words = quads ? h->gmed_on : h->tmed_on;
+  const int *tmed = words.now || words.ok(recording(h)) ? h->tmed : nullptr;
   const TileMap &tm = quads ? h->tm_default : h->tm;
   int e = h->mode == FDTD_MODE_EXACT ? exact::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream)
                                      : fast::launch_e(h->g, tm, tmed, yee, c, a, src, h->stream);
@@ -1786,7 +1800,8 @@ int run_h(fdtd_handle *h, int yee, int cpml, int ade, const PassSrc *src = nullp
     if (!a) return FDTD_OK;
     yee = c = 0;
   }
-  const int *tmed = (quads ? h->gmed_ready : h->tmed_ready) ? h->tmed : nullptr;
+  const BuiltIn &words = quads ? h->gmed_on : h->tmed_on;
+  const int *tmed = words.now || words.ok(recording(h)) ? h->tmed : nullptr;
   const TileMap &tm = quads ? h->tm_default : h->tm;
   int e = h->mode == FDTD_MODE_EXACT ? exact::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream)
                                      : fast::launch_h(h->g, tm, tmed, yee, c, a, src, h->stream);
@@ -1858,12 +1873,6 @@ int run_nodal(fdtd_handle *h, int half, int n, const int *dn) {
   return FDTD_OK;
 }
 
-// is a caller recording the grid's stream
-bool stream_capturing(const fdtd_handle *h) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(h->stream, &st) == hipSuccess && st == hipStreamCaptureStatusActive;
-}
-
 // do the passes of the grid's own steps read the TF/SF terms
 bool inline_faces(const fdtd_handle *h) {
   return ((h->psrc_on[0] && h->psrc[0].nface) || (h->psrc_on[1] && h->psrc[1].nface));
@@ -1873,7 +1882,7 @@ bool inline_faces(const fdtd_handle *h) {
 // these calls: it records the launch, and from then on any replay may have
 // written the buffer, so every call writes the terms it needs.
 bool have_terms(fdtd_handle *h, int n) {
-  h->pw_recorded = h->pw_recorded || stream_capturing(h);
+  h->pw_recorded = h->pw_recorded || recording(h);
   return !h->pw_recorded && h->pw_terms_n == n;
 }
 
@@ -2393,7 +2402,7 @@ int fdtd_update_observation(fdtd_handle *h, int32_t n) {
   // a step outside the time vector still samples the probes
   const bool in = n >= 0 && n < (int)h->tiempo.size();
   // the terms of the next step ride along when the steps run call by call
-  const bool pw = in && h->tmed_ready && inline_faces(h) && n + 1 < (int)h->tiempo.size() &&
+  const bool pw = in && h->tmed_on.now && inline_faces(h) && n + 1 < (int)h->tiempo.size() &&
                   have_terms(h, n);
   if ((rc = run_observe(h, h->g, observe_part(h, 2, n, nullptr, true, in, pw)))) return rc;
   if (pw) h->pw_terms_n = n + 1;

@@ -205,3 +205,61 @@ def test_recording_outlives_what_drops_the_graphs(rec, tiling):
             step(s, n)
         assert same(fields(s), want)
     s.close()
+
+
+@pytest.mark.parametrize("tiling", [None, (2, 4, 1)])
+def test_direct_steps_after_a_recording_not_replayed(rec, tiling):
+    """What a recording would renew has not been renewed until it is replayed:
+    media written, steps recorded, and direct steps instead."""
+    pb = wave_problem()
+    s, ref = sf.Solver(pb, stream=rec.stream), sf.Solver(pb)
+    if tiling:
+        s.set_tiling(*tiling)
+    for q in (s, ref):
+        for n in range(12):
+            step(q, n)
+        assert q.lib.fdtd_media_paint_box(q.h, 8, 30, 6, 22, 8, 20, 2, 3, ptr(PRIO, i32p)) == 0
+    two = rec.record(lambda: [step(s, n) for n in (12, 13)])
+    for n in range(12, 16):
+        step(s, n)
+    for n in range(12, 16):
+        step(ref, n)
+    want = fields(ref)
+    assert np.abs(want[0]).max() > 0 and same(fields(s), want)
+    start = s.save_state()
+    for k in range(2):                               # and the recording itself
+        s.load_state(start)
+        rec.replay(two)
+        if k == 0:
+            again = fields(s)
+    assert same(fields(s), again)
+    s.close()
+
+
+def test_granular_calls_recorded_first(rec):
+    """The granular calls first made inside a recording, on a grid whose steps
+    so far were fused ones; recorded after a media change; and directly."""
+    pb = wave_problem(nodal=True)
+    names = ("advance_e_yee", "advance_e_cpml", "advance_planewave_e", "advance_nodal_e",
+             "advance_h_yee", "advance_h_cpml", "advance_planewave_h", "advance_nodal_h")
+
+    def granular(s, n):
+        for name in names:
+            f = getattr(s.lib, "fdtd_" + name)
+            assert (f(s.h, n) if "planewave" in name or "nodal" in name else f(s.h)) == 0, name
+
+    s, ref = sf.Solver(pb, stream=rec.stream), sf.Solver(pb)
+    for q in (s, ref):
+        for n in range(12):
+            step(q, n)
+    two = rec.record(lambda: [granular(s, n) for n in (12, 13)])
+    rec.replay(two)
+    for n in range(14, 17):
+        granular(s, n)
+    pb2 = rec.record(lambda: granular(s, 17))
+    rec.replay(pb2)
+    for n in range(12, 18):
+        step(ref, n)
+    want = fields(ref)
+    assert np.abs(want[0]).max() > 0 and same(fields(s), want)
+    s.close()
