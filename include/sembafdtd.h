@@ -183,7 +183,8 @@ int fdtd_time_halves(fdtd_handle *h, int32_t reps, float ms[3]);
  * second copy held for the purpose (fields, CPML psi and pole state: twice
  * the state's memory).  fdtd_run advances pairs of steps so that the state is
  * back in its usual place when it returns; an odd last step runs the two
- * passes.  The results equal the two-pass step bit for bit.  fp32 storage
+ * passes, and every step does where a TF/SF box reaches the grid's edge (its
+ * faces then act on cells outside the sweeps).  The results equal the two-pass step bit for bit.  fp32 storage
  * only.  No counterpart in the reference. */
 int fdtd_set_step_mode(fdtd_handle *h, int32_t rows, int32_t zchunk);
 int fdtd_get_step_mode(const fdtd_handle *h, int32_t *rows, int32_t *zchunk);

@@ -792,7 +792,10 @@ int fdtd_batch_step(fdtd_batch *b, int32_t nsteps) {
   int rc = build_descriptors(b);
   if (rc) return rc;
   // one launch per step: pairs A -> B -> A, an odd last step on the two passes
-  const int pairs = b->step_rows > 0 ? nsteps / 2 : 0;
+  // (as every step where a grid's TF/SF box reaches its edge)
+  bool edge = false;
+  for (fdtd_handle *h : b->slots) edge = edge || (h && h->pw_edge);
+  const int pairs = b->step_rows > 0 && !edge ? nsteps / 2 : 0;
   const int singles = nsteps - 2 * pairs;
   if (pairs > 0) {
     if ((rc = build_step_descriptors(b))) return rc;

@@ -151,6 +151,9 @@ struct fdtd_handle {
   float *dphys = nullptr;
   int pstride = 0;
   double *dtiempo = nullptr;
+  // some face has cells outside its component's sweep (a box on the grid's edge):
+  // the two passes' own launches reach them, the one-launch step does not
+  bool pw_edge = false;
   // the faces of each half as the face passes apply them inline (pw_masks:
   // at most kPassFaces, all inside their components' sweeps), and the buffer
   // of both halves' terms, which holds those of step pw_terms_n (-1: none) until

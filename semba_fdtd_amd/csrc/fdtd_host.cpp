@@ -1225,7 +1225,10 @@ static void build_pw_masks(fdtd_handle *h, const std::vector<PwWave> &waves, PwM
       if (cells) {
         // the passes run the components' sweeps: a face outside (a box on
         // the grid's edge) keeps its own launch
-        for (int a = 0; a < 3; ++a) ok = ok && lo[a] >= 0 && hi[a] <= sweep_last(h, f.comp, a);
+        bool in = true;
+        for (int a = 0; a < 3; ++a) in = in && lo[a] >= 0 && hi[a] <= sweep_last(h, f.comp, a);
+        h->pw_edge = h->pw_edge || !in;
+        ok = ok && in;
         ok = ok && w.start.back() + cells < 0x40000000LL;
         if (ok) {
           for (int a = 0; a < 3; ++a)
@@ -1494,6 +1497,7 @@ int build_planewaves(fdtd_handle *h) {
   h->pw_faces[0].clear();
   h->pw_faces[1].clear();
   h->pw_masks[0] = h->pw_masks[1] = false;
+  h->pw_edge = false;
   h->pw_terms = PwTerms{};
   h->pw_terms_n = -1;
   h->dwaves = nullptr; h->dphys = nullptr; h->dtiempo = nullptr;
@@ -2520,7 +2524,7 @@ int fdtd_run(fdtd_handle *h, int32_t n0, int32_t nsteps) {
   if (launch_set_step(h->dstep, n0, h->stream)) return fail(h, FDTD_ERR_HIP, "step launch failed");
   // one-launch steps go in pairs (A -> B -> A); an odd last step, and every
   // step when they are off, replays the two-pass step
-  const bool paired = h->step_rows > 0 && nsteps >= 2;
+  const bool paired = h->step_rows > 0 && nsteps >= 2 && !h->pw_edge;
   const int pairs = paired ? nsteps / 2 : 0;
   const int singles = paired ? nsteps % 2 : nsteps;
   if (pairs > 0 && !h->pexec) {
