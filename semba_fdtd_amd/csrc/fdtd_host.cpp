@@ -547,6 +547,7 @@ int build_ade(fdtd_handle *h) {
     if (rc) return rc;
   }
   if (h->g.ade[0].has || h->g.ade[1].has) ++h->src_gen;
+  h->prev_exact = true;   // (the stored previous fields start at zero again)
   h->ade_ready = true;
   return FDTD_OK;
 }
